@@ -52,6 +52,13 @@ int64_t near_grid(size_t lds) {
   return (int64_t)per_cu * num_cus();
 }
 
+// LDS of the far-field kernel: r2 slots, moment tables, a tile's rows, core terms
+template <int CORE, bool GRAD>
+constexpr size_t ff_far_lds() {
+  return (size_t)256 * FF_SL * sizeof(__bf16) + (size_t)2 * ff_rows<ff_form<CORE, GRAD>()>() * FF_TP * sizeof(_Float16) +
+         512 * sizeof(float4) + (CORE == CORE_WL || CORE == CORE_V2 ? 256 * sizeof(float) : 0);
+}
+
 // RAII pair of events for the optional stage timing
 struct Ev {
   hipEvent_t e = nullptr;
@@ -79,6 +86,18 @@ struct Layout {
   size_t bytes;
 };
 
+// Near-field items per block: about 4,096 in all, three rounds of the workgroups that the
+// GPU holds (an item of FF_M0 tiles is 262,144 pairs), and at least 2 per block
+int near_split(int64_t nb) { return (int)std::max<int64_t>(2, std::min<int64_t>(16, 4096 / nb)); }
+
+// Slices of the far field: blocks x slices workgroups, at least about four rounds of the
+// two that a CU holds, so that the last round is short beside the whole and few blocks
+// (a collection of 65,536: 256) still fill every slot.
+int far_slices(int64_t nb, int64_t mwords) {
+  const int64_t want = (8 * (int64_t)num_cus() + nb - 1) / nb;
+  return (int)std::max<int64_t>(1, std::min<int64_t>({want, mwords, 8}));
+}
+
 Layout layout(char* base, int64_t ns, int64_t nt, bool same, int T, size_t tmp_bytes) {
   const int64_t nb = (nt + FF_TB - 1) / FF_TB;
   const int64_t ntiles = (ns + T - 1) / T;
@@ -95,8 +114,8 @@ Layout layout(char* base, int64_t ns, int64_t nt, bool same, int T, size_t tmp_b
   L.it_in = same ? nullptr : cv.take<int>(nt);
   L.it_out = same ? nullptr : cv.take<int>(nt);
   L.tmp = cv.take<char>(tmp_bytes);
-  L.sp = cv.take<float4>(ns);
-  L.sa = cv.take<float4>(ns);
+  L.sp = cv.take<float4>((size_t)ntiles * T);
+  L.sa = cv.take<float4>((size_t)ntiles * T);
   L.tq = cv.take<float4>(nt);
   L.tsph = cv.take<float4>(ntiles);
   L.tcs = cv.take<float>(ntiles);
@@ -104,7 +123,7 @@ Layout layout(char* base, int64_t ns, int64_t nt, bool same, int T, size_t tmp_b
   L.bsph = cv.take<float4>(nb);
   L.bcs = cv.take<float>(nb);
   L.mask = cv.take<unsigned>((size_t)(nb * mwords));
-  L.farv = cv.take<double>((size_t)12 * nt);
+  L.farv = cv.take<double>((size_t)12 * far_slices(nb, mwords) * nt);
   L.npair = cv.take<unsigned long long>(1);
   L.nn = cv.take<int>(nb);
   L.noff = cv.take<int>(nb);
@@ -112,7 +131,7 @@ Layout layout(char* base, int64_t ns, int64_t nt, bool same, int T, size_t tmp_b
   L.ioff = cv.take<int>(nb);
   L.mfold = cv.take<int>(1);
   L.ctr = cv.take<unsigned>(1);
-  L.part = cv.take<double>((size_t)3 * nb * 12 * FF_TB);   // at most 3 items per block
+  L.part = cv.take<double>((size_t)(near_split(nb) + 1) * nb * 12 * FF_TB);
   L.bytes = cv.off;
   return L;
 }
@@ -174,7 +193,9 @@ int run(const o3d_points* src, o3d_points* targ, bool self_excl, int T, hipStrea
       return rc;
     tperm = tp;
   }
-  hipLaunchKernelGGL((k_ff_gather_src<CORE>), dim3(grid_of(ns, 256)), dim3(256), 0, st, sv, sperm, ns, L.sp, L.sa);
+  const int64_t npad = (int64_t)ntiles * T;
+  hipLaunchKernelGGL((k_ff_gather_src<CORE>), dim3(grid_of(npad, 256)), dim3(256), 0, st, sv, sperm, ns, npad, L.sp, L.sa,
+                     L.bb + 6);
   hipLaunchKernelGGL((k_ff_gather_tgt<CORE, THICK>), dim3(grid_of(nt, 256)), dim3(256), 0, st, tv, tperm, nt, L.tq);
   hipLaunchKernelGGL(k_ff_bounds, dim3((unsigned)ntiles), dim3(256), 0, st, L.sp, L.sa, ns, T, L.tsph, L.tcs, L.tam);
   hipLaunchKernelGGL(k_ff_bounds, dim3((unsigned)nb), dim3(256), 0, st, L.tq, (const float4*)nullptr, nt, FF_TB, L.bsph,
@@ -184,7 +205,8 @@ int run(const o3d_points* src, o3d_points* targ, bool self_excl, int T, hipStrea
   hipLaunchKernelGGL(k_ff_plan_count, dim3(grid_of(nb, 256)), dim3(256), 0, st, L.mask, nb, mwords, ntiles, L.nn);
   HIPCHK(hipGetLastError());
   if ((rc = exclusive_scan_i32(L.nn, L.noff, nb, st)) != O3D_OK) return rc;
-  hipLaunchKernelGGL(k_ff_plan_items, dim3(grid_of(nb, 256)), dim3(256), 0, st, L.nn, L.noff, nb, L.items, L.mfold);
+  hipLaunchKernelGGL(k_ff_plan_items, dim3(grid_of(nb, 256)), dim3(256), 0, st, L.nn, L.noff, nb, near_split(nb), L.items,
+                     L.mfold);
   HIPCHK(hipGetLastError());
   if ((rc = exclusive_scan_i32(L.items, L.ioff, nb, st)) != O3D_OK) return rc;
   hipLaunchKernelGGL(k_ff_zero_u32, dim3(1), dim3(64), 0, st, L.ctr);
@@ -193,19 +215,22 @@ int run(const o3d_points* src, o3d_points* targ, bool self_excl, int T, hipStrea
   FFArgs a{};
   a.sp = L.sp; a.sa = L.sa; a.tq = L.tq; a.tperm = tperm;
   a.tsph = L.tsph; a.tcs = L.tcs; a.tam = L.tam; a.bsph = L.bsph; a.bcs = L.bcs;
-  a.mask = L.mask; a.farv = L.farv;
+  a.mask = L.mask; a.farv = L.farv; a.sign = L.bb + 6;
   a.nn = L.nn; a.items = L.items; a.ioff = L.ioff; a.mfold = L.mfold; a.ctr = L.ctr; a.part = L.part;
   a.s = sv; a.t = tv;
   a.ns = ns; a.nt = nt;
   a.tile = T; a.mwords = mwords; a.ntiles = ntiles;
   a.self_excl = self_excl ? 1 : 0;
-  const size_t lds_far = (size_t)256 * FF_SL * sizeof(__bf16) + (size_t)2 * 32 * FF_TP * sizeof(_Float16);
+  const int nslice = far_slices(nb, mwords);
+  a.wslice = (mwords + nslice - 1) / nslice;
+  a.nslice = (mwords + a.wslice - 1) / a.wslice;
+  const size_t lds_far = ff_far_lds<CORE, true>();
   if (prof) HIPCHK(hipEventRecord(ev[1].e, st));
-  hipLaunchKernelGGL((k_ff_far<CORE, THICK, PREC>), dim3((unsigned)nb), dim3(FF_FAR_THREADS), lds_far, st, a);
+  hipLaunchKernelGGL((k_ff_far<CORE, true>), dim3((unsigned)nb, (unsigned)a.nslice), dim3(FF_FAR_THREADS), lds_far, st, a);
   HIPCHK(hipGetLastError());
   if (prof) HIPCHK(hipEventRecord(ev[2].e, st));
   const size_t lds_near = (size_t)T * 2 * sizeof(float4);
-  const unsigned gnear = (unsigned)std::min<int64_t>(3 * nb, near_grid<CORE, PREC>(lds_near));
+  const unsigned gnear = (unsigned)std::min<int64_t>((near_split(nb) + 1) * nb, near_grid<CORE, PREC>(lds_near));
   hipLaunchKernelGGL((k_ff_near<CORE, PREC>), dim3(gnear), dim3(FF_TB), lds_near, st, a);
   HIPCHK(hipGetLastError());
   hipLaunchKernelGGL((k_ff_combine<CORE, PREC>), dim3((unsigned)nb), dim3(FF_TB), 0, st, a);
@@ -297,7 +322,8 @@ int sorted_sources(const o3d_points* src, const int32_t* perm, int tile, void* w
   float4* sph = (float4*)(p + 2 * r(sizeof(float4) * (size_t)n));
   float* cs = (float*)(p + 2 * r(sizeof(float4) * (size_t)n) + r(sizeof(float4) * (size_t)ntiles));
   const SrcView sv{src->x[0], src->x[1], src->x[2], src->r, src->s[0], src->s[1], src->s[2]};
-  hipLaunchKernelGGL((k_ff_gather_src<CORE_EXP>), dim3(grid_of(n, 256)), dim3(256), 0, st, sv, perm, n, sp, sa);
+  hipLaunchKernelGGL((k_ff_gather_src<CORE_EXP>), dim3(grid_of(n, 256)), dim3(256), 0, st, sv, perm, n, n, sp, sa,
+                     (unsigned*)nullptr);
   hipLaunchKernelGGL(k_ff_bounds, dim3((unsigned)ntiles), dim3(256), 0, st, (const float4*)sp, (const float4*)nullptr,
                      n, tile, sph, cs, (float*)nullptr);
   HIPCHK(hipGetLastError());

@@ -201,3 +201,21 @@ def test_factored_random_clouds(infl, core, kind, n):
     print(f"plain: factored vel {efv} grad {efg}; direct vel {edv} grad {edg}", flush=True)
     assert efv[0] <= 2 * edv[0] + 1e-6 and efg[0] <= 2 * edg[0] + 1e-6
     assert not np.array_equal(g, infl.p2p(core, pos, st, rad, pos, rad, True, "comp", method="direct")[1])
+
+
+@pytest.mark.parametrize("core", ["rm", "exp"])
+@pytest.mark.parametrize("n", [2049, 30011])
+def test_factored_negation_and_zero_strengths(infl, core, n):
+    """Negating every strength negates every result exactly (the far field takes all
+    strengths times the sign of the first nonzero one), and whole tiles of particles with
+    no strength, in sorted order, add nothing: compensated within 2e-6 of the oracle."""
+    p = scenes.colliding_rings(n_each=(n + 1) // 2, sigma=0.03, seed=n)
+    st = p.str * (p.pos[2] > -1.02)      # the lower part of one ring: no strength
+    print(f"case: {core} N={p.n}", flush=True)
+    call = lambda s: infl.p2p(core, p.pos, s, p.rad, p.pos, p.rad, True, "comp", method="factored")
+    v, g = call(st)
+    vn, gn = call(-st)
+    assert np.array_equal(vn, -v) and np.array_equal(gn, -g)
+    sel = _sel(p.n, 512)
+    ov, og = oracle.p2p(core, p.pos, st, p.rad, p.pos[:, sel], p.rad[sel], True, "f64")
+    assert rel_errors(v[:, sel], ov)[0] <= 2e-6 and rel_errors(g[:, sel], og)[0] <= 2e-6
