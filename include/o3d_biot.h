@@ -65,7 +65,9 @@ enum o3d_self { O3D_SELF_INCLUDE = 0, O3D_SELF_EXCLUDE = 1 };
  *             cores; other pairs as in DIRECT.  RM and EXP cores, velocity and
  *             gradient, FP32 or compensated precision; tile 64, 128 or 256.
  *   AUTO:     FACTORED where it applies and both counts are >= 65536 with tile
- *             and tpt left at 0, DIRECT otherwise.
+ *             and tpt left at 0, DIRECT otherwise.  In compensated precision AUTO
+ *             takes the far tiles of the other cores (WL, V2) and of velocities
+ *             alone to the matrix cores as well, at the same counts.
  * For panel sources (o3d_panels_affect_points[_dev]) the field selects the rule:
  *   AUTO / DIRECT:      the reference's recursive centroid rule (Kernels.h:1028-1211);
  *   O3D_PANEL_GAUSS7:   no counterpart in the reference -- per (target, panel) pair a

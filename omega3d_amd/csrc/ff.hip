@@ -43,10 +43,10 @@ struct Carve {
 unsigned grid_of(int64_t n, int per) { return (unsigned)std::max<int64_t>(1, (n + per - 1) / per); }
 
 // workgroups of the persistent near-field kernel: every slot of every CU
-template <int CORE, int PREC>
+template <int CORE, bool GRAD, int PREC>
 int64_t near_grid(size_t lds) {
   int per_cu = 0;
-  if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, k_ff_near<CORE, PREC>, FF_TB, lds) != hipSuccess ||
+  if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, k_ff_near<CORE, GRAD, PREC>, FF_TB, lds) != hipSuccess ||
       per_cu < 1)
     per_cu = 1;
   return (int64_t)per_cu * num_cus();
@@ -80,7 +80,7 @@ struct Layout {
   int *is_in, *is_out, *it_in, *it_out, *nn, *noff, *items, *ioff, *mfold;
   void* tmp;
   float4 *sp, *sa, *tq, *tsph, *bsph;
-  float *tcs, *tam, *bcs;
+  float *tcs, *tam, *tsg, *bcs;
   double *farv, *part;
   unsigned long long* npair;
   size_t bytes;
@@ -98,7 +98,7 @@ int far_slices(int64_t nb, int64_t mwords) {
   return (int)std::max<int64_t>(1, std::min<int64_t>({want, mwords, 8}));
 }
 
-Layout layout(char* base, int64_t ns, int64_t nt, bool same, int T, size_t tmp_bytes) {
+Layout layout(char* base, int64_t ns, int64_t nt, bool same, int T, size_t tmp_bytes, int nout) {
   const int64_t nb = (nt + FF_TB - 1) / FF_TB;
   const int64_t ntiles = (ns + T - 1) / T;
   const int64_t mwords = (ntiles + 31) / 32;
@@ -120,10 +120,11 @@ Layout layout(char* base, int64_t ns, int64_t nt, bool same, int T, size_t tmp_b
   L.tsph = cv.take<float4>(ntiles);
   L.tcs = cv.take<float>(ntiles);
   L.tam = cv.take<float>(ntiles);
+  L.tsg = cv.take<float>(ntiles);
   L.bsph = cv.take<float4>(nb);
   L.bcs = cv.take<float>(nb);
   L.mask = cv.take<unsigned>((size_t)(nb * mwords));
-  L.farv = cv.take<double>((size_t)12 * far_slices(nb, mwords) * nt);
+  L.farv = cv.take<double>((size_t)nout * far_slices(nb, mwords) * nt);
   L.npair = cv.take<unsigned long long>(1);
   L.nn = cv.take<int>(nb);
   L.noff = cv.take<int>(nb);
@@ -131,14 +132,14 @@ Layout layout(char* base, int64_t ns, int64_t nt, bool same, int T, size_t tmp_b
   L.ioff = cv.take<int>(nb);
   L.mfold = cv.take<int>(1);
   L.ctr = cv.take<unsigned>(1);
-  L.part = cv.take<double>((size_t)(near_split(nb) + 1) * nb * 12 * FF_TB);
+  L.part = cv.take<double>((size_t)(near_split(nb) + 1) * nb * nout * FF_TB);
   L.bytes = cv.off;
   return L;
 }
 
 // ws == nullptr: the stream's own workspace (caller holds g_ws_mu); otherwise the
 // caller's, of ws_bytes
-template <int CORE, bool THICK, int PREC>
+template <int CORE, bool THICK, bool GRAD, int PREC>
 int run(const o3d_points* src, o3d_points* targ, bool self_excl, int T, hipStream_t st, o3d_factored_profile* prof,
         void* ws, size_t ws_bytes) {
   const int64_t ns = src->n, nt = targ->n;
@@ -149,7 +150,7 @@ int run(const o3d_points* src, o3d_points* targ, bool self_excl, int T, hipStrea
 
   const size_t tmp_bytes = lib_tmp_bytes(ns, nt, same);
 
-  Layout L = layout(nullptr, ns, nt, same, T, tmp_bytes);
+  Layout L = layout(nullptr, ns, nt, same, T, tmp_bytes, GRAD ? 12 : 3);
   char* base = static_cast<char*>(ws);
   if (ws) {
     if (ws_bytes < L.bytes) return fail(O3D_EINVAL, "factored path: workspace of %zu bytes, %zu needed", ws_bytes, L.bytes);
@@ -159,13 +160,13 @@ int run(const o3d_points* src, o3d_points* targ, bool self_excl, int T, hipStrea
     if (rc != O3D_OK) return rc;
     base = static_cast<char*>(p);
   }
-  L = layout(base, ns, nt, same, T, tmp_bytes);
+  L = layout(base, ns, nt, same, T, tmp_bytes, GRAD ? 12 : 3);
 
   SrcView sv{src->x[0], src->x[1], src->x[2], src->r, src->s[0], src->s[1], src->s[2]};
   TgtView tv{};
   tv.x = targ->x[0]; tv.y = targ->x[1]; tv.z = targ->x[2]; tv.r = targ->r;
   tv.u = targ->u[0]; tv.v = targ->u[1]; tv.w = targ->u[2];
-  for (int k = 0; k < 9; ++k) tv.g[k] = targ->ug[k];
+  for (int k = 0; k < 9; ++k) tv.g[k] = GRAD ? targ->ug[k] : nullptr;
 
   Ev ev[4];
   if (prof) {
@@ -194,12 +195,12 @@ int run(const o3d_points* src, o3d_points* targ, bool self_excl, int T, hipStrea
     tperm = tp;
   }
   const int64_t npad = (int64_t)ntiles * T;
-  hipLaunchKernelGGL((k_ff_gather_src<CORE>), dim3(grid_of(npad, 256)), dim3(256), 0, st, sv, sperm, ns, npad, L.sp, L.sa,
-                     L.bb + 6);
+  hipLaunchKernelGGL((k_ff_gather_src<CORE>), dim3(grid_of(npad, 256)), dim3(256), 0, st, sv, sperm, ns, npad, L.sp, L.sa);
   hipLaunchKernelGGL((k_ff_gather_tgt<CORE, THICK>), dim3(grid_of(nt, 256)), dim3(256), 0, st, tv, tperm, nt, L.tq);
-  hipLaunchKernelGGL(k_ff_bounds, dim3((unsigned)ntiles), dim3(256), 0, st, L.sp, L.sa, ns, T, L.tsph, L.tcs, L.tam);
+  hipLaunchKernelGGL(k_ff_bounds, dim3((unsigned)ntiles), dim3(256), 0, st, L.sp, L.sa, ns, T, L.tsph, L.tcs, L.tam,
+                     L.tsg);
   hipLaunchKernelGGL(k_ff_bounds, dim3((unsigned)nb), dim3(256), 0, st, L.tq, (const float4*)nullptr, nt, FF_TB, L.bsph,
-                     L.bcs, (float*)nullptr);
+                     L.bcs, (float*)nullptr, (float*)nullptr);
   hipLaunchKernelGGL((k_ff_classify<CORE>), dim3(grid_of(nb * mwords, 256)), dim3(256), 0, st, L.bsph, L.bcs, nb, L.tsph,
                      L.tcs, ntiles, mwords, L.mask);
   hipLaunchKernelGGL(k_ff_plan_count, dim3(grid_of(nb, 256)), dim3(256), 0, st, L.mask, nb, mwords, ntiles, L.nn);
@@ -215,7 +216,7 @@ int run(const o3d_points* src, o3d_points* targ, bool self_excl, int T, hipStrea
   FFArgs a{};
   a.sp = L.sp; a.sa = L.sa; a.tq = L.tq; a.tperm = tperm;
   a.tsph = L.tsph; a.tcs = L.tcs; a.tam = L.tam; a.bsph = L.bsph; a.bcs = L.bcs;
-  a.mask = L.mask; a.farv = L.farv; a.sign = L.bb + 6;
+  a.mask = L.mask; a.farv = L.farv; a.tsg = L.tsg;
   a.nn = L.nn; a.items = L.items; a.ioff = L.ioff; a.mfold = L.mfold; a.ctr = L.ctr; a.part = L.part;
   a.s = sv; a.t = tv;
   a.ns = ns; a.nt = nt;
@@ -224,16 +225,16 @@ int run(const o3d_points* src, o3d_points* targ, bool self_excl, int T, hipStrea
   const int nslice = far_slices(nb, mwords);
   a.wslice = (mwords + nslice - 1) / nslice;
   a.nslice = (mwords + a.wslice - 1) / a.wslice;
-  const size_t lds_far = ff_far_lds<CORE, true>();
+  const size_t lds_far = ff_far_lds<CORE, GRAD>();
   if (prof) HIPCHK(hipEventRecord(ev[1].e, st));
-  hipLaunchKernelGGL((k_ff_far<CORE, true>), dim3((unsigned)nb, (unsigned)a.nslice), dim3(FF_FAR_THREADS), lds_far, st, a);
+  hipLaunchKernelGGL((k_ff_far<CORE, GRAD>), dim3((unsigned)nb, (unsigned)a.nslice), dim3(FF_FAR_THREADS), lds_far, st, a);
   HIPCHK(hipGetLastError());
   if (prof) HIPCHK(hipEventRecord(ev[2].e, st));
   const size_t lds_near = (size_t)T * 2 * sizeof(float4);
-  const unsigned gnear = (unsigned)std::min<int64_t>((near_split(nb) + 1) * nb, near_grid<CORE, PREC>(lds_near));
-  hipLaunchKernelGGL((k_ff_near<CORE, PREC>), dim3(gnear), dim3(FF_TB), lds_near, st, a);
+  const unsigned gnear = (unsigned)std::min<int64_t>((near_split(nb) + 1) * nb, near_grid<CORE, GRAD, PREC>(lds_near));
+  hipLaunchKernelGGL((k_ff_near<CORE, GRAD, PREC>), dim3(gnear), dim3(FF_TB), lds_near, st, a);
   HIPCHK(hipGetLastError());
-  hipLaunchKernelGGL((k_ff_combine<CORE, PREC>), dim3((unsigned)nb), dim3(FF_TB), 0, st, a);
+  hipLaunchKernelGGL((k_ff_combine<CORE, GRAD>), dim3((unsigned)nb), dim3(FF_TB), 0, st, a);
   HIPCHK(hipGetLastError());
   if (prof) {
     HIPCHK(hipEventRecord(ev[3].e, st));
@@ -258,14 +259,18 @@ int run(const o3d_points* src, o3d_points* targ, bool self_excl, int T, hipStrea
   return O3D_OK;
 }
 
-template <int CORE>
+// plain FP32 sums come here for the cores and results that the method FACTORED serves;
+// the others only in compensated precision
+template <int CORE, bool GRAD>
 int run_core(const o3d_points* src, o3d_points* targ, bool thick, int prec, bool self_excl, int T, hipStream_t st,
              o3d_factored_profile* prof, void* ws, size_t wsb) {
-  if (thick)
-    return prec == PREC_COMP ? run<CORE, true, PREC_COMP>(src, targ, self_excl, T, st, prof, ws, wsb)
-                             : run<CORE, true, PREC_FP32>(src, targ, self_excl, T, st, prof, ws, wsb);
-  return prec == PREC_COMP ? run<CORE, false, PREC_COMP>(src, targ, self_excl, T, st, prof, ws, wsb)
-                           : run<CORE, false, PREC_FP32>(src, targ, self_excl, T, st, prof, ws, wsb);
+  if (prec == PREC_COMP)
+    return thick ? run<CORE, true, GRAD, PREC_COMP>(src, targ, self_excl, T, st, prof, ws, wsb)
+                 : run<CORE, false, GRAD, PREC_COMP>(src, targ, self_excl, T, st, prof, ws, wsb);
+  if constexpr (GRAD && (CORE == CORE_RM || CORE == CORE_EXP))
+    return thick ? run<CORE, true, GRAD, PREC_FP32>(src, targ, self_excl, T, st, prof, ws, wsb)
+                 : run<CORE, false, GRAD, PREC_FP32>(src, targ, self_excl, T, st, prof, ws, wsb);
+  return fail(O3D_EINVAL, "internal: plain FP32 sums of core %d routed to the factored path", CORE);
 }
 
 }  // namespace
@@ -322,10 +327,9 @@ int sorted_sources(const o3d_points* src, const int32_t* perm, int tile, void* w
   float4* sph = (float4*)(p + 2 * r(sizeof(float4) * (size_t)n));
   float* cs = (float*)(p + 2 * r(sizeof(float4) * (size_t)n) + r(sizeof(float4) * (size_t)ntiles));
   const SrcView sv{src->x[0], src->x[1], src->x[2], src->r, src->s[0], src->s[1], src->s[2]};
-  hipLaunchKernelGGL((k_ff_gather_src<CORE_EXP>), dim3(grid_of(n, 256)), dim3(256), 0, st, sv, perm, n, n, sp, sa,
-                     (unsigned*)nullptr);
+  hipLaunchKernelGGL((k_ff_gather_src<CORE_EXP>), dim3(grid_of(n, 256)), dim3(256), 0, st, sv, perm, n, n, sp, sa);
   hipLaunchKernelGGL(k_ff_bounds, dim3((unsigned)ntiles), dim3(256), 0, st, (const float4*)sp, (const float4*)nullptr,
-                     n, tile, sph, cs, (float*)nullptr);
+                     n, tile, sph, cs, (float*)nullptr, (float*)nullptr);
   HIPCHK(hipGetLastError());
   a->sp = sp;
   a->sa = sa;
@@ -389,10 +393,13 @@ bool ff_supported(int core, bool grad, int prec) {
   return (core == CORE_RM || core == CORE_EXP) && grad && (prec == PREC_FP32 || prec == PREC_COMP);
 }
 
+// what AUTO may send here besides
+bool ff_auto_supported(int core, bool grad, int prec) { return prec == PREC_COMP || ff_supported(core, grad, prec); }
+
 namespace {
 int check_factored(const o3d_points* src, const o3d_points* targ, const o3d_opts* o, int* T) {
   const bool grad = o->results == O3D_VELANDGRAD;
-  if (!ff_supported(o->core, grad, o->precision))
+  if (o->method == O3D_METHOD_FACTORED && !ff_supported(o->core, grad, o->precision))
     return fail(O3D_EINVAL, "factored method: needs the RM or EXP core, velocity and gradient, and FP32 or "
                             "compensated precision");
   if (src->n > INT_MAX || targ->n > INT_MAX)
@@ -402,12 +409,23 @@ int check_factored(const o3d_points* src, const o3d_points* targ, const o3d_opts
   return O3D_OK;
 }
 
-int dispatch(const o3d_points* src, o3d_points* targ, const o3d_opts* o, int T, hipStream_t st,
-             o3d_factored_profile* prof, void* ws, size_t wsb) {
+template <bool GRAD>
+int dispatch_grad(const o3d_points* src, o3d_points* targ, const o3d_opts* o, int T, hipStream_t st,
+                  o3d_factored_profile* prof, void* ws, size_t wsb) {
   const bool thick = targ->r != nullptr;
   const bool self_excl = o->self_term == O3D_SELF_EXCLUDE;
-  if (o->core == CORE_RM) return run_core<CORE_RM>(src, targ, thick, o->precision, self_excl, T, st, prof, ws, wsb);
-  return run_core<CORE_EXP>(src, targ, thick, o->precision, self_excl, T, st, prof, ws, wsb);
+  switch (o->core) {
+    case CORE_RM: return run_core<CORE_RM, GRAD>(src, targ, thick, o->precision, self_excl, T, st, prof, ws, wsb);
+    case CORE_WL: return run_core<CORE_WL, GRAD>(src, targ, thick, o->precision, self_excl, T, st, prof, ws, wsb);
+    case CORE_EXP: return run_core<CORE_EXP, GRAD>(src, targ, thick, o->precision, self_excl, T, st, prof, ws, wsb);
+    default: return run_core<CORE_V2, GRAD>(src, targ, thick, o->precision, self_excl, T, st, prof, ws, wsb);
+  }
+}
+
+int dispatch(const o3d_points* src, o3d_points* targ, const o3d_opts* o, int T, hipStream_t st,
+             o3d_factored_profile* prof, void* ws, size_t wsb) {
+  return o->results == O3D_VELANDGRAD ? dispatch_grad<true>(src, targ, o, T, st, prof, ws, wsb)
+                                      : dispatch_grad<false>(src, targ, o, T, st, prof, ws, wsb);
 }
 }  // namespace
 
@@ -430,9 +448,9 @@ int p2p_factored_ws(const o3d_points* src, o3d_points* targ, const o3d_opts* o, 
   return dispatch(src, targ, o, T, st, nullptr, ws, ws_bytes);
 }
 
-size_t ff_workspace_bytes(int64_t ns, int64_t nt, bool same, int tile) {
+size_t ff_workspace_bytes(int64_t ns, int64_t nt, bool same, int tile, bool grad) {
   const int T = tile > 0 ? tile : 256;
-  return layout(nullptr, ns, nt, same, T, lib_tmp_bytes(ns, nt, same)).bytes;
+  return layout(nullptr, ns, nt, same, T, lib_tmp_bytes(ns, nt, same), grad ? 12 : 3).bytes;
 }
 
 }  // namespace o3d

@@ -45,20 +45,15 @@
 
 #include <type_traits>
 
-// the far field's schedule of one phase (k_ff_far): two products of squared distances
-// and n of moments, each followed by its share of the phase's vector work, the
-// quarter-rate square roots first
-#define FF_SCHED(n)                                                          \
-  _Pragma("unroll") for (int q_ = 0; q_ < (n) + 2; ++q_) {                   \
+// the far field's schedule of one phase (k_ff_far): n matrix products, each followed by
+// its share (tr, va) of the phase's vector work, the quarter-rate square roots first
+#define FF_SCHED(n, tr, va)                                                  \
+  _Pragma("unroll") for (int q_ = 0; q_ < (n); ++q_) {                   \
     __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);                       \
-    __builtin_amdgcn_sched_group_barrier(0x400, FF_TR(n), 0);                \
-    __builtin_amdgcn_sched_group_barrier(0x002, FF_VA(n), 0);                \
+    __builtin_amdgcn_sched_group_barrier(0x400, (tr), 0);                    \
+    __builtin_amdgcn_sched_group_barrier(0x002, (va), 0);                    \
   }                                                                          \
   __builtin_amdgcn_sched_barrier(0)
-#ifndef FF_TR
-#define FF_TR(n) 2
-#define FF_VA(n) 10
-#endif
 
 namespace o3d {
 
@@ -69,17 +64,20 @@ typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
 constexpr int FF_TB = 256;          // targets per workgroup: 4 waves x 64
 constexpr float FF_KAPPA = 1.0f;    // minimum gap, in block radii
 // near field, compensated: sources per FP32 partial.  Gradient error against FP64 on two
-// rings of 1,048,576 particles, EXP: 5.9e-8 at 32, 5.0e-8 at 16 (near field 30.3 and 31.5
-// ms); RM, 262,144: 4.5e-8 and 4.3e-8, with the near field 6% slower at 16
-template <int CORE>
-constexpr int ff_fold() { return CORE == CORE_EXP ? 16 : 32; }
+// rings: EXP, 1,048,576 particles, 5.9e-8 at 32 and 5.0e-8 at 16 (near field 30.3 and
+// 31.5 ms); RM, 262,144, 4.5e-8 and 4.3e-8, with the near field 6% slower at 16; WL,
+// 131,070, 5.6e-8 at 32, 5.2e-8 at 16, 4.9e-8 at 8 (the call 0 and 1% slower)
+template <int CORE, bool GRAD>
+constexpr int ff_fold() { return !GRAD || CORE == CORE_WL ? 8 : CORE == CORE_RM ? 32 : 16; }
 constexpr int FF_M0 = 4;            // near field: fewest tiles per work item
 constexpr int FF_FAR_THREADS = 256; // far field: 4 waves of 64 targets per block
 constexpr int FF_TP = 264;          // far field: LDS row of the FP16 moment tables (halves, tile <= 256)
 constexpr int FF_SL = 40;           // far field: LDS row of a source's BF16 r2 slots (32 used, 80 bytes)
 // far field: most consecutive tiles per fold into FP64.  Two rings, 262,144 particles, RM:
-// velocity error 5.9e-8 at 8 tiles, 5.2e-8 at 4, 4.9e-8 at 2; far field 19.2, 19.7, 20.2 ms
-constexpr int FF_MERGE = 4;
+// velocity error 4.5e-8 at 8 tiles, 4.2e-8 at 4; far field 20.2 and 20.5 ms.
+// Cores that the direct kernel sums otherwise (4.6e-8): 2
+template <int CORE, bool GRAD>
+constexpr int ff_merge() { return GRAD && (CORE == CORE_RM || CORE == CORE_EXP) ? 4 : 2; }
 
 struct FFArgs {
   const float4* sp;    // sorted sources {x, y, z, core_term}, up to a whole tile: the last one again
@@ -93,7 +91,7 @@ struct FFArgs {
   const float* bcs;    // per target block: largest core term
   const unsigned* mask;  // far bit per (block, tile), mwords words per block
   double* farv;        // per slice: 12 x nt (3 x nt), sorted target order: far-field velocity and gradient
-  const unsigned* sign;  // odd: the first strength's first nonzero component is negative
+  const float* tsg;    // per source tile: sign of its first nonzero strength, 0: none
   int32_t nslice;      // slices of the far field: slice y takes mask words [y * wslice, (y + 1) * wslice)
   int32_t wslice;
   const int* nn;       // near tiles per block
@@ -121,7 +119,7 @@ __device__ __forceinline__ float fdec(unsigned e) {
 }
 
 __global__ void k_ff_bbox_init(unsigned* bb) {
-  if (threadIdx.x < 3 || threadIdx.x == 6) bb[threadIdx.x] = 0xffffffffu;
+  if (threadIdx.x < 3) bb[threadIdx.x] = 0xffffffffu;
   else if (threadIdx.x < 6) bb[threadIdx.x] = 0u;
 }
 
@@ -192,26 +190,15 @@ __global__ __launch_bounds__(256) void k_ff_keys(const float* x, const float* y,
   if (idx) idx[i] = (int)i;
 }
 
-// rows n .. npad - 1: the last source's place with no strength; sign (optional): the
-// smallest 2 i + (its first nonzero component is negative) over the sources i with a
-// strength, in sorted order
+// rows n .. npad - 1: the last source's place with no strength
 template <int CORE>
 __global__ __launch_bounds__(256) void k_ff_gather_src(SrcView s, const int* perm, int64_t n, int64_t npad, float4* sp,
-                                                       float4* sa, unsigned* sign) {
+                                                       float4* sa) {
   const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
   if (i >= npad) return;
   const int j = perm[i < n ? i : n - 1];
   sp[i] = make_float4(s.x[j], s.y[j], s.z[j], core_term<CORE>(s.r[j]));
-  const float4 A = i < n ? make_float4(s.ax[j], s.ay[j], s.az[j], 0.0f) : make_float4(0.0f, 0.0f, 0.0f, 0.0f);
-  sa[i] = A;
-  if (sign) {
-    const float lead = A.x != 0.0f ? A.x : A.y != 0.0f ? A.y : A.z;
-    const uint64_t any = __builtin_amdgcn_ballot_w64(lead != 0.0f);
-    if (any != 0 && (threadIdx.x & 63) == (unsigned)__builtin_ctzll(any)) {
-      const unsigned key = 2u * (unsigned)i + (lead < 0.0f ? 1u : 0u);
-      if (key < __hip_atomic_load(sign, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)) atomicMin(sign, key);
-    }
-  }
+  sa[i] = i < n ? make_float4(s.ax[j], s.ay[j], s.az[j], 0.0f) : make_float4(0.0f, 0.0f, 0.0f, 0.0f);
 }
 
 template <int CORE, bool THICK>
@@ -234,11 +221,14 @@ __device__ __forceinline__ float wg_max(float v, float* red) {
 __device__ __forceinline__ float wg_min(float v, float* red) { return -wg_max(-v, red); }
 
 // bounding sphere (bbox centre, largest distance), largest core term and (when pa
-// is given) largest |alpha| of each group of `group` consecutive sorted points;
-// one workgroup per group
+// is given) largest |alpha| and the sign of the first nonzero strength (0: none), by
+// its first nonzero component, of each group of `group` consecutive sorted points; one
+// workgroup per group
 __global__ __launch_bounds__(256) void k_ff_bounds(const float4* p, const float4* pa, int64_t n, int group,
-                                                   float4* sph, float* cs, float* amax) {
+                                                   float4* sph, float* cs, float* amax, float* sign) {
   __shared__ float red[4];
+  __shared__ unsigned lead;   // smallest 2 i + (negative) over the group's points i with a strength
+  if (threadIdx.x == 0) lead = 0xffffffffu;
   const int64_t b0 = (int64_t)blockIdx.x * group;
   const int64_t b1 = (b0 + group) < n ? (b0 + group) : n;
   float lo[3] = {__builtin_huge_valf(), __builtin_huge_valf(), __builtin_huge_valf()};
@@ -271,13 +261,16 @@ __global__ __launch_bounds__(256) void k_ff_bounds(const float4* p, const float4
     for (int64_t i = b0 + threadIdx.x; i < b1; i += blockDim.x) {
       const float4 q = pa[i];
       a2 = fmaxf(a2, fmaf(q.z, q.z, fmaf(q.y, q.y, q.x * q.x)));
+      const float f = q.x != 0.0f ? q.x : q.y != 0.0f ? q.y : q.z;
+      if (f != 0.0f) atomicMin(&lead, 2u * (unsigned)(i - b0) + (f < 0.0f ? 1u : 0u));
     }
-  a2 = wg_max(a2, red);
+  a2 = wg_max(a2, red);   // its barriers order the atomics too
   if (threadIdx.x == 0) {
     // margin for the rounding of the distances above
     sph[blockIdx.x] = make_float4(c[0], c[1], c[2], __fsqrt_rn(r2) * 1.00001f + 1e-30f);
     cs[blockIdx.x] = cmax;
     if (amax) amax[blockIdx.x] = __fsqrt_rn(a2) * 1.00001f;
+    if (sign) sign[blockIdx.x] = lead == 0xffffffffu ? 0.0f : (lead & 1u) ? -1.0f : 1.0f;
   }
 }
 
@@ -435,11 +428,14 @@ __device__ __forceinline__ void split_bf3(float x, __bf16& hi, __bf16& mid, __bf
 // squared distances on the matrix cores: r2 = sum_c S_c T_c over the five terms
 // S = (-2 s'x, -2 s'y, -2 s'z, b, 1) (per source) and T = (t'x, t'y, t'z, 1, a) (per
 // target), both pre-scaled by the tile's r2 scale, each split into BF16 hi/mid/lo
-// and multiplied as hi hi + hi mid + mid hi + hi lo + lo hi + mid mid (about 24 bits:
-// the accuracy of the FP32 expression it replaces).  Slot q < 30 of the K = 32
-// product holds term q / 5 of component q % 5; the parts taken per term:
-__device__ __forceinline__ int ff_src_part(int term) { return term == 2 || term == 5 ? 1 : (term == 4 ? 2 : 0); }
-__device__ __forceinline__ int ff_tgt_part(int term) { return term == 1 || term == 5 ? 1 : (term == 3 ? 2 : 0); }
+// and multiplied as hi lo + lo hi + mid mid + hi mid + mid hi + hi hi (about 24 bits: the
+// accuracy of the FP32 expression it replaces).  Slot q < 30 of the K = 32 product
+// holds term q / 5 of component q % 5, the small terms first: a product of the first 16
+// slots has no large term, against which the matrix cores would cut the small ones off
+// (large terms first: an error of 4e-8 in K that the targets' own parts decide, the
+// same for all far sources).  The parts taken per term:
+__device__ __forceinline__ int ff_src_part(int term) { return term == 1 ? 2 : (term == 2 || term == 4 ? 1 : 0); }
+__device__ __forceinline__ int ff_tgt_part(int term) { return term == 0 ? 2 : (term == 2 || term == 3 ? 1 : 0); }
 
 // source position of tile slot p in the FP16 moment tables: inside each group of 16
 // sources, slot 16g + 8h + e holds source 16g + 4h + (e % 4) + 8 (e / 4), so that the
@@ -470,6 +466,22 @@ __device__ __forceinline__ void ff_weights(float r, float tau, float& K, float& 
   }
 }
 
+// Relative errors with a mean, which a sum over many pairs keeps while the rest of them
+// averages out; the folds take it out of the sums of Bp and of K.  v_rsq_f32: -6.98e-9
+// over all mantissas of two octaves weighted by 1 / x (rms 2.6e-8, largest 9.4e-8);
+// v_sqrt_f32: -1.43e-8 likewise; the squared distance: -1.97e-8, as the matrix cores cut
+// off what does not fit the sum (from K of far clouds of particles in FP64).
+constexpr double FF_RSQ_MEAN = -6.98e-9, FF_SQRT_MEAN = -1.43e-8, FF_R2_MEAN = -1.97e-8;
+template <int CORE>
+constexpr double ff_mean_b() {
+  return 1.0 - (CORE == CORE_V2 ? 2.5 * FF_RSQ_MEAN + FF_SQRT_MEAN : 5.0 * FF_RSQ_MEAN) + 2.5 * FF_R2_MEAN;
+}
+template <int CORE>
+constexpr double ff_mean_k() {
+  return 1.0 - (CORE == CORE_V2 ? 1.5 * FF_RSQ_MEAN + FF_SQRT_MEAN : (CORE == CORE_WL ? 5.0 : 3.0) * FF_RSQ_MEAN) +
+         1.5 * FF_R2_MEAN;
+}
+
 // 16 bytes per lane from memory to LDS without a register: lane l's from src to dst + l
 // (dst the same in every lane); done when the wave's loads are
 __device__ __forceinline__ void ff_load_lds16(const float4* src, float4* dst) {
@@ -492,7 +504,7 @@ __device__ __forceinline__ void ff_load_lds16(const float4* src, float4* dst) {
 // a, so Bp takes 2^(5 jw / 2) and K 2^(3 jw / 2) (from Bp <= 3.5 gap^-5), and each moment
 // group by 2^eg (from the tile's largest |alpha| and source distance), so that every
 // FP16 factor stays below 2^16.  Consecutive tiles keep the scales of the first as
-// long as they fit (FF_MERGE tiles at most) and share one fold into FP64, where the
+// long as they fit (ff_merge tiles at most) and share one fold into FP64, where the
 // scales are removed.  All strengths are taken times the sign of the first nonzero one
 // (in sorted order, its first nonzero component) and the result times that sign again:
 // the matrix cores do not round a product and its negative alike, and so negating
@@ -508,15 +520,15 @@ __device__ __forceinline__ void ff_load_lds16(const float4* src, float4* dst) {
 // of 16 lanes cover all 64 banks, the rows of the next tile, and (WL, V2) the scaled
 // core term per source.
 //
-// The loop over chunks is a pipeline: while one set's weights are formed on the vector
-// ALUs, the matrix cores take the other set's moment products and the next squared
-// distances.  A wave issues in order, so each product is followed by its share of the
+// The loop over chunks is a pipeline: while the weights of one set and half are formed on
+// the vector ALUs, the matrix cores take the moment products of the half before and the
+// next squared distances.  A wave issues in order, so each product is followed by its share of the
 // vector work (FF_SCHED).  Measured cycles per wave instruction with two waves per SIMD:
 // product 32; add, multiply, fmac 2.3; conversions and v_fma_mix_f32 4.5; v_rsq_f32 and
 // v_fma_mixlo/mixhi_f16 8.3.  A product beside 2 rsq, 6 multiplies and 4 conversions
 // takes 64.5, the twelve alone 57: this loop runs at 69.  The tile's tables cost about
 // 200 vector instructions per wave, the loop 1,700; what a run (ff_fold and the target
-// slots) costs is shared by FF_MERGE tiles.
+// slots) costs is shared by ff_merge tiles.
 template <int CORE, bool GRAD>
 __global__ __launch_bounds__(FF_FAR_THREADS, 2) void k_ff_far(FFArgs a) {
   constexpr int FORM = ff_form<CORE, GRAD>();
@@ -540,8 +552,9 @@ __global__ __launch_bounds__(FF_FAR_THREADS, 2) void k_ff_far(FFArgs a) {
   const int64_t blk = blockIdx.x;
   const int64_t base = blk * FF_TB + w * 64;
   const float4 cb = a.bsph[blk];
-  const unsigned lead = *a.sign;
-  const float sgn = lead != 0xffffffffu && (lead & 1u) ? -1.0f : 1.0f;
+  float sgn = a.tsg[0];   // of the first nonzero strength of all
+  for (int t = 1; sgn == 0.0f && t < a.ntiles; ++t) sgn = a.tsg[t];
+  sgn = sgn < 0.0f ? -1.0f : 1.0f;
 
   float tx[2], ty[2], tz[2], tt[2], al[2];
 #pragma unroll
@@ -553,10 +566,16 @@ __global__ __launch_bounds__(FF_FAR_THREADS, 2) void k_ff_far(FFArgs a) {
     tt[s] = CORE == CORE_EXP ? 0.0f : q.w;
     al[s] = fmaf(tz[s], tz[s], fmaf(ty[s], ty[s], fmaf(tx[s], tx[s], COREA ? tt[s] : 0.0f)));
   }
-  f32x16 accB[2], accK[2];
-  double sum[NOUT];
+  f32x16 accB[2], accK[2], accR[2];
+  // the folds add up in registers, or (both weights: no registers left) in the results' place
+  constexpr bool INMEM = FORM == FF_KB;
+  double sum[INMEM ? 1 : NOUT];
+  bool first = true;
+  if (!INMEM)
 #pragma unroll
-  for (int k = 0; k < NOUT; ++k) sum[k] = 0.0;
+    for (int k = 0; k < NOUT; ++k) sum[k] = 0.0;
+  const int64_t own = base + lane;
+  double* dst = a.farv + (int64_t)blockIdx.y * NOUT * a.nt + own;
 
   const unsigned* mrow = a.mask + blk * a.mwords;
   int jw = 0, eg[NG];
@@ -587,98 +606,103 @@ __global__ __launch_bounds__(FF_FAR_THREADS, 2) void k_ff_far(FFArgs a) {
     double c[32], ck[32], out[12];
     if (HASB) {
       // 2^(-5 jw / 2)
-      const double wb = ldexp(jw & 1 ? 0.70710678118654752440 : 1.0, -2 * jw - (jw >> 1));
+      const double wb = ldexp(jw & 1 ? 0.70710678118654752440 : 1.0, -2 * jw - (jw >> 1)) * ff_mean_b<CORE>();
+      if (FORM == FF_B)
+#pragma unroll
+        for (int s = 0; s < 2; ++s)
+#pragma unroll
+          for (int r = 0; r < 16; ++r) accB[s][r] += accR[s][r];
       rows_of(accB, c);
 #pragma unroll
       for (int i = 0; i < COLS; ++i) c[i] *= sc[ff_group(i)] * wb;
     }
     if (HASK) {
       // 2^(-3 jw / 2)
-      const double wk = ldexp(jw & 1 ? 0.70710678118654752440 : 1.0, -jw - (jw >> 1));
+      const double wk = ldexp(jw & 1 ? 0.70710678118654752440 : 1.0, -jw - (jw >> 1)) * ff_mean_k<CORE>();
       rows_of(accK, ck);
 #pragma unroll
       for (int i = 0; i < 6; ++i) ck[i] = (ck[i] + ck[16 + i]) * (sc[ff_group(i)] * wk);
     }
     if constexpr (FORM == FF_B) ff_epilogue(c, ox, oy, oz, oa, out);
     else ff_epilogue_k<GRAD>(ck, c, ox, oy, oz, out);
+    if constexpr (INMEM) {
+      if (own < a.nt) {
 #pragma unroll
-    for (int k = 0; k < NOUT; ++k) sum[k] += out[k];
+        for (int k = 0; k < NOUT; ++k) dst[(int64_t)k * a.nt] = (first ? 0.0 : dst[(int64_t)k * a.nt]) + out[k];
+      }
+      first = false;
+    } else {
+#pragma unroll
+      for (int k = 0; k < NOUT; ++k) sum[k] += out[k];
+    }
   };
-  // one chunk of 32 sources: the slots and moment operands of this lane, the weights of
-  // each set split by halves of 16 sources
+  // one chunk of 32 sources: its slots and moment operands (two halves of 16 sources) of
+  // this lane, its squared distances per set, and the weights of two consecutive halves
   struct Frag {
-    f16x8 bh[2], bl[2], kh[2], kl[2];
+    f16x8 bh, bl, kh, kl;
   };
   bf16x8 sa[2];
   f16x8 mb[2][2], mk[2];
   f32x16 r2[2];
   Frag f[2];
-  auto load_slots = [&](int k0) {
-    const __bf16* srow = sl + (k0 + col) * FF_SL + 8 * half;
-    sa[0] = *reinterpret_cast<const bf16x8*>(srow);
-    sa[1] = *reinterpret_cast<const bf16x8*>(srow + 16);
+  auto load_slots = [&](int k0, int part) {
+    sa[part] = *reinterpret_cast<const bf16x8*>(sl + (k0 + col) * FF_SL + 8 * half + 16 * part);
   };
-  auto load_moments = [&](int k0) {
-#pragma unroll
-    for (int kb = 0; kb < 2; ++kb) {
-      const int pbase = k0 + 16 * kb + 8 * half;
-      if (HASB) {
-        mb[kb][0] = *reinterpret_cast<const f16x8*>(mh + col * TP + pbase);
-        mb[kb][1] = *reinterpret_cast<const f16x8*>(ml + col * TP + pbase);
-      }
-      // rows 0-15 the leading parts of the first 16 columns, rows 16-31 their remainders
-      if (HASK)
-        mk[kb] = *reinterpret_cast<const f16x8*>((col < 16 ? mh + col * TP : ml + (col - 16) * TP) + pbase);
+  auto load_moments = [&](int k0, int kb) {
+    const int pbase = k0 + 16 * kb + 8 * half;
+    if (HASB) {
+      mb[kb][0] = *reinterpret_cast<const f16x8*>(mh + col * TP + pbase);
+      mb[kb][1] = *reinterpret_cast<const f16x8*>(ml + col * TP + pbase);
     }
+    // rows 0-15 the leading parts of the first 16 columns, rows 16-31 their remainders
+    if (HASK) mk[kb] = *reinterpret_cast<const f16x8*>((col < 16 ? mh + col * TP : ml + (col - 16) * TP) + pbase);
   };
-  // squared distances of the 32 sources of sa to this lane's target of set s
-  auto dist = [&](int s) {
+  // squared distances of the 32 sources of sa to this lane's target of set s, in two parts
+  auto dist = [&](int s, int part) {
     const f32x16 z = {};
-    r2[s] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(sa[0], tb[s][0], z, 0, 0, 0);
-    r2[s] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(sa[1], tb[s][1], r2[s], 0, 0, 0);
+    r2[s] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(sa[part], tb[s][part], part == 0 ? z : r2[s], 0, 0, 0);
   };
-  auto weigh = [&](int s, int k0) {
-#pragma unroll
-    for (int kb = 0; kb < 2; ++kb) {
-      float tau[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
-      if (TAU) {
-        const float4 t0 = *reinterpret_cast<const float4*>(tc + k0 + 16 * kb + 4 * half);
-        const float4 t1 = *reinterpret_cast<const float4*>(tc + k0 + 16 * kb + 8 + 4 * half);
-        tau[0] = t0.x; tau[1] = t0.y; tau[2] = t0.z; tau[3] = t0.w;
-        tau[4] = t1.x; tau[5] = t1.y; tau[6] = t1.z; tau[7] = t1.w;
-      }
-#pragma unroll
-      for (int e = 0; e < 8; e += 2) {
-        float K0, K1, B0, B1;
-        ff_weights<CORE, FORM>(r2[s][8 * kb + e], tau[e] + tts[s], K0, B0);
-        ff_weights<CORE, FORM>(r2[s][8 * kb + e + 1], tau[e + 1] + tts[s], K1, B1);
-        if (HASB) split16x2(B0, B1, f[s].bh[kb], f[s].bl[kb], e);
-        if (HASK) split16x2(K0, K1, f[s].kh[kb], f[s].kl[kb], e);
-      }
+  // scaled core terms of the 8 sources that the lane weighs next
+  float tau[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
+  auto load_tau = [&](int k0, int kb) {
+    if (TAU) {
+      const float4 t0 = *reinterpret_cast<const float4*>(tc + k0 + 16 * kb + 4 * half);
+      const float4 t1 = *reinterpret_cast<const float4*>(tc + k0 + 16 * kb + 8 + 4 * half);
+      tau[0] = t0.x; tau[1] = t0.y; tau[2] = t0.z; tau[3] = t0.w;
+      tau[4] = t1.x; tau[5] = t1.y; tau[6] = t1.z; tau[7] = t1.w;
     }
   };
-  auto moments = [&](int s) {
+  auto weigh = [&](int s, int kb) {
 #pragma unroll
-    for (int kb = 0; kb < 2; ++kb) {
-      if (HASB) {
-        accB[s] = __builtin_amdgcn_mfma_f32_32x32x16_f16(mb[kb][0], f[s].bh[kb], accB[s], 0, 0, 0);
-        accB[s] = __builtin_amdgcn_mfma_f32_32x32x16_f16(mb[kb][0], f[s].bl[kb], accB[s], 0, 0, 0);
-        accB[s] = __builtin_amdgcn_mfma_f32_32x32x16_f16(mb[kb][1], f[s].bh[kb], accB[s], 0, 0, 0);
-      }
-      if (HASK) {
-        accK[s] = __builtin_amdgcn_mfma_f32_32x32x16_f16(mk[kb], f[s].kh[kb], accK[s], 0, 0, 0);
-        accK[s] = __builtin_amdgcn_mfma_f32_32x32x16_f16(mk[kb], f[s].kl[kb], accK[s], 0, 0, 0);
-      }
+    for (int e = 0; e < 8; e += 2) {
+      float K0, K1, B0, B1;
+      ff_weights<CORE, FORM>(r2[s][8 * kb + e], tau[e] + tts[s], K0, B0);
+      ff_weights<CORE, FORM>(r2[s][8 * kb + e + 1], tau[e + 1] + tts[s], K1, B1);
+      if (HASB) split16x2(B0, B1, f[kb].bh, f[kb].bl, e);
+      if (HASK) split16x2(K0, K1, f[kb].kh, f[kb].kl, e);
+    }
+  };
+  auto moments = [&](int s, int kb) {
+    if (HASB) {
+      accB[s] = __builtin_amdgcn_mfma_f32_32x32x16_f16(mb[kb][0], f[kb].bh, accB[s], 0, 0, 0);
+      // the products with a remainder in sums of their own (FF_B: there are registers for
+      // it): the matrix cores cut off every sum they add to, so the large one is cut once
+      // per 16 sources instead of three times (far clouds of particles, RM and EXP with
+      // gradient: error 7.4e-8 -> 4.5e-8)
+      f32x16& rest = FORM == FF_B ? accR[s] : accB[s];
+      rest = __builtin_amdgcn_mfma_f32_32x32x16_f16(mb[kb][0], f[kb].bl, rest, 0, 0, 0);
+      rest = __builtin_amdgcn_mfma_f32_32x32x16_f16(mb[kb][1], f[kb].bh, rest, 0, 0, 0);
+    }
+    if (HASK) {
+      accK[s] = __builtin_amdgcn_mfma_f32_32x32x16_f16(mk[kb], f[kb].kh, accK[s], 0, 0, 0);
+      accK[s] = __builtin_amdgcn_mfma_f32_32x32x16_f16(mk[kb], f[kb].kl, accK[s], 0, 0, 0);
     }
   };
   // nothing pending: zero weights (and operands) for the moments of a chunk before the first
   auto none_pending = [&]() {
     const f16x8 z = {};
-#pragma unroll
-    for (int kb = 0; kb < 2; ++kb) {
-      if (HASB) { f[1].bh[kb] = z; f[1].bl[kb] = z; mb[kb][0] = z; mb[kb][1] = z; }
-      if (HASK) { f[1].kh[kb] = z; f[1].kl[kb] = z; mk[kb] = z; }
-    }
+    if (HASB) { f[1].bh = z; f[1].bl = z; mb[1][0] = z; mb[1][1] = z; }
+    if (HASK) { f[1].kh = z; f[1].kl = z; mk[1] = z; }
   };
   // the next far tile of this slice of the block (-1: none).  A mask word at a time, lane
   // l works out the scales that tile l of the word wants: the largest weight and moment
@@ -764,7 +788,7 @@ __global__ __launch_bounds__(FF_FAR_THREADS, 2) void k_ff_far(FFArgs a) {
 #pragma unroll
     for (int s = 0; s < 2; ++s)
 #pragma unroll
-      for (int r = 0; r < 16; ++r) { accB[s][r] = 0.0f; accK[s][r] = 0.0f; }
+      for (int r = 0; r < 16; ++r) { accB[s][r] = 0.0f; accK[s][r] = 0.0f; accR[s][r] = 0.0f; }
     none_pending();
     int run = 0;
     bool more;
@@ -846,39 +870,58 @@ __global__ __launch_bounds__(FF_FAR_THREADS, 2) void k_ff_far(FFArgs a) {
     ti = next_tile();
     if (ti >= 0) fetch(ti);
 
-    // phases of 32 sources x 32 targets: while set 0 of a chunk is weighed the matrix
-    // cores take set 1's distances and the moments of set 1 of the chunk before (for the
-    // first chunk: of the tile before, or zeros); while set 1 is weighed, set 0's
-    // distances of the next chunk and the moments of set 0
-    constexpr int NM = (HASB ? 6 : 0) + (HASK ? 4 : 0);
-    load_slots(0);
-    dist(0);
+    // Four phases per chunk of 32 sources, one per set and half: while a half is weighed,
+    // the matrix cores take the moments of the half before (in the first phase: of the
+    // chunk or tile before, or zeros) and half of the distances that the phase after next
+    // needs.
+    constexpr int NM = (HASB ? 3 : 0) + (HASK ? 2 : 0) + 1;
+    constexpr int TR = FORM == FF_K || CORE == CORE_V2 ? 3 : 2;
+    constexpr int VA = FORM == FF_B ? 10 : FORM == FF_K ? (CORE == CORE_WL ? 16 : 12) : CORE == CORE_WL ? 18 : 12;
+    load_slots(0, 0);
+    load_slots(0, 1);
+    load_tau(0, 0);
+    dist(0, 0);
+    dist(0, 1);
     for (int k0 = 0; k0 < T; k0 += 32) {
+      const int kn = k0 + 32 < T ? k0 + 32 : 0;   // after the last chunk: distances that nothing uses
       __builtin_amdgcn_sched_barrier(0);
-      dist(1);
-      moments(1);
-      weigh(0, k0);
-      load_slots(k0 + 32 < T ? k0 + 32 : 0);
-      load_moments(k0);
-      FF_SCHED(NM);
-      dist(0);
-      moments(0);
-      weigh(1, k0);
-      FF_SCHED(NM);
+      dist(1, 0);
+      moments(1, 1);
+      weigh(0, 0);
+      load_tau(k0, 1);
+      load_moments(k0, 0);
+      FF_SCHED(NM, TR, VA);
+      dist(1, 1);
+      moments(0, 0);
+      weigh(0, 1);
+      load_tau(k0, 0);
+      load_moments(k0, 1);
+      load_slots(kn, 0);
+      FF_SCHED(NM, TR, VA);
+      dist(0, 0);
+      moments(0, 1);
+      weigh(1, 0);
+      load_tau(k0, 1);
+      load_slots(kn, 1);
+      FF_SCHED(NM, TR, VA);
+      dist(0, 1);
+      moments(1, 0);
+      weigh(1, 1);
+      load_tau(kn, 0);
+      FF_SCHED(NM, TR, VA);
     }
     // the run's scales fit a further tile when no factor passes 2^16 and none loses more
     // than 4 of its leading bits
-    more = ti >= 0 && ++run < FF_MERGE && (unsigned)(jw - wj + 1) <= 2u;
+    more = ti >= 0 && ++run < ff_merge<CORE, GRAD>() && (unsigned)(jw - wj + 1) <= 2u;
 #pragma unroll
     for (int g = 0; g < NG; ++g) more = more && (unsigned)(eg[g] - wg[g] + 4) <= 6u;
     } while (more);
-    moments(1);
+    moments(1, 1);
     fold();
   }
-  const int64_t i = base + lane;
-  if (i < a.nt) {
+  if (own < a.nt && (!INMEM || first)) {
 #pragma unroll
-    for (int k = 0; k < NOUT; ++k) a.farv[((int64_t)blockIdx.y * NOUT + k) * a.nt + i] = sum[k];
+    for (int k = 0; k < NOUT; ++k) dst[(int64_t)k * a.nt] = INMEM ? 0.0 : sum[k];
   }
 }
 
@@ -921,7 +964,7 @@ __global__ void k_ff_zero_u32(unsigned* p) {
 }
 
 // per-target partial of one item: near tiles of rank [r0, r1) among block b's
-template <int CORE, int PREC>
+template <int CORE, bool GRAD, int PREC>
 __device__ __forceinline__ void near_item(const FFArgs& a, int64_t b, int r0, int r1, float4* sh, double* r) {
   const int T = a.tile;
   const int tid = threadIdx.x;
@@ -962,17 +1005,17 @@ __device__ __forceinline__ void near_item(const FFArgs& a, int64_t b, int r0, in
         // gradient's into FP64 and the velocity's into its TwoSum pair (the velocity
         // once per tile: error against FP64 on 65,536-131,072 particles in two rings
         // 9.1e-8 to 1.2e-7 instead of 4.8e-8 to 6.0e-8, near field 0-1% faster).
-        constexpr int FOLD = ff_fold<CORE>();
+        constexpr int FOLD = ff_fold<CORE, GRAD>();
         for (int j0 = 0; j0 < cnt; j0 += FOLD) {
           const int j1 = j0 + FOLD < cnt ? j0 + FOLD : cnt;
           for (int j = j0; j < j1; ++j)
-            source_acc<CORE, true, 1>(tx, ty, tz, tt, thr, sh[2 * j], sh[2 * j + 1], acc);
-          fold_grad_raw(acc[0], gr);
+            source_acc<CORE, GRAD, 1>(tx, ty, tz, tt, thr, sh[2 * j], sh[2 * j + 1], acc);
+          if (GRAD) fold_grad_raw(acc[0], gr);
           fold_vel_comp(acc[0], hi, lo);
         }
       } else {
         for (int j = 0; j < cnt; ++j)
-          source_acc<CORE, true, 1>(tx, ty, tz, tt, thr, sh[2 * j], sh[2 * j + 1], acc);
+          source_acc<CORE, GRAD, 1>(tx, ty, tz, tt, thr, sh[2 * j], sh[2 * j + 1], acc);
       }
     }
   }
@@ -980,18 +1023,20 @@ __device__ __forceinline__ void near_item(const FFArgs& a, int64_t b, int r0, in
     r[0] = (double)hi[0] + (double)lo[0];
     r[1] = (double)hi[1] + (double)lo[1];
     r[2] = (double)hi[2] + (double)lo[2];
-    grad_from<double>(gr, r + 3);
+    if (GRAD) grad_from<double>(gr, r + 3);
   } else {
-    float g[9];
-    grad_from<float>(acc[0], g);
     r[0] = acc[0][0]; r[1] = acc[0][1]; r[2] = acc[0][2];
+    if (GRAD) {
+      float g[9];
+      grad_from<float>(acc[0], g);
 #pragma unroll
-    for (int c = 0; c < 9; ++c) r[3 + c] = g[c];
+      for (int c = 0; c < 9; ++c) r[3 + c] = g[c];
+    }
   }
 }
 
 // persistent: every workgroup takes items from the queue until none is left
-template <int CORE, int PREC>
+template <int CORE, bool GRAD, int PREC>
 __global__ __launch_bounds__(256) void k_ff_near(FFArgs a) {
   extern __shared__ float4 sh[];
   __shared__ int s_item;
@@ -1017,46 +1062,50 @@ __global__ __launch_bounds__(256) void k_ff_near(FFArgs a) {
     const int nnb = a.nn[b];
     const int r1 = r0 + m < nnb ? r0 + m : nnb;
     double r[12];
-    near_item<CORE, PREC>(a, b, r0, r1, sh, r);
-    double* slot = a.part + (int64_t)item * 12 * FF_TB;
+    near_item<CORE, GRAD, PREC>(a, b, r0, r1, sh, r);
+    constexpr int NOUT = GRAD ? 12 : 3;
+    double* slot = a.part + (int64_t)item * NOUT * FF_TB;
 #pragma unroll
-    for (int c = 0; c < 12; ++c) slot[c * FF_TB + threadIdx.x] = r[c];
+    for (int c = 0; c < NOUT; ++c) slot[c * FF_TB + threadIdx.x] = r[c];
   }
 }
 
 // one workgroup per block: near partials in item order, far part, self-pair
 // exclusion, then accumulate into the caller's arrays at the original index
-template <int CORE, int PREC>
+template <int CORE, bool GRAD>
 __global__ __launch_bounds__(256) void k_ff_combine(FFArgs a) {
+  constexpr int NOUT = GRAD ? 12 : 3;
   const int64_t b = blockIdx.x;
   const int64_t i = b * FF_TB + threadIdx.x;
   if (i >= a.nt) return;
-  double r[12];
+  double r[NOUT];
 #pragma unroll
-  for (int c = 0; c < 12; ++c) r[c] = a.farv[(int64_t)c * a.nt + i];
+  for (int c = 0; c < NOUT; ++c) r[c] = a.farv[(int64_t)c * a.nt + i];
   for (int y = 1; y < a.nslice; ++y) {
 #pragma unroll
-    for (int c = 0; c < 12; ++c) r[c] += a.farv[((int64_t)y * 12 + c) * a.nt + i];
+    for (int c = 0; c < NOUT; ++c) r[c] += a.farv[((int64_t)y * NOUT + c) * a.nt + i];
   }
   const int n_it = a.items[b], off = a.ioff[b];
   for (int k = 0; k < n_it; ++k) {
-    const double* slot = a.part + (int64_t)(off + k) * 12 * FF_TB;
+    const double* slot = a.part + (int64_t)(off + k) * NOUT * FF_TB;
 #pragma unroll
-    for (int c = 0; c < 12; ++c) r[c] += slot[c * FF_TB + threadIdx.x];
+    for (int c = 0; c < NOUT; ++c) r[c] += slot[c * FF_TB + threadIdx.x];
   }
   const int io = a.tperm[i];
-  if (a.self_excl) {
-    // the self pair entered only W (velocity and dyad vanish at d = 0)
-    float ks, Bp;
-    kb<CORE>(0.0f, core_term<CORE>(a.s.r[io]) + a.tq[i].w, 0.0f, ks, Bp);
-    const double kx = (double)ks * a.s.ax[io], ky = (double)ks * a.s.ay[io], kz = (double)ks * a.s.az[io];
-    r[4] -= kz; r[5] += ky; r[6] += kz; r[8] -= kx; r[9] -= ky; r[10] += kx;
-  }
   a.t.u[io] = (float)((double)a.t.u[io] + r[0]);
   a.t.v[io] = (float)((double)a.t.v[io] + r[1]);
   a.t.w[io] = (float)((double)a.t.w[io] + r[2]);
+  if constexpr (GRAD) {
+    if (a.self_excl) {
+      // the self pair entered only W (velocity and dyad vanish at d = 0)
+      float ks, Bp;
+      kb<CORE>(0.0f, core_term<CORE>(a.s.r[io]) + a.tq[i].w, 0.0f, ks, Bp);
+      const double kx = (double)ks * a.s.ax[io], ky = (double)ks * a.s.ay[io], kz = (double)ks * a.s.az[io];
+      r[4] -= kz; r[5] += ky; r[6] += kz; r[8] -= kx; r[9] -= ky; r[10] += kx;
+    }
 #pragma unroll
-  for (int c = 0; c < 9; ++c) a.t.g[c][io] = (float)((double)a.t.g[c][io] + r[3 + c]);
+    for (int c = 0; c < 9; ++c) a.t.g[c][io] = (float)((double)a.t.g[c][io] + r[3 + c]);
+  }
 }
 
 // number of (target, source) pairs the far-field kernel takes: one thread per block

@@ -30,12 +30,14 @@ int check_opts(const o3d_opts* o);
 // host-memory panels: every node index below nn (device panels are the caller's to keep in range)
 int check_node_indices(const o3d_panels* p, const char* what);
 void fill_stats(o3d_stats* stats, double secs, double flops, double inter);
+// method FACTORED serves it; method AUTO may take the factored path for it
 bool ff_supported(int core, bool grad, int prec);
+bool ff_auto_supported(int core, bool grad, int prec);
 int p2p_factored(const o3d_points* src, o3d_points* targ, const o3d_opts* o, hipStream_t st,
                  o3d_factored_profile* prof = nullptr);
 int p2p_factored_ws(const o3d_points* src, o3d_points* targ, const o3d_opts* o, hipStream_t st, void* ws,
                     size_t ws_bytes);
-size_t ff_workspace_bytes(int64_t ns, int64_t nt, bool same, int tile);
+size_t ff_workspace_bytes(int64_t ns, int64_t nt, bool same, int tile, bool grad = true);
 // sources and targets are one collection (the factored method sorts it once)
 bool ff_same_points(const o3d_points* src, const o3d_points* targ);
 // one growable device workspace per stream (calls on a stream are ordered, so they

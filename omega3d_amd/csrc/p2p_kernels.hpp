@@ -179,7 +179,8 @@ __device__ __forceinline__ void kb_d(float dx, float dy, float dz, float st, flo
       const float top = fmaf(1.5f, st, dd);
       const float dn5 = ir2 * ir2 * ir;
       K = top * dn5;
-      Bp = dn5 * fmaf((float)(5.0 / 3.0), top * ir2, (float)(-2.0 / 3.0));
+      // (5 top / dd - 2) / 3 with top = dd + 1.5 st, without its difference of near numbers
+      Bp = dn5 * fmaf(2.5f * st, ir2, 1.0f);
     }
   } else {
     kb<CORE>(fmaf(dz, dz, fmaf(dy, dy, dx * dx)), st, thr, K, Bp);

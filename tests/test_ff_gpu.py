@@ -219,3 +219,31 @@ def test_factored_negation_and_zero_strengths(infl, core, n):
     sel = _sel(p.n, 512)
     ov, og = oracle.p2p(core, p.pos, st, p.rad, p.pos[:, sel], p.rad[sel], True, "f64")
     assert rel_errors(v[:, sel], ov)[0] <= 2e-6 and rel_errors(g[:, sel], og)[0] <= 2e-6
+
+
+@pytest.mark.parametrize("core,grads", [("wl", True), ("v2", True), ("rm", False), ("wl", False), ("exp", False),
+                                        ("v2", False)])
+@pytest.mark.parametrize("ns,nt", [(65536, 65536), (66001, 70017)])
+def test_auto_takes_far_tiles_of_other_cores_and_velocities(infl, core, grads, ns, nt):
+    """AUTO at 65,536 and more, compensated: the two-weight form (WL, V2 with gradient) and
+    the velocity form, on one collection with varied core radii and on point targets of
+    another: within 2e-6 of the oracle and of the direct method, other bits than the
+    direct method's, and the self pair left out where asked."""
+    same = ns == nt
+    c = scenes.colliding_rings(n_each=(ns + 1) // 2, sigma=0.03)
+    rad = (c.rad * np.linspace(0.7, 1.3, c.n)[np.random.default_rng(2).permutation(c.n)]).astype(np.float32)[:ns]
+    pos, st = c.pos[:, :ns], c.str[:, :ns]
+    tp = pos if same else scenes.ring(nt, R=1.2, a=0.4, seed=9).pos
+    tr = rad if same else None
+    print(f"case: {core} grads={grads} ns={ns} nt={nt}", flush=True)
+    args = (core, pos, st, rad, tp, tr, grads, "comp")
+    v, g = infl.p2p(*args, self_term=int(same))
+    vd, gd = infl.p2p(*args, self_term=int(same), method="direct")
+    sel = _sel(tp.shape[1], 512)
+    ov, og = oracle.p2p(core, pos, st, rad, tp[:, sel], None if tr is None else tr[sel], grads, "f64")
+    assert rel_errors(v[:, sel], ov)[0] <= 2e-6 and rel_errors(v, vd)[0] <= 2e-6
+    assert not np.array_equal(v, vd)
+    if grads:
+        if same:
+            og = og - self_term_gradient(core, st[:, sel], rad[sel])
+        assert rel_errors(g[:, sel], og)[0] <= 2e-6 and rel_errors(g, gd)[0] <= 2e-6
