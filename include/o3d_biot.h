@@ -70,6 +70,9 @@ enum o3d_self { O3D_SELF_INCLUDE = 0, O3D_SELF_EXCLUDE = 1 };
  *             alone to the matrix cores as well, at the same counts.
  * For panel sources (o3d_panels_affect_points[_dev]) the field selects the rule:
  *   AUTO / DIRECT:      the reference's recursive centroid rule (Kernels.h:1028-1211);
+ *             AUTO takes the separated pairs of large calls with tile 0, of both rules
+ *             and of particles on panels, to the matrix cores (the same decision for
+ *             every pair);
  *   O3D_PANEL_GAUSS7:   no counterpart in the reference -- per (target, panel) pair a
  *             7-point degree-5 rule (Strang & Fix; Dunavant) when the target is at
  *             least twice the panel's longest edge from its centroid, otherwise the

@@ -28,20 +28,6 @@ struct Work {
 std::mutex g_ws_mu;
 std::map<hipStream_t, Work> g_ws;
 
-// sequential sub-allocation of the workspace, 256-byte aligned
-struct Carve {
-  char* base;
-  size_t off = 0;
-  template <class T>
-  T* take(size_t count) {
-    T* p = base ? reinterpret_cast<T*>(base + off) : nullptr;
-    off += (count * sizeof(T) + 255) & ~(size_t)255;
-    return p;
-  }
-};
-
-unsigned grid_of(int64_t n, int per) { return (unsigned)std::max<int64_t>(1, (n + per - 1) / per); }
-
 // workgroups of the persistent near-field kernel: every slot of every CU
 template <int CORE, bool GRAD, int PREC>
 int64_t near_grid(size_t lds) {
@@ -50,13 +36,6 @@ int64_t near_grid(size_t lds) {
       per_cu < 1)
     per_cu = 1;
   return (int64_t)per_cu * num_cus();
-}
-
-// LDS of the far-field kernel: r2 slots, moment tables, a tile's rows, core terms
-template <int CORE, bool GRAD>
-constexpr size_t ff_far_lds() {
-  return (size_t)256 * FF_SL * sizeof(__bf16) + (size_t)2 * ff_rows<ff_form<CORE, GRAD>()>() * FF_TP * sizeof(_Float16) +
-         512 * sizeof(float4) + (CORE == CORE_WL || CORE == CORE_V2 ? 256 * sizeof(float) : 0);
 }
 
 // RAII pair of events for the optional stage timing
@@ -86,18 +65,6 @@ struct Layout {
   size_t bytes;
 };
 
-// Near-field items per block: about 4,096 in all, three rounds of the workgroups that the
-// GPU holds (an item of FF_M0 tiles is 262,144 pairs), and at least 2 per block
-int near_split(int64_t nb) { return (int)std::max<int64_t>(2, std::min<int64_t>(16, 4096 / nb)); }
-
-// Slices of the far field: blocks x slices workgroups, at least about four rounds of the
-// two that a CU holds, so that the last round is short beside the whole and few blocks
-// (a collection of 65,536: 256) still fill every slot.
-int far_slices(int64_t nb, int64_t mwords) {
-  const int64_t want = (8 * (int64_t)num_cus() + nb - 1) / nb;
-  return (int)std::max<int64_t>(1, std::min<int64_t>({want, mwords, 8}));
-}
-
 Layout layout(char* base, int64_t ns, int64_t nt, bool same, int T, size_t tmp_bytes, int nout) {
   const int64_t nb = (nt + FF_TB - 1) / FF_TB;
   const int64_t ntiles = (ns + T - 1) / T;
@@ -124,7 +91,7 @@ Layout layout(char* base, int64_t ns, int64_t nt, bool same, int T, size_t tmp_b
   L.bsph = cv.take<float4>(nb);
   L.bcs = cv.take<float>(nb);
   L.mask = cv.take<unsigned>((size_t)(nb * mwords));
-  L.farv = cv.take<double>((size_t)nout * far_slices(nb, mwords) * nt);
+  L.farv = cv.take<double>((size_t)nout * far_slices(nb, mwords, num_cus()) * nt);
   L.npair = cv.take<unsigned long long>(1);
   L.nn = cv.take<int>(nb);
   L.noff = cv.take<int>(nb);
@@ -222,7 +189,7 @@ int run(const o3d_points* src, o3d_points* targ, bool self_excl, int T, hipStrea
   a.ns = ns; a.nt = nt;
   a.tile = T; a.mwords = mwords; a.ntiles = ntiles;
   a.self_excl = self_excl ? 1 : 0;
-  const int nslice = far_slices(nb, mwords);
+  const int nslice = far_slices(nb, mwords, num_cus());
   a.wslice = (mwords + nslice - 1) / nslice;
   a.nslice = (mwords + a.wslice - 1) / a.wslice;
   const size_t lds_far = ff_far_lds<CORE, GRAD>();

@@ -43,6 +43,7 @@
 #pragma once
 #include "p2p_kernels.hpp"
 
+#include <algorithm>
 #include <type_traits>
 
 // the far field's schedule of one phase (k_ff_far): n matrix products, each followed by
@@ -61,6 +62,9 @@ typedef float f32x16 __attribute__((ext_vector_type(16)));
 typedef _Float16 f16x8 __attribute__((ext_vector_type(8)));
 typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
 
+// the singular kernel of panel points: K = r^-3, Bp = r^-5, no core terms; the core term
+// of a row is the distance from there beyond which a pair is a plain point pair
+constexpr int CORE_SING = 0;
 constexpr int FF_TB = 256;          // targets per workgroup: 4 waves x 64
 constexpr float FF_KAPPA = 1.0f;    // minimum gap, in block radii
 // near field, compensated: sources per FP32 partial.  Gradient error against FP64 on two
@@ -77,16 +81,16 @@ constexpr int FF_SL = 40;           // far field: LDS row of a source's BF16 r2 
 // velocity error 4.5e-8 at 8 tiles, 4.2e-8 at 4; far field 20.2 and 20.5 ms.
 // Cores that the direct kernel sums otherwise (4.6e-8): 2
 template <int CORE, bool GRAD>
-constexpr int ff_merge() { return GRAD && (CORE == CORE_RM || CORE == CORE_EXP) ? 4 : 2; }
+constexpr int ff_merge() { return GRAD && (CORE == CORE_RM || CORE == CORE_EXP || CORE == CORE_SING) ? 4 : 2; }
 
 struct FFArgs {
   const float4* sp;    // sorted sources {x, y, z, core_term}, up to a whole tile: the last one again
-  const float4* sa;    // sorted sources {ax, ay, az, 0}, up to a whole tile: zeros
+  const float4* sa;    // sorted sources {ax, ay, az, q}, up to a whole tile: zeros (q: source strength of panels, or 0)
   const float4* tq;    // sorted targets {x, y, z, core_term or 0 for point targets}
   const int* tperm;    // sorted target -> original target index
   const float4* tsph;  // per source tile: bounding sphere {cx, cy, cz, r}
   const float* tcs;    // per source tile: largest core term
-  const float* tam;    // per source tile: largest |alpha|
+  const float* tam;    // per source tile: largest |alpha| and |q|
   const float4* bsph;  // per target block: bounding sphere
   const float* bcs;    // per target block: largest core term
   const unsigned* mask;  // far bit per (block, tile), mwords words per block
@@ -118,7 +122,7 @@ __device__ __forceinline__ float fdec(unsigned e) {
   return __uint_as_float((e & 0x80000000u) ? (e & 0x7fffffffu) : ~e);
 }
 
-__global__ void k_ff_bbox_init(unsigned* bb) {
+static __global__ void k_ff_bbox_init(unsigned* bb) {
   if (threadIdx.x < 3) bb[threadIdx.x] = 0xffffffffu;
   else if (threadIdx.x < 6) bb[threadIdx.x] = 0u;
 }
@@ -128,7 +132,7 @@ __global__ void k_ff_bbox_init(unsigned* bb) {
 // issues 6 atomics, so a launch of FF_BBOX_GRID workgroups makes few atomics on
 // the 6 shared words (one per wave took ~0.5 ms at N = 1M).
 constexpr unsigned FF_BBOX_GRID = 512;
-__global__ __launch_bounds__(256) void k_ff_bbox(const float* x, const float* y, const float* z, int64_t n,
+static __global__ __launch_bounds__(256) void k_ff_bbox(const float* x, const float* y, const float* z, int64_t n,
                                                  unsigned* bb) {
   __shared__ float red[4][6];
   float lo[3] = {__builtin_huge_valf(), __builtin_huge_valf(), __builtin_huge_valf()};
@@ -172,7 +176,7 @@ __device__ __forceinline__ unsigned spread10(unsigned v) {
 }
 
 // 30-bit Morton keys on the common bounding box, and the identity permutation
-__global__ __launch_bounds__(256) void k_ff_keys(const float* x, const float* y, const float* z, int64_t n,
+static __global__ __launch_bounds__(256) void k_ff_keys(const float* x, const float* y, const float* z, int64_t n,
                                                  const unsigned* bb, unsigned* keys, int* idx) {
   const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
   if (i >= n) return;
@@ -221,10 +225,10 @@ __device__ __forceinline__ float wg_max(float v, float* red) {
 __device__ __forceinline__ float wg_min(float v, float* red) { return -wg_max(-v, red); }
 
 // bounding sphere (bbox centre, largest distance), largest core term and (when pa
-// is given) largest |alpha| and the sign of the first nonzero strength (0: none), by
+// is given) a bound of |alpha| and |q| and the sign of the first nonzero strength (0: none), by
 // its first nonzero component, of each group of `group` consecutive sorted points; one
 // workgroup per group
-__global__ __launch_bounds__(256) void k_ff_bounds(const float4* p, const float4* pa, int64_t n, int group,
+static __global__ __launch_bounds__(256) void k_ff_bounds(const float4* p, const float4* pa, int64_t n, int group,
                                                    float4* sph, float* cs, float* amax, float* sign) {
   __shared__ float red[4];
   __shared__ unsigned lead;   // smallest 2 i + (negative) over the group's points i with a strength
@@ -256,20 +260,20 @@ __global__ __launch_bounds__(256) void k_ff_bounds(const float4* p, const float4
     r2 = fmaxf(r2, fmaf(dz, dz, fmaf(dy, dy, dx * dx)));
   }
   r2 = wg_max(r2, red);
-  float a2 = 0.0f;
+  float am = 0.0f;   // largest component: no square that could leave the range
   if (pa)
     for (int64_t i = b0 + threadIdx.x; i < b1; i += blockDim.x) {
       const float4 q = pa[i];
-      a2 = fmaxf(a2, fmaf(q.z, q.z, fmaf(q.y, q.y, q.x * q.x)));
-      const float f = q.x != 0.0f ? q.x : q.y != 0.0f ? q.y : q.z;
+      am = fmaxf(fmaxf(fmaxf(am, fabsf(q.x)), fmaxf(fabsf(q.y), fabsf(q.z))), fabsf(q.w));
+      const float f = q.x != 0.0f ? q.x : q.y != 0.0f ? q.y : q.z != 0.0f ? q.z : q.w;
       if (f != 0.0f) atomicMin(&lead, 2u * (unsigned)(i - b0) + (f < 0.0f ? 1u : 0u));
     }
-  a2 = wg_max(a2, red);   // its barriers order the atomics too
+  am = wg_max(am, red);   // its barriers order the atomics too
   if (threadIdx.x == 0) {
     // margin for the rounding of the distances above
     sph[blockIdx.x] = make_float4(c[0], c[1], c[2], __fsqrt_rn(r2) * 1.00001f + 1e-30f);
     cs[blockIdx.x] = cmax;
-    if (amax) amax[blockIdx.x] = __fsqrt_rn(a2) * 1.00001f;
+    if (amax) amax[blockIdx.x] = am * 1.7321f;   // sqrt 3, rounded up
     if (sign) sign[blockIdx.x] = lead == 0xffffffffu ? 0.0f : (lead & 1u) ? -1.0f : 1.0f;
   }
 }
@@ -294,6 +298,7 @@ __global__ __launch_bounds__(256) void k_ff_classify(const float4* bsph, const f
     const float gap = __fsqrt_rn(fmaf(dz, dz, fmaf(dy, dy, dx * dx))) - cb.w - ct.w;
     bool far = gap > 0.0f && gap > FF_KAPPA * cb.w;
     if (CORE == CORE_EXP) far = far && gap * gap > exp_threshold(csb + tcs[ti]);
+    if (CORE == CORE_SING) far = far && gap > fmaxf(csb, tcs[ti]);
     if (far) bits |= 1u << k;
   }
   mask[g] = bits;
@@ -363,34 +368,74 @@ __device__ __forceinline__ void ff_epilogue_k(const double* k, const double* c, 
   grad_from<double>(a, out + 3);
 }
 
+// ... and for panels with source strengths q: K sums of alpha 0-2, m 3-5, q 6, q s' 7-9,
+// Bp sums of these and of s' x alpha 10-18, s' x m 19-26, q s' s' 27-31 (00, 01, 02, 11,
+// 12).  With X_ij = sum Bp q d_i d_j, whose trace is sum K q: u += sum K q d and
+// g_ji += -3 X_ji + delta_ji sum K q
+template <bool GRAD>
+__device__ __forceinline__ void ff_epilogue_sheet(const double* k, const double* c, double tx, double ty, double tz,
+                                                  double* out) {
+  const double t[3] = {tx, ty, tz};
+  if (GRAD) {
+    double p[23];   // the vortex part's own columns
+#pragma unroll
+    for (int i = 0; i < 23; ++i) p[i] = c[i < 6 ? i : i + 4];
+    ff_epilogue_k<true>(k, p, tx, ty, tz, out);
+    const double X00 = t[0] * t[0] * c[6] - 2.0 * t[0] * c[7] + c[27];
+    const double X01 = t[0] * t[1] * c[6] - t[0] * c[8] - t[1] * c[7] + c[28];
+    const double X02 = t[0] * t[2] * c[6] - t[0] * c[9] - t[2] * c[7] + c[29];
+    const double X11 = t[1] * t[1] * c[6] - 2.0 * t[1] * c[8] + c[30];
+    const double X12 = t[1] * t[2] * c[6] - t[1] * c[9] - t[2] * c[8] + c[31];
+    const double X22 = k[6] - X00 - X11;
+    out[3] += k[6] - 3.0 * X00; out[4] -= 3.0 * X01; out[5] -= 3.0 * X02;
+    out[6] -= 3.0 * X01; out[7] += k[6] - 3.0 * X11; out[8] -= 3.0 * X12;
+    out[9] -= 3.0 * X02; out[10] -= 3.0 * X12; out[11] += k[6] - 3.0 * X22;
+  } else {
+    ff_epilogue_k<false>(k, c, tx, ty, tz, out);
+  }
+#pragma unroll
+  for (int d = 0; d < 3; ++d) out[d] += k[6] * t[d] - k[7 + d];
+}
+
 // ---- far field: the three forms ------------------------------------------------
 // FF_B: one weight per pair, Bp; K comes back as Bp r2 (RM and EXP with gradient).
 // FF_K: one weight, K, and the velocity alone.
-// FF_KB: both weights, for the cores whose K is no product of Bp with r2 (WL, V2).
+// FF_KB: both weights, for the cores whose K is no product of Bp with r2 (WL, V2), and for
+// panels with source strengths (SHEET), whose moments fill the 32 rows with K beside them.
 enum { FF_B = 0, FF_K = 1, FF_KB = 2 };
-template <int CORE, bool GRAD>
+template <int CORE, bool GRAD, bool SHEET>
 constexpr int ff_form() {
-  return !GRAD ? FF_K : (CORE == CORE_RM || CORE == CORE_EXP ? FF_B : FF_KB);
+  return !GRAD ? FF_K : SHEET || CORE == CORE_WL || CORE == CORE_V2 ? FF_KB : FF_B;
 }
 // columns of the moment table (rows of the matrix product):
 //   FF_B   alpha 0-2, m 3-5, s' x alpha 6-14, s' x m 15-22, b alpha 23-25, b m 26-28
-//   FF_KB  the first 23 (K multiplies alpha and m, Bp all of them)
-//   FF_K   alpha and m, in 16 rows of leading parts and 16 rows of remainders
-template <int FORM>
-constexpr int ff_cols() { return FORM == FF_B ? 29 : FORM == FF_KB ? 23 : 6; }
+//   FF_KB  the first 23 (K multiplies alpha and m, Bp all of them); SHEET: ff_epilogue_sheet
+//   FF_K   what K multiplies, in 16 rows of leading parts and 16 rows of remainders
+template <int FORM, bool SHEET>
+constexpr int ff_cols() { return FORM == FF_B ? 29 : FORM == FF_KB ? (SHEET ? 32 : 23) : (SHEET ? 10 : 6); }
 template <int FORM>
 constexpr int ff_rows() { return FORM == FF_K ? 16 : 32; }
 
-// moment column -> scale group: alpha (0), m and s' alpha (1), s' m (2), b alpha (3),
-// b m (4); padding columns hold zeros
+// moment column -> scale group: alpha and q (0), m, s' alpha and q s' (1), s' m and q s' s'
+// (2), b alpha (3), b m (4); padding columns hold zeros
+template <bool SHEET>
 __host__ __device__ constexpr int ff_group(int col) {
+  if (SHEET) return col < 3 || col == 6 ? 0 : col < 19 ? 1 : 2;
   return col < 3 ? 0 : col < 15 ? 1 : col < 23 ? 2 : col < 26 ? 3 : 4;
 }
 
-// column c of one source: alpha a, s' s, m = alpha x s', b
-__device__ __forceinline__ float ff_column(int c, const float* a, const float* s, const float* m, float b) {
+// column c of one source: alpha a, q, s' s, m = alpha x s', b
+template <bool SHEET>
+__device__ __forceinline__ float ff_column(int c, const float* a, float q, const float* s, const float* m, float b) {
   if (c < 3) return a[c];
   if (c < 6) return m[c - 3];
+  if (SHEET) {
+    if (c == 6) return q;
+    if (c < 10) return q * s[c - 7];
+    if (c < 19) return s[(c - 10) / 3] * a[(c - 10) % 3];
+    if (c < 27) return s[(c - 19) / 3] * m[(c - 19) % 3];
+    return q * s[c < 30 ? 0 : 1] * s[c < 30 ? c - 27 : c - 29];
+  }
   if (c < 15) return s[(c - 6) / 3] * a[(c - 6) % 3];
   if (c < 23) return s[(c - 15) / 3] * m[(c - 15) % 3];
   if (c < 26) return b * a[c - 23];
@@ -448,11 +493,12 @@ __device__ __forceinline__ int ff_quad_slot(int q) { return 16 * (q >> 2) + 8 * 
 // tau (WL, V2): the pair's scaled core term
 template <int CORE, int FORM>
 __device__ __forceinline__ void ff_weights(float r, float tau, float& K, float& Bp) {
-  if (CORE == CORE_RM || CORE == CORE_EXP) {
+  if (CORE == CORE_RM || CORE == CORE_EXP || CORE == CORE_SING) {
     const float ir = frsq(r);
     const float ir2 = ir * ir;
-    if (FORM == FF_K) K = ir2 * ir;
-    else Bp = (ir2 * ir2) * ir;
+    if (FORM != FF_B) K = ir2 * ir;
+    if (FORM == FF_KB) Bp = K * ir2;
+    if (FORM == FF_B) Bp = (ir2 * ir2) * ir;
   } else if (CORE == CORE_WL) {     // CoreFunc.h:265-274 with D = rho^2 + tau = r
     const float ir = frsq(r);
     const float ir2 = ir * ir;
@@ -529,10 +575,11 @@ __device__ __forceinline__ void ff_load_lds16(const float4* src, float4* dst) {
 // takes 64.5, the twelve alone 57: this loop runs at 69.  The tile's tables cost about
 // 200 vector instructions per wave, the loop 1,700; what a run (ff_fold and the target
 // slots) costs is shared by ff_merge tiles.
-template <int CORE, bool GRAD>
+template <int CORE, bool GRAD, bool SHEET = false>
 __global__ __launch_bounds__(FF_FAR_THREADS, 2) void k_ff_far(FFArgs a) {
-  constexpr int FORM = ff_form<CORE, GRAD>();
-  constexpr int ROWS = ff_rows<FORM>(), COLS = ff_cols<FORM>();
+  constexpr int FORM = ff_form<CORE, GRAD, SHEET>();
+  constexpr int ROWS = ff_rows<FORM>(), COLS = ff_cols<FORM, SHEET>();
+  constexpr int KCOLS = SHEET ? 10 : 6;   // of them, the first KCOLS take K
   constexpr bool HASB = FORM != FF_K, HASK = FORM != FF_B;
   constexpr bool TAU = CORE == CORE_WL || CORE == CORE_V2;
   constexpr bool COREA = CORE == CORE_RM || CORE == CORE_WL;   // core terms are part of r2
@@ -563,7 +610,7 @@ __global__ __launch_bounds__(FF_FAR_THREADS, 2) void k_ff_far(FFArgs a) {
     i = i < a.nt ? i : a.nt - 1;
     const float4 q = a.tq[i];
     tx[s] = q.x - cb.x; ty[s] = q.y - cb.y; tz[s] = q.z - cb.z;
-    tt[s] = CORE == CORE_EXP ? 0.0f : q.w;
+    tt[s] = COREA || TAU ? q.w : 0.0f;
     al[s] = fmaf(tz[s], tz[s], fmaf(ty[s], ty[s], fmaf(tx[s], tx[s], COREA ? tt[s] : 0.0f)));
   }
   f32x16 accB[2], accK[2], accR[2];
@@ -614,16 +661,17 @@ __global__ __launch_bounds__(FF_FAR_THREADS, 2) void k_ff_far(FFArgs a) {
           for (int r = 0; r < 16; ++r) accB[s][r] += accR[s][r];
       rows_of(accB, c);
 #pragma unroll
-      for (int i = 0; i < COLS; ++i) c[i] *= sc[ff_group(i)] * wb;
+      for (int i = 0; i < COLS; ++i) c[i] *= sc[ff_group<SHEET>(i)] * wb;
     }
     if (HASK) {
       // 2^(-3 jw / 2)
       const double wk = ldexp(jw & 1 ? 0.70710678118654752440 : 1.0, -jw - (jw >> 1)) * ff_mean_k<CORE>();
       rows_of(accK, ck);
 #pragma unroll
-      for (int i = 0; i < 6; ++i) ck[i] = (ck[i] + ck[16 + i]) * (sc[ff_group(i)] * wk);
+      for (int i = 0; i < KCOLS; ++i) ck[i] = (ck[i] + ck[16 + i]) * (sc[ff_group<SHEET>(i)] * wk);
     }
-    if constexpr (FORM == FF_B) ff_epilogue(c, ox, oy, oz, oa, out);
+    if constexpr (SHEET) ff_epilogue_sheet<GRAD>(ck, c, ox, oy, oz, out);
+    else if constexpr (FORM == FF_B) ff_epilogue(c, ox, oy, oz, oa, out);
     else ff_epilogue_k<GRAD>(ck, c, ox, oy, oz, out);
     if constexpr (INMEM) {
       if (own < a.nt) {
@@ -724,13 +772,16 @@ __global__ __launch_bounds__(FF_FAR_THREADS, 2) void k_ff_far(FFArgs a) {
       const float lgap = __builtin_amdgcn_logf(fmaxf(dc - cb.w - ct.w, 1e-37f));   // gap > 0 for a far tile
       const float rs = dc + ct.w;                                                // |s'| bound
       const float lrs = __builtin_amdgcn_logf(rs);
-      const float lam = fmaxf(__builtin_amdgcn_logf(a.tam[t]), -100.0f);
+      // strengths by exponent and mantissa, so that scaling all by a power of two moves the
+      // scales by just that and the results with them, exactly
+      int ea;
+      const float lam = __builtin_amdgcn_logf(fmaxf(frexpf(a.tam[t], &ea), 0.5f));
       const float lbm = __builtin_amdgcn_logf(fmaf(rs, rs, COREA ? a.tcs[t] : 0.0f));
       const float top = (TAU ? 11.0f : 13.0f) * (HASB ? 1.0f / 5.0f : 1.0f / 3.0f);
       const float lg[5] = {lam, lam + lrs, lam + 2.0f * lrs, lam + lbm, lam + lbm + lrs};
       int wg[5];
 #pragma unroll
-      for (int g = 0; g < 5; ++g) wg[g] = (int)fminf(fmaxf(floorf(13.0f - lg[g]), -110.0f), 110.0f) & 255;
+      for (int g = 0; g < 5; ++g) wg[g] = (int)fminf(fmaxf(floorf(13.0f - lg[g]) - (float)ea, -126.0f), 126.0f) & 255;
       pk0 = ((int)floorf(2.0f * (lgap + top)) << 16) | (wg[1] << 8) | wg[0];
       pk1 = (wg[4] << 16) | (wg[3] << 8) | wg[2];
     }
@@ -811,10 +862,11 @@ __global__ __launch_bounds__(FF_FAR_THREADS, 2) void k_ff_far(FFArgs a) {
             const float s[3] = {P.x - cb.x, P.y - cb.y, P.z - cb.z};
             const float b = fmaf(s[2], s[2], fmaf(s[1], s[1], fmaf(s[0], s[0], COREA ? P.w : 0.0f)));
             // strengths take their group's power of two first: exact, one product per group and component
-            float al3[NG][3], m[NG][3];
+            float al3[NG][3], m[NG][3], qs[NG];
 #pragma unroll
             for (int g = 0; g < NG; ++g) {
               const float ax = A.x * gs[g], ay = A.y * gs[g], az = A.z * gs[g];
+              qs[g] = SHEET ? A.w * gs[g] : 0.0f;
               al3[g][0] = ax; al3[g][1] = ay; al3[g][2] = az;
               m[g][0] = fmaf(ay, s[2], -az * s[1]);
               m[g][1] = fmaf(az, s[0], -ax * s[2]);
@@ -823,8 +875,8 @@ __global__ __launch_bounds__(FF_FAR_THREADS, 2) void k_ff_far(FFArgs a) {
 #pragma unroll
             for (int c = 0; c < CW; ++c) {
               constexpr int last = COLS - 1;
-              const int cc = C0 + c < COLS ? C0 + c : last, g = ff_group(cc);
-              cv[c][u] = C0 + c < COLS ? ff_column(cc, al3[g], s, m[g], b) : 0.0f;
+              const int cc = C0 + c < COLS ? C0 + c : last, g = ff_group<SHEET>(cc);
+              cv[c][u] = C0 + c < COLS ? ff_column<SHEET>(cc, al3[g], qs[g], s, m[g], b) : 0.0f;
             }
           }
           const int pos = ff_quad_slot(lane);
@@ -941,7 +993,7 @@ __device__ __forceinline__ int near_tiles_of(const unsigned* mrow, int mwords, i
 }
 
 // nn[b] = number of near tiles of block b
-__global__ __launch_bounds__(256) void k_ff_plan_count(const unsigned* mask, int64_t nb, int mwords, int ntiles,
+static __global__ __launch_bounds__(256) void k_ff_plan_count(const unsigned* mask, int64_t nb, int mwords, int ntiles,
                                                        int* nn) {
   const int64_t b = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
   if (b < nb) nn[b] = near_tiles_of(mask + b * mwords, mwords, ntiles);
@@ -949,7 +1001,7 @@ __global__ __launch_bounds__(256) void k_ff_plan_count(const unsigned* mask, int
 
 // after the exclusive scan noff of nn: M = max(FF_M0, ceil(total / (split nb))) and the
 // item count of every block (at most (split + 1) nb items in all)
-__global__ __launch_bounds__(256) void k_ff_plan_items(const int* nn, const int* noff, int64_t nb, int split,
+static __global__ __launch_bounds__(256) void k_ff_plan_items(const int* nn, const int* noff, int64_t nb, int split,
                                                        int* items, int* mfold) {
   const int64_t b = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
   const int64_t total = (int64_t)noff[nb - 1] + nn[nb - 1];
@@ -959,7 +1011,7 @@ __global__ __launch_bounds__(256) void k_ff_plan_items(const int* nn, const int*
   if (b < nb) items[b] = (int)((nn[b] + m - 1) / m);
 }
 
-__global__ void k_ff_zero_u32(unsigned* p) {
+static __global__ void k_ff_zero_u32(unsigned* p) {
   if (threadIdx.x == 0) *p = 0u;
 }
 
@@ -1109,7 +1161,7 @@ __global__ __launch_bounds__(256) void k_ff_combine(FFArgs a) {
 }
 
 // number of (target, source) pairs the far-field kernel takes: one thread per block
-__global__ __launch_bounds__(256) void k_ff_count(const unsigned* mask, int64_t nb, int mwords, int ntiles, int T,
+static __global__ __launch_bounds__(256) void k_ff_count(const unsigned* mask, int64_t nb, int mwords, int ntiles, int T,
                                                   int64_t ns, int64_t nt, unsigned long long* out) {
   const int64_t b = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
   if (b >= nb) return;
@@ -1127,8 +1179,45 @@ __global__ __launch_bounds__(256) void k_ff_count(const unsigned* mask, int64_t 
   atomicAdd(out, sum);
 }
 
-__global__ void k_ff_zero_u64(unsigned long long* p) {
+static __global__ void k_ff_zero_u64(unsigned long long* p) {
   if (threadIdx.x == 0) *p = 0ull;
 }
+
+// ---- host side shared by the factored calls ----------------------------------------
+
+// sequential sub-allocation of a workspace, 256-byte aligned
+struct Carve {
+  char* base;
+  size_t off = 0;
+  template <class T>
+  T* take(size_t count) {
+    T* p = base ? reinterpret_cast<T*>(base + off) : nullptr;
+    off += (count * sizeof(T) + 255) & ~(size_t)255;
+    return p;
+  }
+};
+
+inline unsigned grid_of(int64_t n, int per) { return (unsigned)std::max<int64_t>(1, (n + per - 1) / per); }
+
+// LDS of the far-field kernel: r2 slots, moment tables, a tile's rows, core terms
+template <int CORE, bool GRAD, bool SHEET = false>
+constexpr size_t ff_far_lds() {
+  return (size_t)256 * FF_SL * sizeof(__bf16) +
+         (size_t)2 * ff_rows<ff_form<CORE, GRAD, SHEET>()>() * FF_TP * sizeof(_Float16) + 512 * sizeof(float4) +
+         (CORE == CORE_WL || CORE == CORE_V2 ? 256 * sizeof(float) : 0);
+}
+
+// Near-field items per block: about 4,096 in all, three rounds of the workgroups that the
+// GPU holds (an item of FF_M0 tiles is 262,144 pairs), and at least 2 per block
+inline int near_split(int64_t nb) { return (int)std::max<int64_t>(2, std::min<int64_t>(16, 4096 / nb)); }
+
+// Slices of the far field: blocks x slices workgroups, at least about four rounds of the
+// two that a CU holds, so that the last round is short beside the whole and few blocks
+// (a collection of 65,536: 256) still fill every slot.
+inline int far_slices(int64_t nb, int64_t mwords, int cus) {
+  const int64_t want = (8 * (int64_t)cus + nb - 1) / nb;
+  return (int)std::max<int64_t>(1, std::min<int64_t>({want, mwords, 32}));
+}
+
 
 }  // namespace o3d

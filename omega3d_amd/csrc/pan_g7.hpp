@@ -69,40 +69,41 @@ __device__ __forceinline__ void panel_vertices(const PanArgs& a, int64_t p, floa
   v[6] = a.nx[i2]; v[7] = a.ny[i2]; v[8] = a.nz[i2];
 }
 
-// stage panels [p0, p0 + cnt):
+// a panel's record:
 //   f0..f5.x  the seven points (21 floats, computed in FP64 and rounded)
 //   f5.yzw    centroid (float, the decision's arithmetic)
 //   f6        {tsx, tsy, tsz, ss * area}   absolute vortex and source strengths
 //   f7        {4 D^2, v0x, v0y, v0z}       f8 {v1x, v1y, v1z, v2x}
 //   f9        {v2y, v2z, area, ss}
+__device__ __forceinline__ void g7_record(const PanArgs& a, int64_t p, float4* s) {
+  float v[9];
+  panel_vertices(a, p, v);
+  float pts[21];
+#pragma unroll
+  for (int q = 0; q < 7; ++q)
+#pragma unroll
+    for (int d = 0; d < 3; ++d)
+      pts[3 * q + d] = (float)(g7_bary(q, 0) * (double)v[d] + g7_bary(q, 1) * (double)v[3 + d] +
+                               g7_bary(q, 2) * (double)v[6 + d]);
+  const float4 geo = g7_geometry(v);
+  const float cx = geo.x, cy = geo.y, cz = geo.z, lim = geo.w;
+  const float ar = a.area[p];
+  const float sg = a.ss ? a.ss[p] : 0.0f;
+  s[0] = make_float4(pts[0], pts[1], pts[2], pts[3]);
+  s[1] = make_float4(pts[4], pts[5], pts[6], pts[7]);
+  s[2] = make_float4(pts[8], pts[9], pts[10], pts[11]);
+  s[3] = make_float4(pts[12], pts[13], pts[14], pts[15]);
+  s[4] = make_float4(pts[16], pts[17], pts[18], pts[19]);
+  s[5] = make_float4(pts[20], cx, cy, cz);
+  s[6] = make_float4(a.tsx[p], a.tsy[p], a.tsz[p], sg * ar);
+  s[7] = make_float4(lim, v[0], v[1], v[2]);
+  s[8] = make_float4(v[3], v[4], v[5], v[6]);
+  s[9] = make_float4(v[7], v[8], ar, sg);
+}
+
+// stage panels [p0, p0 + cnt)
 __device__ __forceinline__ void stage_g7(const PanArgs& a, int64_t p0, int cnt, float4* sh) {
-  for (int j = threadIdx.x; j < cnt; j += BLOCK) {
-    const int64_t p = p0 + j;
-    float v[9];
-    panel_vertices(a, p, v);
-    float pts[21];
-#pragma unroll
-    for (int q = 0; q < 7; ++q)
-#pragma unroll
-      for (int d = 0; d < 3; ++d)
-        pts[3 * q + d] = (float)(g7_bary(q, 0) * (double)v[d] + g7_bary(q, 1) * (double)v[3 + d] +
-                                 g7_bary(q, 2) * (double)v[6 + d]);
-    const float4 geo = g7_geometry(v);
-    const float cx = geo.x, cy = geo.y, cz = geo.z, lim = geo.w;
-    const float ar = a.area[p];
-    const float sg = a.ss ? a.ss[p] : 0.0f;
-    float4* s = sh + G7_F4 * j;
-    s[0] = make_float4(pts[0], pts[1], pts[2], pts[3]);
-    s[1] = make_float4(pts[4], pts[5], pts[6], pts[7]);
-    s[2] = make_float4(pts[8], pts[9], pts[10], pts[11]);
-    s[3] = make_float4(pts[12], pts[13], pts[14], pts[15]);
-    s[4] = make_float4(pts[16], pts[17], pts[18], pts[19]);
-    s[5] = make_float4(pts[20], cx, cy, cz);
-    s[6] = make_float4(a.tsx[p], a.tsy[p], a.tsz[p], sg * ar);
-    s[7] = make_float4(lim, v[0], v[1], v[2]);
-    s[8] = make_float4(v[3], v[4], v[5], v[6]);
-    s[9] = make_float4(v[7], v[8], ar, sg);
-  }
+  for (int j = threadIdx.x; j < cnt; j += BLOCK) g7_record(a, p0 + j, sh + G7_F4 * j);
 }
 
 __device__ __forceinline__ bool g7_is_near(float tx, float ty, float tz, const float4* s) {
@@ -370,7 +371,7 @@ __global__ __launch_bounds__(BLOCK) void k_pan_g7(PanArgs a) {
 }
 
 // the decision's geometry of every panel, for k_pan_g7_near
-__global__ __launch_bounds__(BLOCK) void k_pan_g7_geom(PanArgs a, float4* geom) {
+static __global__ __launch_bounds__(BLOCK) void k_pan_g7_geom(PanArgs a, float4* geom) {
   const int64_t p = (int64_t)blockIdx.x * BLOCK + threadIdx.x;
   if (p >= a.np) return;
   float v[9];
@@ -439,7 +440,7 @@ __global__ __launch_bounds__(BLOCK) void k_pan_g7_near(PanArgs a, const float4* 
   if (nnear && mine) atomicAdd(nnear, mine);
 }
 
-__global__ void k_pan_g7_zero(unsigned int* c) {
+static __global__ void k_pan_g7_zero(unsigned int* c) {
   if (threadIdx.x == 0 && blockIdx.x == 0) *c = 0u;
 }
 

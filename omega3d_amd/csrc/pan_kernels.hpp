@@ -351,6 +351,44 @@ __device__ __forceinline__ void pan_root_pair(const float4* s, R tx, R ty, R tz,
 
 constexpr int PAN_UNROLL = 4;   // panels per step of k_pan's separated-pair loop
 
+// the staged panels 0 .. cnt - 1 acting on one target per lane
+template <class R, bool GRAD>
+__device__ __forceinline__ void pan_root_tile(const float4* shp, int cnt, R tx, R ty, R tz, int maxlev, bool active,
+                                              R* acc, bool& has_near) {
+  int j = 0;
+  if constexpr (sizeof(R) == 4) {
+    // PAN_UNROLL panels at a time while every lane's pairs are surely leaves at the
+    // root (d2 beyond the far band): one wave-uniform branch, the leaves with no
+    // per-pair mask, the LDS address in a vector register (made so by an opaque
+    // zero) with immediate offsets.  The same leaves, in the same order and with
+    // the same bits, as the per-pair path below; an idle lane's sums are dropped.
+    int vz;
+    asm volatile("v_mov_b32 %0, 0" : "=v"(vz));
+    const float4* q = shp + vz;
+    for (; j + PAN_UNROLL <= cnt; j += PAN_UNROLL, q += PAN_F4 * PAN_UNROLL) {
+      float4 g[PAN_UNROLL], c[PAN_UNROLL];
+      uint64_t near = 0;   // lanes with a pair not surely a leaf, as a scalar mask
+#pragma unroll
+      for (int u = 0; u < PAN_UNROLL; ++u) {
+        g[u] = q[PAN_F4 * u + 2];
+        c[u] = q[PAN_F4 * u + 3];
+        const float ex = tx - c[u].x, ey = ty - c[u].y, ez = tz - c[u].z;
+        near |= __builtin_amdgcn_ballot_w64(!(fmaf(ez, ez, fmaf(ey, ey, ex * ex)) > c[u].w));
+      }
+      if (near == 0) {
+#pragma unroll
+        for (int u = 0; u < PAN_UNROLL; ++u)
+          leaf_acc<R, GRAD>(tx, ty, tz, c[u].x, c[u].y, c[u].z, g[u].x, g[u].y, g[u].z, g[u].w, acc);
+      } else {
+#pragma unroll
+        for (int u = 0; u < PAN_UNROLL; ++u) pan_root_pair<R, GRAD>(q + PAN_F4 * u, tx, ty, tz, maxlev, active,
+                                                                    acc, has_near);
+      }
+    }
+  }
+  for (; j < cnt; ++j) pan_root_pair<R, GRAD>(shp + PAN_F4 * j, tx, ty, tz, maxlev, active, acc, has_near);
+}
+
 // rec: the records of all panels (k_pan_geom).  At least 5 waves per SIMD (96
 // VGPRs; the FP64 gradient sums spill once per tile, outside the panel loop): on
 // the icosphere 1.7% faster than the 103 VGPRs and 4 waves the compiler chooses,
@@ -374,38 +412,7 @@ __global__ __launch_bounds__(BLOCK, 5) void k_pan(PanArgs a, const float4* rec) 
     __syncthreads();
     stage_panels(rec, p0, cnt, shp);
     __syncthreads();
-    int j = 0;
-    if constexpr (sizeof(R) == 4) {
-      // PAN_UNROLL panels at a time while every lane's pairs are surely leaves at the
-      // root (d2 beyond the far band): one wave-uniform branch, the leaves with no
-      // per-pair mask, the LDS address in a vector register (made so by an opaque
-      // zero) with immediate offsets.  The same leaves, in the same order and with
-      // the same bits, as the per-pair path below; an idle lane's sums are dropped.
-      int vz;
-      asm volatile("v_mov_b32 %0, 0" : "=v"(vz));
-      const float4* q = shp + vz;
-      for (; j + PAN_UNROLL <= cnt; j += PAN_UNROLL, q += PAN_F4 * PAN_UNROLL) {
-        float4 g[PAN_UNROLL], c[PAN_UNROLL];
-        uint64_t near = 0;   // lanes with a pair not surely a leaf, as a scalar mask
-#pragma unroll
-        for (int u = 0; u < PAN_UNROLL; ++u) {
-          g[u] = q[PAN_F4 * u + 2];
-          c[u] = q[PAN_F4 * u + 3];
-          const float ex = tx - c[u].x, ey = ty - c[u].y, ez = tz - c[u].z;
-          near |= __builtin_amdgcn_ballot_w64(!(fmaf(ez, ez, fmaf(ey, ey, ex * ex)) > c[u].w));
-        }
-        if (near == 0) {
-#pragma unroll
-          for (int u = 0; u < PAN_UNROLL; ++u)
-            leaf_acc<R, GRAD>(tx, ty, tz, c[u].x, c[u].y, c[u].z, g[u].x, g[u].y, g[u].z, g[u].w, acc);
-        } else {
-#pragma unroll
-          for (int u = 0; u < PAN_UNROLL; ++u) pan_root_pair<R, GRAD>(q + PAN_F4 * u, tx, ty, tz, a.maxlev, active,
-                                                                      acc, has_near);
-        }
-      }
-    }
-    for (; j < cnt; ++j) pan_root_pair<R, GRAD>(shp + PAN_F4 * j, tx, ty, tz, a.maxlev, active, acc, has_near);
+    pan_root_tile<R, GRAD>(shp, cnt, tx, ty, tz, a.maxlev, active, acc, has_near);
     if (PREC == PREC_COMP) {
       two_sum(hi[0], lo[0], (float)acc[0]);
       two_sum(hi[1], lo[1], (float)acc[1]);

@@ -5,6 +5,7 @@
 #include "o3d_api_internal.hpp"
 #include "pan_g7.hpp"
 #include "pan_kernels.hpp"
+#include "panfar.hpp"
 
 #include <algorithm>
 #include <chrono>
@@ -175,15 +176,18 @@ static int pan_dev(const o3d_panels* p, o3d_points* t, const o3d_opts* o, int pr
   PanArgs a = pan_args(p, t, grad, out64);
   a.tile = o->tile > 0 ? o->tile : 128;
   a.maxlev = ml;
+  std::lock_guard<std::mutex> lk(stream_ws_mutex());
+  const int rule = g7 ? PANFAR_POINTS7 : PANFAR_POINTS;
+  void* ws = nullptr;
+  if (panfar_pays(rule, a.np, a.nt, o->method, o->tile, prec) && panfar_scratch(panfar_bytes(rule, a.np, a.nt, grad), st, &ws))
+    return panfar_points(a, rule, grad, prec, ws, st);
   if (g7) {
-    std::lock_guard<std::mutex> lk(stream_ws_mutex());
     float4* geom = nullptr;
     if ((rc = g7_scratch(&a, st, &geom)) != O3D_OK) return rc;
     const hipError_t e = launch_pan_g7(a, grad, prec, true, st, geom);
     if (e != hipSuccess) return fail(O3D_EDEVICE, "panel launch failed: %s", hipGetErrorString(e));
     return O3D_OK;
   }
-  std::lock_guard<std::mutex> lk(stream_ws_mutex());
   float4* rec = nullptr;
   if ((rc = g7_scratch(&a, st, &rec, PAN_F4 + 1)) != O3D_OK) return rc;
   const hipError_t e = launch_pan(a, grad, prec, st, rec);
@@ -247,13 +251,18 @@ static int pap_dev(const o3d_panels* src, const o3d_panels* targ, float* const v
   a.maxlev = ml;
   std::lock_guard<std::mutex> lk(stream_ws_mutex());
   float4* rec = nullptr;
-  void* tail = nullptr;
-  if ((rc = g7_scratch(&a, st, &rec, PAN_F4 + 1, sizeof(float) * 3 * (size_t)nt, &tail)) != O3D_OK) return rc;
+  void *tail = nullptr, *ws = nullptr;
+  const size_t pts = (sizeof(float) * 3 * (size_t)nt + 255) & ~(size_t)255;
+  const bool far = panfar_pays(PANFAR_POINTS, a.np, nt, o->method, o->tile, o->precision) &&
+                   panfar_scratch(pts + panfar_bytes(PANFAR_POINTS, a.np, nt, false), st, &ws);
+  if (far) tail = ws;
+  else if ((rc = g7_scratch(&a, st, &rec, PAN_F4 + 1, pts, &tail)) != O3D_OK) return rc;
   float* px = (float*)tail;
   a.tx = px; a.ty = px + nt; a.tz = px + 2 * nt;
   hipLaunchKernelGGL(k_colocation, dim3(g), dim3(BLOCK), 0, st, targ->x[0], targ->x[1], targ->x[2], targ->idx, nt,
                      COLOCATION_OFFSET, px, px + nt, px + 2 * nt);
   HIPCHK(hipGetLastError());
+  if (far) return panfar_points(a, PANFAR_POINTS, false, o->precision, (char*)ws + pts, st);
   const hipError_t e = launch_pan(a, false, o->precision, st, rec);
   if (e != hipSuccess) return fail(O3D_EDEVICE, "panel launch failed: %s", hipGetErrorString(e));
   return O3D_OK;

@@ -1,0 +1,618 @@
+// panfar.hip -- the panel sums with their separated pairs on the matrix cores.
+//
+// A panel far from a target is one singular point (recursive rule, pan_kernels.hpp; the
+// roles reversed for particles -> panels, ptpan.hip) or seven of them (7-point rule,
+// pan_g7.hpp).  Panels and points are put in Morton order, and a block of 256 targets
+// takes the tiles of sources that lie a block radius away, and beyond every distance at
+// which one of the pairs would not be plain, through k_ff_far (ff_kernels.hpp).  The
+// other tiles go through the code of the direct kernels, tile by tile in work items of a
+// queue: each item leaves its sums per target, and lists the targets that have pairs
+// which need the recursion (or the closed form); a second kernel gives each of those
+// entries 16 lanes, which gather the entry's pairs and walk them 16 at a time, and adds
+// to the item's sums.  All decisions per pair are the direct kernels'.
+//
+// The direct kernels are bound by the issue of about 40 vector instructions per pair (35
+// per point of the 7-point rule); a far pair takes one square root, three products and the
+// weight's split beside the matrix products (2.5e12 pairs/s with 128 panels per tile).
+// Compensated: 20,480 panels on 524,288 points, velocity and gradient 12.1 -> 6.2 ms (far
+// 3.74, items 1.49, walks 0.91); 5,120 panels with source strengths on 200,003 points,
+// 7-point rule 7.7 -> 4.3 ms (2.74, 1.28, 0.32); 524,288 particles on 20,480 panels 6.4 ->
+// 5.7 ms (2.31, 2.54, 1.06).  Errors against FP64 as before or smaller (1.2e-7 -> 0.9e-7).
+#include "ff_kernels.hpp"
+#include "o3d_api_internal.hpp"
+#include "pan_g7.hpp"
+#include "panfar.hpp"
+#include "ptpan_kernels.hpp"
+
+namespace o3d {
+namespace {
+
+constexpr int PF_FOLD = 64;   // panels or particles per FP32 partial of the compensated sums: half the direct tile, near terms being the large ones
+
+struct PanFarArgs {
+  FFArgs f;            // targets: points (PANFAR_POINTS7: too) or panels
+  PanArgs p;           // panels as sources
+  PtPanArgs t;         // panels as targets
+  float4* rec;         // records of the panels in sorted order (targets: rows of tq are enough)
+  float4* cen;         // panels as sources: what the near test needs first
+  unsigned* list;      // entries (item * 256 + target of the block) with pairs to walk
+  unsigned* count;
+  int* iblk;           // block of every item
+  int64_t units;       // panels or particles that are sources
+  int32_t unit;        // of them, per tile
+};
+
+// what makes a pair of a panel with a point plain: the distance of the point from the
+// panel's centroid, with a margin far above the rounding of the distances compared; a
+// limit that is no number keeps the panel out of the far field
+__device__ __forceinline__ float plain_limit(float lim) { return lim >= 0.0f ? lim * 1.00001f : __builtin_huge_valf(); }
+
+// centroids of the panels for the Morton order (as the decisions take them)
+__global__ __launch_bounds__(256) void k_pf_centroids(PanArgs a, float* x, float* y, float* z) {
+  const int64_t p = (int64_t)blockIdx.x * 256 + threadIdx.x;
+  if (p >= a.np) return;
+  float v[9], cx, cy, cz;
+  panel_vertices(a, p, v);
+  centroid_exact(v[0], v[1], v[2], v[3], v[4], v[5], v[6], v[7], v[8], cx, cy, cz);
+  x[p] = cx; y[p] = cy; z[p] = cz;
+}
+
+// source rows 0 .. npad - 1 in sorted order, and the panels' records and near-test rows
+template <int RULE>
+__global__ __launch_bounds__(256) void k_pf_sources(PanFarArgs a, const int* perm, float4* sp, float4* sa) {
+  const int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x;
+  if (RULE == PANFAR_PARTICLES) {
+    if (i >= (int64_t)a.f.ntiles * a.f.tile) return;
+    const int j = perm[i < a.units ? i : a.units - 1];
+    sp[i] = make_float4(a.t.sx[j], a.t.sy[j], a.t.sz[j], 0.0f);
+    sa[i] = i < a.units ? make_float4(a.t.ax[j], a.t.ay[j], a.t.az[j], 0.0f) : make_float4(0.f, 0.f, 0.f, 0.f);
+    return;
+  }
+  if (i >= (int64_t)a.f.ntiles * a.unit) return;
+  const bool real = i < a.units;
+  const int64_t p = perm[real ? i : a.units - 1];
+  if (RULE == PANFAR_POINTS) {
+    float4 s[PAN_F4];
+    panel_record(a.p, p, s);
+    sp[i] = make_float4(s[3].x, s[3].y, s[3].z, plain_limit(s[4].z * 4.0f));
+    sa[i] = real ? s[2] : make_float4(0.f, 0.f, 0.f, 0.f);
+    if (!real) return;
+#pragma unroll
+    for (int k = 0; k < PAN_F4; ++k) a.rec[PAN_F4 * i + k] = s[k];
+    a.cen[i] = s[3];
+    return;
+  }
+  // seven rows per panel, the last of a tile's panels filling the tile up
+  float4 s[G7_F4];
+  g7_record(a.p, p, s);
+  const float lim = plain_limit(sqrtf(s[7].x));
+  const float pt[21] = {s[0].x, s[0].y, s[0].z, s[0].w, s[1].x, s[1].y, s[1].z, s[1].w, s[2].x, s[2].y, s[2].z,
+                        s[2].w, s[3].x, s[3].y, s[3].z, s[3].w, s[4].x, s[4].y, s[4].z, s[4].w, s[5].x};
+  const int64_t t = i / a.unit;
+  const int j = (int)(i - t * a.unit);
+  const int64_t row = t * a.f.tile + 7 * j;
+#pragma unroll
+  for (int q = 0; q < 7; ++q) {
+    const float w = real ? (float)g7_weight(q) : 0.0f;
+    sp[row + q] = make_float4(pt[3 * q], pt[3 * q + 1], pt[3 * q + 2], lim);
+    sa[row + q] = real ? make_float4(w * s[6].x, w * s[6].y, w * s[6].z, w * s[6].w) : make_float4(0.f, 0.f, 0.f, 0.f);
+  }
+  if (j == a.unit - 1)
+    for (int k = 7 * a.unit; k < a.f.tile; ++k) {
+      sp[t * a.f.tile + k] = make_float4(pt[0], pt[1], pt[2], lim);
+      sa[t * a.f.tile + k] = make_float4(0.f, 0.f, 0.f, 0.f);
+    }
+  if (!real) return;
+#pragma unroll
+  for (int k = 0; k < G7_F4; ++k) a.rec[G7_F4 * i + k] = s[k];
+  a.cen[i] = make_float4(s[5].y, s[5].z, s[5].w, s[7].x);
+}
+
+// targets in sorted order: points, or panels' centroids with their limit
+template <int RULE>
+__global__ __launch_bounds__(256) void k_pf_targets(PanFarArgs a, const int* perm, float4* tq) {
+  const int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x;
+  if (i >= a.f.nt) return;
+  const int j = perm[i];
+  if (RULE == PANFAR_PARTICLES) {
+    float4 s[PAN_F4];
+    ptpan_record(a.t, j, s);
+    tq[i] = make_float4(s[3].x, s[3].y, s[3].z, plain_limit(s[4].z * 4.0f));
+  } else {
+    tq[i] = make_float4(a.p.tx[j], a.p.ty[j], a.p.tz[j], 0.0f);
+  }
+}
+
+// block b's near tiles of rank [r0, r1), in order: next() gives -1 after the last
+struct NearTiles {
+  const unsigned* mrow;
+  int mwords, ntiles, r0, r1, w = -1, rank = 0;
+  unsigned bits = 0u;
+  __device__ __forceinline__ NearTiles(const FFArgs& f, int64_t b, int r0_, int r1_)
+      : mrow(f.mask + b * f.mwords), mwords(f.mwords), ntiles(f.ntiles), r0(r0_), r1(r1_) {}
+  __device__ __forceinline__ int next() {
+    for (;;) {
+      while (bits == 0u) {
+        if (rank >= r1 || ++w >= mwords) return -1;
+        const int left = ntiles - 32 * w;
+        bits = ~mrow[w] & (left >= 32 ? 0xffffffffu : (1u << left) - 1u);
+        const int c = __popc(bits);
+        if (rank + c <= r0) { rank += c; bits = 0u; }
+      }
+      const int t = 32 * w + __builtin_ctz(bits);
+      bits &= bits - 1u;
+      if (rank++ < r0) continue;
+      return rank <= r1 ? t : -1;
+    }
+  }
+};
+
+// one item: the pairs of a block with some of its near tiles, as the direct kernel takes
+// them (k_pan, k_pan_g7, k_ptpan)
+template <int RULE, bool GRAD, int PREC>
+__device__ __forceinline__ void pf_item(const PanFarArgs& a, int64_t b, int item, int r0, int r1, float4* sh) {
+  constexpr int NOUT = GRAD ? 12 : 3;
+  constexpr int F4 = RULE == PANFAR_POINTS ? PAN_F4 : RULE == PANFAR_POINTS7 ? G7_F4 : 2;
+  const int tid = threadIdx.x;
+  const int64_t i = b * FF_TB + tid;
+  const bool active = i < a.f.nt;
+  const int64_t ic = active ? i : a.f.nt - 1;
+  const float4 q = a.f.tq[ic];
+  float4 s[PAN_F4];
+  if (RULE == PANFAR_PARTICLES) ptpan_record(a.t, a.f.tperm[ic], s);
+  float acc[16];
+  float hi[3] = {0.f, 0.f, 0.f}, lo[3] = {0.f, 0.f, 0.f};
+  double gd[9] = {0, 0, 0, 0, 0, 0, 0, 0, 0};
+  bool has_near = false;
+#pragma unroll
+  for (int c = 0; c < 16; ++c) acc[c] = 0.0f;
+  NearTiles tiles(a.f, b, r0, r1);
+  for (int t = tiles.next(); t >= 0; t = tiles.next()) {
+    const int64_t p0 = (int64_t)t * a.unit;
+    const int cnt = (int)(a.units - p0 < a.unit ? a.units - p0 : a.unit);
+    __syncthreads();
+    if (RULE == PANFAR_PARTICLES) {
+      for (int j = tid; j < cnt; j += FF_TB) {
+        sh[2 * j] = a.f.sp[p0 + j];
+        sh[2 * j + 1] = a.f.sa[p0 + j];
+      }
+    } else {
+      for (int j = tid; j < F4 * cnt; j += FF_TB) sh[j] = a.rec[F4 * p0 + j];
+    }
+    __syncthreads();
+    for (int j0 = 0; j0 < cnt; j0 += PF_FOLD) {
+      const int n = cnt - j0 < PF_FOLD ? cnt - j0 : PF_FOLD;
+      const float4* w = sh + F4 * j0;
+      if constexpr (RULE == PANFAR_POINTS) {
+        pan_root_tile<float, GRAD>(w, n, q.x, q.y, q.z, a.p.maxlev, active, acc, has_near);
+      } else if constexpr (RULE == PANFAR_POINTS7) {
+        for (int j = 0; j < n; ++j) {
+          const bool near = g7_is_near(q.x, q.y, q.z, w + G7_F4 * j);
+          has_near |= near;
+          g7_far_pair<float, GRAD>(q.x, q.y, q.z, w + G7_F4 * j, near ? 0.0f : 1.0f, acc);
+        }
+      } else {
+        int nnear = 0;
+        ptpan_root_tile<PREC, false>(w, n, p0 + j0, s, a.t.maxlev, active, acc, nullptr, nnear);
+        has_near |= nnear > 0;
+      }
+      if (PREC == PREC_COMP) {
+        two_sum(hi[0], lo[0], acc[0]);
+        two_sum(hi[1], lo[1], acc[1]);
+        two_sum(hi[2], lo[2], acc[2]);
+        if (GRAD) {
+          float g[9];
+          if (RULE == PANFAR_POINTS7) {
+#pragma unroll
+            for (int k = 0; k < 9; ++k) g[k] = acc[3 + k];
+          } else {
+            grad_of<float>(acc, g);
+          }
+#pragma unroll
+          for (int k = 0; k < 9; ++k) gd[k] += (double)g[k];
+        }
+#pragma unroll
+        for (int c = 0; c < 16; ++c) acc[c] = 0.0f;
+      }
+    }
+  }
+  // particles -> panels: the pairs were summed with the roles reversed
+  const double sg = RULE == PANFAR_PARTICLES ? -1.0 : 1.0;
+  double* slot = a.f.part + (int64_t)item * NOUT * FF_TB + tid;
+#pragma unroll
+  for (int d = 0; d < 3; ++d)
+    slot[d * FF_TB] = sg * (PREC == PREC_COMP ? (double)hi[d] + (double)lo[d] : (double)acc[d]);
+  if (GRAD) {
+    float g[9];
+    if (PREC != PREC_COMP) {
+      if (RULE == PANFAR_POINTS7) {
+#pragma unroll
+        for (int k = 0; k < 9; ++k) g[k] = acc[3 + k];
+      } else {
+        grad_of<float>(acc, g);
+      }
+    }
+#pragma unroll
+    for (int k = 0; k < 9; ++k) slot[(3 + k) * FF_TB] = PREC == PREC_COMP ? gd[k] : (double)g[k];
+  }
+  if (has_near && active) a.list[atomicAdd(a.count, 1u)] = (unsigned)item * FF_TB + tid;
+}
+
+// persistent: every workgroup takes items from the queue until none is left
+template <int RULE, bool GRAD, int PREC>
+__global__ __launch_bounds__(FF_TB) void k_pf_items(PanFarArgs a) {
+  extern __shared__ float4 sh[];
+  __shared__ int s_item;
+  const int64_t nb = (a.f.nt + FF_TB - 1) / FF_TB;
+  const int total = a.f.ioff[nb - 1] + a.f.items[nb - 1];
+  const int m = *a.f.mfold;
+  for (;;) {
+    __syncthreads();
+    if (threadIdx.x == 0) s_item = (int)atomicAdd(a.f.ctr, 1u);
+    __syncthreads();
+    const int item = s_item;
+    if (item >= total) break;
+    // block b: the last with ioff[b] <= item (blocks without items share the offset of the next)
+    int64_t lo = 0, hi = nb;
+    while (hi - lo > 1) {
+      const int64_t mid = (lo + hi) / 2;
+      if (a.f.ioff[mid] <= item) lo = mid; else hi = mid;
+    }
+    if (threadIdx.x == 0) a.iblk[item] = (int)lo;
+    const int r0 = (item - a.f.ioff[lo]) * m;
+    const int nnb = a.f.nn[lo];
+    pf_item<RULE, GRAD, PREC>(a, lo, item, r0, r0 + m < nnb ? r0 + m : nnb, sh);
+  }
+}
+
+// The listed entries' pairs that need the recursion or the closed form.  Each quarter
+// of a wave takes an entry: its 16 lanes test the item's panels (particles) in turn,
+// queue those that are near and walk them when 16 are there or none is left, hit h in
+// lane h mod 16, so that the lanes walk together however the near ones lie.  A fixed
+// butterfly adds the lanes' sums in FP64; the order in which entries were listed decides
+// nothing.
+template <int RULE, bool GRAD, int PREC>
+__global__ __launch_bounds__(BLOCK) void k_pf_walk(PanFarArgs a) {
+  constexpr int NOUT = GRAD ? 12 : 3;
+  __shared__ int ring[BLOCK / 16][32];
+  const int lane = threadIdx.x & 63, ql = lane & 15, q0 = lane & 48;
+  int* mine = ring[threadIdx.x >> 4];
+  const int64_t wave = ((int64_t)blockIdx.x * BLOCK + threadIdx.x) >> 6;
+  const int64_t nwaves = ((int64_t)gridDim.x * BLOCK) >> 6;
+  const int64_t listed = *a.count;
+  const int m = *a.f.mfold;
+  for (int64_t e = wave; 4 * e < listed; e += nwaves) {
+    const int64_t li = 4 * e + (lane >> 4);
+    const bool has = li < listed;
+    const unsigned entry = a.list[has ? li : 4 * e];
+    const int item = (int)(entry / FF_TB), tid = (int)(entry % FF_TB);
+    const int64_t b = a.iblk[item];
+    const int r0 = (item - a.f.ioff[b]) * m;
+    const int r1 = has ? (r0 + m < a.f.nn[b] ? r0 + m : a.f.nn[b]) : r0;
+    const float4 q = a.f.tq[b * FF_TB + tid];
+    float4 s[PAN_F4];
+    float far2 = 0.0f;
+    if (RULE == PANFAR_PARTICLES) {
+      ptpan_record(a.t, a.f.tperm[b * FF_TB + tid], s);
+      far2 = s[3].w;
+    }
+    float acc[16];
+    double u[3] = {0, 0, 0}, g[9] = {0, 0, 0, 0, 0, 0, 0, 0, 0};
+#pragma unroll
+    for (int c = 0; c < 16; ++c) acc[c] = 0.0f;
+    // whether pair p is near, from its near-test row
+    auto is_near = [&](int64_t p, const float4 c) {
+      if constexpr (RULE == PANFAR_POINTS7) {
+        float d2;
+        {
+#pragma clang fp contract(off)
+          const float ex = q.x - c.x, ey = q.y - c.y, ez = q.z - c.z;
+          d2 = ex * ex + ey * ey + ez * ez;
+        }
+        return d2 < c.w;
+      } else {
+        constexpr bool PART = RULE == PANFAR_PARTICLES;
+        const float4 P = PART ? c : q, C = PART ? q : c;
+        const float ex = P.x - C.x, ey = P.y - C.y, ez = P.z - C.z;
+        if (fmaf(ez, ez, fmaf(ey, ey, ex * ex)) > (PART ? far2 : c.w)) return false;
+        float gx, gy, gz, gs, cx0, cy0, cz0, lim;
+        RootLim rl;
+        panel_root<float>(PART ? s : a.rec + PAN_F4 * p, gx, gy, gz, gs, cx0, cy0, cz0, lim, rl);
+        return !root_leaf<float>(P.x, P.y, P.z, cx0, cy0, cz0, lim, rl, PART ? a.t.maxlev : a.p.maxlev, true);
+      }
+    };
+    auto walk = [&](int64_t p) {
+      if constexpr (RULE == PANFAR_POINTS) {
+        walk_panel<float, GRAD>(q.x, q.y, q.z, a.rec + PAN_F4 * p, a.p.maxlev, true, acc);
+      } else if constexpr (RULE == PANFAR_POINTS7) {
+        const float4* r = a.rec + G7_F4 * p;
+        const float4 f6 = r[6], f7 = r[7], f8 = r[8], f9 = r[9];
+        const float v[9] = {f7.y, f7.z, f7.w, f8.x, f8.y, f8.z, f8.w, f9.x, f9.y};
+        const float ts[3] = {f6.x, f6.y, f6.z};
+        g7_near_pair<GRAD>(q.x, q.y, q.z, v, ts, f9.z, f9.w, u, g);
+      } else {
+        const float4 P = a.f.sp[p], A = a.f.sa[p];
+        ptpan_strength<PREC>(s, A);
+        walk_panel<float, false>(P.x, P.y, P.z, s, a.t.maxlev, true, acc);
+      }
+    };
+    int head = 0, tail = 0;   // hits walked and found, alike in the quarter's lanes
+    auto drain = [&]() {
+      const int h = head + ((ql - head) & 15);
+      __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+      if (h < tail) walk(mine[h & 31]);
+      __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+      head = head + 16 < tail ? head + 16 : tail;
+    };
+    NearTiles tiles(a.f, b, r0, r1);
+    for (int t = tiles.next(); wave_any(t >= 0); t = t >= 0 ? tiles.next() : -1) {
+      const int64_t p0 = (int64_t)t * a.unit;
+      const int cnt = t < 0 ? 0 : (int)(a.units - p0 < a.unit ? a.units - p0 : a.unit);
+      for (int j0 = 0; j0 < a.unit; j0 += 64) {
+        float4 c[4];
+#pragma unroll
+        for (int k = 0; k < 4; ++k) {
+          const int j = j0 + 16 * k + ql;
+          c[k] = RULE == PANFAR_PARTICLES ? a.f.sp[j < cnt ? p0 + j : 0] : a.cen[j < cnt ? p0 + j : 0];
+        }
+#pragma unroll
+        for (int k = 0; k < 4; ++k) {
+          const int j = j0 + 16 * k + ql;
+          const bool near = j < cnt && is_near(p0 + j, c[k]);
+          const unsigned hits = (unsigned)(__builtin_amdgcn_ballot_w64(near) >> q0) & 0xffffu;
+          if (near) mine[(tail + __popc(hits & ((1u << ql) - 1u))) & 31] = (int)(p0 + j);
+          tail += __popc(hits);
+          while (wave_any(tail - head >= 16)) drain();
+        }
+      }
+    }
+    while (wave_any(head < tail)) drain();
+    if (RULE != PANFAR_POINTS7) {
+#pragma unroll
+      for (int d = 0; d < 3; ++d) u[d] = (RULE == PANFAR_PARTICLES ? -1.0 : 1.0) * (double)acc[d];
+      if (GRAD) {
+        float gl[9];
+        grad_of<float>(acc, gl);
+#pragma unroll
+        for (int k = 0; k < 9; ++k) g[k] = (double)gl[k];
+      }
+    }
+    double* slot = a.f.part + (int64_t)item * NOUT * FF_TB + tid;
+#pragma unroll
+    for (int d = 0; d < 3; ++d) u[d] = quarter_sum(u[d]);
+    if (GRAD) {
+#pragma unroll
+      for (int k = 0; k < 9; ++k) g[k] = quarter_sum(g[k]);
+    }
+    if (ql != 0 || !has) continue;
+#pragma unroll
+    for (int d = 0; d < 3; ++d) slot[d * FF_TB] += u[d];
+    if (GRAD) {
+#pragma unroll
+      for (int k = 0; k < 9; ++k) slot[(3 + k) * FF_TB] += g[k];
+    }
+  }
+}
+
+struct PanFarLayout {
+  unsigned *bb, *ks_in, *ks_out, *kt_in, *kt_out, *mask, *ctr, *list, *count;
+  int *is_in, *is_out, *it_in, *it_out, *nn, *noff, *items, *ioff, *mfold, *iblk;
+  void* tmp;
+  float *cx, *cy, *cz, *tcs, *tam, *tsg, *bcs;
+  float4 *sp, *sa, *tq, *tsph, *bsph, *rec, *cen;
+  double *farv, *part;
+  size_t bytes;
+};
+
+// sources per tile and panels per tile.  128 panels lie within 0.3 radii on the sphere of
+// 20,480, 256 within 0.42: 87 and 82% of the pairs of 524,288 points around it are far
+int tile_of(int rule) { return rule == PANFAR_POINTS ? 128 : 256; }
+int unit_of(int rule) { return rule == PANFAR_POINTS7 ? tile_of(rule) / 7 : tile_of(rule); }
+
+PanFarLayout layout(char* base, int rule, int64_t units, int64_t nt, int nout) {
+  const int T = tile_of(rule), U = unit_of(rule);
+  const int64_t np = rule == PANFAR_PARTICLES ? nt : units;
+  const int64_t nb = (nt + FF_TB - 1) / FF_TB;
+  const int64_t ntiles = (units + U - 1) / U;
+  const int64_t mwords = (ntiles + 31) / 32;
+  const int64_t maxitems = (near_split(nb) + 1) * nb;
+  const int f4 = rule == PANFAR_POINTS ? PAN_F4 : rule == PANFAR_POINTS7 ? G7_F4 : 0;
+  Carve cv{base};
+  PanFarLayout L{};
+  L.bb = cv.take<unsigned>(8);
+  L.cx = cv.take<float>(np);
+  L.cy = cv.take<float>(np);
+  L.cz = cv.take<float>(np);
+  L.ks_in = cv.take<unsigned>(units);
+  L.ks_out = cv.take<unsigned>(units);
+  L.is_in = cv.take<int>(units);
+  L.is_out = cv.take<int>(units);
+  L.kt_in = cv.take<unsigned>(nt);
+  L.kt_out = cv.take<unsigned>(nt);
+  L.it_in = cv.take<int>(nt);
+  L.it_out = cv.take<int>(nt);
+  L.tmp = cv.take<char>(radix_tmp_bytes(std::max(units, nt)));
+  L.sp = cv.take<float4>((size_t)ntiles * T);
+  L.sa = cv.take<float4>((size_t)ntiles * T);
+  L.rec = cv.take<float4>((size_t)f4 * units);
+  L.cen = cv.take<float4>(f4 ? units : 0);
+  L.tq = cv.take<float4>(nt);
+  L.tsph = cv.take<float4>(ntiles);
+  L.tcs = cv.take<float>(ntiles);
+  L.tam = cv.take<float>(ntiles);
+  L.tsg = cv.take<float>(ntiles);
+  L.bsph = cv.take<float4>(nb);
+  L.bcs = cv.take<float>(nb);
+  L.mask = cv.take<unsigned>((size_t)(nb * mwords));
+  L.farv = cv.take<double>((size_t)nout * far_slices(nb, mwords, num_cus()) * nt);
+  L.nn = cv.take<int>(nb);
+  L.noff = cv.take<int>(nb);
+  L.items = cv.take<int>(nb);
+  L.ioff = cv.take<int>(nb);
+  L.mfold = cv.take<int>(1);
+  L.ctr = cv.take<unsigned>(1);
+  L.count = cv.take<unsigned>(1);
+  L.iblk = cv.take<int>(maxitems);
+  L.list = cv.take<unsigned>((size_t)maxitems * FF_TB);
+  L.part = cv.take<double>((size_t)maxitems * nout * FF_TB);
+  L.bytes = cv.off;
+  return L;
+}
+
+template <int RULE, bool GRAD, int PREC>
+int64_t items_grid(size_t lds) {
+  int per_cu = 0;
+  if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, k_pf_items<RULE, GRAD, PREC>, FF_TB, lds) != hipSuccess ||
+      per_cu < 1)
+    per_cu = 1;
+  return (int64_t)per_cu * num_cus();
+}
+
+template <int RULE, bool GRAD, bool SHEET, int PREC>
+int run(const PanArgs* p, const PtPanArgs* t, void* ws, hipStream_t st) {
+  constexpr bool PART = RULE == PANFAR_PARTICLES;
+  PanFarArgs a{};
+  if (p) a.p = *p;
+  if (t) {
+    a.t = *t;
+    a.p.nx = t->nx; a.p.ny = t->ny; a.p.nz = t->nz;
+    a.p.idx = t->idx; a.p.np = t->np;
+  }
+  const int T = tile_of(RULE), U = unit_of(RULE);
+  const int64_t units = PART ? t->ns : p->np, nt = PART ? t->np : p->nt;
+  const int64_t nb = (nt + FF_TB - 1) / FF_TB;
+  const int ntiles = (int)((units + U - 1) / U), mwords = (ntiles + 31) / 32;
+  const PanFarLayout L = layout(static_cast<char*>(ws), RULE, units, nt, GRAD ? 12 : 3);
+  FFArgs& f = a.f;
+  f.sp = L.sp; f.sa = L.sa; f.tq = L.tq;
+  f.tsph = L.tsph; f.tcs = L.tcs; f.tam = L.tam; f.tsg = L.tsg; f.bsph = L.bsph; f.bcs = L.bcs;
+  f.mask = L.mask; f.farv = L.farv;
+  f.nn = L.nn; f.items = L.items; f.ioff = L.ioff; f.mfold = L.mfold; f.ctr = L.ctr; f.part = L.part;
+  f.nt = nt; f.ns = (int64_t)ntiles * T;
+  f.tile = T; f.mwords = mwords; f.ntiles = ntiles;
+  f.t.u = (float*)(PART ? t->u : p->u); f.t.v = (float*)(PART ? t->v : p->v); f.t.w = (float*)(PART ? t->w : p->w);
+  for (int k = 0; k < 9; ++k) f.t.g[k] = GRAD ? (float*)p->g[k] : nullptr;
+  a.rec = L.rec; a.cen = L.cen; a.list = L.list; a.count = L.count; a.iblk = L.iblk;
+  a.units = units; a.unit = U;
+
+  const int64_t npan = a.p.np;
+  const float* cen[3] = {L.cx, L.cy, L.cz};
+  const float* pts[3] = {PART ? t->sx : p->tx, PART ? t->sy : p->ty, PART ? t->sz : p->tz};
+  const int64_t npts = PART ? units : nt;
+  const float* const* src = PART ? pts : cen;
+  const float* const* tgt = PART ? cen : pts;
+  hipLaunchKernelGGL(k_pf_centroids, dim3(grid_of(npan, 256)), dim3(256), 0, st, a.p, L.cx, L.cy, L.cz);
+  hipLaunchKernelGGL(k_ff_bbox_init, dim3(1), dim3(64), 0, st, L.bb);
+  hipLaunchKernelGGL(k_ff_bbox, dim3(std::min(grid_of(npan, 256), FF_BBOX_GRID)), dim3(256), 0, st, cen[0], cen[1],
+                     cen[2], npan, L.bb);
+  hipLaunchKernelGGL(k_ff_bbox, dim3(std::min(grid_of(npts, 256), FF_BBOX_GRID)), dim3(256), 0, st, pts[0], pts[1],
+                     pts[2], npts, L.bb);
+  hipLaunchKernelGGL(k_ff_keys, dim3(grid_of(units, 256)), dim3(256), 0, st, src[0], src[1], src[2], units, L.bb,
+                     L.ks_in, L.is_in);
+  hipLaunchKernelGGL(k_ff_keys, dim3(grid_of(nt, 256)), dim3(256), 0, st, tgt[0], tgt[1], tgt[2], nt, L.bb, L.kt_in,
+                     L.it_in);
+  HIPCHK(hipGetLastError());
+  unsigned* keys = nullptr;
+  int *sperm = nullptr, *tperm = nullptr;
+  int rc = radix_sort_pairs(L.ks_in, L.is_in, L.ks_out, L.is_out, units, 30, L.tmp, st, &keys, &sperm);
+  if (rc != O3D_OK) return rc;
+  if ((rc = radix_sort_pairs(L.kt_in, L.it_in, L.kt_out, L.it_out, nt, 30, L.tmp, st, &keys, &tperm)) != O3D_OK)
+    return rc;
+  f.tperm = tperm;
+  hipLaunchKernelGGL((k_pf_sources<RULE>), dim3(grid_of((int64_t)ntiles * U, 256)), dim3(256), 0, st, a, sperm, L.sp,
+                     L.sa);
+  hipLaunchKernelGGL((k_pf_targets<RULE>), dim3(grid_of(nt, 256)), dim3(256), 0, st, a, tperm, L.tq);
+  hipLaunchKernelGGL(k_ff_bounds, dim3((unsigned)ntiles), dim3(256), 0, st, L.sp, L.sa, f.ns, T, L.tsph, L.tcs, L.tam,
+                     L.tsg);
+  hipLaunchKernelGGL(k_ff_bounds, dim3((unsigned)nb), dim3(256), 0, st, L.tq, (const float4*)nullptr, nt, FF_TB, L.bsph,
+                     L.bcs, (float*)nullptr, (float*)nullptr);
+  hipLaunchKernelGGL((k_ff_classify<CORE_SING>), dim3(grid_of(nb * mwords, 256)), dim3(256), 0, st, L.bsph, L.bcs, nb,
+                     L.tsph, L.tcs, ntiles, mwords, L.mask);
+  hipLaunchKernelGGL(k_ff_plan_count, dim3(grid_of(nb, 256)), dim3(256), 0, st, L.mask, nb, mwords, ntiles, L.nn);
+  HIPCHK(hipGetLastError());
+  if ((rc = exclusive_scan_i32(L.nn, L.noff, nb, st)) != O3D_OK) return rc;
+  hipLaunchKernelGGL(k_ff_plan_items, dim3(grid_of(nb, 256)), dim3(256), 0, st, L.nn, L.noff, nb, near_split(nb), L.items,
+                     L.mfold);
+  HIPCHK(hipGetLastError());
+  if ((rc = exclusive_scan_i32(L.items, L.ioff, nb, st)) != O3D_OK) return rc;
+  hipLaunchKernelGGL(k_ff_zero_u32, dim3(1), dim3(64), 0, st, L.ctr);
+  hipLaunchKernelGGL(k_ff_zero_u32, dim3(1), dim3(64), 0, st, L.count);
+
+  const int nslice = far_slices(nb, mwords, num_cus());
+  f.wslice = (mwords + nslice - 1) / nslice;
+  f.nslice = (mwords + f.wslice - 1) / f.wslice;
+  hipLaunchKernelGGL((k_ff_far<CORE_SING, GRAD, SHEET>), dim3((unsigned)nb, (unsigned)f.nslice), dim3(FF_FAR_THREADS),
+                     (ff_far_lds<CORE_SING, GRAD, SHEET>()), st, f);
+  HIPCHK(hipGetLastError());
+  const size_t lds = (size_t)U * (RULE == PANFAR_POINTS ? PAN_F4 : RULE == PANFAR_POINTS7 ? G7_F4 : 2) * sizeof(float4);
+  const int64_t maxitems = (near_split(nb) + 1) * nb;
+  const unsigned gitems = (unsigned)std::min<int64_t>(maxitems, items_grid<RULE, GRAD, PREC>(lds));
+  hipLaunchKernelGGL((k_pf_items<RULE, GRAD, PREC>), dim3(gitems), dim3(FF_TB), lds, st, a);
+  HIPCHK(hipGetLastError());
+  // at most 16 waves per CU
+  const unsigned gwalk = (unsigned)std::min<int64_t>((maxitems * FF_TB + 15) / 16, 4 * (int64_t)num_cus());
+  hipLaunchKernelGGL((k_pf_walk<RULE, GRAD, PREC>), dim3(gwalk), dim3(BLOCK), 0, st, a);
+  HIPCHK(hipGetLastError());
+  hipLaunchKernelGGL((k_ff_combine<CORE_SING, GRAD>), dim3((unsigned)nb), dim3(FF_TB), 0, st, f);
+  HIPCHK(hipGetLastError());
+  return O3D_OK;
+}
+
+template <int RULE, bool GRAD>
+int run_points(const PanArgs& p, int prec, void* ws, hipStream_t st) {
+  if (prec == PREC_COMP)
+    return p.ss ? run<RULE, GRAD, true, PREC_COMP>(&p, nullptr, ws, st) : run<RULE, GRAD, false, PREC_COMP>(&p, nullptr, ws, st);
+  return p.ss ? run<RULE, GRAD, true, PREC_FP32>(&p, nullptr, ws, st) : run<RULE, GRAD, false, PREC_FP32>(&p, nullptr, ws, st);
+}
+
+}  // namespace
+
+// Where the far field pays, on spheres of 320 to 20,480 panels and 2,048 to 131,072 points
+// in a shell around them, compensated, direct against here.  Panels on points, recursive:
+// from 1,280 panels at every count (1,280 on 2,048: 901 and 634 us; 20,480 on 2,048: 3,199
+// and 613, on 524,288: 12.1 and 6.2 ms), 320 panels from 32,768 points (1,100 and 1,009 us;
+// on 16,384: 718 and 709).  7-point rule: 1,280 panels likewise (661 and 273 us on 2,048,
+// velocity alone 872 and 825 on 131,072), 320 panels only at 131,072 points (1,269 and
+// 1,038 us; 458 and 544 at 32,768).  Particles on panels: 20,480 panels and 131,072
+// particles 1.63 and 1.74 ms, 524,288 particles 6.4 and 5.7 ms.  A call that
+// names its method or a tile is the direct kernels'.
+// Where the far field pays, on spheres of 320 to 20,480 panels and 2,048 to 131,072 points
+// in a shell around them, compensated, direct against here.  Panels on points, recursive:
+// from 1,280 panels at every count (1,280 on 2,048: 901 and 634 us; 20,480 on 2,048: 3,199
+// and 613, on 524,288: 12.1 and 6.2 ms), 320 panels from 32,768 points (1,100 and 1,009 us;
+// on 16,384: 718 and 709).  7-point rule: 1,280 panels likewise (661 and 273 us on 2,048,
+// velocity alone 872 and 825 on 131,072), 320 panels only at 131,072 points (1,269 and
+// 1,038 us; 458 and 544 at 32,768).  Particles on panels: 20,480 panels and 131,072
+// particles 1.63 and 1.74 ms, 524,288 particles 6.4 and 5.7 ms.  A call that
+// names its method or a tile is the direct kernels'.
+bool panfar_pays(int rule, int64_t units, int64_t nt, int method, int tile, int prec) {
+  if (method != O3D_METHOD_AUTO || tile > 0 || prec == PREC_FP64 || units > (1 << 26) || nt > (1 << 26)) return false;
+  if (rule == PANFAR_PARTICLES) return units >= 262144 && nt >= 16384;
+  if (units < 256 || nt < 2048) return false;
+  return units >= 1024 || units * nt >= (rule == PANFAR_POINTS7 ? 40000000 : 10000000);
+}
+
+size_t panfar_bytes(int rule, int64_t units, int64_t nt, bool grad) {
+  return layout(nullptr, rule, units, nt, grad ? 12 : 3).bytes;
+}
+
+bool panfar_scratch(size_t bytes, hipStream_t st, void** ws) {
+  if (stream_capturing(st) && !stream_workspace_fits(st, bytes)) return false;
+  if (stream_workspace(st, bytes, ws) == O3D_OK) return true;
+  clear_error();
+  (void)hipGetLastError();
+  return false;
+}
+
+int panfar_points(const PanArgs& p, int rule, bool grad, int prec, void* ws, hipStream_t st) {
+  if (rule == PANFAR_POINTS7)
+    return grad ? run_points<PANFAR_POINTS7, true>(p, prec, ws, st) : run_points<PANFAR_POINTS7, false>(p, prec, ws, st);
+  return grad ? run_points<PANFAR_POINTS, true>(p, prec, ws, st) : run_points<PANFAR_POINTS, false>(p, prec, ws, st);
+}
+
+int panfar_particles(const PtPanArgs& t, int prec, void* ws, hipStream_t st) {
+  return prec == PREC_COMP ? run<PANFAR_PARTICLES, false, false, PREC_COMP>(nullptr, &t, ws, st)
+                           : run<PANFAR_PARTICLES, false, false, PREC_FP32>(nullptr, &t, ws, st);
+}
+
+}  // namespace o3d

@@ -17,9 +17,11 @@
 // also keeps the first few such particles of each (slice, panel) in ascending
 // order.  k_ptpan_near gives each listed panel one wave whose lanes walk those
 // pairs with the depth-first tree walk of panels_affect_points (pan_kernels.hpp),
-// so the subdivision decisions are the reference's.
+// so the subdivision decisions are the reference's.  Large calls take the separated
+// pairs to the matrix cores (panfar.hip).
 #include "o3d_api_internal.hpp"
-#include "pan_kernels.hpp"
+#include "panfar.hpp"
+#include "ptpan_kernels.hpp"
 
 #include <algorithm>
 #include <chrono>
@@ -27,69 +29,12 @@
 
 namespace o3d {
 
-struct PtPanArgs {
-  const float* sx; const float* sy; const float* sz;    // particles
-  const float* ax; const float* ay; const float* az;
-  int64_t ns;
-  const float* nx; const float* ny; const float* nz;    // panel nodes
-  const uint32_t* idx;
-  const float* area;
-  int64_t np;
-  void* u; void* v; void* w;   // float (decremented in place) or double (FP64: zeroed scratch)
-  int32_t tile;
-  int32_t maxlev;
-  int32_t* near_list;          // panels with a pair that needs the recursion
-  unsigned int* near_count;
-  double* part;                // per slice: 3 sums per panel
-  int32_t* cnt;                // [panel][slice]: particles that need the recursion
-  int32_t* ent;                // [panel][slice][PTPAN_CAP]: the first of them, ascending
-  int64_t slen;                // particles per slice
-  int32_t nslice;
-};
-
-// particles kept per (slice, panel) for the near kernel; a slice with more is
-// scanned again there
-constexpr int PTPAN_CAP = 8;
-
-// this lane's panel in the staged-panel layout of pan_kernels.hpp (the strength
-// fields are filled per particle)
-__device__ __forceinline__ void ptpan_record(const PtPanArgs& a, int64_t i, float4* s) {
-  const uint32_t i0 = a.idx[3 * i], i1 = a.idx[3 * i + 1], i2 = a.idx[3 * i + 2];
-  const float x0 = a.nx[i0], y0 = a.ny[i0], z0 = a.nz[i0];
-  const float x1 = a.nx[i1], y1 = a.ny[i1], z1 = a.nz[i1];
-  const float x2 = a.nx[i2], y2 = a.ny[i2], z2 = a.nz[i2];
-  const float ar = a.area[i];
-  float cx, cy, cz;
-  centroid_exact(x0, y0, z0, x1, y1, z1, x2, y2, z2, cx, cy, cz);
-  s[0] = make_float4(x0, y0, z0, x1);
-  s[1] = make_float4(y1, z1, x2, y2);
-  s[2] = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
-  float far2, near2;
-  root_bands(sqrtf(ar), far2, near2);
-  s[3] = make_float4(cx, cy, cz, far2);
-  s[4] = make_float4(z2, ar, sqrtf(ar), near2);
-  s[5] = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
-}
-
-// particle j's strength on panel record s at level 0.  FP64: the walk forms
-// (alpha / area) * area in double from s[5].  FP32 and compensated: alpha itself;
-// the reference's float round trip (alpha / area) * area (Influence.h:1198,
-// Kernels.h:1136-1146) moves it by at most one float ulp and costs three IEEE
-// divisions per pair.
-template <int PREC>
-__device__ __forceinline__ void ptpan_strength(float4* s, float4 A) {
-  if (PREC == PREC_FP64) s[5] = make_float4(A.x, A.y, A.z, 0.0f);
-  else { s[2].x = A.x; s[2].y = A.y; s[2].z = A.z; }
-}
-
 // One lane per target panel, particles [y*slen, (y+1)*slen) of slice y =
 // blockIdx.y staged per tile in LDS: the root decision of every (panel, particle)
 // pair -- the reference's, through root_leaf -- and the pairs that are leaves at
 // the root.  Each slice leaves its sum (FP64) in part[y][0..2][panel], the count
 // of pairs that need the recursion in cnt and the first PTPAN_CAP of their
 // particles in ent; k_ptpan_combine adds the slices in order.
-constexpr int PTPAN_UNROLL = 4;   // particles per step of k_ptpan's separated-pair loop
-
 template <int PREC>
 __global__ __launch_bounds__(BLOCK) void k_ptpan(PtPanArgs a) {
   using R = typename std::conditional<PREC == PREC_FP64, double, float>::type;
@@ -99,16 +44,12 @@ __global__ __launch_bounds__(BLOCK) void k_ptpan(PtPanArgs a) {
   const int64_t ic = active ? i : a.np - 1;
   float4 s[PAN_F4];
   ptpan_record(a, ic, s);
-  const float ar = s[4].y;
   R acc[16];
 #pragma unroll
   for (int c = 0; c < 16; ++c) acc[c] = R(0);
   float hi[3] = {0.f, 0.f, 0.f}, lo[3] = {0.f, 0.f, 0.f};
   int nnear = 0;
   int32_t* ent = a.ent + ((int64_t)ic * a.nslice + blockIdx.y) * PTPAN_CAP;
-  R gx, gy, gz, gs, cx0, cy0, cz0, lim;
-  RootLim rl;
-  panel_root<R>(s, gx, gy, gz, gs, cx0, cy0, cz0, lim, rl);
   const int64_t q0 = (int64_t)blockIdx.y * a.slen;
   const int64_t q1 = q0 + a.slen < a.ns ? q0 + a.slen : a.ns;
 
@@ -121,55 +62,7 @@ __global__ __launch_bounds__(BLOCK) void k_ptpan(PtPanArgs a) {
       shs[2 * j + 1] = make_float4(a.ax[g], a.ay[g], a.az[g], 0.0f);
     }
     __syncthreads();
-    // the root decision of particle j of the tile: a leaf is evaluated, a recursed
-    // pair listed
-    auto pair = [&](const float4 P, const float4 A, int j) {
-      if (root_leaf<R>(P.x, P.y, P.z, cx0, cy0, cz0, lim, rl, a.maxlev, active)) {
-        if (!active) return;
-        R ax, ay, az;
-        if (PREC == PREC_FP64) {
-#pragma clang fp contract(off)
-          ax = (R(A.x) / R(ar)) * R(ar); ay = (R(A.y) / R(ar)) * R(ar); az = (R(A.z) / R(ar)) * R(ar);
-        } else {
-          ax = A.x; ay = A.y; az = A.z;
-        }
-        leaf_acc<R, false>(P.x, P.y, P.z, cx0, cy0, cz0, ax, ay, az, R(0), acc);
-      } else if (active) {
-        if (nnear < PTPAN_CAP) ent[nnear] = (int32_t)(p0 + j);
-        ++nnear;
-      }
-    };
-    int j = 0;
-    if constexpr (sizeof(R) == 4) {
-      // PTPAN_UNROLL particles at a time while they are surely beyond every lane's
-      // far band: one scalar branch on the OR of the ballots, the leaves with no
-      // per-pair mask, the LDS address in a vector register (made so by an opaque
-      // zero); the same leaves in the same order as the per-pair path, and an idle
-      // lane's sums are dropped
-      int vz;
-      asm volatile("v_mov_b32 %0, 0" : "=v"(vz));
-      const float4* q = shs + vz;
-      for (; j + PTPAN_UNROLL <= cnt; j += PTPAN_UNROLL, q += 2 * PTPAN_UNROLL) {
-        float4 P[PTPAN_UNROLL], A[PTPAN_UNROLL];
-        uint64_t near = 0;
-#pragma unroll
-        for (int u = 0; u < PTPAN_UNROLL; ++u) {
-          P[u] = q[2 * u];
-          A[u] = q[2 * u + 1];
-          const float ex = P[u].x - cx0, ey = P[u].y - cy0, ez = P[u].z - cz0;
-          near |= __builtin_amdgcn_ballot_w64(!(fmaf(ez, ez, fmaf(ey, ey, ex * ex)) > rl.far2));
-        }
-        if (near == 0) {
-#pragma unroll
-          for (int u = 0; u < PTPAN_UNROLL; ++u)
-            leaf_acc<R, false>(P[u].x, P[u].y, P[u].z, cx0, cy0, cz0, A[u].x, A[u].y, A[u].z, R(0), acc);
-        } else {
-#pragma unroll
-          for (int u = 0; u < PTPAN_UNROLL; ++u) pair(P[u], A[u], j + u);
-        }
-      }
-    }
-    for (; j < cnt; ++j) pair(shs[2 * j], shs[2 * j + 1], j);
+    ptpan_root_tile<PREC, true>(shs, cnt, p0, s, a.maxlev, active, acc, ent, nnear);
     if (PREC == PREC_COMP) {
       two_sum(hi[0], lo[0], (float)acc[0]);
       two_sum(hi[1], lo[1], (float)acc[1]);
@@ -293,7 +186,8 @@ __global__ void k_ptpan_zero(unsigned int* c) {
 // root pairs over particle slices, their combination, then the near pairs of the
 // listed panels; the partial sums, the list and its counter in the stream's
 // workspace.  Enough slices of whole tiles for about 16 workgroups per CU.
-static int launch_ptpan(PtPanArgs a, int prec, hipStream_t st) {
+static int launch_ptpan(PtPanArgs a, const o3d_opts* o, hipStream_t st) {
+  const int prec = o->precision;
   if (a.np <= 0 || a.ns <= 0) return O3D_OK;
   if (a.np > INT32_MAX) return fail(O3D_EINVAL, "points_affect_panels takes at most %d panels", INT32_MAX);
   if (a.ns > INT32_MAX) return fail(O3D_EINVAL, "points_affect_panels takes at most %d particles", INT32_MAX);
@@ -305,6 +199,9 @@ static int launch_ptpan(PtPanArgs a, int prec, hipStream_t st) {
   a.nslice = (int32_t)((a.ns + a.slen - 1) / a.slen);
   std::lock_guard<std::mutex> lk(stream_ws_mutex());
   void* ws = nullptr;
+  if (panfar_pays(PANFAR_PARTICLES, a.ns, a.np, o->method, o->tile, prec) &&
+      panfar_scratch(panfar_bytes(PANFAR_PARTICLES, a.ns, a.np, false), st, &ws))
+    return panfar_particles(a, prec, ws, st);
   const size_t list = (sizeof(int32_t) * (size_t)a.np + 255) & ~(size_t)255;
   const size_t part = sizeof(double) * 3 * (size_t)a.nslice * (size_t)a.np;
   const size_t cnt = (sizeof(int32_t) * (size_t)a.nslice * (size_t)a.np + 255) & ~(size_t)255;
@@ -522,7 +419,7 @@ int o3d_points_affect_panels(const o3d_points* src, const o3d_panels* targ, floa
     if (!f64)
       for (int k = 0; k < 3; ++k)
         HIPCHK(hipMemcpyAsync(vb + vsz * np * k, vel[k], sizeof(float) * np, hipMemcpyHostToDevice, st));
-    if ((rc = launch_ptpan(a, o->precision, st)) != O3D_OK) return rc;
+    if ((rc = launch_ptpan(a, o, st)) != O3D_OK) return rc;
     if (f64) {
       std::vector<double> h((size_t)3 * np);
       HIPCHK(hipMemcpyAsync(h.data(), vb, vbytes, hipMemcpyDeviceToHost, st));
@@ -552,7 +449,7 @@ int o3d_points_affect_panels_dev(const o3d_points* src, const o3d_panels* targ, 
   if (src->n > 0 && targ->np > 0) {
     PtPanArgs a = ptpan_args(src, targ, o);
     a.u = vel[0]; a.v = vel[1]; a.w = vel[2];
-    if ((rc = launch_ptpan(a, o->precision, (hipStream_t)o->stream)) != O3D_OK) return rc;
+    if ((rc = launch_ptpan(a, o, (hipStream_t)o->stream)) != O3D_OK) return rc;
   }
   fill_stats(stats, 0.0, ptpan_flops(targ->np, src->n), (double)targ->np * (double)src->n);
   return O3D_OK;
@@ -598,7 +495,7 @@ int o3d_bem_rhs_dev(const o3d_points* vort, int32_t nvort, const o3d_panels* bdr
     if (vort[k].n == 0) continue;
     PtPanArgs pa = ptpan_args(&vort[k], bdry, opts);
     pa.u = pu[0]; pa.v = pu[1]; pa.w = pu[2];
-    if ((rc = launch_ptpan(pa, opts->precision, st)) != O3D_OK) return rc;
+    if ((rc = launch_ptpan(pa, opts, st)) != O3D_OK) return rc;
   }
   hipLaunchKernelGGL(k_bem_rhs, dim3((unsigned)((a.np + BLOCK - 1) / BLOCK)), dim3(BLOCK), 0, st, a);
   HIPCHK(hipGetLastError());

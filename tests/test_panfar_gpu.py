@@ -1,0 +1,110 @@
+"""Panel sums whose separated pairs go to the matrix cores (panfar.hip): large calls with
+the tile left open, against the oracle on some targets and against the direct kernels (a
+tile given) on all.
+
+Bars, in units of the largest value: the oracle's as for the direct kernels
+(test_pan_gpu.py: max(2e-6, 3 x the float reference's own distance from FP64); 7-point
+rule 2e-6); between the two GPU paths, which take the same decision for every pair, twice
+2e-6 in compensated precision, and in FP32, whose direct kernel adds up to `np` (7 np)
+terms in one float, 2e-6 + 4e-6 as for a random walk of 2,500 roundings of 6e-8.
+"""
+import ctypes as C
+
+import numpy as np
+import pytest
+
+import oracle
+from omega3d_amd import scenes
+from omega3d_amd.metrics import rel_errors
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.fixture(scope="module")
+def mods():
+    torch = pytest.importorskip("torch")
+    from omega3d_amd import _lib, influence
+    assert _lib.lib.o3d_init(-1) == 0, _lib.last_error()
+    return torch, _lib, influence
+
+
+def _call(mods, pan, n, tp, grads, prec, method, tile, ss=True, maxlev=-1, scale=1.0, area=None):
+    """panels_affect_points on device arrays: velocity and gradient (12 or 3, nt)"""
+    torch, _lib, influence = mods
+    dev = lambda x: torch.tensor(np.ascontiguousarray(x), device="cuda")
+    nodes, idx = dev(pan.nodes.astype(np.float32)), dev(pan.idx[:3 * n].astype(np.int32))
+    ts = dev((pan.ts[:, :n] * scale).astype(np.float32))
+    ar = dev((pan.area if area is None else area)[:n].astype(np.float32))
+    s = dev((pan.ss[:n] * scale).astype(np.float32)) if ss else None
+    t, out = dev(tp.astype(np.float32)), torch.zeros(12 if grads else 3, tp.shape[1], device="cuda")
+    p, q = _lib.Panels(), _lib.Points()
+    p.np, p.nn, p.idx, p.area = n, nodes.shape[1], idx.data_ptr(), ar.data_ptr()
+    p.ss = s.data_ptr() if ss else None
+    q.n = tp.shape[1]
+    for d in range(3):
+        p.x[d], p.ts[d], q.x[d], q.u[d] = (a[d].data_ptr() for a in (nodes, ts, t, out))
+    for k in range(9 if grads else 0):
+        q.ug[k] = out[3 + k].data_ptr()
+    o = _lib.make_opts("rm", grads, prec, method=method, tile=tile, maxlev=maxlev)
+    _lib.check(_lib.lib.o3d_panels_affect_points_dev(C.byref(p), C.byref(q), C.byref(o), None))
+    torch.cuda.synchronize()
+    return out.cpu().numpy()
+
+
+def _surface():
+    pan = scenes.icosphere_panels(levels=3)   # 1,280 panels
+    pan.ss = (0.3 * np.random.default_rng(3).normal(size=pan.np)).astype(np.float32)
+    return pan
+
+
+def _bar(a, b, tol):
+    for rows in ([slice(0, 3)] if a.shape[0] == 3 else [slice(0, 3), slice(3, 12)]):
+        assert rel_errors(a[rows], b[rows])[0] <= tol
+
+
+@pytest.mark.parametrize("method", ["auto", "gauss7"])
+@pytest.mark.parametrize("n,nt,grads,ss,prec,maxlev", [
+    (1280, 2048, True, True, "comp", -1),     # whole tiles and blocks
+    (1280, 2049, True, False, "comp", 2),     # a block of one target
+    (1281 - 256, 2303, False, True, "comp", -1),   # a tile of one panel
+    (1024, 5000, False, False, "comp", 0),
+    (1153, 2304, True, True, "fp32", -1),
+    (1279, 2100, False, False, "fp32", 1)])
+def test_separated_panels(mods, method, n, nt, grads, ss, prec, maxlev):
+    pan = _surface()
+    tp = scenes.shell_points(nt, 1.02, 3.0, seed=nt)
+    a = _call(mods, pan, n, tp, grads, prec, method, 0, ss, maxlev)
+    b = _call(mods, pan, n, tp, grads, prec, method, 128, ss, maxlev)
+    assert not np.array_equal(a, b)   # the far field took part
+    _bar(a, b, 6e-6 if prec == "fp32" else 4e-6)
+    k = np.random.default_rng(1).choice(nt, 150, replace=False)
+    if method == "gauss7":
+        o = oracle.pan_g7(pan.nodes, pan.idx[:3 * n], pan.ts[:, :n], pan.area[:n], pan.ss[:n] if ss else None, tp[:, k],
+                          grads=grads)
+        _bar(a[:, k], np.concatenate(o[:2] if grads else o[:1]), 6e-6 if prec == "fp32" else 2e-6)
+    else:
+        args = ("rm", pan.nodes, pan.idx[:3 * n], pan.ts[:, :n], pan.area[:n], pan.ss[:n] if ss else None, tp[:, k], grads)
+        o64, o32 = (np.concatenate([x for x in oracle.pan(*args, mode, maxlev=3 if maxlev < 0 else maxlev) if x is not None])
+                    for mode in ("f64", "f32d"))
+        for rows in ([slice(0, 3), slice(3, 12)] if grads else [slice(0, 3)]):
+            bar = max(2e-6 if prec == "comp" else 6e-6, 3 * rel_errors(o32[rows], o64[rows])[0])
+            assert rel_errors(a[rows][:, k], o64[rows])[0] <= bar
+
+
+@pytest.mark.parametrize("method", ["auto", "gauss7"])
+def test_scaling_and_places(mods, method):
+    """strengths times -1 and times powers of two give just that, and points far away, all in
+    one place or beside panels whose area is no number are summed as the direct kernels do"""
+    pan = _surface()
+    n, tp = pan.np, scenes.shell_points(3000, 1.02, 1.5, seed=9)
+    a = _call(mods, pan, n, tp, True, "comp", method, 0)
+    for f in (-1.0, 2.0, -2.0 ** -20, 2.0 ** 80):
+        assert np.array_equal(_call(mods, pan, n, tp, True, "comp", method, 0, scale=f), a * np.float32(f))
+    for far in (tp + 50.0, np.repeat(tp[:, :1], 2500, 1), np.concatenate([tp[:, :1300], 1e4 * tp[:, :1300]], 1)):
+        _bar(_call(mods, pan, n, far, True, "comp", method, 0), _call(mods, pan, n, far, True, "comp", method, 128), 4e-6)
+    if method == "auto":
+        area = pan.area.copy()
+        area[77] = -area[77]
+        x = _call(mods, pan, n, tp, True, "comp", method, 0, area=area, maxlev=1)
+        y = _call(mods, pan, n, tp, True, "comp", method, 128, area=area, maxlev=1)
+        _bar(x, y, 4e-6)
