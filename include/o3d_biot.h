@@ -58,7 +58,7 @@ enum o3d_self { O3D_SELF_INCLUDE = 0, O3D_SELF_EXCLUDE = 1 };
  *   DIRECT:   one pair at a time on the vector ALUs, sources in index order (an
  *             EXP call of >= 32,768 targets on one collection, tile and tpt left
  *             at 0, reads them in the targets' Morton order instead).
- *   FACTORED: particles in Morton order; a source tile well separated from a
+ *   FACTORED: particles in Hilbert order; a source tile well separated from a
  *             target block is summed through an exact factorisation
  *             K = Bp (|t'|^2 - 2 t'.s' + |s'|^2 + cores) as a product of the pair
  *             weights with a 29-column per-source moment table on the matrix
@@ -290,7 +290,7 @@ int o3d_bem_matrix_profile_dev(const o3d_panels* src, const o3d_panels* targ, in
 
 /* Diagnostics of the factored method (no counterpart in the reference): runs one
  * o3d_points_affect_points_dev evaluation with method FACTORED on device arrays,
- * synchronises, and reports the time of its stages (preparation: box, Morton keys,
+ * synchronises, and reports the time of its stages (preparation: box, Hilbert keys,
  * sort, gathers, bounds, classification; far field on the matrix cores; near field
  * and output) and the number of (target, source) pairs taken by the far field.
  * Results are accumulated as by the plain call. */

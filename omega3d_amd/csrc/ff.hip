@@ -1,7 +1,7 @@
 // ff.hip -- host side of the factored far-field evaluation (method "factored").
 //
 // One call enqueues, on the caller's stream and without synchronising:
-//   bounding box -> Morton keys -> radix sort (sort.hip) of sources (and of targets
+//   bounding box -> Hilbert keys -> radix sort (sort.hip) of sources (and of targets
 //   when they are a different collection) -> gather into sorted float4 rows ->
 //   bounding spheres of source tiles and target blocks -> far/near bit per
 //   (block, tile) -> far-field kernel (matrix cores) -> near-field kernel, which
@@ -145,7 +145,7 @@ int run(const o3d_points* src, o3d_points* targ, bool self_excl, int T, hipStrea
   if (!same)
     hipLaunchKernelGGL(k_ff_bbox, dim3(std::min(grid_of(nt, 256), FF_BBOX_GRID)), dim3(256), 0, st, tv.x, tv.y, tv.z, nt,
                        L.bb);
-  hipLaunchKernelGGL(k_ff_keys, dim3(grid_of(ns, 256)), dim3(256), 0, st, sv.x, sv.y, sv.z, ns, L.bb, L.ks_in, L.is_in);
+  hipLaunchKernelGGL((k_ff_keys<true>), dim3(grid_of(ns, 256)), dim3(256), 0, st, sv.x, sv.y, sv.z, ns, L.bb, L.ks_in, L.is_in);
   HIPCHK(hipGetLastError());
   unsigned* skeys = nullptr;
   int* sperm = nullptr;
@@ -153,7 +153,7 @@ int run(const o3d_points* src, o3d_points* targ, bool self_excl, int T, hipStrea
   if (rc != O3D_OK) return rc;
   const int* tperm = sperm;
   if (!same) {
-    hipLaunchKernelGGL(k_ff_keys, dim3(grid_of(nt, 256)), dim3(256), 0, st, tv.x, tv.y, tv.z, nt, L.bb, L.kt_in, L.it_in);
+    hipLaunchKernelGGL((k_ff_keys<true>), dim3(grid_of(nt, 256)), dim3(256), 0, st, tv.x, tv.y, tv.z, nt, L.bb, L.kt_in, L.it_in);
     HIPCHK(hipGetLastError());
     unsigned* tkeys = nullptr;
     int* tp = nullptr;
@@ -262,7 +262,7 @@ int point_order(const float* x, const float* y, const float* z, int64_t n, void*
   void* tmp = p + 256 + 4 * a;
   hipLaunchKernelGGL(k_ff_bbox_init, dim3(1), dim3(64), 0, st, bb);
   hipLaunchKernelGGL(k_ff_bbox, dim3(std::min(grid_of(n, 256), FF_BBOX_GRID)), dim3(256), 0, st, x, y, z, n, bb);
-  hipLaunchKernelGGL(k_ff_keys, dim3(grid_of(n, 256)), dim3(256), 0, st, x, y, z, n, bb, kin, iin);
+  hipLaunchKernelGGL((k_ff_keys<false>), dim3(grid_of(n, 256)), dim3(256), 0, st, x, y, z, n, bb, kin, iin);
   HIPCHK(hipGetLastError());
   unsigned* sk = nullptr;
   int* sp = nullptr;
@@ -439,7 +439,7 @@ extern "C" int o3d_morton_order_dev(const float* x, const float* y, const float*
   if ((rc = point_order(x, y, z, n, ws, st, &p)) != O3D_OK) return rc;
   HIPCHK(hipMemcpyAsync(perm, p, sizeof(int32_t) * (size_t)n, hipMemcpyDeviceToDevice, st));
   // the keys in index order, from the same box (point_order left it at the workspace's start)
-  hipLaunchKernelGGL(k_ff_keys, dim3(grid_of(n, 256)), dim3(256), 0, st, x, y, z, n, (const unsigned*)ws,
+  hipLaunchKernelGGL((k_ff_keys<false>), dim3(grid_of(n, 256)), dim3(256), 0, st, x, y, z, n, (const unsigned*)ws,
                      (unsigned*)keys, (int*)nullptr);
   HIPCHK(hipGetLastError());
   return O3D_OK;

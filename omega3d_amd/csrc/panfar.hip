@@ -2,7 +2,7 @@
 //
 // A panel far from a target is one singular point (recursive rule, pan_kernels.hpp; the
 // roles reversed for particles -> panels, ptpan.hip) or seven of them (7-point rule,
-// pan_g7.hpp).  Panels and points are put in Morton order, and a block of 256 targets
+// pan_g7.hpp).  Panels and points are sorted along a Hilbert curve, and a block of 256 targets
 // takes the tiles of sources that lie a block radius away, and beyond every distance at
 // which one of the pairs would not be plain, through k_ff_far (ff_kernels.hpp).  The
 // other tiles go through the code of the direct kernels, tile by tile in work items of a
@@ -47,7 +47,7 @@ struct PanFarArgs {
 // limit that is no number keeps the panel out of the far field
 __device__ __forceinline__ float plain_limit(float lim) { return lim >= 0.0f ? lim * 1.00001f : __builtin_huge_valf(); }
 
-// centroids of the panels for the Morton order (as the decisions take them)
+// centroids of the panels for the order (as the decisions take them)
 __global__ __launch_bounds__(256) void k_pf_centroids(PanArgs a, float* x, float* y, float* z) {
   const int64_t p = (int64_t)blockIdx.x * 256 + threadIdx.x;
   if (p >= a.np) return;
@@ -507,9 +507,9 @@ int run(const PanArgs* p, const PtPanArgs* t, void* ws, hipStream_t st) {
                      cen[2], npan, L.bb);
   hipLaunchKernelGGL(k_ff_bbox, dim3(std::min(grid_of(npts, 256), FF_BBOX_GRID)), dim3(256), 0, st, pts[0], pts[1],
                      pts[2], npts, L.bb);
-  hipLaunchKernelGGL(k_ff_keys, dim3(grid_of(units, 256)), dim3(256), 0, st, src[0], src[1], src[2], units, L.bb,
+  hipLaunchKernelGGL((k_ff_keys<true>), dim3(grid_of(units, 256)), dim3(256), 0, st, src[0], src[1], src[2], units, L.bb,
                      L.ks_in, L.is_in);
-  hipLaunchKernelGGL(k_ff_keys, dim3(grid_of(nt, 256)), dim3(256), 0, st, tgt[0], tgt[1], tgt[2], nt, L.bb, L.kt_in,
+  hipLaunchKernelGGL((k_ff_keys<true>), dim3(grid_of(nt, 256)), dim3(256), 0, st, tgt[0], tgt[1], tgt[2], nt, L.bb, L.kt_in,
                      L.it_in);
   HIPCHK(hipGetLastError());
   unsigned* keys = nullptr;
