@@ -158,8 +158,9 @@ __device__ __forceinline__ void pf_item(const PanFarArgs& a, int64_t b, int item
   const bool active = i < a.f.nt;
   const int64_t ic = active ? i : a.f.nt - 1;
   const float4 q = a.f.tq[ic];
-  float4 s[PAN_F4];
+  float4 s[PAN_F4] = {};
   if (RULE == PANFAR_PARTICLES) ptpan_record(a.t, a.f.tperm[ic], s);
+  const PtRoot<float> root(s);
   float acc[16];
   float hi[3] = {0.f, 0.f, 0.f}, lo[3] = {0.f, 0.f, 0.f};
   double gd[9] = {0, 0, 0, 0, 0, 0, 0, 0, 0};
@@ -193,7 +194,7 @@ __device__ __forceinline__ void pf_item(const PanFarArgs& a, int64_t b, int item
         }
       } else {
         int nnear = 0;
-        ptpan_root_tile<PREC, false>(w, n, p0 + j0, s, a.t.maxlev, active, acc, nullptr, nnear);
+        ptpan_root_tile<PREC, false>(w, n, p0 + j0, root, a.t.maxlev, active, acc, nullptr, nnear);
         has_near |= nnear > 0;
       }
       if (PREC == PREC_COMP) {

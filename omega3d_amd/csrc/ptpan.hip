@@ -44,6 +44,7 @@ __global__ __launch_bounds__(BLOCK) void k_ptpan(PtPanArgs a) {
   const int64_t ic = active ? i : a.np - 1;
   float4 s[PAN_F4];
   ptpan_record(a, ic, s);
+  const PtRoot<R> root(s);
   R acc[16];
 #pragma unroll
   for (int c = 0; c < 16; ++c) acc[c] = R(0);
@@ -62,7 +63,7 @@ __global__ __launch_bounds__(BLOCK) void k_ptpan(PtPanArgs a) {
       shs[2 * j + 1] = make_float4(a.ax[g], a.ay[g], a.az[g], 0.0f);
     }
     __syncthreads();
-    ptpan_root_tile<PREC, true>(shs, cnt, p0, s, a.maxlev, active, acc, ent, nnear);
+    ptpan_root_tile<PREC, true>(shs, cnt, p0, root, a.maxlev, active, acc, ent, nnear);
     if (PREC == PREC_COMP) {
       two_sum(hi[0], lo[0], (float)acc[0]);
       two_sum(hi[1], lo[1], (float)acc[1]);

@@ -63,29 +63,40 @@ __device__ __forceinline__ void ptpan_strength(float4* s, float4 A) {
 
 constexpr int PTPAN_UNROLL = 4;   // particles per step of the separated-pair loop
 
-// the staged particles 0 .. cnt - 1 ({x, y, z}, {alpha} in turn; numbered from p0) on this
-// lane's panel (record s): the pairs that are leaves at the root are added to acc, the
-// particles of the others counted in nnear and, with LIST, the first PTPAN_CAP noted in ent
-template <int PREC, bool LIST, class R>
-__device__ __forceinline__ void ptpan_root_tile(const float4* shs, int cnt, int64_t p0, const float4* s, int maxlev,
-                                                bool active, R* acc, int32_t* ent, int& nnear) {
-  const float ar = s[4].y;
-  R gx, gy, gz, gs, cx0, cy0, cz0, lim;
+// what the root decision of a target panel needs of its record
+template <class R>
+struct PtRoot {
+  R cx, cy, cz, lim;
   RootLim rl;
-  panel_root<R>(s, gx, gy, gz, gs, cx0, cy0, cz0, lim, rl);
+  float area;
+  __device__ __forceinline__ explicit PtRoot(const float4* s) : area(s[4].y) {
+    R gx, gy, gz, gs;
+    panel_root<R>(s, gx, gy, gz, gs, cx, cy, cz, lim, rl);
+  }
+};
+
+// the staged particles 0 .. cnt - 1 ({x, y, z}, {alpha} in turn; numbered from p0) on this
+// lane's panel: the pairs that are leaves at the root are added to sums, the
+// particles of the others counted in listed and, with LIST, the first PTPAN_CAP noted in ent
+template <int PREC, bool LIST, class R>
+__device__ __forceinline__ void ptpan_root_tile(const float4* shs, int cnt, int64_t p0, const PtRoot<R>& t, int maxlev,
+                                                bool active, R* sums, int32_t* ent, int& listed) {
+  R acc[3] = {sums[0], sums[1], sums[2]};   // local copies stay in registers
+  int nnear = listed;
   // the root decision of particle j of the tile: a leaf is evaluated, a recursed
   // pair listed
   auto pair = [&](const float4 P, const float4 A, int j) {
-    if (root_leaf<R>(P.x, P.y, P.z, cx0, cy0, cz0, lim, rl, maxlev, active)) {
+    if (root_leaf<R>(P.x, P.y, P.z, t.cx, t.cy, t.cz, t.lim, t.rl, maxlev, active)) {
       if (!active) return;
       R ax, ay, az;
       if (PREC == PREC_FP64) {
 #pragma clang fp contract(off)
-        ax = (R(A.x) / R(ar)) * R(ar); ay = (R(A.y) / R(ar)) * R(ar); az = (R(A.z) / R(ar)) * R(ar);
+        const R ar = t.area;
+        ax = (R(A.x) / ar) * ar; ay = (R(A.y) / ar) * ar; az = (R(A.z) / ar) * ar;
       } else {
         ax = A.x; ay = A.y; az = A.z;
       }
-      leaf_acc<R, false>(P.x, P.y, P.z, cx0, cy0, cz0, ax, ay, az, R(0), acc);
+      leaf_acc<R, false>(P.x, P.y, P.z, t.cx, t.cy, t.cz, ax, ay, az, R(0), acc);
     } else if (active) {
       if (LIST && nnear < PTPAN_CAP) ent[nnear] = (int32_t)(p0 + j);
       ++nnear;
@@ -108,13 +119,13 @@ __device__ __forceinline__ void ptpan_root_tile(const float4* shs, int cnt, int6
       for (int u = 0; u < PTPAN_UNROLL; ++u) {
         P[u] = q[2 * u];
         A[u] = q[2 * u + 1];
-        const float ex = P[u].x - cx0, ey = P[u].y - cy0, ez = P[u].z - cz0;
-        near |= __builtin_amdgcn_ballot_w64(!(fmaf(ez, ez, fmaf(ey, ey, ex * ex)) > rl.far2));
+        const float ex = P[u].x - t.cx, ey = P[u].y - t.cy, ez = P[u].z - t.cz;
+        near |= __builtin_amdgcn_ballot_w64(!(fmaf(ez, ez, fmaf(ey, ey, ex * ex)) > t.rl.far2));
       }
       if (near == 0) {
 #pragma unroll
         for (int u = 0; u < PTPAN_UNROLL; ++u)
-          leaf_acc<R, false>(P[u].x, P[u].y, P[u].z, cx0, cy0, cz0, A[u].x, A[u].y, A[u].z, R(0), acc);
+          leaf_acc<R, false>(P[u].x, P[u].y, P[u].z, t.cx, t.cy, t.cz, A[u].x, A[u].y, A[u].z, R(0), acc);
       } else {
 #pragma unroll
         for (int u = 0; u < PTPAN_UNROLL; ++u) pair(P[u], A[u], j + u);
@@ -122,6 +133,8 @@ __device__ __forceinline__ void ptpan_root_tile(const float4* shs, int cnt, int6
     }
   }
   for (; j < cnt; ++j) pair(shs[2 * j], shs[2 * j + 1], j);
+  sums[0] = acc[0]; sums[1] = acc[1]; sums[2] = acc[2];
+  listed = nnear;
 }
 
 }  // namespace o3d
