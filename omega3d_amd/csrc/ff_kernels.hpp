@@ -37,6 +37,14 @@
 // the direct per-pair code in original coordinates, so near pairs keep exact
 // differences t - s.
 //
+// The centre may be any point: a tile that is smaller than the block and one of its own
+// radii away is far as well, with its own centre in place of the block's (the same bound
+// by symmetry).  It is then summed by itself, and its gap is at least a third of the
+// block's radius, so that the block's weights, scaled for the nearest target, keep their
+// 22 bits at the farthest ((1 / 7)^5 of 2^13 is above 2^-3).  Few targets, wide blocks:
+// pairs left near 21 -> 11% for 524,288 particles on 20,480 panels, 15 -> 8% for 65,537
+// points in a box around two rings of 100,002 (whole calls 5.13 -> 4.58 and 2.16 -> 2.00 ms).
+//
 // Particles are sorted along a Hilbert curve first (keys on a 10-bit grid per axis) so
 // that blocks and tiles are compact; the decision per (block, tile) is computed
 // once into a bit mask read by both kernels.  The curve has no jumps: in Morton order a
@@ -69,7 +77,8 @@ typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
 // of a row is the distance from there beyond which a pair is a plain point pair
 constexpr int CORE_SING = 0;
 constexpr int FF_TB = 256;          // targets per workgroup: 4 waves x 64
-constexpr float FF_KAPPA = 1.0f;    // minimum gap, in block radii
+constexpr float FF_KAPPA = 1.0f;    // minimum gap, in radii of the block or the tile, whichever is smaller
+constexpr float FF_SPREAD = 1.0f / 3.0f;   // and in block radii, so that one scale serves the block's weights
 // near field, compensated: sources per FP32 partial.  Gradient error against FP64 on two
 // rings: EXP, 1,048,576 particles, 5.9e-8 at 32 and 5.0e-8 at 16 (near field 30.3 and
 // 31.5 ms); RM, 262,144, 4.5e-8 and 4.3e-8, with the near field 6% slower at 16; WL,
@@ -326,7 +335,7 @@ __global__ __launch_bounds__(256) void k_ff_classify(const float4* bsph, const f
     const float4 ct = tsph[ti];
     const float dx = cb.x - ct.x, dy = cb.y - ct.y, dz = cb.z - ct.z;
     const float gap = __fsqrt_rn(fmaf(dz, dz, fmaf(dy, dy, dx * dx))) - cb.w - ct.w;
-    bool far = gap > 0.0f && gap > FF_KAPPA * cb.w;
+    bool far = gap > 0.0f && gap > FF_KAPPA * fmaxf(fminf(cb.w, ct.w), FF_SPREAD * cb.w);
     if (CORE == CORE_EXP) far = far && gap * gap > exp_threshold(csb + tcs[ti]);
     if (CORE == CORE_SING) far = far && gap > fmaxf(csb, tcs[ti]);
     if (far) bits |= 1u << k;
@@ -633,15 +642,16 @@ __global__ __launch_bounds__(FF_FAR_THREADS, 2) void k_ff_far(FFArgs a) {
   for (int t = 1; sgn == 0.0f && t < a.ntiles; ++t) sgn = a.tsg[t];
   sgn = sgn < 0.0f ? -1.0f : 1.0f;
 
-  float tx[2], ty[2], tz[2], tt[2], al[2];
+  // targets; and the current run's centre, the block's or its one tile's
+  float qx[2], qy[2], qz[2], tt[2];
+  float cx = cb.x, cy = cb.y, cz = cb.z;
 #pragma unroll
   for (int s = 0; s < 2; ++s) {
     int64_t i = base + 32 * s + col;
     i = i < a.nt ? i : a.nt - 1;
     const float4 q = a.tq[i];
-    tx[s] = q.x - cb.x; ty[s] = q.y - cb.y; tz[s] = q.z - cb.z;
+    qx[s] = q.x; qy[s] = q.y; qz[s] = q.z;
     tt[s] = COREA || TAU ? q.w : 0.0f;
-    al[s] = fmaf(tz[s], tz[s], fmaf(ty[s], ty[s], fmaf(tx[s], tx[s], COREA ? tt[s] : 0.0f)));
   }
   f32x16 accB[2], accK[2], accR[2];
   // the folds add up in registers, or (both weights: no registers left) in the results' place
@@ -675,7 +685,7 @@ __global__ __launch_bounds__(FF_FAR_THREADS, 2) void k_ff_far(FFArgs a) {
     }
   };
   auto fold = [&]() {
-    const double ox = half ? tx[1] : tx[0], oy = half ? ty[1] : ty[0], oz = half ? tz[1] : tz[0];
+    const double ox = (half ? qx[1] : qx[0]) - cx, oy = (half ? qy[1] : qy[0]) - cy, oz = (half ? qz[1] : qz[0]) - cz;
     const double oa = ox * ox + oy * oy + oz * oz + (COREA ? (double)(half ? tt[1] : tt[0]) : 0.0);
     double sc[NG];
 #pragma unroll
@@ -799,8 +809,10 @@ __global__ __launch_bounds__(FF_FAR_THREADS, 2) void k_ff_far(FFArgs a) {
       const float4 ct = a.tsph[t];
       const float ddx = cb.x - ct.x, ddy = cb.y - ct.y, ddz = cb.z - ct.z;
       const float dc = __fsqrt_rn(fmaf(ddz, ddz, fmaf(ddy, ddy, ddx * ddx)));
-      const float lgap = __builtin_amdgcn_logf(fmaxf(dc - cb.w - ct.w, 1e-37f));   // gap > 0 for a far tile
-      const float rs = dc + ct.w;                                                // |s'| bound
+      const float gap = dc - cb.w - ct.w;   // > 0 for a far tile
+      const float lgap = __builtin_amdgcn_logf(fmaxf(gap, 1e-37f));
+      const bool own = !(gap > FF_KAPPA * cb.w);   // a tile nearer than the block is wide: its own centre
+      const float rs = own ? fmaxf(ct.w, gap * 0x1p-12f) : dc + ct.w;   // |s'| bound
       const float lrs = __builtin_amdgcn_logf(rs);
       // strengths by exponent and mantissa, so that scaling all by a power of two moves the
       // scales by just that and the results with them, exactly
@@ -813,7 +825,7 @@ __global__ __launch_bounds__(FF_FAR_THREADS, 2) void k_ff_far(FFArgs a) {
 #pragma unroll
       for (int g = 0; g < 5; ++g) wg[g] = (int)fminf(fmaxf(floorf(13.0f - lg[g]) - (float)ea, -126.0f), 126.0f) & 255;
       pk0 = ((int)floorf(2.0f * (lgap + top)) << 16) | (wg[1] << 8) | wg[0];
-      pk1 = (wg[4] << 16) | (wg[3] << 8) | wg[2];
+      pk1 = (own ? 1 << 24 : 0) | (wg[4] << 16) | (wg[3] << 8) | wg[2];
     }
     const int t = __builtin_ctz(bits);
     bits &= bits - 1u;
@@ -822,11 +834,13 @@ __global__ __launch_bounds__(FF_FAR_THREADS, 2) void k_ff_far(FFArgs a) {
   // a tile's rows on their way to LDS, straight from memory, while the tile before is
   // summed; and the scales it wants
   int wj = 0, wg[5] = {0, 0, 0, 0, 0};
+  bool wown = false;
   auto fetch = [&](int t) {
     const int p0 = __builtin_amdgcn_readlane(pk0, t & 31), p1 = __builtin_amdgcn_readlane(pk1, t & 31);
     wj = p0 >> 16;
     wg[0] = (int8_t)p0; wg[1] = (int8_t)(p0 >> 8);
     wg[2] = (int8_t)p1; wg[3] = (int8_t)(p1 >> 8); wg[4] = (int8_t)(p1 >> 16);
+    wown = (p1 >> 24) != 0;
     if (w * 64 < T) {
       const int i = w * 64 + lane, q4 = T / 4;   // slot i: source 4 (i mod T/4) + i / (T/4)
       const int64_t g = (int64_t)t * T + 4 * (i & (q4 - 1)) + i / q4;
@@ -839,6 +853,11 @@ __global__ __launch_bounds__(FF_FAR_THREADS, 2) void k_ff_far(FFArgs a) {
   while (ti >= 0) {
     // a run: consecutive tiles summed under the scales of the first
     jw = wj;
+    const bool own = wown;
+    {
+      const float4 c = own ? a.tsph[ti] : cb;
+      cx = c.x; cy = c.y; cz = c.z;
+    }
 #pragma unroll
     for (int g = 0; g < NG; ++g) eg[g] = wg[g];
     const float rsc = ldexpf(1.0f, -jw);
@@ -850,7 +869,9 @@ __global__ __launch_bounds__(FF_FAR_THREADS, 2) void k_ff_far(FFArgs a) {
       // and 16 + 8 half + e)
 #pragma unroll
       for (int s = 0; s < 2; ++s) {
-        const float tv[5] = {tx[s], ty[s], tz[s], 1.0f, al[s] * rsc};
+        const float tx = qx[s] - cx, ty = qy[s] - cy, tz = qz[s] - cz;
+        const float al = fmaf(tz, tz, fmaf(ty, ty, fmaf(tx, tx, COREA ? tt[s] : 0.0f)));
+        const float tv[5] = {tx, ty, tz, 1.0f, al * rsc};
         __bf16 part[3][5];
 #pragma unroll
         for (int c = 0; c < 5; ++c) split_bf3(tv[c], part[0][c], part[1][c], part[2][c]);
@@ -889,7 +910,7 @@ __global__ __launch_bounds__(FF_FAR_THREADS, 2) void k_ff_far(FFArgs a) {
           for (int u = 0; u < 4; ++u) {
             const float4 P = raw[u * (T / 4) + lane];   // source 4 lane + u
             const float4 A = raw[256 + u * (T / 4) + lane];
-            const float s[3] = {P.x - cb.x, P.y - cb.y, P.z - cb.z};
+            const float s[3] = {P.x - cx, P.y - cy, P.z - cz};
             const float b = fmaf(s[2], s[2], fmaf(s[1], s[1], fmaf(s[0], s[0], COREA ? P.w : 0.0f)));
             // strengths take their group's power of two first: exact, one product per group and component
             float al3[NG][3], m[NG][3], qs[NG];
@@ -930,7 +951,7 @@ __global__ __launch_bounds__(FF_FAR_THREADS, 2) void k_ff_far(FFArgs a) {
     // r2 slots (and core terms) of one source per lane
     if (tid < T) {
       const float4 P = raw[(tid & 3) * (T / 4) + (tid >> 2)];
-      const float sx = P.x - cb.x, sy = P.y - cb.y, sz = P.z - cb.z;
+      const float sx = P.x - cx, sy = P.y - cy, sz = P.z - cz;
       const float b = fmaf(sz, sz, fmaf(sy, sy, fmaf(sx, sx, COREA ? P.w : 0.0f)));
       const float sv5[5] = {-2.0f * sx * rsc, -2.0f * sy * rsc, -2.0f * sz * rsc, b * rsc, 1.0f};   // exact scalings
       __bf16 part[3][5];
@@ -994,7 +1015,7 @@ __global__ __launch_bounds__(FF_FAR_THREADS, 2) void k_ff_far(FFArgs a) {
     }
     // the run's scales fit a further tile when no factor passes 2^16 and none loses more
     // than 4 of its leading bits
-    more = ti >= 0 && ++run < ff_merge<CORE, GRAD>() && (unsigned)(jw - wj + 1) <= 2u;
+    more = ti >= 0 && !own && !wown && ++run < ff_merge<CORE, GRAD>() && (unsigned)(jw - wj + 1) <= 2u;
 #pragma unroll
     for (int g = 0; g < NG; ++g) more = more && (unsigned)(eg[g] - wg[g] + 4) <= 6u;
     } while (more);
