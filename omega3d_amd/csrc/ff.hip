@@ -99,7 +99,7 @@ Layout layout(char* base, int64_t ns, int64_t nt, bool same, int T, size_t tmp_b
   L.ioff = cv.take<int>(nb);
   L.mfold = cv.take<int>(1);
   L.ctr = cv.take<unsigned>(1);
-  L.part = cv.take<double>((size_t)(near_split(nb) + 1) * nb * nout * FF_TB);
+  L.part = cv.take<double>((size_t)(near_split(nb, ntiles) + 1) * nb * nout * FF_TB);
   L.bytes = cv.off;
   return L;
 }
@@ -173,7 +173,7 @@ int run(const o3d_points* src, o3d_points* targ, bool self_excl, int T, hipStrea
   hipLaunchKernelGGL(k_ff_plan_count, dim3(grid_of(nb, 256)), dim3(256), 0, st, L.mask, nb, mwords, ntiles, L.nn);
   HIPCHK(hipGetLastError());
   if ((rc = exclusive_scan_i32(L.nn, L.noff, nb, st)) != O3D_OK) return rc;
-  hipLaunchKernelGGL(k_ff_plan_items, dim3(grid_of(nb, 256)), dim3(256), 0, st, L.nn, L.noff, nb, near_split(nb), L.items,
+  hipLaunchKernelGGL(k_ff_plan_items, dim3(grid_of(nb, 256)), dim3(256), 0, st, L.nn, L.noff, nb, near_split(nb, ntiles), L.items,
                      L.mfold);
   HIPCHK(hipGetLastError());
   if ((rc = exclusive_scan_i32(L.items, L.ioff, nb, st)) != O3D_OK) return rc;
@@ -198,7 +198,7 @@ int run(const o3d_points* src, o3d_points* targ, bool self_excl, int T, hipStrea
   HIPCHK(hipGetLastError());
   if (prof) HIPCHK(hipEventRecord(ev[2].e, st));
   const size_t lds_near = (size_t)T * 2 * sizeof(float4);
-  const unsigned gnear = (unsigned)std::min<int64_t>((near_split(nb) + 1) * nb, near_grid<CORE, GRAD, PREC>(lds_near));
+  const unsigned gnear = (unsigned)std::min<int64_t>((near_split(nb, ntiles) + 1) * nb, near_grid<CORE, GRAD, PREC>(lds_near));
   hipLaunchKernelGGL((k_ff_near<CORE, GRAD, PREC>), dim3(gnear), dim3(FF_TB), lds_near, st, a);
   HIPCHK(hipGetLastError());
   hipLaunchKernelGGL((k_ff_combine<CORE, GRAD>), dim3((unsigned)nb), dim3(FF_TB), 0, st, a);

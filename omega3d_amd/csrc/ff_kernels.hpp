@@ -1049,14 +1049,17 @@ static __global__ __launch_bounds__(256) void k_ff_plan_count(const unsigned* ma
   if (b < nb) nn[b] = near_tiles_of(mask + b * mwords, mwords, ntiles);
 }
 
-// after the exclusive scan noff of nn: M = max(FF_M0, ceil(total / (split nb))) and the
-// item count of every block (at most (split + 1) nb items in all)
+// after the exclusive scan noff of nn: M = max(ceil(total / (split nb)), FF_M0, or fewer
+// while that makes less than 2,048 items) and the item count of every block (at most
+// (split + 1) nb items in all)
 static __global__ __launch_bounds__(256) void k_ff_plan_items(const int* nn, const int* noff, int64_t nb, int split,
                                                        int* items, int* mfold) {
   const int64_t b = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
   const int64_t total = (int64_t)noff[nb - 1] + nn[nb - 1];
   int64_t m = (total + split * nb - 1) / (split * nb);
-  m = m < FF_M0 ? FF_M0 : m;
+  const int64_t m0 = (total + 2047) / 2048 < FF_M0 ? (total + 2047) / 2048 : FF_M0;
+  m = m < m0 ? m0 : m;
+  m = m < 1 ? 1 : m;
   if (b == 0) *mfold = (int)m;
   if (b < nb) items[b] = (int)((nn[b] + m - 1) / m);
 }
@@ -1258,8 +1261,12 @@ constexpr size_t ff_far_lds() {
 }
 
 // Near-field items per block: about 4,096 in all, three rounds of the workgroups that the
-// GPU holds (an item of FF_M0 tiles is 262,144 pairs), and at least 2 per block
-inline int near_split(int64_t nb) { return (int)std::max<int64_t>(2, std::min<int64_t>(16, 4096 / nb)); }
+// GPU holds (an item of FF_M0 tiles is 262,144 pairs), and at least 2 per block; 2,048 in
+// all where there are few blocks, but no more per block than it has tiles
+inline int near_split(int64_t nb, int64_t ntiles) {
+  return (int)std::max<int64_t>(2, std::min<int64_t>(std::max<int64_t>(std::min<int64_t>(16, 4096 / nb), 2048 / nb),
+                                                     ntiles));
+}
 
 // Slices of the far field: blocks x slices workgroups, at least about four rounds of the
 // two that a CU holds, so that the last round is short beside the whole and few blocks

@@ -12,9 +12,7 @@
 // LDS, decides every root pair and evaluates the pairs that are leaves at the
 // root, and lists the targets that have a pair needing the recursion (those near
 // the surface).  k_pan_near then gives each listed target one wave whose lanes
-// take the panels in turn and walk the near ones: a lane walks the tree in
-// depth-first order with an explicit (level, path) cursor -- no recursion, no
-// stack -- recomputing a node's vertices from the panel's corners along its path.
+// take the panels in turn and split the near ones' nodes together (NodeStack).
 // Walking inside k_pan instead held a whole wave of targets for the deepest walk
 // of any of its lanes.  Every quantity that decides the tree
 // shape (midpoints, centroid, sqrt(area), distance) is computed in correctly
@@ -279,59 +277,79 @@ __device__ __forceinline__ bool root_leaf(R tx, R ty, R tz, R cx0, R cy0, R cz0,
   return leaf0 || maxlev == 0;
 }
 
-// one (target, panel) tree walk, accumulating into acc
+// ---- the recursion ------------------------------------------------------------
+// A wave takes the tree walks of one target (panels on points) or one panel (particles on
+// panels) together: nodes known to be split wait on a stack in LDS, and up to 64 of them
+// at a time are split, one per lane.  A lane forms its node's corners from the panel's
+// along the path, then the four children: a leaf goes to the lane's sums, the others back
+// on the stack.  So lanes stay busy however deep each pair's tree goes (one lane per
+// pair held the wave for the deepest tree, and formed the corners of every node from the
+// root), and the corners are formed once for four children.  Which node a lane takes
+// depends on its target's own pairs alone, so results do not depend on scheduling.
+// Whole calls before and after: 1,280 panels on 131,072 points 2.36 -> 0.62 ms, 320 panels on
+// 8,192 0.65 -> 0.12; 131,072 particles on 1,280 panels 4.5 -> 0.47, on 320 panels 83 -> 1.7.
+struct NodeStack {
+  int2* st;    // {panel (particle), level << 16 | path}, node_cap(maxlev) entries
+  int n = 0;
+  int cap;
+  __device__ __forceinline__ void push(bool yes, int p, unsigned node) {
+    const uint64_t m = __builtin_amdgcn_ballot_w64(yes);
+    if (yes) st[n + __builtin_amdgcn_mbcnt_hi((unsigned)(m >> 32), __builtin_amdgcn_mbcnt_lo((unsigned)m, 0))] =
+        make_int2(p, (int)node);
+    n += __builtin_popcountll(m);
+  }
+  // the topmost nodes, one per lane; fewer near the cap, where a single node at a time
+  // needs at most three places per level
+  __device__ __forceinline__ bool pop(int2& node) {
+    const int room = (cap - 24 - n) / 3;
+    const int k = min(min(64, n), max(1, room));
+    const int lane = threadIdx.x & 63;
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    node = st[lane < k ? n - k + lane : 0];
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    n -= k;
+    return lane < k;
+  }
+};
+// 127 nodes of the scan, and 192 more per level for 64 split at a time
+__host__ __device__ constexpr int node_cap(int maxlev) { return 160 + 192 * maxlev; }
+constexpr size_t node_lds(int maxlev) { return (BLOCK / 64) * node_cap(maxlev) * sizeof(int2); }
+
+// split one node (has: this lane has one) of the panel with record s for target t
 template <class R, bool GRAD>
-__device__ __forceinline__ void walk_panel(R tx, R ty, R tz, const float4* s, int maxlev, bool active, R* acc) {
+__device__ __forceinline__ void split_node(bool has, int2 node, R tx, R ty, R tz, const float4* s, int maxlev, R* acc,
+                                           NodeStack& stack) {
+  const int lev = (node.y >> 16) + 1;   // of the children
+  const unsigned path = (unsigned)node.y & 0xffffu;
   const float4 f0 = s[0], f1 = s[1], f4 = s[4];
-  const R ar = f4.y;
   R gx, gy, gz, gs, cx0, cy0, cz0, lim;
   RootLim rl;
   panel_root<R>(s, gx, gy, gz, gs, cx0, cy0, cz0, lim, rl);
-  const bool leaf0 = root_leaf<R>(tx, ty, tz, cx0, cy0, cz0, lim, rl, maxlev, active);
-  if (!wave_any(!leaf0 && active)) {
-    if (active) leaf_acc<R, GRAD>(tx, ty, tz, cx0, cy0, cz0, gx, gy, gz, gs, acc);
-    return;
+  R t[9] = {R(f0.x), R(f0.y), R(f0.z), R(f0.w), R(f1.x), R(f1.y), R(f1.z), R(f1.w), R(f4.x)};
+  R sa = R(0.25) * R(f4.y), scale = R(0.25);
+  for (int l = 1; l < lev; ++l) {
+    child_of<R>(t, (path >> (2 * (l - 1))) & 3);
+    sa = R(0.25) * sa;
+    scale = R(0.25) * scale;
   }
-  // depth-first walk; lev = 0 is the root (already decided above)
-  int lev = 0, path = 0;
-  bool done = !active;
-  bool first = true;
-  while (wave_any(!done)) {
-    if (!done) {
-      bool leaf;
-      R cx, cy, cz;
-      R scale = R(1);
-      if (first) {
-        leaf = leaf0;
-        cx = cx0; cy = cy0; cz = cz0;
-      } else {
-        R t[9] = {R(f0.x), R(f0.y), R(f0.z), R(f0.w), R(f1.x), R(f1.y), R(f1.z), R(f1.w), R(f4.x)};
-        R sa = ar;
-        for (int l = 1; l <= lev; ++l) {
-          child_of<R>(t, (path >> (2 * (l - 1))) & 3);
-          sa = R(0.25) * sa;
-          scale = R(0.25) * scale;
-        }
-        centroid_exact<R>(t[0], t[1], t[2], t[3], t[4], t[5], t[6], t[7], t[8], cx, cy, cz);
-        leaf = lev == maxlev || dist_exact<R>(tx, ty, tz, cx, cy, cz) > sqrt(sa) * R(4);
-      }
-      first = false;
-      if (leaf) {
-        if (lev == 0) leaf_acc<R, GRAD>(tx, ty, tz, cx, cy, cz, gx, gy, gz, gs, acc);
-        else leaf_acc<R, GRAD>(tx, ty, tz, cx, cy, cz, gx * scale, gy * scale, gz * scale, gs * scale, acc);
-        // advance to the next node in preorder after this subtree
-        while (lev > 0) {
-          const int sh = 2 * (lev - 1);
-          const int c = (path >> sh) & 3;
-          if (c < 3) { path += 1 << sh; break; }
-          path &= ~(3 << sh);
-          --lev;
-        }
-        if (lev == 0) done = true;
-      } else {
-        ++lev;   // first child: digit 0
-      }
-    }
+  gx = gx * scale; gy = gy * scale; gz = gz * scale; gs = gs * scale;
+  const R sq = sqrt(sa);
+  lim = sq * R(4);
+  if constexpr (sizeof(R) == 4) {
+    rl.lim = lim;
+    root_bands(sq, rl.far2, rl.near2);
+  }
+#pragma unroll
+  for (int c = 0; c < 4; ++c) {
+    R v[9];
+#pragma unroll
+    for (int k = 0; k < 9; ++k) v[k] = t[k];
+    child_of<R>(v, c);
+    R cx, cy, cz;
+    centroid_exact<R>(v[0], v[1], v[2], v[3], v[4], v[5], v[6], v[7], v[8], cx, cy, cz);
+    const bool leaf = root_leaf<R>(tx, ty, tz, cx, cy, cz, lim, rl, lev == maxlev ? 0 : 1, has);
+    if (has && leaf) leaf_acc<R, GRAD>(tx, ty, tz, cx, cy, cz, gx, gy, gz, gs, acc);
+    stack.push(has && !leaf, node.x, (unsigned)lev << 16 | path | (unsigned)c << (2 * (lev - 1)));
   }
 }
 
@@ -460,69 +478,61 @@ __global__ __launch_bounds__(BLOCK, 5) void k_pan(PanArgs a, const float4* rec) 
 }
 
 // The pairs of the listed targets that the root decision sends into the
-// recursion, added to the outputs after k_pan.  One wave per 4 listed targets, one
-// per 16-lane quarter: lane l of a quarter takes panels l, l + 16, ..., so the
-// quarters load the same panels in the same instruction.  A panel whose centroid
+// recursion, added to the outputs after k_pan.  One wave per listed target: its lanes
+// take the panels in turn.  A panel whose centroid
 // lies beyond its far band (cen: the fused d2 of root_leaf against the same band)
 // is a leaf at the root, which k_pan evaluated; the others are decided as k_pan
-// did and the near ones walked (Kernels.h:1028-1211).  A fixed butterfly adds each
-// quarter's sums in FP64, so results do not depend on scheduling.  Grid-stride
+// did and the near ones split (Kernels.h:1028-1211).  A fixed butterfly adds the
+// lanes' sums in FP64, so results do not depend on scheduling.  Grid-stride
 // over the list, whose length k_pan left in near_count.
 template <bool GRAD, int PREC>
 __global__ __launch_bounds__(BLOCK) void k_pan_near(PanArgs a, const float4* rec, const float4* cen) {
   using R = typename std::conditional<PREC == PREC_FP64, double, float>::type;
+  extern __shared__ int2 shn[];
   const int lane = threadIdx.x & 63;
-  const int ql = lane & 15;
   const int64_t wave = ((int64_t)blockIdx.x * BLOCK + threadIdx.x) >> 6;
   const int64_t nwaves = ((int64_t)gridDim.x * BLOCK) >> 6;
   const int64_t listed = *a.near_count;
-  const int64_t groups = (listed + 3) / 4;
-  for (int64_t e = wave; e < groups; e += nwaves) {
-    const int64_t li = 4 * e + (lane >> 4);
-    const bool has = li < listed;
-    const int64_t i = a.near_list[has ? li : 4 * e];
+  NodeStack stack{shn + (threadIdx.x >> 6) * node_cap(a.maxlev), 0, node_cap(a.maxlev)};
+  for (int64_t e = wave; e < listed; e += nwaves) {
+    const int64_t i = a.near_list[e];
     const R tx = a.tx[i], ty = a.ty[i], tz = a.tz[i];
     R acc[16];
 #pragma unroll
     for (int c = 0; c < 16; ++c) acc[c] = R(0);
-    if (has) {
-      // four panels per step: their prefilter loads are issued together, then the
-      // candidates are decided and walked in ascending order
-      for (int64_t p = ql; p < a.np; p += 64) {
-        unsigned m = 0;
-#pragma unroll
-        for (int k = 0; k < 4; ++k) {
-          const int64_t pk = p + 16 * k;
-          if (pk >= a.np) continue;
-          if constexpr (sizeof(R) == 4) {
-            const float4 c = cen[pk];
-            const float ex = tx - c.x, ey = ty - c.y, ez = tz - c.z;
-            if (fmaf(ez, ez, fmaf(ey, ey, ex * ex)) > c.w) continue;
-          }
-          m |= 1u << k;
-        }
-        while (m) {
-          const int k = __builtin_ctz(m);
-          m &= m - 1;
-          const float4* s = rec + PAN_F4 * (p + 16 * k);
-          R gx, gy, gz, gs, cx0, cy0, cz0, lim;
-          RootLim rl;
-          panel_root<R>(s, gx, gy, gz, gs, cx0, cy0, cz0, lim, rl);
-          if (!root_leaf<R>(tx, ty, tz, cx0, cy0, cz0, lim, rl, a.maxlev, true))
-            walk_panel<R, GRAD>(tx, ty, tz, s, a.maxlev, true, acc);
-        }
+    auto split = [&]() {
+      int2 node;
+      const bool has = stack.pop(node);
+      split_node<R, GRAD>(has, node, tx, ty, tz, rec + PAN_F4 * (has ? (int64_t)node.x : 0), a.maxlev, acc, stack);
+    };
+    for (int64_t p0 = 0; p0 < a.np; p0 += 64) {
+      const int64_t p = p0 + lane;
+      bool near = p < a.np;
+      if constexpr (sizeof(R) == 4) {
+        const float4 c = cen[near ? p : 0];
+        const float ex = tx - c.x, ey = ty - c.y, ez = tz - c.z;
+        near = near && !(fmaf(ez, ez, fmaf(ey, ey, ex * ex)) > c.w);
       }
+      if (near) {
+        R gx, gy, gz, gs, cx0, cy0, cz0, lim;
+        RootLim rl;
+        panel_root<R>(rec + PAN_F4 * p, gx, gy, gz, gs, cx0, cy0, cz0, lim, rl);
+        near = !root_leaf<R>(tx, ty, tz, cx0, cy0, cz0, lim, rl, a.maxlev, true);
+      }
+      stack.push(near, (int)p, 0u);
+      while (stack.n >= 64) split();
     }
+    while (stack.n > 0) split();
     double u[3], g[9];
 #pragma unroll
-    for (int d = 0; d < 3; ++d) u[d] = quarter_sum((double)acc[d]);
+    for (int d = 0; d < 3; ++d) u[d] = wave_sum((double)acc[d]);
     if (GRAD) {
       R gl[9];
       grad_of<R>(acc, gl);
 #pragma unroll
-      for (int k = 0; k < 9; ++k) g[k] = quarter_sum((double)gl[k]);
+      for (int k = 0; k < 9; ++k) g[k] = wave_sum((double)gl[k]);
     }
-    if (ql != 0 || !has) continue;
+    if (lane != 0) continue;
     if (PREC == PREC_FP64) {
       double* uu = (double*)a.u; double* vv = (double*)a.v; double* ww = (double*)a.w;
       uu[i] += u[0]; vv[i] += u[1]; ww[i] += u[2];

@@ -27,8 +27,8 @@ static hipError_t launch_pan(const PanArgs& a, bool grad, int prec, hipStream_t 
   if (!a.near_list || !a.near_count || !rec) return hipErrorInvalidValue;
   const size_t lds = (size_t)a.tile * PAN_F4 * sizeof(float4);
   const dim3 grid((unsigned)((a.nt + BLOCK - 1) / BLOCK));
-  // one wave per 4 listed targets, grid-stride: at most 16 waves per CU
-  const dim3 grid_near((unsigned)std::min<int64_t>((a.nt + 15) / 16, 4 * (int64_t)num_cus()));
+  // one wave per listed target, grid-stride: at most 16 waves per CU
+  const dim3 grid_near((unsigned)std::min<int64_t>((a.nt + 3) / 4, 4 * (int64_t)num_cus()));
   float4* cen = rec + PAN_F4 * a.np;
   hipLaunchKernelGGL(k_pan_g7_zero, dim3(1), dim3(64), 0, st, a.near_count);
   hipLaunchKernelGGL(k_pan_geom, dim3((unsigned)((a.np + BLOCK - 1) / BLOCK)), dim3(BLOCK), 0, st, a, rec, cen);
@@ -38,7 +38,7 @@ static hipError_t launch_pan(const PanArgs& a, bool grad, int prec, hipStream_t 
     hipLaunchKernelGGL((k_pan<G, P>), grid, dim3(BLOCK), lds, st, a, (const float4*)rec);  \
     e = hipGetLastError();                                                                \
     if (e == hipSuccess) {                                                                \
-      hipLaunchKernelGGL((k_pan_near<G, P>), grid_near, dim3(BLOCK), 0, st, a, (const float4*)rec, \
+      hipLaunchKernelGGL((k_pan_near<G, P>), grid_near, dim3(BLOCK), node_lds(a.maxlev), st, a, (const float4*)rec, \
                          (const float4*)cen);                                             \
       e = hipGetLastError();                                                              \
     }                                                                                     \

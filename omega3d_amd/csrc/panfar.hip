@@ -7,9 +7,8 @@
 // which one of the pairs would not be plain, through k_ff_far (ff_kernels.hpp).  The
 // other tiles go through the code of the direct kernels, tile by tile in work items of a
 // queue: each item leaves its sums per target, and lists the targets that have pairs
-// which need the recursion (or the closed form); a second kernel gives each of those
-// entries 16 lanes, which gather the entry's pairs and walk them 16 at a time, and adds
-// to the item's sums.  All decisions per pair are the direct kernels'.
+// which need the recursion (or the closed form); a second kernel takes those pairs entry
+// by entry and adds to the item's sums.  All decisions per pair are the direct kernels'.
 //
 // The direct kernels are bound by the issue of about 40 vector instructions per pair (35
 // per point of the 7-point rule); a far pair takes one square root, three products and the
@@ -17,7 +16,8 @@
 // Compensated: 20,480 panels on 524,288 points, velocity and gradient 12.1 -> 6.2 ms (far
 // 3.74, items 1.49, walks 0.91); 5,120 panels with source strengths on 200,003 points,
 // 7-point rule 7.7 -> 4.3 ms (2.74, 1.28, 0.32); 524,288 particles on 20,480 panels 6.4 ->
-// 5.7 ms (2.31, 2.54, 1.06).  Errors against FP64 as before or smaller (1.2e-7 -> 0.9e-7).
+// 5.7 ms (2.31, 2.54, 1.06); with Hilbert blocks, tiles' own centres and the node stack
+// 5.0, 4.0 and 4.0 ms.  Errors against FP64 as before or smaller (1.2e-7 -> 0.9e-7).
 #include "ff_kernels.hpp"
 #include "o3d_api_internal.hpp"
 #include "pan_g7.hpp"
@@ -266,14 +266,105 @@ __global__ __launch_bounds__(FF_TB) void k_pf_items(PanFarArgs a) {
   }
 }
 
-// The listed entries' pairs that need the recursion or the closed form.  Each quarter
-// of a wave takes an entry: its 16 lanes test the item's panels (particles) in turn,
-// queue those that are near and walk them when 16 are there or none is left, hit h in
-// lane h mod 16, so that the lanes walk together however the near ones lie.  A fixed
-// butterfly adds the lanes' sums in FP64; the order in which entries were listed decides
-// nothing.
+// an entry's block, item, target row and tiles
+struct PfEntry {
+  int64_t b;
+  int item, tid, r0, r1;
+  __device__ __forceinline__ PfEntry(const PanFarArgs& a, unsigned e) : item((int)(e / FF_TB)), tid((int)(e % FF_TB)) {
+    b = a.iblk[item];
+    const int m = *a.f.mfold;
+    r0 = (item - a.f.ioff[b]) * m;
+    r1 = r0 + m < a.f.nn[b] ? r0 + m : a.f.nn[b];
+  }
+};
+
+// The listed entries' pairs that need the recursion: one wave per entry, whose lanes test
+// the item's panels (particles) in turn and split the near ones' nodes together
+// (NodeStack).  A fixed butterfly adds the lanes' sums in FP64; the order in which entries
+// were listed decides nothing.
 template <int RULE, bool GRAD, int PREC>
 __global__ __launch_bounds__(BLOCK) void k_pf_walk(PanFarArgs a) {
+  constexpr int NOUT = GRAD ? 12 : 3;
+  constexpr bool PART = RULE == PANFAR_PARTICLES;
+  extern __shared__ int2 shn[];
+  const int maxlev = PART ? a.t.maxlev : a.p.maxlev;
+  NodeStack stack{shn + (threadIdx.x >> 6) * node_cap(maxlev), 0, node_cap(maxlev)};
+  const int lane = threadIdx.x & 63;
+  const int64_t wave = ((int64_t)blockIdx.x * BLOCK + threadIdx.x) >> 6;
+  const int64_t nwaves = ((int64_t)gridDim.x * BLOCK) >> 6;
+  const int64_t listed = *a.count;
+  for (int64_t e = wave; e < listed; e += nwaves) {
+    const PfEntry n(a, a.list[e]);
+    const float4 q = a.f.tq[n.b * FF_TB + n.tid];
+    float4 s[PAN_F4] = {};
+    if (PART) ptpan_record(a.t, a.f.tperm[n.b * FF_TB + n.tid], s);
+    const PtRoot<float> root(s);
+    float acc[16];
+#pragma unroll
+    for (int c = 0; c < 16; ++c) acc[c] = 0.0f;
+    auto split = [&]() {
+      int2 node;
+      const bool has = stack.pop(node);
+      const int64_t p = has ? node.x : 0;
+      if constexpr (PART) {
+        const float4 P = a.f.sp[p];
+        ptpan_strength<PREC>(s, a.f.sa[p]);
+        split_node<float, false>(has, node, P.x, P.y, P.z, s, maxlev, acc, stack);
+      } else {
+        split_node<float, GRAD>(has, node, q.x, q.y, q.z, a.rec + PAN_F4 * p, maxlev, acc, stack);
+      }
+    };
+    NearTiles tiles(a.f, n.b, n.r0, n.r1);
+    for (int t = tiles.next(); t >= 0; t = tiles.next()) {
+      const int64_t p0 = (int64_t)t * a.unit;
+      const int cnt = (int)(a.units - p0 < a.unit ? a.units - p0 : a.unit);
+      for (int j0 = 0; j0 < cnt; j0 += 64) {
+        const int64_t p = p0 + j0 + lane;
+        bool near = j0 + lane < cnt;
+        const float4 c = PART ? a.f.sp[near ? p : 0] : a.cen[near ? p : 0];
+        const float4 P = PART ? c : q;
+        if constexpr (PART) {
+          near = near && !root_leaf<float>(P.x, P.y, P.z, root.cx, root.cy, root.cz, root.lim, root.rl, maxlev, near);
+        } else {
+          const float ex = P.x - c.x, ey = P.y - c.y, ez = P.z - c.z;
+          near = near && !(fmaf(ez, ez, fmaf(ey, ey, ex * ex)) > c.w);
+          if (near) {
+            float gx, gy, gz, gs, cx0, cy0, cz0, lim;
+            RootLim rl;
+            panel_root<float>(a.rec + PAN_F4 * p, gx, gy, gz, gs, cx0, cy0, cz0, lim, rl);
+            near = !root_leaf<float>(P.x, P.y, P.z, cx0, cy0, cz0, lim, rl, maxlev, true);
+          }
+        }
+        stack.push(near, (int)p, 0u);
+        while (stack.n >= 64) split();
+      }
+    }
+    while (stack.n > 0) split();
+    double* slot = a.f.part + (int64_t)n.item * NOUT * FF_TB + n.tid;
+    double u[3], g[9];
+#pragma unroll
+    for (int d = 0; d < 3; ++d) u[d] = wave_sum((PART ? -1.0 : 1.0) * (double)acc[d]);
+    if (GRAD) {
+      float gl[9];
+      grad_of<float>(acc, gl);
+#pragma unroll
+      for (int k = 0; k < 9; ++k) g[k] = wave_sum((double)gl[k]);
+    }
+    if (lane != 0) continue;
+#pragma unroll
+    for (int d = 0; d < 3; ++d) slot[d * FF_TB] += u[d];
+    if (GRAD) {
+#pragma unroll
+      for (int k = 0; k < 9; ++k) slot[(3 + k) * FF_TB] += g[k];
+    }
+  }
+}
+
+// The 7-point rule's near pairs in closed form, FP64.  Each quarter of a wave takes an
+// entry: its 16 lanes test the item's panels in turn, queue those that are near and
+// evaluate them when 16 are there or none is left, hit h in lane h mod 16.  Summed as above.
+template <bool GRAD>
+__global__ __launch_bounds__(BLOCK) void k_pf_near7(PanFarArgs a) {
   constexpr int NOUT = GRAD ? 12 : 3;
   __shared__ int ring[BLOCK / 16][32];
   const int lane = threadIdx.x & 63, ql = lane & 15, q0 = lane & 48;
@@ -281,104 +372,48 @@ __global__ __launch_bounds__(BLOCK) void k_pf_walk(PanFarArgs a) {
   const int64_t wave = ((int64_t)blockIdx.x * BLOCK + threadIdx.x) >> 6;
   const int64_t nwaves = ((int64_t)gridDim.x * BLOCK) >> 6;
   const int64_t listed = *a.count;
-  const int m = *a.f.mfold;
   for (int64_t e = wave; 4 * e < listed; e += nwaves) {
     const int64_t li = 4 * e + (lane >> 4);
     const bool has = li < listed;
-    const unsigned entry = a.list[has ? li : 4 * e];
-    const int item = (int)(entry / FF_TB), tid = (int)(entry % FF_TB);
-    const int64_t b = a.iblk[item];
-    const int r0 = (item - a.f.ioff[b]) * m;
-    const int r1 = has ? (r0 + m < a.f.nn[b] ? r0 + m : a.f.nn[b]) : r0;
-    const float4 q = a.f.tq[b * FF_TB + tid];
-    float4 s[PAN_F4];
-    float far2 = 0.0f;
-    if (RULE == PANFAR_PARTICLES) {
-      ptpan_record(a.t, a.f.tperm[b * FF_TB + tid], s);
-      far2 = s[3].w;
-    }
-    float acc[16];
+    const PfEntry n(a, a.list[has ? li : 4 * e]);
+    const float4 q = a.f.tq[n.b * FF_TB + n.tid];
     double u[3] = {0, 0, 0}, g[9] = {0, 0, 0, 0, 0, 0, 0, 0, 0};
-#pragma unroll
-    for (int c = 0; c < 16; ++c) acc[c] = 0.0f;
-    // whether pair p is near, from its near-test row
-    auto is_near = [&](int64_t p, const float4 c) {
-      if constexpr (RULE == PANFAR_POINTS7) {
+    int head = 0, tail = 0;   // hits evaluated and found, alike in the quarter's lanes
+    auto drain = [&]() {
+      const int h = head + ((ql - head) & 15);
+      __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+      if (h < tail) {
+        const float4* r = a.rec + G7_F4 * (int64_t)mine[h & 31];
+        const float4 f6 = r[6], f7 = r[7], f8 = r[8], f9 = r[9];
+        const float v[9] = {f7.y, f7.z, f7.w, f8.x, f8.y, f8.z, f8.w, f9.x, f9.y};
+        const float ts[3] = {f6.x, f6.y, f6.z};
+        g7_near_pair<GRAD>(q.x, q.y, q.z, v, ts, f9.z, f9.w, u, g);
+      }
+      __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+      head = head + 16 < tail ? head + 16 : tail;
+    };
+    NearTiles tiles(a.f, n.b, n.r0, has ? n.r1 : n.r0);
+    for (int t = tiles.next(); wave_any(t >= 0); t = t >= 0 ? tiles.next() : -1) {
+      const int64_t p0 = (int64_t)t * a.unit;
+      const int cnt = t < 0 ? 0 : (int)(a.units - p0 < a.unit ? a.units - p0 : a.unit);
+      for (int j0 = 0; j0 < a.unit; j0 += 16) {
+        const int j = j0 + ql;
+        const float4 c = a.cen[j < cnt ? p0 + j : 0];
         float d2;
         {
 #pragma clang fp contract(off)
           const float ex = q.x - c.x, ey = q.y - c.y, ez = q.z - c.z;
           d2 = ex * ex + ey * ey + ez * ez;
         }
-        return d2 < c.w;
-      } else {
-        constexpr bool PART = RULE == PANFAR_PARTICLES;
-        const float4 P = PART ? c : q, C = PART ? q : c;
-        const float ex = P.x - C.x, ey = P.y - C.y, ez = P.z - C.z;
-        if (fmaf(ez, ez, fmaf(ey, ey, ex * ex)) > (PART ? far2 : c.w)) return false;
-        float gx, gy, gz, gs, cx0, cy0, cz0, lim;
-        RootLim rl;
-        panel_root<float>(PART ? s : a.rec + PAN_F4 * p, gx, gy, gz, gs, cx0, cy0, cz0, lim, rl);
-        return !root_leaf<float>(P.x, P.y, P.z, cx0, cy0, cz0, lim, rl, PART ? a.t.maxlev : a.p.maxlev, true);
-      }
-    };
-    auto walk = [&](int64_t p) {
-      if constexpr (RULE == PANFAR_POINTS) {
-        walk_panel<float, GRAD>(q.x, q.y, q.z, a.rec + PAN_F4 * p, a.p.maxlev, true, acc);
-      } else if constexpr (RULE == PANFAR_POINTS7) {
-        const float4* r = a.rec + G7_F4 * p;
-        const float4 f6 = r[6], f7 = r[7], f8 = r[8], f9 = r[9];
-        const float v[9] = {f7.y, f7.z, f7.w, f8.x, f8.y, f8.z, f8.w, f9.x, f9.y};
-        const float ts[3] = {f6.x, f6.y, f6.z};
-        g7_near_pair<GRAD>(q.x, q.y, q.z, v, ts, f9.z, f9.w, u, g);
-      } else {
-        const float4 P = a.f.sp[p], A = a.f.sa[p];
-        ptpan_strength<PREC>(s, A);
-        walk_panel<float, false>(P.x, P.y, P.z, s, a.t.maxlev, true, acc);
-      }
-    };
-    int head = 0, tail = 0;   // hits walked and found, alike in the quarter's lanes
-    auto drain = [&]() {
-      const int h = head + ((ql - head) & 15);
-      __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
-      if (h < tail) walk(mine[h & 31]);
-      __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
-      head = head + 16 < tail ? head + 16 : tail;
-    };
-    NearTiles tiles(a.f, b, r0, r1);
-    for (int t = tiles.next(); wave_any(t >= 0); t = t >= 0 ? tiles.next() : -1) {
-      const int64_t p0 = (int64_t)t * a.unit;
-      const int cnt = t < 0 ? 0 : (int)(a.units - p0 < a.unit ? a.units - p0 : a.unit);
-      for (int j0 = 0; j0 < a.unit; j0 += 64) {
-        float4 c[4];
-#pragma unroll
-        for (int k = 0; k < 4; ++k) {
-          const int j = j0 + 16 * k + ql;
-          c[k] = RULE == PANFAR_PARTICLES ? a.f.sp[j < cnt ? p0 + j : 0] : a.cen[j < cnt ? p0 + j : 0];
-        }
-#pragma unroll
-        for (int k = 0; k < 4; ++k) {
-          const int j = j0 + 16 * k + ql;
-          const bool near = j < cnt && is_near(p0 + j, c[k]);
-          const unsigned hits = (unsigned)(__builtin_amdgcn_ballot_w64(near) >> q0) & 0xffffu;
-          if (near) mine[(tail + __popc(hits & ((1u << ql) - 1u))) & 31] = (int)(p0 + j);
-          tail += __popc(hits);
-          while (wave_any(tail - head >= 16)) drain();
-        }
+        const bool near = j < cnt && d2 < c.w;
+        const unsigned hits = (unsigned)(__builtin_amdgcn_ballot_w64(near) >> q0) & 0xffffu;
+        if (near) mine[(tail + __popc(hits & ((1u << ql) - 1u))) & 31] = (int)(p0 + j);
+        tail += __popc(hits);
+        while (wave_any(tail - head >= 16)) drain();
       }
     }
     while (wave_any(head < tail)) drain();
-    if (RULE != PANFAR_POINTS7) {
-#pragma unroll
-      for (int d = 0; d < 3; ++d) u[d] = (RULE == PANFAR_PARTICLES ? -1.0 : 1.0) * (double)acc[d];
-      if (GRAD) {
-        float gl[9];
-        grad_of<float>(acc, gl);
-#pragma unroll
-        for (int k = 0; k < 9; ++k) g[k] = (double)gl[k];
-      }
-    }
-    double* slot = a.f.part + (int64_t)item * NOUT * FF_TB + tid;
+    double* slot = a.f.part + (int64_t)n.item * NOUT * FF_TB + n.tid;
 #pragma unroll
     for (int d = 0; d < 3; ++d) u[d] = quarter_sum(u[d]);
     if (GRAD) {
@@ -416,7 +451,7 @@ PanFarLayout layout(char* base, int rule, int64_t units, int64_t nt, int nout) {
   const int64_t nb = (nt + FF_TB - 1) / FF_TB;
   const int64_t ntiles = (units + U - 1) / U;
   const int64_t mwords = (ntiles + 31) / 32;
-  const int64_t maxitems = (near_split(nb) + 1) * nb;
+  const int64_t maxitems = (near_split(nb, ntiles) + 1) * nb;
   const int f4 = rule == PANFAR_POINTS ? PAN_F4 : rule == PANFAR_POINTS7 ? G7_F4 : 0;
   Carve cv{base};
   PanFarLayout L{};
@@ -532,7 +567,7 @@ int run(const PanArgs* p, const PtPanArgs* t, void* ws, hipStream_t st) {
   hipLaunchKernelGGL(k_ff_plan_count, dim3(grid_of(nb, 256)), dim3(256), 0, st, L.mask, nb, mwords, ntiles, L.nn);
   HIPCHK(hipGetLastError());
   if ((rc = exclusive_scan_i32(L.nn, L.noff, nb, st)) != O3D_OK) return rc;
-  hipLaunchKernelGGL(k_ff_plan_items, dim3(grid_of(nb, 256)), dim3(256), 0, st, L.nn, L.noff, nb, near_split(nb), L.items,
+  hipLaunchKernelGGL(k_ff_plan_items, dim3(grid_of(nb, 256)), dim3(256), 0, st, L.nn, L.noff, nb, near_split(nb, ntiles), L.items,
                      L.mfold);
   HIPCHK(hipGetLastError());
   if ((rc = exclusive_scan_i32(L.items, L.ioff, nb, st)) != O3D_OK) return rc;
@@ -546,13 +581,16 @@ int run(const PanArgs* p, const PtPanArgs* t, void* ws, hipStream_t st) {
                      (ff_far_lds<CORE_SING, GRAD, SHEET>()), st, f);
   HIPCHK(hipGetLastError());
   const size_t lds = (size_t)U * (RULE == PANFAR_POINTS ? PAN_F4 : RULE == PANFAR_POINTS7 ? G7_F4 : 2) * sizeof(float4);
-  const int64_t maxitems = (near_split(nb) + 1) * nb;
+  const int64_t maxitems = (near_split(nb, ntiles) + 1) * nb;
   const unsigned gitems = (unsigned)std::min<int64_t>(maxitems, items_grid<RULE, GRAD, PREC>(lds));
   hipLaunchKernelGGL((k_pf_items<RULE, GRAD, PREC>), dim3(gitems), dim3(FF_TB), lds, st, a);
   HIPCHK(hipGetLastError());
   // at most 16 waves per CU
   const unsigned gwalk = (unsigned)std::min<int64_t>((maxitems * FF_TB + 15) / 16, 4 * (int64_t)num_cus());
-  hipLaunchKernelGGL((k_pf_walk<RULE, GRAD, PREC>), dim3(gwalk), dim3(BLOCK), 0, st, a);
+  if constexpr (RULE == PANFAR_POINTS7)
+    hipLaunchKernelGGL((k_pf_near7<GRAD>), dim3(gwalk), dim3(BLOCK), 0, st, a);
+  else
+    hipLaunchKernelGGL((k_pf_walk<RULE, GRAD, PREC>), dim3(gwalk), dim3(BLOCK), node_lds(PART ? t->maxlev : p->maxlev), st, a);
   HIPCHK(hipGetLastError());
   hipLaunchKernelGGL((k_ff_combine<CORE_SING, GRAD>), dim3((unsigned)nb), dim3(FF_TB), 0, st, f);
   HIPCHK(hipGetLastError());
@@ -568,29 +606,29 @@ int run_points(const PanArgs& p, int prec, void* ws, hipStream_t st) {
 
 }  // namespace
 
-// Where the far field pays, on spheres of 320 to 20,480 panels and 2,048 to 131,072 points
-// in a shell around them, compensated, direct against here.  Panels on points, recursive:
-// from 1,280 panels at every count (1,280 on 2,048: 901 and 634 us; 20,480 on 2,048: 3,199
-// and 613, on 524,288: 12.1 and 6.2 ms), 320 panels from 32,768 points (1,100 and 1,009 us;
-// on 16,384: 718 and 709).  7-point rule: 1,280 panels likewise (661 and 273 us on 2,048,
-// velocity alone 872 and 825 on 131,072), 320 panels only at 131,072 points (1,269 and
-// 1,038 us; 458 and 544 at 32,768).  Particles on panels: 20,480 panels and 131,072
-// particles 1.63 and 1.74 ms, 524,288 particles 6.4 and 5.7 ms.  A call that
-// names its method or a tile is the direct kernels'.
-// Where the far field pays, on spheres of 320 to 20,480 panels and 2,048 to 131,072 points
-// in a shell around them, compensated, direct against here.  Panels on points, recursive:
-// from 1,280 panels at every count (1,280 on 2,048: 901 and 634 us; 20,480 on 2,048: 3,199
-// and 613, on 524,288: 12.1 and 6.2 ms), 320 panels from 32,768 points (1,100 and 1,009 us;
-// on 16,384: 718 and 709).  7-point rule: 1,280 panels likewise (661 and 273 us on 2,048,
-// velocity alone 872 and 825 on 131,072), 320 panels only at 131,072 points (1,269 and
-// 1,038 us; 458 and 544 at 32,768).  Particles on panels: 20,480 panels and 131,072
-// particles 1.63 and 1.74 ms, 524,288 particles 6.4 and 5.7 ms.  A call that
-// names its method or a tile is the direct kernels'.
+// Where the far field pays, compensated, direct against here, spheres and points in a shell
+// around them.  Panels on points, recursive: the direct kernel takes 0.14 us per panel with
+// few points, here 0.2 ms: 960 panels on 2,048 points 233 and 211 us, 5,120 panels on 32
+// points 690 and 218, 20,480 on 2,048 points 3.2 and 0.44 ms.  With many points the near
+// field of few, coarse panels decides: 1,280 panels on 16,384 points 333 and 318 us, on
+// 65,536 449 and 553; 1,600 panels (a patch) on 16,384 282 and 295; 2,560 on 262,144 0.90
+// and 0.89 ms; 3,600 on 262,144 1.30 and 1.11, 5,120 1.89 and 1.33.  7-point rule: 960
+// panels on 1,024 points 511 and 212 us, 1,280 on 131,072 1.45 and 1.03 ms (velocity alone
+// 0.87 and 0.77); 640 panels on 65,536 520 and 498 us (311 and 429), 320 on 524,288 points
+// 4.86 and 2.57 ms.  Particles on panels: 20 panels and 8,192 particles 751 and 309 us, 320
+// and 16,384 257 and 292, 320 and 32,768 447 and 351, 20,480 and 180,000 1.85 and 1.63 ms,
+// 5,120 and 262,144 0.85 and 1.14, 524,288 2.43 and 1.89; 1,280 and 400,000 2.42 and 1.37,
+// 2,560 and 400,000 0.76 and 1.05.  A call that names its method or a tile is the direct
+// kernels'.
 bool panfar_pays(int rule, int64_t units, int64_t nt, int method, int tile, int prec) {
   if (method != O3D_METHOD_AUTO || tile > 0 || prec == PREC_FP64 || units > (1 << 26) || nt > (1 << 26)) return false;
-  if (rule == PANFAR_PARTICLES) return units >= 262144 && nt >= 16384;
-  if (units < 256 || nt < 2048) return false;
-  return units >= 1024 || units * nt >= (rule == PANFAR_POINTS7 ? 40000000 : 10000000);
+  if (rule == PANFAR_PARTICLES) {
+    if (nt < 512) return units >= 8192 && units >= 100 * nt;
+    return units * nt >= 2500000000LL || (units >= 400000 && nt <= 2048);
+  }
+  if (nt < 32) return false;
+  if (rule == PANFAR_POINTS7) return units >= 1024 || units * nt >= 160000000LL;
+  return units >= 3072 || (units >= 1024 && nt <= 8 * units);
 }
 
 size_t panfar_bytes(int rule, int64_t units, int64_t nt, bool grad) {

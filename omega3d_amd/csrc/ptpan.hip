@@ -15,8 +15,8 @@
 // evaluates the one-leaf pairs.  k_ptpan_combine adds the slices in order and
 // lists the panels that have particles near enough for the recursion; k_ptpan
 // also keeps the first few such particles of each (slice, panel) in ascending
-// order.  k_ptpan_near gives each listed panel one wave whose lanes walk those
-// pairs with the depth-first tree walk of panels_affect_points (pan_kernels.hpp),
+// order.  k_ptpan_near gives each listed panel one wave that walks those
+// pairs with the node stack of panels_affect_points (pan_kernels.hpp),
 // so the subdivision decisions are the reference's.  Large calls take the separated
 // pairs to the matrix cores (panfar.hip).
 #include "o3d_api_internal.hpp"
@@ -112,41 +112,47 @@ __global__ __launch_bounds__(BLOCK) void k_ptpan_combine(PtPanArgs a) {
 }
 
 // The near pairs of the listed panels, after k_ptpan_combine.  One wave per listed
-// panel: lane l takes slices l, l + 64, ... and walks the particles k_ptpan kept
+// panel: lane l takes slices l, l + 64, ... with the particles k_ptpan kept
 // for its slice, in ascending order; a slice with more than PTPAN_CAP such
 // particles is scanned again by the whole wave (lane l takes its particles l,
-// l + 64, ..., decides each root pair as k_ptpan did).  The walk is the depth-first
-// tree walk of panels_affect_points (Kernels.h:1028-1211).  A fixed butterfly
+// l + 64, ..., decides each root pair as k_ptpan did).  The trees are those
+// of panels_affect_points (Kernels.h:1028-1211), their nodes split together
+// (NodeStack).  A fixed butterfly
 // adds the lanes' sums in FP64, subtracted from the panel's velocity.
 template <int PREC>
 __global__ __launch_bounds__(BLOCK) void k_ptpan_near(PtPanArgs a) {
   using R = typename std::conditional<PREC == PREC_FP64, double, float>::type;
+  extern __shared__ int2 shn[];
   const int lane = threadIdx.x & 63;
   const int64_t wave = ((int64_t)blockIdx.x * BLOCK + threadIdx.x) >> 6;
   const int64_t nwaves = ((int64_t)gridDim.x * BLOCK) >> 6;
   const int64_t listed = *a.near_count;
+  NodeStack stack{shn + (threadIdx.x >> 6) * node_cap(a.maxlev), 0, node_cap(a.maxlev)};
   for (int64_t e = wave; e < listed; e += nwaves) {
     const int64_t i = a.near_list[e];
     float4 s[PAN_F4];
     ptpan_record(a, i, s);
-    R acc[3] = {R(0), R(0), R(0)};
-    // one walk of particle p on this panel, added to acc
-    auto walk = [&](int64_t p) {
-      const float px = a.sx[p], py = a.sy[p], pz = a.sz[p];
-      ptpan_strength<PREC>(s, make_float4(a.ax[p], a.ay[p], a.az[p], 0.0f));
-      R t16[16];
+    const PtRoot<R> root(s);
+    R acc[16];
 #pragma unroll
-      for (int c = 0; c < 16; ++c) t16[c] = R(0);
-      walk_panel<R, false>(px, py, pz, s, a.maxlev, true, t16);
-      acc[0] += t16[0]; acc[1] += t16[1]; acc[2] += t16[2];
+    for (int c = 0; c < 16; ++c) acc[c] = R(0);
+    auto split = [&]() {
+      int2 node;
+      const bool has = stack.pop(node);
+      const int p = has ? node.x : 0;
+      ptpan_strength<PREC>(s, make_float4(a.ax[p], a.ay[p], a.az[p], 0.0f));
+      split_node<R, false>(has, node, a.sx[p], a.sy[p], a.sz[p], s, a.maxlev, acc, stack);
     };
     const int32_t* cnt = a.cnt + i * a.nslice;
     for (int64_t y0 = 0; y0 < a.nslice; y0 += 64) {
       const int64_t y = y0 + lane;
       const int n = y < a.nslice ? cnt[y] : 0;
-      if (n <= PTPAN_CAP) {
-        const int32_t* ent = a.ent + (i * a.nslice + y) * PTPAN_CAP;
-        for (int c = 0; c < n; ++c) walk(ent[c]);
+      const int32_t* ent = a.ent + (i * a.nslice + y) * PTPAN_CAP;
+      for (int c = 0; c < PTPAN_CAP; ++c) {
+        const bool kept = n <= PTPAN_CAP && c < n;
+        if (!wave_any(kept)) break;
+        stack.push(kept, kept ? ent[c] : 0, 0u);
+        while (stack.n >= 64) split();
       }
       // slices whose particles did not all fit: the whole wave, one slice at a time
       uint64_t over = __builtin_amdgcn_ballot_w64(n > PTPAN_CAP);
@@ -155,14 +161,16 @@ __global__ __launch_bounds__(BLOCK) void k_ptpan_near(PtPanArgs a) {
         over &= over - 1;
         const int64_t q0 = (y0 + l) * a.slen;
         const int64_t q1 = q0 + a.slen < a.ns ? q0 + a.slen : a.ns;
-        for (int64_t p = q0 + lane; p < q1; p += 64) {
-          R gx, gy, gz, gs, cx0, cy0, cz0, lim;
-          RootLim rl;
-          panel_root<R>(s, gx, gy, gz, gs, cx0, cy0, cz0, lim, rl);
-          if (!root_leaf<R>(a.sx[p], a.sy[p], a.sz[p], cx0, cy0, cz0, lim, rl, a.maxlev, true)) walk(p);
+        for (int64_t p0 = q0; p0 < q1; p0 += 64) {
+          const int64_t p = p0 + lane;
+          const bool near = p < q1 && !root_leaf<R>(a.sx[p], a.sy[p], a.sz[p], root.cx, root.cy, root.cz, root.lim,
+                                                    root.rl, a.maxlev, true);
+          stack.push(near, (int)p, 0u);
+          while (stack.n >= 64) split();
         }
       }
     }
+    while (stack.n > 0) split();
     double u[3];
 #pragma unroll
     for (int d = 0; d < 3; ++d) u[d] = wave_sum((double)acc[d]);
@@ -224,7 +232,7 @@ static int launch_ptpan(PtPanArgs a, const o3d_opts* o, hipStream_t st) {
   if (prec == P) {                                                                 \
     hipLaunchKernelGGL((k_ptpan<P>), grid, dim3(BLOCK), lds, st, a);               \
     hipLaunchKernelGGL((k_ptpan_combine<P>), grid1, dim3(BLOCK), 0, st, a);        \
-    hipLaunchKernelGGL((k_ptpan_near<P>), grid_near, dim3(BLOCK), 0, st, a);       \
+    hipLaunchKernelGGL((k_ptpan_near<P>), grid_near, dim3(BLOCK), node_lds(a.maxlev), st, a);       \
   }
   O3D_PP(PREC_FP32) O3D_PP(PREC_COMP) O3D_PP(PREC_FP64)
 #undef O3D_PP

@@ -186,3 +186,57 @@ def test_tiles_smaller_than_the_block(mods, core, grads):
         e = rel_errors(a, b)
         print(core, grads, e)
         assert e[0] <= 2e-6 and e[1] <= 2.4e-7
+
+
+def _ptpan(mods, pan, sp, ss, prec, method, tile, maxlev):
+    """points_affect_panels on device arrays: velocities (3, np)"""
+    torch, _lib, _ = mods
+    dev = lambda x: torch.tensor(np.ascontiguousarray(x), device="cuda")
+    nodes, idx, ar = dev(pan.nodes.astype(np.float32)), dev(pan.idx.astype(np.int32)), dev(pan.area)
+    pos, a, out = dev(sp), dev(ss), torch.zeros(3, pan.np, device="cuda")
+    p, q = _lib.Panels(), _lib.Points()
+    p.np, p.nn, p.idx, p.area, q.n = pan.np, nodes.shape[1], idx.data_ptr(), ar.data_ptr(), sp.shape[1]
+    for d in range(3):
+        p.x[d], q.x[d], q.s[d] = nodes[d].data_ptr(), pos[d].data_ptr(), a[d].data_ptr()
+    vel = (C.c_void_p * 3)(*[out[d].data_ptr() for d in range(3)])
+    o = _lib.make_opts("rm", False, prec, method=method, tile=tile, maxlev=maxlev)
+    _lib.check(_lib.lib.o3d_points_affect_panels_dev(C.byref(q), C.byref(p), vel, C.byref(o), None))
+    torch.cuda.synchronize()
+    return out.cpu().numpy()
+
+
+@pytest.mark.parametrize("levels,ns,prec,maxlev", [(1, 8192, "comp", -1), (2, 32769, "comp", 2), (2, 40001, "fp32", -1),
+                                                   (0, 8193, "comp", 8)])
+def test_separated_particles_on_panels(mods, levels, ns, prec, maxlev):
+    """few panels, many particles, a good part of them near: against the direct kernel and,
+    with the first particles alone, the oracle"""
+    pan = scenes.icosphere_panels(levels=levels)
+    sp = scenes.shell_points(ns, 1.01, 2.5, seed=ns).astype(np.float32)
+    ss = (np.random.default_rng(5).normal(size=(3, ns)) / ns).astype(np.float32)
+    a = _ptpan(mods, pan, sp, ss, prec, "auto", 0, maxlev)
+    b = _ptpan(mods, pan, sp, ss, prec, "auto", 256, maxlev)
+    assert not np.array_equal(a, b)
+    assert rel_errors(a, b)[0] <= (6e-6 if prec == "fp32" else 4e-6)
+    assert np.array_equal(_ptpan(mods, pan, sp, -2 * ss, prec, "auto", 0, maxlev), -2 * a)
+    m = 2000
+    lev = 3 if maxlev < 0 else maxlev
+    o64, o32 = (oracle.ptpan("rm", sp[:, :m], ss[:, :m], pan.nodes, pan.idx, pan.area, mode, maxlev=lev)
+                for mode in ("f64", "f32d"))
+    ss[:, m:] = 0
+    bar = max(2e-6 if prec == "comp" else 6e-6, 3 * rel_errors(o32, o64)[0])
+    assert rel_errors(_ptpan(mods, pan, sp, ss, prec, "auto", 0, maxlev), o64)[0] <= bar
+
+
+@pytest.mark.parametrize("maxlev,tile", [(1, 128), (3, 128), (6, 0), (8, 128), (8, 0)])
+def test_deep_trees(mods, maxlev, tile):
+    """points so near the surface that trees reach every level (the stack of nodes at its
+    fullest), direct and separated, against the oracle"""
+    pan = _surface()
+    k = np.arange(40)
+    tp = scenes.shell_points(1100, 1.0002, 1.02, seed=maxlev)
+    v = _call(mods, pan, pan.np, tp, True, "comp", "auto", tile, True, maxlev)
+    args = ("rm", pan.nodes, pan.idx, pan.ts, pan.area, pan.ss, tp[:, k], True)
+    o64, o32 = (np.concatenate(oracle.pan(*args, mode, maxlev=maxlev)) for mode in ("f64", "f32d"))
+    for rows in (slice(0, 3), slice(3, 12)):
+        bar = max(2e-6, 3 * rel_errors(o32[rows], o64[rows])[0])
+        assert rel_errors(v[rows][:, k], o64[rows])[0] <= bar
