@@ -529,7 +529,7 @@ __device__ __forceinline__ int ff_tgt_part(int term) { return term == 0 ? 2 : (t
 __device__ __forceinline__ int ff_quad_slot(int q) { return 16 * (q >> 2) + 8 * (q & 1) + 4 * ((q >> 1) & 1); }
 
 // the pair weights of one scaled squared distance r (RM, WL: core terms included);
-// tau (WL, V2): the pair's scaled core term
+// tau (WL, V2): the pair's scaled core term, of WL 2.5 times
 template <int CORE, int FORM>
 __device__ __forceinline__ void ff_weights(float r, float tau, float& K, float& Bp) {
   if (CORE == CORE_RM || CORE == CORE_EXP || CORE == CORE_SING) {
@@ -542,8 +542,8 @@ __device__ __forceinline__ void ff_weights(float r, float tau, float& K, float& 
     const float ir = frsq(r);
     const float ir2 = ir * ir;
     const float i5 = (ir2 * ir2) * ir;
-    K = i5 * fmaf(1.5f, tau, r);
-    if (FORM == FF_KB) Bp = i5 * fmaf(tau * 2.5f, ir2, 1.0f);
+    K = i5 * fmaf(0.6f, tau, r);    // tau: 2.5 times the core term
+    if (FORM == FF_KB) Bp = i5 * fmaf(tau, ir2, 1.0f);
   } else {                          // CoreFunc.h:317-328
     const float rs = frsq(fmaf(r, r, tau));
     K = rs * fsqrt(rs);
@@ -654,13 +654,9 @@ __global__ __launch_bounds__(FF_FAR_THREADS, 2) void k_ff_far(FFArgs a) {
     tt[s] = COREA || TAU ? q.w : 0.0f;
   }
   f32x16 accB[2], accK[2], accR[2];
-  // the folds add up in registers, or (both weights: no registers left) in the results' place
-  constexpr bool INMEM = FORM == FF_KB;
-  double sum[INMEM ? 1 : NOUT];
-  bool first = true;
-  if (!INMEM)
+  double sum[NOUT];
 #pragma unroll
-    for (int k = 0; k < NOUT; ++k) sum[k] = 0.0;
+  for (int k = 0; k < NOUT; ++k) sum[k] = 0.0;
   const int64_t own = base + lane;
   double* dst = a.farv + (int64_t)blockIdx.y * NOUT * a.nt + own;
 
@@ -713,16 +709,8 @@ __global__ __launch_bounds__(FF_FAR_THREADS, 2) void k_ff_far(FFArgs a) {
     if constexpr (SHEET) ff_epilogue_sheet<GRAD>(ck, c, ox, oy, oz, out);
     else if constexpr (FORM == FF_B) ff_epilogue(c, ox, oy, oz, oa, out);
     else ff_epilogue_k<GRAD>(ck, c, ox, oy, oz, out);
-    if constexpr (INMEM) {
-      if (own < a.nt) {
 #pragma unroll
-        for (int k = 0; k < NOUT; ++k) dst[(int64_t)k * a.nt] = (first ? 0.0 : dst[(int64_t)k * a.nt]) + out[k];
-      }
-      first = false;
-    } else {
-#pragma unroll
-      for (int k = 0; k < NOUT; ++k) sum[k] += out[k];
-    }
+    for (int k = 0; k < NOUT; ++k) sum[k] += out[k];
   };
   // one chunk of 32 sources: its slots and moment operands (two halves of 16 sources) of
   // this lane, its squared distances per set, and the weights of two consecutive halves
@@ -884,7 +872,7 @@ __global__ __launch_bounds__(FF_FAR_THREADS, 2) void k_ff_far(FFArgs a) {
             const __bf16 v1 = q1 < 30 ? part[ff_tgt_part(q1 / 5)][q1 % 5] : (__bf16)0.0f;
             tb[s][m][e] = half ? v1 : v0;
           }
-        if (TAU) tts[s] = tt[s] * rsc * (CORE == CORE_V2 ? rsc : 1.0f);
+        if (TAU) tts[s] = tt[s] * rsc * (CORE == CORE_V2 ? rsc : 2.5f);
       }
     }
 #pragma unroll
@@ -967,7 +955,7 @@ __global__ __launch_bounds__(FF_FAR_THREADS, 2) void k_ff_far(FFArgs a) {
         }
         *reinterpret_cast<bf16x8*>(sl + tid * FF_SL + 8 * v) = row;
       }
-      if (TAU) tc[tid] = P.w * rsc * (CORE == CORE_V2 ? rsc : 1.0f);
+      if (TAU) tc[tid] = P.w * rsc * (CORE == CORE_V2 ? rsc : 2.5f);
     }
     __syncthreads();
     ti = next_tile();
@@ -1022,9 +1010,9 @@ __global__ __launch_bounds__(FF_FAR_THREADS, 2) void k_ff_far(FFArgs a) {
     moments(1, 1);
     fold();
   }
-  if (own < a.nt && (!INMEM || first)) {
+  if (own < a.nt) {
 #pragma unroll
-    for (int k = 0; k < NOUT; ++k) dst[(int64_t)k * a.nt] = INMEM ? 0.0 : sum[k];
+    for (int k = 0; k < NOUT; ++k) dst[(int64_t)k * a.nt] = sum[k];
   }
 }
 

@@ -440,13 +440,14 @@ struct PanFarLayout {
   size_t bytes;
 };
 
-// sources per tile and panels per tile.  128 panels lie within 0.3 radii on the sphere of
-// 20,480, 256 within 0.42: 87 and 82% of the pairs of 524,288 points around it are far
-int tile_of(int rule) { return rule == PANFAR_POINTS ? 128 : 256; }
-int unit_of(int rule) { return rule == PANFAR_POINTS7 ? tile_of(rule) / 7 : tile_of(rule); }
+// sources per tile and panels per tile.  A tile of fewer panels is smaller, but its tables
+// are made for fewer pairs.  5,120 panels on 262,144 points: 1.44 ms with 256 and 1.34 with
+// 128; 20,480 panels on 524,288 4.96 and 5.00, on 2,048 0.38 and 0.44
+int tile_of(int rule, int64_t units) { return rule == PANFAR_POINTS && units < 8192 ? 128 : 256; }
+int unit_of(int rule, int64_t units) { return rule == PANFAR_POINTS7 ? tile_of(rule, units) / 7 : tile_of(rule, units); }
 
 PanFarLayout layout(char* base, int rule, int64_t units, int64_t nt, int nout) {
-  const int T = tile_of(rule), U = unit_of(rule);
+  const int T = tile_of(rule, units), U = unit_of(rule, units);
   const int64_t np = rule == PANFAR_PARTICLES ? nt : units;
   const int64_t nb = (nt + FF_TB - 1) / FF_TB;
   const int64_t ntiles = (units + U - 1) / U;
@@ -514,8 +515,8 @@ int run(const PanArgs* p, const PtPanArgs* t, void* ws, hipStream_t st) {
     a.p.nx = t->nx; a.p.ny = t->ny; a.p.nz = t->nz;
     a.p.idx = t->idx; a.p.np = t->np;
   }
-  const int T = tile_of(RULE), U = unit_of(RULE);
   const int64_t units = PART ? t->ns : p->np, nt = PART ? t->np : p->nt;
+  const int T = tile_of(RULE, units), U = unit_of(RULE, units);
   const int64_t nb = (nt + FF_TB - 1) / FF_TB;
   const int ntiles = (int)((units + U - 1) / U), mwords = (ntiles + 31) / 32;
   const PanFarLayout L = layout(static_cast<char*>(ws), RULE, units, nt, GRAD ? 12 : 3);
