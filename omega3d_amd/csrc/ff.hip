@@ -4,7 +4,7 @@
 //   bounding box -> Hilbert keys -> radix sort (sort.hip) of sources (and of targets
 //   when they are a different collection) -> gather into sorted float4 rows ->
 //   bounding spheres of source tiles and target blocks -> far/near bit per
-//   (block, tile) -> far-field kernel (matrix cores) -> near-field kernel, which
+//   (block, tile) -> near-field plan -> far-field kernel (matrix cores) -> near-field kernel, which
 //   also adds the far part and accumulates into the caller's arrays.
 // Scratch lives in one device workspace per stream (calls on one stream are
 // ordered, so they can share it); it grows when a larger call comes, after the
@@ -48,18 +48,16 @@ bool same_points(const o3d_points* src, const o3d_points* targ) {
   return src->n == targ->n && src->x[0] == targ->x[0] && src->x[1] == targ->x[1] && src->x[2] == targ->x[2];
 }
 
-// scratch of the radix sorts of one call (the scans need none)
-size_t lib_tmp_bytes(int64_t ns, int64_t nt, bool same) {
-  return radix_tmp_bytes(same ? ns : std::max(ns, nt));
-}
+// scratch of the radix sort of one call
+size_t lib_tmp_bytes(int64_t ns, int64_t nt, bool same) { return radix_tmp_bytes(same ? ns : ns + nt); }
 
 // the workspace's sub-arrays in order; with base == nullptr only .bytes is meaningful
 struct Layout {
-  unsigned *bb, *ks_in, *ks_out, *kt_in, *kt_out, *mask, *ctr;
-  int *is_in, *is_out, *it_in, *it_out, *nn, *noff, *items, *ioff, *mfold;
+  unsigned *k_in, *k_out, *mask, *ctr;
+  int *i_in, *i_out, *nn, *items, *ioff, *mfold;
   void* tmp;
   float4 *sp, *sa, *tq, *tsph, *bsph;
-  float *tcs, *tam, *tsg, *bcs;
+  float *box, *tcs, *tam, *tsg, *bcs;
   double *farv, *part;
   unsigned long long* npair;
   size_t bytes;
@@ -71,15 +69,12 @@ Layout layout(char* base, int64_t ns, int64_t nt, bool same, int T, size_t tmp_b
   const int64_t mwords = (ntiles + 31) / 32;
   Carve cv{base};
   Layout L{};
-  L.bb = cv.take<unsigned>(8);
-  L.ks_in = cv.take<unsigned>(ns);
-  L.ks_out = cv.take<unsigned>(ns);
-  L.is_in = cv.take<int>(ns);
-  L.is_out = cv.take<int>(ns);
-  L.kt_in = same ? nullptr : cv.take<unsigned>(nt);
-  L.kt_out = same ? nullptr : cv.take<unsigned>(nt);
-  L.it_in = same ? nullptr : cv.take<int>(nt);
-  L.it_out = same ? nullptr : cv.take<int>(nt);
+  const int64_t n = same ? ns : ns + nt;
+  L.box = cv.take<float>(6 * FF_BOX_GRID);
+  L.k_in = cv.take<unsigned>(n);
+  L.k_out = cv.take<unsigned>(n);
+  L.i_in = cv.take<int>(n);
+  L.i_out = cv.take<int>(n);
   L.tmp = cv.take<char>(tmp_bytes);
   L.sp = cv.take<float4>((size_t)ntiles * T);
   L.sa = cv.take<float4>((size_t)ntiles * T);
@@ -94,7 +89,6 @@ Layout layout(char* base, int64_t ns, int64_t nt, bool same, int T, size_t tmp_b
   L.farv = cv.take<double>((size_t)nout * far_slices(nb, mwords, num_cus()) * nt);
   L.npair = cv.take<unsigned long long>(1);
   L.nn = cv.take<int>(nb);
-  L.noff = cv.take<int>(nb);
   L.items = cv.take<int>(nb);
   L.ioff = cv.take<int>(nb);
   L.mfold = cv.take<int>(1);
@@ -140,44 +134,20 @@ int run(const o3d_points* src, o3d_points* targ, bool self_excl, int T, hipStrea
     for (auto& e : ev) HIPCHK(hipEventCreate(&e.e));
     HIPCHK(hipEventRecord(ev[0].e, st));
   }
-  hipLaunchKernelGGL(k_ff_bbox_init, dim3(1), dim3(64), 0, st, L.bb);
-  hipLaunchKernelGGL(k_ff_bbox, dim3(std::min(grid_of(ns, 256), FF_BBOX_GRID)), dim3(256), 0, st, sv.x, sv.y, sv.z, ns, L.bb);
-  if (!same)
-    hipLaunchKernelGGL(k_ff_bbox, dim3(std::min(grid_of(nt, 256), FF_BBOX_GRID)), dim3(256), 0, st, tv.x, tv.y, tv.z, nt,
-                       L.bb);
-  hipLaunchKernelGGL((k_ff_keys<true>), dim3(grid_of(ns, 256)), dim3(256), 0, st, sv.x, sv.y, sv.z, ns, L.bb, L.ks_in, L.is_in);
-  HIPCHK(hipGetLastError());
-  unsigned* skeys = nullptr;
-  int* sperm = nullptr;
-  int rc = radix_sort_pairs(L.ks_in, L.is_in, L.ks_out, L.is_out, ns, 30, L.tmp, st, &skeys, &sperm);
+  FFSets sets{};
+  sets.x[0] = sv.x; sets.y[0] = sv.y; sets.z[0] = sv.z; sets.n[0] = ns;
+  sets.x[1] = tv.x; sets.y[1] = tv.y; sets.z[1] = tv.z; sets.n[1] = same ? 0 : nt;
+  const int* perm = nullptr;
+  int rc = factored_order(sets, L.box, L.k_in, L.i_in, L.k_out, L.i_out, L.tmp, st, &perm);
   if (rc != O3D_OK) return rc;
-  const int* tperm = sperm;
-  if (!same) {
-    hipLaunchKernelGGL((k_ff_keys<true>), dim3(grid_of(nt, 256)), dim3(256), 0, st, tv.x, tv.y, tv.z, nt, L.bb, L.kt_in, L.it_in);
-    HIPCHK(hipGetLastError());
-    unsigned* tkeys = nullptr;
-    int* tp = nullptr;
-    if ((rc = radix_sort_pairs(L.kt_in, L.it_in, L.kt_out, L.it_out, nt, 30, L.tmp, st, &tkeys, &tp)) != O3D_OK)
-      return rc;
-    tperm = tp;
-  }
-  const int64_t npad = (int64_t)ntiles * T;
-  hipLaunchKernelGGL((k_ff_gather_src<CORE>), dim3(grid_of(npad, 256)), dim3(256), 0, st, sv, sperm, ns, npad, L.sp, L.sa);
-  hipLaunchKernelGGL((k_ff_gather_tgt<CORE, THICK>), dim3(grid_of(nt, 256)), dim3(256), 0, st, tv, tperm, nt, L.tq);
-  hipLaunchKernelGGL(k_ff_bounds, dim3((unsigned)ntiles), dim3(256), 0, st, L.sp, L.sa, ns, T, L.tsph, L.tcs, L.tam,
-                     L.tsg);
-  hipLaunchKernelGGL(k_ff_bounds, dim3((unsigned)nb), dim3(256), 0, st, L.tq, (const float4*)nullptr, nt, FF_TB, L.bsph,
-                     L.bcs, (float*)nullptr, (float*)nullptr);
+  const int *sperm = perm, *tperm = same ? perm : perm + ns;
+  hipLaunchKernelGGL((k_ff_rows<CORE, THICK>), dim3((unsigned)(ntiles + nb)), dim3(256), 0, st, sv, tv, sperm, tperm, ns,
+                     nt, T, ntiles, L.sp, L.sa, L.tq, FFBounds{L.tsph, L.tcs, L.tam, L.tsg},
+                     FFBounds{L.bsph, L.bcs, nullptr, nullptr}, L.nn);
   hipLaunchKernelGGL((k_ff_classify<CORE>), dim3(grid_of(nb * mwords, 256)), dim3(256), 0, st, L.bsph, L.bcs, nb, L.tsph,
-                     L.tcs, ntiles, mwords, L.mask);
-  hipLaunchKernelGGL(k_ff_plan_count, dim3(grid_of(nb, 256)), dim3(256), 0, st, L.mask, nb, mwords, ntiles, L.nn);
-  HIPCHK(hipGetLastError());
-  if ((rc = exclusive_scan_i32(L.nn, L.noff, nb, st)) != O3D_OK) return rc;
-  hipLaunchKernelGGL(k_ff_plan_items, dim3(grid_of(nb, 256)), dim3(256), 0, st, L.nn, L.noff, nb, near_split(nb, ntiles), L.items,
-                     L.mfold);
-  HIPCHK(hipGetLastError());
-  if ((rc = exclusive_scan_i32(L.items, L.ioff, nb, st)) != O3D_OK) return rc;
-  hipLaunchKernelGGL(k_ff_zero_u32, dim3(1), dim3(64), 0, st, L.ctr);
+                     L.tcs, ntiles, mwords, L.mask, L.nn);
+  hipLaunchKernelGGL(k_ff_plan, dim3(1), dim3(FF_PLAN_THREADS), 0, st, L.nn, nb, near_split(nb, ntiles), L.items, L.ioff,
+                     L.mfold, L.ctr, (unsigned*)nullptr);
   HIPCHK(hipGetLastError());
 
   FFArgs a{};
@@ -242,6 +212,24 @@ int run_core(const o3d_points* src, o3d_points* targ, bool thick, int prec, bool
 
 }  // namespace
 
+// the order of one or two sets along the curve: *perm gets the first set's permutation and
+// the second's after it.  box, keys and indices in the caller's scratch
+int factored_order(const FFSets& s, float* box, unsigned* ka, int* va, unsigned* kb, int* vb, void* tmp, hipStream_t st,
+                   const int** perm) {
+  const int64_t n = s.n[0] + s.n[1];
+  const int bits = key_bits(n, s.n[1] > 0);
+  const unsigned g = std::min<unsigned>(FF_BOX_GRID, grid_of(n, 1024));
+  hipLaunchKernelGGL(k_ff_box, dim3(g), dim3(256), 0, st, s, box);
+  hipLaunchKernelGGL(k_ff_hkeys, dim3(std::min(1024u, grid_of(n, 256))), dim3(256), 0, st, s, box, (int)g,
+                     s.n[1] > 0 ? bits - 1 : bits, ka, va);
+  HIPCHK(hipGetLastError());
+  unsigned* keys = nullptr;
+  int* vals = nullptr;
+  const int rc = radix_sort_pairs(ka, va, kb, vb, n, bits, tmp, st, &keys, &vals);
+  *perm = vals;
+  return rc;
+}
+
 // Morton order of n points (the direct kernel's target order): workspace bytes,
 // and the order itself, written into ws (bounding box, keys, indices and the
 // sort's scratch; *perm points into ws)
@@ -262,7 +250,7 @@ int point_order(const float* x, const float* y, const float* z, int64_t n, void*
   void* tmp = p + 256 + 4 * a;
   hipLaunchKernelGGL(k_ff_bbox_init, dim3(1), dim3(64), 0, st, bb);
   hipLaunchKernelGGL(k_ff_bbox, dim3(std::min(grid_of(n, 256), FF_BBOX_GRID)), dim3(256), 0, st, x, y, z, n, bb);
-  hipLaunchKernelGGL((k_ff_keys<false>), dim3(grid_of(n, 256)), dim3(256), 0, st, x, y, z, n, bb, kin, iin);
+  hipLaunchKernelGGL(k_ff_keys, dim3(grid_of(n, 256)), dim3(256), 0, st, x, y, z, n, bb, kin, iin);
   HIPCHK(hipGetLastError());
   unsigned* sk = nullptr;
   int* sp = nullptr;
@@ -294,9 +282,8 @@ int sorted_sources(const o3d_points* src, const int32_t* perm, int tile, void* w
   float4* sph = (float4*)(p + 2 * r(sizeof(float4) * (size_t)n));
   float* cs = (float*)(p + 2 * r(sizeof(float4) * (size_t)n) + r(sizeof(float4) * (size_t)ntiles));
   const SrcView sv{src->x[0], src->x[1], src->x[2], src->r, src->s[0], src->s[1], src->s[2]};
-  hipLaunchKernelGGL((k_ff_gather_src<CORE_EXP>), dim3(grid_of(n, 256)), dim3(256), 0, st, sv, perm, n, n, sp, sa);
-  hipLaunchKernelGGL(k_ff_bounds, dim3((unsigned)ntiles), dim3(256), 0, st, (const float4*)sp, (const float4*)nullptr,
-                     n, tile, sph, cs, (float*)nullptr, (float*)nullptr);
+  hipLaunchKernelGGL((k_ff_gather_src<CORE_EXP>), dim3(grid_of(n, 256)), dim3(256), 0, st, sv, perm, n, sp, sa);
+  hipLaunchKernelGGL(k_ff_bounds, dim3((unsigned)ntiles), dim3(256), 0, st, (const float4*)sp, n, tile, sph, cs);
   HIPCHK(hipGetLastError());
   a->sp = sp;
   a->sa = sa;
@@ -439,7 +426,7 @@ extern "C" int o3d_morton_order_dev(const float* x, const float* y, const float*
   if ((rc = point_order(x, y, z, n, ws, st, &p)) != O3D_OK) return rc;
   HIPCHK(hipMemcpyAsync(perm, p, sizeof(int32_t) * (size_t)n, hipMemcpyDeviceToDevice, st));
   // the keys in index order, from the same box (point_order left it at the workspace's start)
-  hipLaunchKernelGGL((k_ff_keys<false>), dim3(grid_of(n, 256)), dim3(256), 0, st, x, y, z, n, (const unsigned*)ws,
+  hipLaunchKernelGGL(k_ff_keys, dim3(grid_of(n, 256)), dim3(256), 0, st, x, y, z, n, (const unsigned*)ws,
                      (unsigned*)keys, (int*)nullptr);
   HIPCHK(hipGetLastError());
   return O3D_OK;

@@ -215,10 +215,8 @@ __device__ __forceinline__ unsigned hilbert30(unsigned x, unsigned y, unsigned z
   return (spread10(c[0] ^ t) << 2) | (spread10(c[1] ^ t) << 1) | spread10(c[2] ^ t);
 }
 
-// 30-bit keys on the common bounding box (Morton order, or along the Hilbert curve), and
-// the identity permutation
-template <bool HILBERT>
-__global__ __launch_bounds__(256) void k_ff_keys(const float* x, const float* y, const float* z, int64_t n,
+// 30-bit Morton keys on the common bounding box, and the identity permutation
+static __global__ __launch_bounds__(256) void k_ff_keys(const float* x, const float* y, const float* z, int64_t n,
                                                  const unsigned* bb, unsigned* keys, int* idx) {
   const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
   if (i >= n) return;
@@ -226,30 +224,109 @@ __global__ __launch_bounds__(256) void k_ff_keys(const float* x, const float* y,
   const float ext = fmaxf(fmaxf(fdec(bb[3]) - lx, fdec(bb[4]) - ly), fdec(bb[5]) - lz);
   const float sc = ext > 0.0f ? 1023.0f / ext : 0.0f;
   const float q[3] = {(x[i] - lx) * sc, (y[i] - ly) * sc, (z[i] - lz) * sc};
-  unsigned c[3];
+  unsigned k = 0;
 #pragma unroll
-  for (int d = 0; d < 3; ++d) c[d] = (unsigned)fminf(fmaxf(q[d], 0.0f), 1023.0f);   // NaN -> 0
-  keys[i] = HILBERT ? hilbert30(c[0], c[1], c[2]) : spread10(c[0]) | (spread10(c[1]) << 1) | (spread10(c[2]) << 2);
+  for (int d = 0; d < 3; ++d) {
+    const float c = fminf(fmaxf(q[d], 0.0f), 1023.0f);   // NaN -> 0
+    k |= spread10((unsigned)c) << d;
+  }
+  keys[i] = k;
   if (idx) idx[i] = (int)i;
 }
 
-// rows n .. npad - 1: the last source's place with no strength
-template <int CORE>
-__global__ __launch_bounds__(256) void k_ff_gather_src(SrcView s, const int* perm, int64_t n, int64_t npad, float4* sp,
-                                                       float4* sa) {
-  const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (i >= npad) return;
-  const int j = perm[i < n ? i : n - 1];
-  sp[i] = make_float4(s.x[j], s.y[j], s.z[j], core_term<CORE>(s.r[j]));
-  sa[i] = i < n ? make_float4(s.ax[j], s.ay[j], s.az[j], 0.0f) : make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+// ---- the factored calls' preparation ------------------------------------------------
+// Sources and targets (one set where they are the same collection) are sorted in one go,
+// the set as the top bit of the key, and each step is one launch for both: box, keys,
+// the sort's passes, rows and bounds, far bits, plan.  A small call waits for its launches,
+// about 4 us each.  Two sets of 2,048 and 5,120: 40 launches before, 14 now.
+struct FFSets {
+  const float *x[2], *y[2], *z[2];
+  int64_t n[2];          // n[1] = 0: one set
+  const uint32_t* idx;   // set `pan` is panels: three node indices each, x, y, z the nodes
+  int32_t pan;
+};
+__device__ __forceinline__ void ff_position(const FFSets& s, int set, int64_t i, float* p) {
+  if (s.idx && set == s.pan) {   // about the centroid: it only decides the order
+    const uint32_t a = s.idx[3 * i], b = s.idx[3 * i + 1], c = s.idx[3 * i + 2];
+    p[0] = (s.x[set][a] + s.x[set][b] + s.x[set][c]) * (1.0f / 3.0f);
+    p[1] = (s.y[set][a] + s.y[set][b] + s.y[set][c]) * (1.0f / 3.0f);
+    p[2] = (s.z[set][a] + s.z[set][b] + s.z[set][c]) * (1.0f / 3.0f);
+  } else {
+    p[0] = s.x[set][i]; p[1] = s.y[set][i]; p[2] = s.z[set][i];
+  }
 }
 
-template <int CORE, bool THICK>
-__global__ __launch_bounds__(256) void k_ff_gather_tgt(TgtView t, const int* perm, int64_t n, float4* tq) {
+// largest of each of N values over the workgroup's four waves, in every thread
+template <int N>
+__device__ __forceinline__ void wg_max_n(float* v) {
+  __shared__ float red[4][N];
+#pragma unroll
+  for (int off = 32; off > 0; off >>= 1)
+#pragma unroll
+    for (int k = 0; k < N; ++k) v[k] = fmaxf(v[k], __shfl_xor(v[k], off));
+  __syncthreads();
+  if ((threadIdx.x & 63) == 0)
+#pragma unroll
+    for (int k = 0; k < N; ++k) red[threadIdx.x >> 6][k] = v[k];
+  __syncthreads();
+#pragma unroll
+  for (int k = 0; k < N; ++k) v[k] = fmaxf(fmaxf(red[0][k], red[1][k]), fmaxf(red[2][k], red[3][k]));
+}
+
+// each workgroup's box {-lo, hi} over its strided share of both sets
+constexpr int FF_BOX_GRID = 256;
+static __global__ __launch_bounds__(256) void k_ff_box(FFSets s, float* part) {
+  float v[6];
+#pragma unroll
+  for (int d = 0; d < 6; ++d) v[d] = -__builtin_huge_valf();
+  for (int set = 0; set < 2; ++set)
+    for (int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x; i < s.n[set]; i += (int64_t)gridDim.x * 256) {
+      float p[3];
+      ff_position(s, set, i, p);
+#pragma unroll
+      for (int d = 0; d < 3; ++d) { v[d] = fmaxf(v[d], -p[d]); v[3 + d] = fmaxf(v[3 + d], p[d]); }
+    }
+  wg_max_n<6>(v);
+  if (threadIdx.x == 0)
+#pragma unroll
+    for (int d = 0; d < 6; ++d) part[6 * blockIdx.x + d] = v[d];
+}
+
+// the top `bits` bits of the 30-bit Hilbert keys on the common box, below the set's bit,
+// and each set's identity permutation
+static __global__ __launch_bounds__(256) void k_ff_hkeys(FFSets s, const float* part, int nparts, int bits,
+                                                  unsigned* keys, int* idx) {
+  float v[6];
+#pragma unroll
+  for (int d = 0; d < 6; ++d) v[d] = -__builtin_huge_valf();
+  for (int k = threadIdx.x; k < nparts; k += 256)
+#pragma unroll
+    for (int d = 0; d < 6; ++d) v[d] = fmaxf(v[d], part[6 * k + d]);
+  wg_max_n<6>(v);
+  const float ext = fmaxf(fmaxf(v[3] + v[0], v[4] + v[1]), v[5] + v[2]);
+  const float sc = ext > 0.0f ? 1023.0f / ext : 0.0f;
+  const int64_t n = s.n[0] + s.n[1];
+  for (int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x; i < n; i += (int64_t)gridDim.x * 256) {
+    const int set = i >= s.n[0];
+    const int64_t j = set ? i - s.n[0] : i;
+    float p[3];
+    ff_position(s, set, j, p);
+    unsigned c[3];
+#pragma unroll
+    for (int d = 0; d < 3; ++d) c[d] = (unsigned)fminf(fmaxf((p[d] + v[d]) * sc, 0.0f), 1023.0f);   // NaN -> 0
+    keys[i] = ((unsigned)set << bits) | (hilbert30(c[0], c[1], c[2]) >> (30 - bits));
+    idx[i] = (int)j;
+  }
+}
+
+// sources as rows in a given order (the direct EXP kernel's)
+template <int CORE>
+__global__ __launch_bounds__(256) void k_ff_gather_src(SrcView s, const int* perm, int64_t n, float4* sp, float4* sa) {
   const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
   if (i >= n) return;
   const int j = perm[i];
-  tq[i] = make_float4(t.x[j], t.y[j], t.z[j], THICK ? core_term<CORE>(t.r[j]) : 0.0f);
+  sp[i] = make_float4(s.x[j], s.y[j], s.z[j], core_term<CORE>(s.r[j]));
+  sa[i] = make_float4(s.ax[j], s.ay[j], s.az[j], 0.0f);
 }
 
 // workgroup-wide reductions over 256 threads (4 waves), result in every thread
@@ -263,15 +340,10 @@ __device__ __forceinline__ float wg_max(float v, float* red) {
 }
 __device__ __forceinline__ float wg_min(float v, float* red) { return -wg_max(-v, red); }
 
-// bounding sphere (bbox centre, largest distance), largest core term and (when pa
-// is given) a bound of |alpha| and |q| and the sign of the first nonzero strength (0: none), by
-// its first nonzero component, of each group of `group` consecutive sorted points; one
-// workgroup per group
-static __global__ __launch_bounds__(256) void k_ff_bounds(const float4* p, const float4* pa, int64_t n, int group,
-                                                   float4* sph, float* cs, float* amax, float* sign) {
+// bounding sphere (bbox centre, largest distance) and largest core term of each group of
+// `group` consecutive sorted points; one workgroup per group
+static __global__ __launch_bounds__(256) void k_ff_bounds(const float4* p, int64_t n, int group, float4* sph, float* cs) {
   __shared__ float red[4];
-  __shared__ unsigned lead;   // smallest 2 i + (negative) over the group's points i with a strength
-  if (threadIdx.x == 0) lead = 0xffffffffu;
   const int64_t b0 = (int64_t)blockIdx.x * group;
   const int64_t b1 = (b0 + group) < n ? (b0 + group) : n;
   float lo[3] = {__builtin_huge_valf(), __builtin_huge_valf(), __builtin_huge_valf()};
@@ -299,29 +371,98 @@ static __global__ __launch_bounds__(256) void k_ff_bounds(const float4* p, const
     r2 = fmaxf(r2, fmaf(dz, dz, fmaf(dy, dy, dx * dx)));
   }
   r2 = wg_max(r2, red);
-  float am = 0.0f;   // largest component: no square that could leave the range
-  if (pa)
-    for (int64_t i = b0 + threadIdx.x; i < b1; i += blockDim.x) {
-      const float4 q = pa[i];
-      am = fmaxf(fmaxf(fmaxf(am, fabsf(q.x)), fmaxf(fabsf(q.y), fabsf(q.z))), fabsf(q.w));
-      const float f = q.x != 0.0f ? q.x : q.y != 0.0f ? q.y : q.z != 0.0f ? q.z : q.w;
-      if (f != 0.0f) atomicMin(&lead, 2u * (unsigned)(i - b0) + (f < 0.0f ? 1u : 0u));
-    }
-  am = wg_max(am, red);   // its barriers order the atomics too
   if (threadIdx.x == 0) {
     // margin for the rounding of the distances above
     sph[blockIdx.x] = make_float4(c[0], c[1], c[2], __fsqrt_rn(r2) * 1.00001f + 1e-30f);
     cs[blockIdx.x] = cmax;
-    if (amax) amax[blockIdx.x] = am * 1.7321f;   // sqrt 3, rounded up
-    if (sign) sign[blockIdx.x] = lead == 0xffffffffu ? 0.0f : (lead & 1u) ? -1.0f : 1.0f;
   }
 }
 
-// far bit of every (target block, source tile): one thread per 32 tiles of a block
+// where a group's bounds go: sphere (bbox centre, largest distance), largest core term,
+// and of sources (am) a bound of |alpha| and |q| and the sign of the first nonzero strength
+// (0: none), by its first nonzero component
+struct FFBounds {
+  float4* sph;
+  float *cs, *am, *sign;
+};
+// the bounds of the workgroup's points, N per thread (valid: this thread has some) with
+// core terms p.w; strengths a, of sources
+template <int N>
+__device__ __forceinline__ void ff_group_bounds(bool valid, const float4* p, const float4* a, const FFBounds& out,
+                                                int64_t g) {
+  const float inf = __builtin_huge_valf();
+  float v[7] = {-inf, -inf, -inf, -inf, -inf, -inf, 0.0f};
+  if (valid)
+#pragma unroll
+    for (int k = 0; k < N; ++k) {
+      const float q[3] = {p[k].x, p[k].y, p[k].z};
+#pragma unroll
+      for (int d = 0; d < 3; ++d) { v[d] = fmaxf(v[d], -q[d]); v[3 + d] = fmaxf(v[3 + d], q[d]); }
+      v[6] = fmaxf(v[6], p[k].w);
+    }
+  wg_max_n<7>(v);
+  const float c[3] = {0.5f * v[3] - 0.5f * v[0], 0.5f * v[4] - 0.5f * v[1], 0.5f * v[5] - 0.5f * v[2]};
+  float w[3] = {0.0f, 0.0f, -inf};   // squared radius, largest component, -(2 i + negative) of the first strength
+  if (valid)
+#pragma unroll
+    for (int k = 0; k < N; ++k) {
+      const float dx = p[k].x - c[0], dy = p[k].y - c[1], dz = p[k].z - c[2];
+      w[0] = fmaxf(w[0], fmaf(dz, dz, fmaf(dy, dy, dx * dx)));
+      if (a) {   // no square that could leave the range
+        w[1] = fmaxf(fmaxf(fmaxf(w[1], fabsf(a[k].x)), fmaxf(fabsf(a[k].y), fabsf(a[k].z))), fabsf(a[k].w));
+        const float f = a[k].x != 0.0f ? a[k].x : a[k].y != 0.0f ? a[k].y : a[k].z != 0.0f ? a[k].z : a[k].w;
+        if (f != 0.0f) w[2] = fmaxf(w[2], -(float)(2 * (N * (int)threadIdx.x + k) + (f < 0.0f ? 1 : 0)));
+      }
+    }
+  wg_max_n<3>(w);
+  if (threadIdx.x != 0) return;
+  // margin for the rounding of the distances above
+  out.sph[g] = make_float4(c[0], c[1], c[2], __fsqrt_rn(w[0]) * 1.00001f + 1e-30f);
+  out.cs[g] = v[6];
+  if (a) {
+    out.am[g] = w[1] * 1.7321f;   // sqrt 3, rounded up
+    out.sign[g] = w[2] == -inf ? 0.0f : ((int)-w[2] & 1) ? -1.0f : 1.0f;
+  }
+}
+
+// rows and bounds, one workgroup per source tile and then one per target block: sources up
+// to a whole tile (the rest: the last one's place with no strength) and targets; the
+// blocks' near counts are cleared for k_ff_classify
+template <int CORE, bool THICK>
+__global__ __launch_bounds__(256) void k_ff_rows(SrcView s, TgtView t, const int* sperm, const int* tperm, int64_t ns,
+                                                 int64_t nt, int tile, int ntiles, float4* sp, float4* sa, float4* tq,
+                                                 FFBounds sb, FFBounds tb, int* nn) {
+  const int tid = threadIdx.x;
+  if ((int)blockIdx.x < ntiles) {
+    const int64_t i = (int64_t)blockIdx.x * tile + tid;
+    float4 p{}, a{};
+    if (tid < tile) {
+      const int j = sperm[i < ns ? i : ns - 1];
+      p = make_float4(s.x[j], s.y[j], s.z[j], core_term<CORE>(s.r[j]));
+      if (i < ns) a = make_float4(s.ax[j], s.ay[j], s.az[j], 0.0f);
+      sp[i] = p;
+      sa[i] = a;
+    }
+    ff_group_bounds<1>(tid < tile, &p, &a, sb, blockIdx.x);
+  } else {
+    const int64_t b = (int64_t)blockIdx.x - ntiles, i = b * FF_TB + tid;
+    float4 p{};
+    if (i < nt) {
+      const int j = tperm[i];
+      p = make_float4(t.x[j], t.y[j], t.z[j], THICK ? core_term<CORE>(t.r[j]) : 0.0f);
+      tq[i] = p;
+    }
+    ff_group_bounds<1>(i < nt, &p, nullptr, tb, b);
+    if (tid == 0) nn[b] = 0;
+  }
+}
+
+// far bit of every (target block, source tile), and the near tiles counted into nn (cleared
+// before): one thread per 32 tiles of a block
 template <int CORE>
 __global__ __launch_bounds__(256) void k_ff_classify(const float4* bsph, const float* bcs, int64_t nb,
                                                      const float4* tsph, const float* tcs, int ntiles, int mwords,
-                                                     unsigned* mask) {
+                                                     unsigned* mask, int* nn) {
   const int64_t g = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
   if (g >= nb * mwords) return;
   const int64_t b = g / mwords;
@@ -329,9 +470,9 @@ __global__ __launch_bounds__(256) void k_ff_classify(const float4* bsph, const f
   const float4 cb = bsph[b];
   const float csb = bcs[b];
   unsigned bits = 0u;
-  for (int k = 0; k < 32; ++k) {
+  const int left = ntiles - 32 * w < 32 ? ntiles - 32 * w : 32;
+  for (int k = 0; k < left; ++k) {
     const int ti = w * 32 + k;
-    if (ti >= ntiles) break;
     const float4 ct = tsph[ti];
     const float dx = cb.x - ct.x, dy = cb.y - ct.y, dz = cb.z - ct.z;
     const float gap = __fsqrt_rn(fmaf(dz, dz, fmaf(dy, dy, dx * dx))) - cb.w - ct.w;
@@ -341,6 +482,7 @@ __global__ __launch_bounds__(256) void k_ff_classify(const float4* bsph, const f
     if (far) bits |= 1u << k;
   }
   mask[g] = bits;
+  atomicAdd(&nn[b], left - __popc(bits));
 }
 
 // velocity and gradient (ug order, g = -3 D + skew(W)) of one target from its 32
@@ -1024,36 +1166,56 @@ __global__ __launch_bounds__(FF_FAR_THREADS, 2) void k_ff_far(FFArgs a) {
 // queue by a persistent kernel and write FP64 partial sums; the combine kernel
 // adds a block's partials in item order, so results do not depend on scheduling.
 
-__device__ __forceinline__ int near_tiles_of(const unsigned* mrow, int mwords, int ntiles) {
-  int far = 0;
-  for (int w = 0; w < mwords; ++w) far += __popc(mrow[w]);
-  return ntiles - far;
-}
-
-// nn[b] = number of near tiles of block b
-static __global__ __launch_bounds__(256) void k_ff_plan_count(const unsigned* mask, int64_t nb, int mwords, int ntiles,
-                                                       int* nn) {
-  const int64_t b = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (b < nb) nn[b] = near_tiles_of(mask + b * mwords, mwords, ntiles);
-}
-
-// after the exclusive scan noff of nn: M = max(ceil(total / (split nb)), FF_M0, or fewer
-// while that makes less than 2,048 items) and the item count of every block (at most
-// (split + 1) nb items in all)
-static __global__ __launch_bounds__(256) void k_ff_plan_items(const int* nn, const int* noff, int64_t nb, int split,
-                                                       int* items, int* mfold) {
-  const int64_t b = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  const int64_t total = (int64_t)noff[nb - 1] + nn[nb - 1];
-  int64_t m = (total + split * nb - 1) / (split * nb);
-  const int64_t m0 = (total + 2047) / 2048 < FF_M0 ? (total + 2047) / 2048 : FF_M0;
+// The plan, by one workgroup: M = max(ceil(total / (split nb)), FF_M0, or fewer while that
+// makes less than 2,048 items), the item count of every block (at most (split + 1) nb items
+// in all) and its exclusive scan; the counters of the kernels that follow cleared
+constexpr int FF_PLAN_THREADS = 1024;
+static __global__ __launch_bounds__(FF_PLAN_THREADS) void k_ff_plan(const int* nn, int64_t nb, int split, int* items,
+                                                             int* ioff, int* mfold, unsigned* ctr, unsigned* count) {
+  __shared__ long long sh[FF_PLAN_THREADS / 64];
+  const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6;
+  // inclusive scan over the workgroup; every thread also gets the sum
+  auto scan = [&](long long x, long long* all) {
+#pragma unroll
+    for (int o = 1; o < 64; o <<= 1) {
+      const long long y = __shfl_up(x, o, 64);
+      if (lane >= o) x += y;
+    }
+    __syncthreads();
+    if (lane == 63) sh[w] = x;
+    __syncthreads();
+    long long before = 0, sum = 0;
+    for (int k = 0; k < FF_PLAN_THREADS / 64; ++k) {
+      before += k < w ? sh[k] : 0;
+      sum += sh[k];
+    }
+    *all = sum;
+    return before + x;
+  };
+  long long mine = 0, total;
+  for (int64_t b = tid; b < nb; b += FF_PLAN_THREADS) mine += nn[b];
+  (void)scan(mine, &total);
+  long long m = (total + split * nb - 1) / (split * nb);
+  const long long m0 = (total + 2047) / 2048 < FF_M0 ? (total + 2047) / 2048 : FF_M0;
   m = m < m0 ? m0 : m;
   m = m < 1 ? 1 : m;
-  if (b == 0) *mfold = (int)m;
-  if (b < nb) items[b] = (int)((nn[b] + m - 1) / m);
-}
-
-static __global__ void k_ff_zero_u32(unsigned* p) {
-  if (threadIdx.x == 0) *p = 0u;
+  if (tid == 0) {
+    *mfold = (int)m;
+    *ctr = 0u;
+    if (count) *count = 0u;
+  }
+  long long carry = 0;
+  for (int64_t b0 = 0; b0 < nb; b0 += FF_PLAN_THREADS) {
+    const int64_t b = b0 + tid;
+    const int it = b < nb ? (int)((nn[b] + m - 1) / m) : 0;
+    long long sum;
+    const long long incl = scan(it, &sum);
+    if (b < nb) {
+      items[b] = it;
+      ioff[b] = (int)(carry + incl - it);
+    }
+    carry += sum;
+  }
 }
 
 // per-target partial of one item: near tiles of rank [r0, r1) among block b's
@@ -1226,6 +1388,11 @@ static __global__ void k_ff_zero_u64(unsigned long long* p) {
 
 // ---- host side shared by the factored calls ----------------------------------------
 
+// Key bits, the set's bit included, of n points in all: up to 131,072 points 24, which sort
+// in three passes (2^8 cells per axis or one bit less hold less than a point each even in a
+// ring), then all 30 or 31 in four
+inline int key_bits(int64_t n, bool two_sets) { return n <= 131072 ? 24 : two_sets ? 31 : 30; }
+
 // sequential sub-allocation of a workspace, 256-byte aligned
 struct Carve {
   char* base;
@@ -1264,5 +1431,9 @@ inline int far_slices(int64_t nb, int64_t mwords, int cus) {
   return (int)std::max<int64_t>(1, std::min<int64_t>({want, mwords, 32}));
 }
 
+// (ff.hip) the order of one or two sets along the curve, in the caller's scratch: *perm gets
+// the first set's permutation and the second's after it
+int factored_order(const FFSets& s, float* box, unsigned* ka, int* va, unsigned* kb, int* vb, void* tmp, hipStream_t st,
+                   const int** perm);
 
 }  // namespace o3d

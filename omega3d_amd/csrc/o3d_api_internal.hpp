@@ -67,8 +67,6 @@ int point_order(const float* x, const float* y, const float* z, int64_t n, void*
 size_t radix_tmp_bytes(int64_t n);
 int radix_sort_pairs(unsigned* ka, int* va, unsigned* kb, int* vb, int64_t n, int bits, void* tmp, hipStream_t st,
                      unsigned** keys, int** vals);
-// exclusive prefix sum of n int32 values (one workgroup; meant for small n)
-int exclusive_scan_i32(const int* in, int* out, int64_t n, hipStream_t st);
 // a collection large enough for the factored method to pay when the caller leaves the choice open
 constexpr int64_t FF_AUTO_MIN_N = 65536;
 // the same for an instance of a batch or a session of the server: their factored work runs on

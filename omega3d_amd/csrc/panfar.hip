@@ -47,80 +47,78 @@ struct PanFarArgs {
 // limit that is no number keeps the panel out of the far field
 __device__ __forceinline__ float plain_limit(float lim) { return lim >= 0.0f ? lim * 1.00001f : __builtin_huge_valf(); }
 
-// centroids of the panels for the order (as the decisions take them)
-__global__ __launch_bounds__(256) void k_pf_centroids(PanArgs a, float* x, float* y, float* z) {
-  const int64_t p = (int64_t)blockIdx.x * 256 + threadIdx.x;
-  if (p >= a.np) return;
-  float v[9], cx, cy, cz;
-  panel_vertices(a, p, v);
-  centroid_exact(v[0], v[1], v[2], v[3], v[4], v[5], v[6], v[7], v[8], cx, cy, cz);
-  x[p] = cx; y[p] = cy; z[p] = cz;
-}
-
-// source rows 0 .. npad - 1 in sorted order, and the panels' records and near-test rows
+// rows, records and bounds, one workgroup per tile of sources and then one per block of
+// targets (ff_kernels.hpp: k_ff_rows): source rows up to a whole tile, the panels' records
+// and near-test rows, and targets: points, or panels' centroids with their limit
 template <int RULE>
-__global__ __launch_bounds__(256) void k_pf_sources(PanFarArgs a, const int* perm, float4* sp, float4* sa) {
-  const int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x;
-  if (RULE == PANFAR_PARTICLES) {
-    if (i >= (int64_t)a.f.ntiles * a.f.tile) return;
-    const int j = perm[i < a.units ? i : a.units - 1];
-    sp[i] = make_float4(a.t.sx[j], a.t.sy[j], a.t.sz[j], 0.0f);
-    sa[i] = i < a.units ? make_float4(a.t.ax[j], a.t.ay[j], a.t.az[j], 0.0f) : make_float4(0.f, 0.f, 0.f, 0.f);
-    return;
-  }
-  if (i >= (int64_t)a.f.ntiles * a.unit) return;
-  const bool real = i < a.units;
-  const int64_t p = perm[real ? i : a.units - 1];
-  if (RULE == PANFAR_POINTS) {
-    float4 s[PAN_F4];
-    panel_record(a.p, p, s);
-    sp[i] = make_float4(s[3].x, s[3].y, s[3].z, plain_limit(s[4].z * 4.0f));
-    sa[i] = real ? s[2] : make_float4(0.f, 0.f, 0.f, 0.f);
-    if (!real) return;
-#pragma unroll
-    for (int k = 0; k < PAN_F4; ++k) a.rec[PAN_F4 * i + k] = s[k];
-    a.cen[i] = s[3];
-    return;
-  }
-  // seven rows per panel, the last of a tile's panels filling the tile up
-  float4 s[G7_F4];
-  g7_record(a.p, p, s);
-  const float lim = plain_limit(sqrtf(s[7].x));
-  const float pt[21] = {s[0].x, s[0].y, s[0].z, s[0].w, s[1].x, s[1].y, s[1].z, s[1].w, s[2].x, s[2].y, s[2].z,
-                        s[2].w, s[3].x, s[3].y, s[3].z, s[3].w, s[4].x, s[4].y, s[4].z, s[4].w, s[5].x};
-  const int64_t t = i / a.unit;
-  const int j = (int)(i - t * a.unit);
-  const int64_t row = t * a.f.tile + 7 * j;
-#pragma unroll
-  for (int q = 0; q < 7; ++q) {
-    const float w = real ? (float)g7_weight(q) : 0.0f;
-    sp[row + q] = make_float4(pt[3 * q], pt[3 * q + 1], pt[3 * q + 2], lim);
-    sa[row + q] = real ? make_float4(w * s[6].x, w * s[6].y, w * s[6].z, w * s[6].w) : make_float4(0.f, 0.f, 0.f, 0.f);
-  }
-  if (j == a.unit - 1)
-    for (int k = 7 * a.unit; k < a.f.tile; ++k) {
-      sp[t * a.f.tile + k] = make_float4(pt[0], pt[1], pt[2], lim);
-      sa[t * a.f.tile + k] = make_float4(0.f, 0.f, 0.f, 0.f);
+__global__ __launch_bounds__(256) void k_pf_rows(PanFarArgs a, const int* sperm, float4* sp, float4* sa, float4* tq,
+                                                 FFBounds sb, FFBounds tb, int* nn) {
+  constexpr int N = RULE == PANFAR_POINTS7 ? 7 : 1;
+  const int tid = threadIdx.x;
+  if ((int)blockIdx.x >= a.f.ntiles) {
+    const int64_t b = (int64_t)blockIdx.x - a.f.ntiles, i = b * FF_TB + tid;
+    float4 p{};
+    if (i < a.f.nt) {
+      const int j = a.f.tperm[i];
+      if (RULE == PANFAR_PARTICLES) {
+        float4 s[PAN_F4];
+        ptpan_record(a.t, j, s);
+        p = make_float4(s[3].x, s[3].y, s[3].z, plain_limit(s[4].z * 4.0f));
+      } else {
+        p = make_float4(a.p.tx[j], a.p.ty[j], a.p.tz[j], 0.0f);
+      }
+      tq[i] = p;
     }
-  if (!real) return;
-#pragma unroll
-  for (int k = 0; k < G7_F4; ++k) a.rec[G7_F4 * i + k] = s[k];
-  a.cen[i] = make_float4(s[5].y, s[5].z, s[5].w, s[7].x);
-}
-
-// targets in sorted order: points, or panels' centroids with their limit
-template <int RULE>
-__global__ __launch_bounds__(256) void k_pf_targets(PanFarArgs a, const int* perm, float4* tq) {
-  const int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x;
-  if (i >= a.f.nt) return;
-  const int j = perm[i];
-  if (RULE == PANFAR_PARTICLES) {
-    float4 s[PAN_F4];
-    ptpan_record(a.t, j, s);
-    tq[i] = make_float4(s[3].x, s[3].y, s[3].z, plain_limit(s[4].z * 4.0f));
-  } else {
-    tq[i] = make_float4(a.p.tx[j], a.p.ty[j], a.p.tz[j], 0.0f);
+    ff_group_bounds<1>(i < a.f.nt, &p, nullptr, tb, b);
+    if (tid == 0) nn[b] = 0;
+    return;
   }
+  const int64_t t = blockIdx.x, i = t * a.unit + tid;
+  const bool has = tid < a.unit, real = has && i < a.units;
+  float4 p[N] = {}, q[N] = {};
+  if (has) {
+    const int64_t j = sperm[real ? i : a.units - 1];
+    if constexpr (RULE == PANFAR_PARTICLES) {
+      p[0] = make_float4(a.t.sx[j], a.t.sy[j], a.t.sz[j], 0.0f);
+      if (real) q[0] = make_float4(a.t.ax[j], a.t.ay[j], a.t.az[j], 0.0f);
+    } else if constexpr (RULE == PANFAR_POINTS) {
+      float4 s[PAN_F4];
+      panel_record(a.p, j, s);
+      p[0] = make_float4(s[3].x, s[3].y, s[3].z, plain_limit(s[4].z * 4.0f));
+      if (real) {
+        q[0] = s[2];
+#pragma unroll
+        for (int k = 0; k < PAN_F4; ++k) a.rec[PAN_F4 * i + k] = s[k];
+        a.cen[i] = s[3];
+      }
+    } else {
+      float4 s[G7_F4];
+      g7_record(a.p, j, s);
+      const float lim = plain_limit(sqrtf(s[7].x));
+      const float pt[21] = {s[0].x, s[0].y, s[0].z, s[0].w, s[1].x, s[1].y, s[1].z, s[1].w, s[2].x, s[2].y, s[2].z,
+                            s[2].w, s[3].x, s[3].y, s[3].z, s[3].w, s[4].x, s[4].y, s[4].z, s[4].w, s[5].x};
+#pragma unroll
+      for (int k = 0; k < 7; ++k) {
+        const float w = (float)g7_weight(k);
+        p[k] = make_float4(pt[3 * k], pt[3 * k + 1], pt[3 * k + 2], lim);
+        if (real) q[k] = make_float4(w * s[6].x, w * s[6].y, w * s[6].z, w * s[6].w);
+      }
+      if (real) {
+#pragma unroll
+        for (int k = 0; k < G7_F4; ++k) a.rec[G7_F4 * i + k] = s[k];
+        a.cen[i] = make_float4(s[5].y, s[5].z, s[5].w, s[7].x);
+      }
+    }
+    const int64_t row = t * a.f.tile + N * tid;
+#pragma unroll
+    for (int k = 0; k < N; ++k) { sp[row + k] = p[k]; sa[row + k] = q[k]; }
+    if (N > 1 && tid == a.unit - 1)   // the last panel of a tile fills it up
+      for (int k = N * a.unit; k < a.f.tile; ++k) {
+        sp[t * a.f.tile + k] = p[0];
+        sa[t * a.f.tile + k] = make_float4(0.f, 0.f, 0.f, 0.f);
+      }
+  }
+  ff_group_bounds<N>(has, p, q, sb, t);
 }
 
 // block b's near tiles of rank [r0, r1), in order: next() gives -1 after the last
@@ -431,10 +429,10 @@ __global__ __launch_bounds__(BLOCK) void k_pf_near7(PanFarArgs a) {
 }
 
 struct PanFarLayout {
-  unsigned *bb, *ks_in, *ks_out, *kt_in, *kt_out, *mask, *ctr, *list, *count;
-  int *is_in, *is_out, *it_in, *it_out, *nn, *noff, *items, *ioff, *mfold, *iblk;
+  unsigned *k_in, *k_out, *mask, *ctr, *list, *count;
+  int *i_in, *i_out, *nn, *items, *ioff, *mfold, *iblk;
   void* tmp;
-  float *cx, *cy, *cz, *tcs, *tam, *tsg, *bcs;
+  float *box, *tcs, *tam, *tsg, *bcs;
   float4 *sp, *sa, *tq, *tsph, *bsph, *rec, *cen;
   double *farv, *part;
   size_t bytes;
@@ -448,7 +446,6 @@ int unit_of(int rule, int64_t units) { return rule == PANFAR_POINTS7 ? tile_of(r
 
 PanFarLayout layout(char* base, int rule, int64_t units, int64_t nt, int nout) {
   const int T = tile_of(rule, units), U = unit_of(rule, units);
-  const int64_t np = rule == PANFAR_PARTICLES ? nt : units;
   const int64_t nb = (nt + FF_TB - 1) / FF_TB;
   const int64_t ntiles = (units + U - 1) / U;
   const int64_t mwords = (ntiles + 31) / 32;
@@ -456,19 +453,12 @@ PanFarLayout layout(char* base, int rule, int64_t units, int64_t nt, int nout) {
   const int f4 = rule == PANFAR_POINTS ? PAN_F4 : rule == PANFAR_POINTS7 ? G7_F4 : 0;
   Carve cv{base};
   PanFarLayout L{};
-  L.bb = cv.take<unsigned>(8);
-  L.cx = cv.take<float>(np);
-  L.cy = cv.take<float>(np);
-  L.cz = cv.take<float>(np);
-  L.ks_in = cv.take<unsigned>(units);
-  L.ks_out = cv.take<unsigned>(units);
-  L.is_in = cv.take<int>(units);
-  L.is_out = cv.take<int>(units);
-  L.kt_in = cv.take<unsigned>(nt);
-  L.kt_out = cv.take<unsigned>(nt);
-  L.it_in = cv.take<int>(nt);
-  L.it_out = cv.take<int>(nt);
-  L.tmp = cv.take<char>(radix_tmp_bytes(std::max(units, nt)));
+  L.box = cv.take<float>(6 * FF_BOX_GRID);
+  L.k_in = cv.take<unsigned>(units + nt);
+  L.k_out = cv.take<unsigned>(units + nt);
+  L.i_in = cv.take<int>(units + nt);
+  L.i_out = cv.take<int>(units + nt);
+  L.tmp = cv.take<char>(radix_tmp_bytes(units + nt));
   L.sp = cv.take<float4>((size_t)ntiles * T);
   L.sa = cv.take<float4>((size_t)ntiles * T);
   L.rec = cv.take<float4>((size_t)f4 * units);
@@ -483,7 +473,6 @@ PanFarLayout layout(char* base, int rule, int64_t units, int64_t nt, int nout) {
   L.mask = cv.take<unsigned>((size_t)(nb * mwords));
   L.farv = cv.take<double>((size_t)nout * far_slices(nb, mwords, num_cus()) * nt);
   L.nn = cv.take<int>(nb);
-  L.noff = cv.take<int>(nb);
   L.items = cv.take<int>(nb);
   L.ioff = cv.take<int>(nb);
   L.mfold = cv.take<int>(1);
@@ -510,11 +499,7 @@ int run(const PanArgs* p, const PtPanArgs* t, void* ws, hipStream_t st) {
   constexpr bool PART = RULE == PANFAR_PARTICLES;
   PanFarArgs a{};
   if (p) a.p = *p;
-  if (t) {
-    a.t = *t;
-    a.p.nx = t->nx; a.p.ny = t->ny; a.p.nz = t->nz;
-    a.p.idx = t->idx; a.p.np = t->np;
-  }
+  if (t) a.t = *t;
   const int64_t units = PART ? t->ns : p->np, nt = PART ? t->np : p->nt;
   const int T = tile_of(RULE, units), U = unit_of(RULE, units);
   const int64_t nb = (nt + FF_TB - 1) / FF_TB;
@@ -532,48 +517,24 @@ int run(const PanArgs* p, const PtPanArgs* t, void* ws, hipStream_t st) {
   a.rec = L.rec; a.cen = L.cen; a.list = L.list; a.count = L.count; a.iblk = L.iblk;
   a.units = units; a.unit = U;
 
-  const int64_t npan = a.p.np;
-  const float* cen[3] = {L.cx, L.cy, L.cz};
-  const float* pts[3] = {PART ? t->sx : p->tx, PART ? t->sy : p->ty, PART ? t->sz : p->tz};
-  const int64_t npts = PART ? units : nt;
-  const float* const* src = PART ? pts : cen;
-  const float* const* tgt = PART ? cen : pts;
-  hipLaunchKernelGGL(k_pf_centroids, dim3(grid_of(npan, 256)), dim3(256), 0, st, a.p, L.cx, L.cy, L.cz);
-  hipLaunchKernelGGL(k_ff_bbox_init, dim3(1), dim3(64), 0, st, L.bb);
-  hipLaunchKernelGGL(k_ff_bbox, dim3(std::min(grid_of(npan, 256), FF_BBOX_GRID)), dim3(256), 0, st, cen[0], cen[1],
-                     cen[2], npan, L.bb);
-  hipLaunchKernelGGL(k_ff_bbox, dim3(std::min(grid_of(npts, 256), FF_BBOX_GRID)), dim3(256), 0, st, pts[0], pts[1],
-                     pts[2], npts, L.bb);
-  hipLaunchKernelGGL((k_ff_keys<true>), dim3(grid_of(units, 256)), dim3(256), 0, st, src[0], src[1], src[2], units, L.bb,
-                     L.ks_in, L.is_in);
-  hipLaunchKernelGGL((k_ff_keys<true>), dim3(grid_of(nt, 256)), dim3(256), 0, st, tgt[0], tgt[1], tgt[2], nt, L.bb, L.kt_in,
-                     L.it_in);
-  HIPCHK(hipGetLastError());
-  unsigned* keys = nullptr;
-  int *sperm = nullptr, *tperm = nullptr;
-  int rc = radix_sort_pairs(L.ks_in, L.is_in, L.ks_out, L.is_out, units, 30, L.tmp, st, &keys, &sperm);
+  FFSets sets{};
+  const int pan = PART ? 1 : 0, pts = 1 - pan;   // sources first
+  sets.x[pan] = PART ? t->nx : p->nx; sets.y[pan] = PART ? t->ny : p->ny; sets.z[pan] = PART ? t->nz : p->nz;
+  sets.x[pts] = PART ? t->sx : p->tx; sets.y[pts] = PART ? t->sy : p->ty; sets.z[pts] = PART ? t->sz : p->tz;
+  sets.n[0] = units; sets.n[1] = nt;
+  sets.idx = PART ? t->idx : p->idx;
+  sets.pan = pan;
+  const int* perm = nullptr;
+  const int rc = factored_order(sets, L.box, L.k_in, L.i_in, L.k_out, L.i_out, L.tmp, st, &perm);
   if (rc != O3D_OK) return rc;
-  if ((rc = radix_sort_pairs(L.kt_in, L.it_in, L.kt_out, L.it_out, nt, 30, L.tmp, st, &keys, &tperm)) != O3D_OK)
-    return rc;
-  f.tperm = tperm;
-  hipLaunchKernelGGL((k_pf_sources<RULE>), dim3(grid_of((int64_t)ntiles * U, 256)), dim3(256), 0, st, a, sperm, L.sp,
-                     L.sa);
-  hipLaunchKernelGGL((k_pf_targets<RULE>), dim3(grid_of(nt, 256)), dim3(256), 0, st, a, tperm, L.tq);
-  hipLaunchKernelGGL(k_ff_bounds, dim3((unsigned)ntiles), dim3(256), 0, st, L.sp, L.sa, f.ns, T, L.tsph, L.tcs, L.tam,
-                     L.tsg);
-  hipLaunchKernelGGL(k_ff_bounds, dim3((unsigned)nb), dim3(256), 0, st, L.tq, (const float4*)nullptr, nt, FF_TB, L.bsph,
-                     L.bcs, (float*)nullptr, (float*)nullptr);
+  f.tperm = perm + units;
+  hipLaunchKernelGGL((k_pf_rows<RULE>), dim3((unsigned)(ntiles + nb)), dim3(256), 0, st, a, perm, L.sp, L.sa, L.tq,
+                     FFBounds{L.tsph, L.tcs, L.tam, L.tsg}, FFBounds{L.bsph, L.bcs, nullptr, nullptr}, L.nn);
   hipLaunchKernelGGL((k_ff_classify<CORE_SING>), dim3(grid_of(nb * mwords, 256)), dim3(256), 0, st, L.bsph, L.bcs, nb,
-                     L.tsph, L.tcs, ntiles, mwords, L.mask);
-  hipLaunchKernelGGL(k_ff_plan_count, dim3(grid_of(nb, 256)), dim3(256), 0, st, L.mask, nb, mwords, ntiles, L.nn);
+                     L.tsph, L.tcs, ntiles, mwords, L.mask, L.nn);
+  hipLaunchKernelGGL(k_ff_plan, dim3(1), dim3(FF_PLAN_THREADS), 0, st, L.nn, nb, near_split(nb, ntiles), L.items, L.ioff,
+                     L.mfold, L.ctr, L.count);
   HIPCHK(hipGetLastError());
-  if ((rc = exclusive_scan_i32(L.nn, L.noff, nb, st)) != O3D_OK) return rc;
-  hipLaunchKernelGGL(k_ff_plan_items, dim3(grid_of(nb, 256)), dim3(256), 0, st, L.nn, L.noff, nb, near_split(nb, ntiles), L.items,
-                     L.mfold);
-  HIPCHK(hipGetLastError());
-  if ((rc = exclusive_scan_i32(L.items, L.ioff, nb, st)) != O3D_OK) return rc;
-  hipLaunchKernelGGL(k_ff_zero_u32, dim3(1), dim3(64), 0, st, L.ctr);
-  hipLaunchKernelGGL(k_ff_zero_u32, dim3(1), dim3(64), 0, st, L.count);
 
   const int nslice = far_slices(nb, mwords, num_cus());
   f.wslice = (mwords + nslice - 1) / nslice;

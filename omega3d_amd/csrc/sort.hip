@@ -1,5 +1,4 @@
-// sort.hip -- stable LSD radix sort of (key, index) pairs and an exclusive scan
-// of int32 counts, for gfx950.
+// sort.hip -- stable LSD radix sort of (key, index) pairs for gfx950.
 //
 // Used for the Morton order of particles (the factored method's sources and
 // targets, the direct EXP kernel's target order) and for the factored method's
@@ -12,6 +11,7 @@
 //                 cnt[digit][tile] (digit-major);
 //   k_rs_rowscan  one workgroup per digit: exclusive scan of its row over the
 //                 tiles, and the digit's total;
+//                 (few tiles: left out, k_rs_scatter adds the rows up itself);
 //   k_rs_scatter  per tile: the digit bases (exclusive scan of the totals) plus
 //                 the row offset, then the tile's keys in RS_I rounds of RS_T
 //                 consecutive keys.  Within a round, a key's rank among equal
@@ -35,6 +35,9 @@ constexpr int RS_TILE = RS_T * RS_I;  // keys per workgroup tile
 constexpr int RS_BITS = 8;
 constexpr int RS_B = 1 << RS_BITS;    // digits per pass (== RS_T: one digit per thread)
 constexpr int RS_W = RS_T / 64;       // waves per workgroup
+// up to here a tile adds up the counts of the tiles before it by itself: a launch less per
+// pass, about 4 us, for nblk loads in flight (131,072 keys have 32 tiles)
+constexpr int RS_FUSE = 48;
 static_assert(RS_B == RS_T, "one digit per thread");
 
 // exclusive prefix of v over the RS_T threads of the workgroup; *total gets the sum.
@@ -61,6 +64,8 @@ __device__ __forceinline__ unsigned wg_excl_scan(unsigned v, unsigned* sh, unsig
   return before + x - v;
 }
 
+// cnt[digit][tile], or (FUSED) cnt[tile][digit]
+template <bool FUSED>
 __global__ __launch_bounds__(RS_T) void k_rs_hist(const unsigned* __restrict__ key, int64_t n, int shift,
                                                   unsigned* __restrict__ cnt, int nblk) {
   __shared__ unsigned h[RS_B];
@@ -73,7 +78,7 @@ __global__ __launch_bounds__(RS_T) void k_rs_hist(const unsigned* __restrict__ k
     if (i < n) atomicAdd(&h[(key[i] >> shift) & (RS_B - 1)], 1u);
   }
   __syncthreads();
-  cnt[(int64_t)threadIdx.x * nblk + blockIdx.x] = h[threadIdx.x];
+  cnt[FUSED ? (int64_t)blockIdx.x * RS_B + threadIdx.x : (int64_t)threadIdx.x * nblk + blockIdx.x] = h[threadIdx.x];
 }
 
 // grid = RS_B workgroups, one per digit row of cnt
@@ -93,6 +98,7 @@ __global__ __launch_bounds__(RS_T) void k_rs_rowscan(unsigned* __restrict__ cnt,
   if (threadIdx.x == 0) tot[blockIdx.x] = carry;
 }
 
+template <bool FUSED>
 __global__ __launch_bounds__(RS_T) void k_rs_scatter(const unsigned* __restrict__ kin, const int* __restrict__ vin,
                                                      unsigned* __restrict__ kout, int* __restrict__ vout, int64_t n,
                                                      int shift, const unsigned* __restrict__ cnt,
@@ -113,8 +119,20 @@ __global__ __launch_bounds__(RS_T) void k_rs_scatter(const unsigned* __restrict_
     v[r] = i < n ? vin[i] : 0;
   }
   unsigned t;
-  const unsigned dbase = wg_excl_scan(tot[tid], sh, &t);
-  off[tid] = dbase + cnt[(int64_t)tid * nblk + blockIdx.x];
+  unsigned sum = 0u, before = 0u;
+  if (FUSED) {
+#pragma unroll 8
+    for (int b = 0; b < nblk; ++b) {
+      const unsigned c = cnt[b * RS_B + tid];
+      sum += c;
+      before += b < (int)blockIdx.x ? c : 0u;
+    }
+  } else {
+    sum = tot[tid];
+    before = cnt[(int64_t)tid * nblk + blockIdx.x];
+  }
+  const unsigned dbase = wg_excl_scan(sum, sh, &t);
+  off[tid] = dbase + before;
 #pragma unroll
   for (int q = 0; q < RS_W; ++q) wc[q][tid] = 0u;
   __syncthreads();
@@ -157,29 +175,6 @@ __global__ __launch_bounds__(RS_T) void k_rs_scatter(const unsigned* __restrict_
   }
 }
 
-// exclusive scan of n int32 values by one workgroup, RS_T * 4 values per step
-__global__ __launch_bounds__(RS_T) void k_scan_i32(const int* __restrict__ in, int* __restrict__ out, int64_t n) {
-  __shared__ unsigned sh[RS_W];
-  unsigned carry = 0u;
-  for (int64_t b0 = 0; b0 < n; b0 += (int64_t)RS_T * 4) {
-    const int64_t i0 = b0 + (int64_t)threadIdx.x * 4;
-    unsigned v[4], s = 0u;
-#pragma unroll
-    for (int j = 0; j < 4; ++j) {
-      v[j] = i0 + j < n ? (unsigned)in[i0 + j] : 0u;
-      s += v[j];
-    }
-    unsigned t;
-    unsigned ex = carry + wg_excl_scan(s, sh, &t);
-#pragma unroll
-    for (int j = 0; j < 4; ++j) {
-      if (i0 + j < n) out[i0 + j] = (int)ex;
-      ex += v[j];
-    }
-    carry += t;
-  }
-}
-
 int blocks_of(int64_t n) { return (int)std::max<int64_t>(1, (n + RS_TILE - 1) / RS_TILE); }
 
 }  // namespace
@@ -201,9 +196,16 @@ int radix_sort_pairs(unsigned* ka, int* va, unsigned* kb, int* vb, int64_t n, in
     unsigned* cnt = static_cast<unsigned*>(tmp);
     unsigned* tot = cnt + (size_t)RS_B * nblk;
     for (int shift = 0; shift < bits; shift += RS_BITS) {
-      hipLaunchKernelGGL(k_rs_hist, dim3(nblk), dim3(RS_T), 0, st, kin, n, shift, cnt, nblk);
-      hipLaunchKernelGGL(k_rs_rowscan, dim3(RS_B), dim3(RS_T), 0, st, cnt, nblk, tot);
-      hipLaunchKernelGGL(k_rs_scatter, dim3(nblk), dim3(RS_T), 0, st, kin, vin, kout, vout, n, shift, cnt, tot, nblk);
+      if (nblk <= RS_FUSE) {
+        hipLaunchKernelGGL((k_rs_hist<true>), dim3(nblk), dim3(RS_T), 0, st, kin, n, shift, cnt, nblk);
+        hipLaunchKernelGGL((k_rs_scatter<true>), dim3(nblk), dim3(RS_T), 0, st, kin, vin, kout, vout, n, shift, cnt, tot,
+                           nblk);
+      } else {
+        hipLaunchKernelGGL((k_rs_hist<false>), dim3(nblk), dim3(RS_T), 0, st, kin, n, shift, cnt, nblk);
+        hipLaunchKernelGGL(k_rs_rowscan, dim3(RS_B), dim3(RS_T), 0, st, cnt, nblk, tot);
+        hipLaunchKernelGGL((k_rs_scatter<false>), dim3(nblk), dim3(RS_T), 0, st, kin, vin, kout, vout, n, shift, cnt, tot,
+                           nblk);
+      }
       HIPCHK(hipGetLastError());
       std::swap(kin, kout);
       std::swap(vin, vout);
@@ -211,13 +213,6 @@ int radix_sort_pairs(unsigned* ka, int* va, unsigned* kb, int* vb, int64_t n, in
   }
   *keys = kin;
   *vals = vin;
-  return O3D_OK;
-}
-
-int exclusive_scan_i32(const int* in, int* out, int64_t n, hipStream_t st) {
-  if (n <= 0) return O3D_OK;
-  hipLaunchKernelGGL(k_scan_i32, dim3(1), dim3(RS_T), 0, st, in, out, n);
-  HIPCHK(hipGetLastError());
   return O3D_OK;
 }
 
