@@ -64,10 +64,12 @@ enum o3d_self { O3D_SELF_INCLUDE = 0, O3D_SELF_EXCLUDE = 1 };
  *             weights with a 29-column per-source moment table on the matrix
  *             cores; other pairs as in DIRECT.  RM and EXP cores, velocity and
  *             gradient, FP32 or compensated precision; tile 64, 128 or 256.
- *   AUTO:     FACTORED where it applies and both counts are >= 65536 with tile
- *             and tpt left at 0, DIRECT otherwise.  In compensated precision AUTO
- *             takes the far tiles of the other cores (WL, V2) and of velocities
- *             alone to the matrix cores as well, at the same counts.
+ *   AUTO:     FACTORED where it applies with tile and tpt left at 0 and enough pairs
+ *             (both counts >= 8192 and, with gradient, about 24,500 particles on
+ *             themselves for EXP and 30,000 for RM), DIRECT otherwise.  In compensated
+ *             precision AUTO takes the far tiles of the other cores (WL, V2: about
+ *             45,000) and of velocities alone (EXP 32,000, RM 47,000, WL and V2 55,000)
+ *             to the matrix cores as well.
  * For panel sources (o3d_panels_affect_points[_dev]) the field selects the rule:
  *   AUTO / DIRECT:      the reference's recursive centroid rule (Kernels.h:1028-1211);
  *             AUTO takes the separated pairs of large calls with tile 0, of both rules
@@ -368,8 +370,9 @@ typedef struct o3d_batch o3d_batch;
 
 /* cores / precs / self_terms: per-instance arrays (NULL = the opts value for all).
  * opts->tile / opts->tpt: 0 = defaults (see o3d_batch_tune).
- * opts->method: AUTO sends every instance of >= 32,768 particles with an RM or EXP
- * core in FP32 or compensated precision to the factored far-field method; FACTORED
+ * opts->method: AUTO sends every instance of >= 32,768 particles with the RM core and of
+ * >= 12,288 with the EXP core, in FP32 or compensated precision, and of >= 32,768 with the
+ * WL or V2 core in compensated precision to the factored far-field method; FACTORED
  * sends all instances there (an instance it cannot take is an error); DIRECT keeps
  * all in the persistent queue.  Factored instances run on up to 8 streams the
  * batch creates here, each with scratch allocated here; they fork from the
@@ -435,7 +438,7 @@ typedef struct o3d_server_opts {
   int32_t adaptive_tick;      /* raise the budget to (workgroup slots x the largest
                                  active chunk) so that large sessions fill the GPU      */
   int32_t method;             /* enum o3d_method.  AUTO (0): a step of a session of
-                                 >= 32,768 particles with the RM or EXP core evaluates
+                                 >= 12,288 particles with the RM or EXP core evaluates
                                  both stages by the factored far-field method on a
                                  second stream, overlapping the ticks; FACTORED: every
                                  RM/EXP session; DIRECT: ticks only.  The factored

@@ -7,9 +7,8 @@
 // item runs the same p2p_chunk as the single-collection kernel, so a target's
 // sums do not depend on the launch that computed it.
 //
-// Instances large enough for the factored far field (method AUTO: 32,768 particles
-// and more, where a single call takes it from 65,536; or all of them with method
-// FACTORED) leave the queue and
+// Instances large enough for the factored far field (method AUTO: batch_takes_factored;
+// or all of them with method FACTORED) leave the queue and
 // run that pipeline on FF_LANES (8) streams of the batch (longest first, each to the
 // least-loaded lane), each lane with scratch of its own.  The lanes fork from the
 // caller's stream after the zero fill and join it at the end, so they overlap
@@ -208,7 +207,7 @@ o3d_opts factored_opts(const BatchInst& I) {
   o.results = O3D_VELANDGRAD;
   o.precision = I.prec;
   o.self_term = I.self_excl;
-  o.method = O3D_METHOD_FACTORED;
+  o.method = O3D_METHOD_AUTO;   // taken already (FACTORED would refuse WL and V2)
   return o;
 }
 
@@ -365,8 +364,9 @@ int o3d_batch_create(o3d_batch** out, int32_t ninst, const int64_t* off, const i
   for (int i : order) {
     const BatchInst& I = b->inst[i];
     const bool ffok = ff_supported(I.core, true, I.prec) && I.n <= INT32_MAX;
-    if (I.n > 0 && ffok &&
-        (opts->method == O3D_METHOD_FACTORED || (opts->method == O3D_METHOD_AUTO && I.n >= LANES_FF_AUTO_MIN_N))) {
+    if (I.n > 0 &&
+        (opts->method == O3D_METHOD_FACTORED ? ffok
+                                             : opts->method == O3D_METHOD_AUTO && batch_takes_factored(I.core, I.prec, I.n))) {
       factored[i] = 1;
       b->ff.push_back(i);
     }

@@ -347,8 +347,22 @@ bool ff_supported(int core, bool grad, int prec) {
   return (core == CORE_RM || core == CORE_EXP) && grad && (prec == PREC_FP32 || prec == PREC_COMP);
 }
 
-// what AUTO may send here besides
-bool ff_auto_supported(int core, bool grad, int prec) { return prec == PREC_COMP || ff_supported(core, grad, prec); }
+// AUTO also sends compensated sums of the other cores and of velocities alone.  The line is
+// drawn in pairs, where both methods' times cross, us direct and factored on one or two
+// rings: EXP 24,576 particles 600-630 and 505; RM 24,576 452 and 468, 32,768 750 and 570-645;
+// WL (V2 alike) 32,768 829 and 798-869, 49,152 1,833 and 1,573-1,641; velocity alone: EXP
+// 24,576 376-396 and 410-420, 32,768 675 and 493-562, RM 32,768 441 and 456-504, 49,152 980
+// and 830-884, WL 49,152 1,105 and 1,063-1,125, 65,536 faster.  100,000 particles on 16,384
+// field points and 8,192 on 262,144 fall on the same lines (less the preparation's recent
+// 0.07 ms: RM 1,134 and 1,064, 1,416 and 1,235; WL 1,235 and 1,402, 1,561 and 1,667), 2,048
+// on 262,144 not (EXP 631 and 645), nor do fewer targets.
+bool ff_auto_pays(int core, bool grad, int prec, int64_t ns, int64_t nt) {
+  if (!(prec == PREC_COMP || ff_supported(core, grad, prec))) return false;
+  if (ns < 8192 || nt < 8192 || ns > INT_MAX || nt > INT_MAX) return false;
+  const double least = core == CORE_EXP ? (grad ? 6.0e8 : 1.0e9) : core == CORE_RM ? (grad ? 9.0e8 : 2.2e9)
+                                                                                 : (grad ? 2.0e9 : 3.0e9);
+  return (double)ns * (double)nt >= least && ns + nt <= INT_MAX;
+}
 
 namespace {
 int check_factored(const o3d_points* src, const o3d_points* targ, const o3d_opts* o, int* T) {

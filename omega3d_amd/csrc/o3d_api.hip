@@ -262,8 +262,8 @@ int p2p_dev(const o3d_points* src, o3d_points* targ, const o3d_opts* o, hipStrea
   if (src->n == 0 || targ->n == 0) return O3D_OK;
   if (o->precision == PREC_FP64) return fail(O3D_EINVAL, "internal: FP64 routed to p2p_dev");
   if (o->method == O3D_METHOD_FACTORED) return p2p_factored(src, targ, o, st);
-  if (o->method == O3D_METHOD_AUTO && !tun && o->tile == 0 && o->tpt == 0 && ff_auto_supported(o->core, grad, o->precision) &&
-      src->n >= FF_AUTO_MIN_N && targ->n >= FF_AUTO_MIN_N && src->n <= INT32_MAX && targ->n <= INT32_MAX) {
+  if (o->method == O3D_METHOD_AUTO && !tun && o->tile == 0 && o->tpt == 0 && 
+      ff_auto_pays(o->core, grad, o->precision, src->n, targ->n)) {
     // under graph capture the stream's workspace cannot grow: when it is too small
     // for the factored method, the direct kernel (which needs none) takes the call
     bool ff = true;

@@ -32,7 +32,6 @@ int check_node_indices(const o3d_panels* p, const char* what);
 void fill_stats(o3d_stats* stats, double secs, double flops, double inter);
 // method FACTORED serves it; method AUTO may take the factored path for it
 bool ff_supported(int core, bool grad, int prec);
-bool ff_auto_supported(int core, bool grad, int prec);
 int p2p_factored(const o3d_points* src, o3d_points* targ, const o3d_opts* o, hipStream_t st,
                  o3d_factored_profile* prof = nullptr);
 int p2p_factored_ws(const o3d_points* src, o3d_points* targ, const o3d_opts* o, hipStream_t st, void* ws,
@@ -67,15 +66,26 @@ int point_order(const float* x, const float* y, const float* z, int64_t n, void*
 size_t radix_tmp_bytes(int64_t n);
 int radix_sort_pairs(unsigned* ka, int* va, unsigned* kb, int* vb, int64_t n, int bits, void* tmp, hipStream_t st,
                      unsigned** keys, int** vals);
-// a collection large enough for the factored method to pay when the caller leaves the choice open
-constexpr int64_t FF_AUTO_MIN_N = 65536;
-// the same for an instance of a batch or a session of the server: their factored work runs on
-// streams of its own while the persistent kernel sums the rest, so the split point that balances
-// the two is lower.  256 RM rings of 2,048-262,144 particles, compensated, graph replay: 682-685 ms
-// at 65,536, 667-668 at 49,152, 665-666 at 40,960, 662-664 at 32,768, 741 at 98,304.  16 served
-// sessions of 1,986-296,912 particles: at 32,768 against 65,536 saturated 2,881-2,905 against
-// 2,853-2,856 G interactions/s, Poisson p50 7.8 against 10.6-11.0 ms, p99 78.5 against 80.3 ms
-constexpr int64_t LANES_FF_AUTO_MIN_N = 32768;
+// whether a call is large enough for the factored method to pay when the caller leaves the
+// choice open (and it can take the call at all)
+bool ff_auto_pays(int core, bool grad, int prec, int64_t ns, int64_t nt);
+// Whether an instance of a batch (AUTO) takes it.  Their factored work runs on
+// streams of its own while the persistent kernel sums the rest, so the line that balances
+// the two is lower.  256 RM rings of 2,048-262,144 particles, compensated, graph replay: 645 ms
+// from 32,768 particles on and 640 from 18,432 or 12,288; 48 of 2,048-81,920 18.3, 17.6 and
+// 17.8 ms; 24 EXP rings of 2,048-60,000 8.5 ms from 32,768, 7.2 from 18,432, 6.4 from 12,288,
+// 6.3 from 8,192; 24 WL rings of 8,192-98,000 34.3 ms in the queue, 24.3 from 32,768,
+// 24.4 from 24,576.  RM keeps its documented line.
+inline bool batch_takes_factored(int core, int prec, int64_t n) {
+  if (n > INT32_MAX || !(prec == PREC_COMP || ((core == CORE_RM || core == CORE_EXP) && prec == PREC_FP32))) return false;
+  return n >= (core == CORE_EXP ? 12288 : 32768);
+}
+// a session of the server (AUTO, RM or EXP) from here on: 8 sessions of 1,024-100,000
+// particles stepped together 18.9 ms from 32,768, 17.2 from 24,576, 12.2 from 12,288, 12.9 from
+// 8,192; 12 of 4,096-24,000 12.6, 12.4, 10.1 and 9.1; 16 served sessions of 1,986-296,912
+// particles, Poisson p50 5.2 ms from 32,768 and 4.9 from 12,288, saturated 3,098 and 3,119 G
+// interactions/s
+constexpr int64_t SERVER_FF_AUTO_MIN_N = 12288;
 // direct EXP calls with at least this many targets visit them in Morton order
 constexpr int64_t TARGET_ORDER_MIN_N = 32768;
 int p2p_dev(const o3d_points* src, o3d_points* targ, const o3d_opts* o, hipStream_t st, const Tuning* tun);

@@ -510,7 +510,7 @@ void finish_request(o3d_server* S, Request& r, int state, int status, double whe
 bool session_factored(const o3d_server* S, const Session& ses) {
   if (ses.core != CORE_RM && ses.core != CORE_EXP) return false;
   if (S->opts.method == O3D_METHOD_FACTORED) return true;
-  return S->opts.method == O3D_METHOD_AUTO && ses.n >= LANES_FF_AUTO_MIN_N;
+  return S->opts.method == O3D_METHOD_AUTO && ses.n >= SERVER_FF_AUTO_MIN_N;
 }
 
 // admit queued requests (arrival order; a request of a session with an admitted

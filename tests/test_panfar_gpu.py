@@ -240,3 +240,43 @@ def test_deep_trees(mods, maxlev, tile):
     for rows in (slice(0, 3), slice(3, 12)):
         bar = max(2e-6, 3 * rel_errors(o32[rows], o64[rows])[0])
         assert rel_errors(v[rows][:, k], o64[rows])[0] <= bar
+
+
+@pytest.mark.parametrize("core,n", [("wl", 32768), ("v2", 33001), ("exp", 12288)])
+def test_batch_takes_other_cores_factored(mods, core, n):
+    """instances from the line on leave the queue, one below it stays; both within the
+    compensated bar of the FP64 sums on some targets"""
+    torch, _lib, influence = mods
+    from omega3d_amd import batch
+    inst = [scenes.ring(n, seed=21), scenes.ring(n - 1 if n != 33001 else 32767, seed=22), scenes.ring(300, seed=23)]
+    b = batch.Batch(inst, core=core, precision="comp")
+    try:
+        assert b.config()["factored_instances"] == 1
+        b.run()
+        for (v, g), p in zip(b.results(), inst):
+            k = np.arange(0, p.n, max(1, p.n // 300))
+            ov, og = oracle.p2p(core, p.pos, p.str, p.rad, p.pos[:, k], p.rad[k], True, "f64")
+            assert rel_errors(v[:, k], ov)[0] <= 1e-6 and rel_errors(g[:, k], og)[0] <= 1e-6
+    finally:
+        b.close()
+
+
+@pytest.mark.parametrize("core,grads,ns,nt", [("exp", True, 24495, 24495), ("exp", True, 8192, 73300), ("rm", True, 30001, 30001),
+                                              ("exp", False, 31700, 31700), ("rm", True, 110000, 8192)])
+def test_auto_line(mods, core, grads, ns, nt):
+    """calls just beyond AUTO's line between the methods: not the direct bits, within the
+    compensated bar of FP64; and just before it the direct bits"""
+    torch, _lib, influence = mods
+    p = scenes.ring(ns, seed=31)
+    t = (p.pos, p.rad) if nt == ns else ((3 * np.random.default_rng(2).random((3, nt)) - 1.5).astype(np.float32), None)
+    call = lambda m: influence.p2p(core, p.pos, p.str, p.rad, t[0], t[1], grads, "comp", method=m)
+    v, g = call("auto")
+    w, h = call("direct")
+    assert not np.array_equal(v, w)
+    k = np.arange(0, nt, nt // 300)
+    ov, og = oracle.p2p(core, p.pos, p.str, p.rad, t[0][:, k], None if t[1] is None else t[1][k], grads, "f64")
+    assert rel_errors(v[:, k], ov)[0] <= 1e-6 and (not grads or rel_errors(g[:, k], og)[0] <= 1e-6)
+    m = 8191
+    a = influence.p2p(core, p.pos[:, :m], p.str[:, :m], p.rad[:m], t[0], t[1], grads, "comp")
+    b = influence.p2p(core, p.pos[:, :m], p.str[:, :m], p.rad[:m], t[0], t[1], grads, "comp", method="direct")
+    assert np.array_equal(a[0], b[0]) and (not grads or np.array_equal(a[1], b[1]))
