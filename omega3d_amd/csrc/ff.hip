@@ -86,7 +86,7 @@ Layout layout(char* base, int64_t ns, int64_t nt, bool same, int T, size_t tmp_b
   L.bsph = cv.take<float4>(nb);
   L.bcs = cv.take<float>(nb);
   L.mask = cv.take<unsigned>((size_t)(nb * mwords));
-  L.farv = cv.take<double>((size_t)nout * far_slices(nb, mwords, num_cus()) * nt);
+  L.farv = cv.take<double>((size_t)nout * far_slices(nb, ntiles, nout == 3 ? 3 : 2, num_cus()) * nt);
   L.npair = cv.take<unsigned long long>(1);
   L.nn = cv.take<int>(nb);
   L.items = cv.take<int>(nb);
@@ -159,9 +159,9 @@ int run(const o3d_points* src, o3d_points* targ, bool self_excl, int T, hipStrea
   a.ns = ns; a.nt = nt;
   a.tile = T; a.mwords = mwords; a.ntiles = ntiles;
   a.self_excl = self_excl ? 1 : 0;
-  const int nslice = far_slices(nb, mwords, num_cus());
-  a.wslice = (mwords + nslice - 1) / nslice;
-  a.nslice = (mwords + a.wslice - 1) / a.wslice;
+  const int nslice = far_slices(nb, ntiles, GRAD ? 2 : 3, num_cus());
+  a.tslice = (ntiles + nslice - 1) / nslice;
+  a.nslice = (ntiles + a.tslice - 1) / a.tslice;
   const size_t lds_far = ff_far_lds<CORE, GRAD>();
   if (prof) HIPCHK(hipEventRecord(ev[1].e, st));
   hipLaunchKernelGGL((k_ff_far<CORE, GRAD>), dim3((unsigned)nb, (unsigned)a.nslice), dim3(FF_FAR_THREADS), lds_far, st, a);

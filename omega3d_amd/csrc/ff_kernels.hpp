@@ -108,8 +108,8 @@ struct FFArgs {
   const unsigned* mask;  // far bit per (block, tile), mwords words per block
   double* farv;        // per slice: 12 x nt (3 x nt), sorted target order: far-field velocity and gradient
   const float* tsg;    // per source tile: sign of its first nonzero strength, 0: none
-  int32_t nslice;      // slices of the far field: slice y takes mask words [y * wslice, (y + 1) * wslice)
-  int32_t wslice;
+  int32_t nslice;      // slices of the far field: slice y takes tiles [y * tslice, (y + 1) * tslice)
+  int32_t tslice;
   const int* nn;       // near tiles per block
   const int* items;    // near-field work items per block
   const int* ioff;     // exclusive scan of items
@@ -804,7 +804,7 @@ __global__ __launch_bounds__(FF_FAR_THREADS, 2) void k_ff_far(FFArgs a) {
 
   const unsigned* mrow = a.mask + blk * a.mwords;
   int jw = 0, eg[NG];
-  bf16x8 tb[2][2];
+  bf16x8 tb[2][2] = {};
   float tts[2] = {0.0f, 0.0f};
   // fold: one v_permlane32_swap per register exchanges the upper 32 lanes of acc[0][r]
   // with the lower 32 of acc[1][r], after which every lane holds its own target's rows
@@ -926,14 +926,17 @@ __global__ __launch_bounds__(FF_FAR_THREADS, 2) void k_ff_far(FFArgs a) {
   // l works out the scales that tile l of the word wants: the largest weight and moment
   // of each group below 2^13 (2^11 where a core adds up to 3.5 times), the logarithms'
   // error being far below the margin.
-  int word = (int)blockIdx.y * a.wslice - 1;
-  const int words = word + 1 + a.wslice < a.mwords ? word + 1 + a.wslice : a.mwords;
+  const int first_tile = (int)blockIdx.y * a.tslice;
+  const int end_tile = first_tile + a.tslice < a.ntiles ? first_tile + a.tslice : a.ntiles;
+  int word = (first_tile >> 5) - 1;
   unsigned bits = 0u;
   int pk0 = 0, pk1 = 0;   // lane l: jw and eg[0..1], eg[2..4] wanted by tile l of the word
   auto next_tile = [&]() {
     while (bits == 0u) {
-      if (++word >= words) return -1;
+      if (32 * ++word >= end_tile) return -1;
       bits = __builtin_amdgcn_readfirstlane(mrow[word]);
+      if (32 * word < first_tile) bits &= ~0u << (first_tile & 31);
+      if (32 * word + 32 > end_tile) bits &= (1u << (end_tile & 31)) - 1u;
       if (bits == 0u) continue;
       const int t = word * 32 + col < a.ntiles ? word * 32 + col : a.ntiles - 1;
       const float4 ct = a.tsph[t];
@@ -978,15 +981,19 @@ __global__ __launch_bounds__(FF_FAR_THREADS, 2) void k_ff_far(FFArgs a) {
       ff_load_lds16(a.sa + g, raw + 256 + w * 64);
     }
   };
+  bool slots = false;   // tb holds slots about the block's centre, scaled by jw
   int ti = next_tile();
   if (ti >= 0) fetch(ti);
   while (ti >= 0) {
-    // a run: consecutive tiles summed under the scales of the first
-    jw = wj;
+    // a run: consecutive tiles summed under the scales of the first, its scale of r2 and its
+    // centre, and with them the targets' slots, those of the run before where they serve
     const bool own = wown;
-    {
+    const bool keep = slots && !own && (unsigned)(jw - wj + 1) <= 2u;
+    slots = !own;
+    if (!keep) {
       const float4 c = own ? a.tsph[ti] : cb;
       cx = c.x; cy = c.y; cz = c.z;
+      jw = wj;
     }
 #pragma unroll
     for (int g = 0; g < NG; ++g) eg[g] = wg[g];
@@ -994,7 +1001,7 @@ __global__ __launch_bounds__(FF_FAR_THREADS, 2) void k_ff_far(FFArgs a) {
     float gs[NG];
 #pragma unroll
     for (int g = 0; g < NG; ++g) gs[g] = ldexpf(sgn, eg[g]);
-    {
+    if (!keep) {
       // this lane's target slots for both sets and both r2 products (K slots 8 half + e
       // and 16 + 8 half + e)
 #pragma unroll
@@ -1423,12 +1430,16 @@ inline int near_split(int64_t nb, int64_t ntiles) {
                                                      ntiles));
 }
 
-// Slices of the far field: blocks x slices workgroups, at least about four rounds of the
-// two that a CU holds, so that the last round is short beside the whole and few blocks
-// (a collection of 65,536: 256) still fill every slot.
-inline int far_slices(int64_t nb, int64_t mwords, int cus) {
-  const int64_t want = (8 * (int64_t)cus + nb - 1) / nb;
-  return (int)std::max<int64_t>(1, std::min<int64_t>({want, mwords, 32}));
+// Slices of the far field: blocks x slices workgroups, at least about eight rounds of those
+// that a CU holds (three of the velocity form, two else), so that the last round is short
+// beside the whole, of eight tiles or more each.  With four rounds of two, in words of 32
+// tiles, 65,537 points and 391 tiles made 1,799 workgroups, 2.3 rounds; us then, and with
+// 4, 8 and 16 rounds: 1,877 and 1,803, 1,758, 1,745; 524,288 particles on 20,480 panels 3,917
+// and 3,646, 3,596, 3,594; WL 131,071 9,209 and 9,199, 8,960, 9,077; RM 65,536 1,611 and
+// 1,609, 1,583, 1,583
+inline int far_slices(int64_t nb, int64_t ntiles, int per_cu, int cus) {
+  const int64_t want = (8 * (int64_t)per_cu * cus + nb - 1) / nb;
+  return (int)std::max<int64_t>(1, std::min<int64_t>({want, ntiles / 8, 64}));
 }
 
 // (ff.hip) the order of one or two sets along the curve, in the caller's scratch: *perm gets

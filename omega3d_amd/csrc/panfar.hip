@@ -471,7 +471,7 @@ PanFarLayout layout(char* base, int rule, int64_t units, int64_t nt, int nout) {
   L.bsph = cv.take<float4>(nb);
   L.bcs = cv.take<float>(nb);
   L.mask = cv.take<unsigned>((size_t)(nb * mwords));
-  L.farv = cv.take<double>((size_t)nout * far_slices(nb, mwords, num_cus()) * nt);
+  L.farv = cv.take<double>((size_t)nout * far_slices(nb, ntiles, nout == 3 ? 3 : 2, num_cus()) * nt);
   L.nn = cv.take<int>(nb);
   L.items = cv.take<int>(nb);
   L.ioff = cv.take<int>(nb);
@@ -536,9 +536,9 @@ int run(const PanArgs* p, const PtPanArgs* t, void* ws, hipStream_t st) {
                      L.mfold, L.ctr, L.count);
   HIPCHK(hipGetLastError());
 
-  const int nslice = far_slices(nb, mwords, num_cus());
-  f.wslice = (mwords + nslice - 1) / nslice;
-  f.nslice = (mwords + f.wslice - 1) / f.wslice;
+  const int nslice = far_slices(nb, ntiles, GRAD ? 2 : 3, num_cus());
+  f.tslice = (ntiles + nslice - 1) / nslice;
+  f.nslice = (ntiles + f.tslice - 1) / f.tslice;
   hipLaunchKernelGGL((k_ff_far<CORE_SING, GRAD, SHEET>), dim3((unsigned)nb, (unsigned)f.nslice), dim3(FF_FAR_THREADS),
                      (ff_far_lds<CORE_SING, GRAD, SHEET>()), st, f);
   HIPCHK(hipGetLastError());
