@@ -54,7 +54,7 @@ size_t lib_tmp_bytes(int64_t ns, int64_t nt, bool same) { return radix_tmp_bytes
 // the workspace's sub-arrays in order; with base == nullptr only .bytes is meaningful
 struct Layout {
   unsigned *k_in, *k_out, *mask, *ctr;
-  int *i_in, *i_out, *nn, *items, *ioff, *mfold;
+  int *i_in, *i_out, *tinv, *nn, *items, *ioff, *mfold;
   void* tmp;
   float4 *sp, *sa, *tq, *tsph, *bsph;
   float *box, *tcs, *tam, *tsg, *bcs;
@@ -75,6 +75,7 @@ Layout layout(char* base, int64_t ns, int64_t nt, bool same, int T, size_t tmp_b
   L.k_out = cv.take<unsigned>(n);
   L.i_in = cv.take<int>(n);
   L.i_out = cv.take<int>(n);
+  L.tinv = cv.take<int>(nt);
   L.tmp = cv.take<char>(tmp_bytes);
   L.sp = cv.take<float4>((size_t)ntiles * T);
   L.sa = cv.take<float4>((size_t)ntiles * T);
@@ -143,7 +144,7 @@ int run(const o3d_points* src, o3d_points* targ, bool self_excl, int T, hipStrea
   const int *sperm = perm, *tperm = same ? perm : perm + ns;
   hipLaunchKernelGGL((k_ff_rows<CORE, THICK>), dim3((unsigned)(ntiles + nb)), dim3(256), 0, st, sv, tv, sperm, tperm, ns,
                      nt, T, ntiles, L.sp, L.sa, L.tq, FFBounds{L.tsph, L.tcs, L.tam, L.tsg},
-                     FFBounds{L.bsph, L.bcs, nullptr, nullptr}, L.nn);
+                     FFBounds{L.bsph, L.bcs, nullptr, nullptr}, L.nn, nt >= FF_ROWS_MIN ? L.tinv : nullptr);
   hipLaunchKernelGGL((k_ff_classify<CORE>), dim3(grid_of(nb * mwords, 256)), dim3(256), 0, st, L.bsph, L.bcs, nb, L.tsph,
                      L.tcs, ntiles, mwords, L.mask, L.nn);
   hipLaunchKernelGGL(k_ff_plan, dim3(1), dim3(FF_PLAN_THREADS), 0, st, L.nn, nb, near_split(nb, ntiles), L.items, L.ioff,
@@ -151,7 +152,7 @@ int run(const o3d_points* src, o3d_points* targ, bool self_excl, int T, hipStrea
   HIPCHK(hipGetLastError());
 
   FFArgs a{};
-  a.sp = L.sp; a.sa = L.sa; a.tq = L.tq; a.tperm = tperm;
+  a.sp = L.sp; a.sa = L.sa; a.tq = L.tq; a.tperm = tperm; a.tinv = L.tinv; a.rows = nt >= FF_ROWS_MIN;
   a.tsph = L.tsph; a.tcs = L.tcs; a.tam = L.tam; a.bsph = L.bsph; a.bcs = L.bcs;
   a.mask = L.mask; a.farv = L.farv; a.tsg = L.tsg;
   a.nn = L.nn; a.items = L.items; a.ioff = L.ioff; a.mfold = L.mfold; a.ctr = L.ctr; a.part = L.part;
@@ -171,7 +172,8 @@ int run(const o3d_points* src, o3d_points* targ, bool self_excl, int T, hipStrea
   const unsigned gnear = (unsigned)std::min<int64_t>((near_split(nb, ntiles) + 1) * nb, near_grid<CORE, GRAD, PREC>(lds_near));
   hipLaunchKernelGGL((k_ff_near<CORE, GRAD, PREC>), dim3(gnear), dim3(FF_TB), lds_near, st, a);
   HIPCHK(hipGetLastError());
-  hipLaunchKernelGGL((k_ff_combine<CORE, GRAD>), dim3((unsigned)nb), dim3(FF_TB), 0, st, a);
+  if (a.rows) hipLaunchKernelGGL((k_ff_combine<CORE, GRAD, true>), dim3((unsigned)nb), dim3(FF_TB), 0, st, a);
+  else hipLaunchKernelGGL((k_ff_combine<CORE, GRAD, false>), dim3((unsigned)nb), dim3(FF_TB), 0, st, a);
   HIPCHK(hipGetLastError());
   if (prof) {
     HIPCHK(hipEventRecord(ev[3].e, st));

@@ -106,7 +106,8 @@ struct FFArgs {
   const float4* bsph;  // per target block: bounding sphere
   const float* bcs;    // per target block: largest core term
   const unsigned* mask;  // far bit per (block, tile), mwords words per block
-  double* farv;        // per slice: 12 x nt (3 x nt), sorted target order: far-field velocity and gradient
+  double* farv;        // per slice and target, sorted: far-field velocity and gradient, 12 (3) (FFSum)
+  const int* tinv;     // original target -> sorted target
   const float* tsg;    // per source tile: sign of its first nonzero strength, 0: none
   int32_t nslice;      // slices of the far field: slice y takes tiles [y * tslice, (y + 1) * tslice)
   int32_t tslice;
@@ -115,7 +116,8 @@ struct FFArgs {
   const int* ioff;     // exclusive scan of items
   const int* mfold;    // near tiles per item
   unsigned* ctr;       // work-queue counter
-  double* part;        // per item: 12 x 256 partial sums
+  double* part;        // per item and target of the block: 12 (3) partial sums (FFSum)
+  int32_t rows;        // a target's sums lie in a row
   SrcView s;           // original sources (self-pair exclusion)
   TgtView t;           // original targets (outputs, accumulated)
   int64_t ns, nt;
@@ -124,6 +126,33 @@ struct FFArgs {
   int32_t ntiles;
   int32_t self_excl;
 };
+
+// NOUT sums of one target: in a row, or each a whole array of n targets apart.  k_ff_combine
+// gathers rows and reads and writes the 12 output arrays in order; from arrays it scatters a
+// float of each to a line of its own, which costs where the outputs do not stay in the
+// caches: 524,288 targets 206 us, the call 4.82 ms, with rows 4.68; 262,144 alike, 65,536
+// with 16 slices 1.66 and 1.69
+constexpr int64_t FF_ROWS_MIN = 393216;
+template <int NOUT>
+__device__ __forceinline__ void ff_sum_store(double* base, int64_t n, int64_t i, bool rows, const double* v) {
+  if (rows) {
+#pragma unroll
+    for (int k = 0; k < NOUT; ++k) base[i * NOUT + k] = v[k];
+  } else {
+#pragma unroll
+    for (int k = 0; k < NOUT; ++k) base[k * n + i] = v[k];
+  }
+}
+template <int NOUT>
+__device__ __forceinline__ void ff_sum_add(const double* base, int64_t n, int64_t i, bool rows, double* v) {
+  if (rows) {
+#pragma unroll
+    for (int k = 0; k < NOUT; ++k) v[k] += base[i * NOUT + k];
+  } else {
+#pragma unroll
+    for (int k = 0; k < NOUT; ++k) v[k] += base[k * n + i];
+  }
+}
 
 // ---- order-preserving float <-> uint (for atomic min / max of floats) ---------
 __device__ __forceinline__ unsigned fenc(float f) {
@@ -431,7 +460,7 @@ __device__ __forceinline__ void ff_group_bounds(bool valid, const float4* p, con
 template <int CORE, bool THICK>
 __global__ __launch_bounds__(256) void k_ff_rows(SrcView s, TgtView t, const int* sperm, const int* tperm, int64_t ns,
                                                  int64_t nt, int tile, int ntiles, float4* sp, float4* sa, float4* tq,
-                                                 FFBounds sb, FFBounds tb, int* nn) {
+                                                 FFBounds sb, FFBounds tb, int* nn, int* tinv) {
   const int tid = threadIdx.x;
   if ((int)blockIdx.x < ntiles) {
     const int64_t i = (int64_t)blockIdx.x * tile + tid;
@@ -451,6 +480,7 @@ __global__ __launch_bounds__(256) void k_ff_rows(SrcView s, TgtView t, const int
       const int j = tperm[i];
       p = make_float4(t.x[j], t.y[j], t.z[j], THICK ? core_term<CORE>(t.r[j]) : 0.0f);
       tq[i] = p;
+      if (tinv) tinv[j] = (int)i;
     }
     ff_group_bounds<1>(i < nt, &p, nullptr, tb, b);
     if (tid == 0) nn[b] = 0;
@@ -800,7 +830,6 @@ __global__ __launch_bounds__(FF_FAR_THREADS, 2) void k_ff_far(FFArgs a) {
 #pragma unroll
   for (int k = 0; k < NOUT; ++k) sum[k] = 0.0;
   const int64_t own = base + lane;
-  double* dst = a.farv + (int64_t)blockIdx.y * NOUT * a.nt + own;
 
   const unsigned* mrow = a.mask + blk * a.mwords;
   int jw = 0, eg[NG];
@@ -1159,10 +1188,7 @@ __global__ __launch_bounds__(FF_FAR_THREADS, 2) void k_ff_far(FFArgs a) {
     moments(1, 1);
     fold();
   }
-  if (own < a.nt) {
-#pragma unroll
-    for (int k = 0; k < NOUT; ++k) dst[(int64_t)k * a.nt] = sum[k];
-  }
+  if (own < a.nt) ff_sum_store<NOUT>(a.farv + (int64_t)blockIdx.y * NOUT * a.nt, a.nt, own, a.rows, sum);
 }
 
 // ---- near field -------------------------------------------------------------
@@ -1326,34 +1352,26 @@ __global__ __launch_bounds__(256) void k_ff_near(FFArgs a) {
     double r[12];
     near_item<CORE, GRAD, PREC>(a, b, r0, r1, sh, r);
     constexpr int NOUT = GRAD ? 12 : 3;
-    double* slot = a.part + (int64_t)item * NOUT * FF_TB;
-#pragma unroll
-    for (int c = 0; c < NOUT; ++c) slot[c * FF_TB + threadIdx.x] = r[c];
+    ff_sum_store<NOUT>(a.part + (int64_t)item * NOUT * FF_TB, FF_TB, threadIdx.x, a.rows, r);
   }
 }
 
-// one workgroup per block: near partials in item order, far part, self-pair
-// exclusion, then accumulate into the caller's arrays at the original index
-template <int CORE, bool GRAD>
+// per target (original order with ROWS, else sorted): far part by slice, near partials in
+// item order, self-pair exclusion, accumulated into the caller's arrays
+template <int CORE, bool GRAD, bool ROWS>
 __global__ __launch_bounds__(256) void k_ff_combine(FFArgs a) {
   constexpr int NOUT = GRAD ? 12 : 3;
-  const int64_t b = blockIdx.x;
-  const int64_t i = b * FF_TB + threadIdx.x;
-  if (i >= a.nt) return;
-  double r[NOUT];
-#pragma unroll
-  for (int c = 0; c < NOUT; ++c) r[c] = a.farv[(int64_t)c * a.nt + i];
-  for (int y = 1; y < a.nslice; ++y) {
-#pragma unroll
-    for (int c = 0; c < NOUT; ++c) r[c] += a.farv[((int64_t)y * NOUT + c) * a.nt + i];
-  }
+  const int64_t g = (int64_t)blockIdx.x * 256 + threadIdx.x;
+  if (g >= a.nt) return;
+  const int64_t i = ROWS ? a.tinv[g] : g, io = ROWS ? g : a.tperm[g];
+  const int64_t b = i / FF_TB;
+  double r[NOUT] = {};
+#pragma unroll 2
+  for (int y = 0; y < a.nslice; ++y) ff_sum_add<NOUT>(a.farv + (int64_t)y * NOUT * a.nt, a.nt, i, ROWS, r);
   const int n_it = a.items[b], off = a.ioff[b];
-  for (int k = 0; k < n_it; ++k) {
-    const double* slot = a.part + (int64_t)(off + k) * NOUT * FF_TB;
-#pragma unroll
-    for (int c = 0; c < NOUT; ++c) r[c] += slot[c * FF_TB + threadIdx.x];
-  }
-  const int io = a.tperm[i];
+#pragma unroll 2
+  for (int k = 0; k < n_it; ++k)
+    ff_sum_add<NOUT>(a.part + (int64_t)(off + k) * NOUT * FF_TB, FF_TB, i % FF_TB, ROWS, r);
   a.t.u[io] = (float)((double)a.t.u[io] + r[0]);
   a.t.v[io] = (float)((double)a.t.v[io] + r[1]);
   a.t.w[io] = (float)((double)a.t.w[io] + r[2]);
@@ -1395,10 +1413,11 @@ static __global__ void k_ff_zero_u64(unsigned long long* p) {
 
 // ---- host side shared by the factored calls ----------------------------------------
 
-// Key bits, the set's bit included, of n points in all: up to 131,072 points 24, which sort
-// in three passes (2^8 cells per axis or one bit less hold less than a point each even in a
-// ring), then all 30 or 31 in four
-inline int key_bits(int64_t n, bool two_sets) { return n <= 131072 ? 24 : two_sets ? 31 : 30; }
+// Key bits, the set's bit included, of n points in all: up to 1,048,576 points 24, which sort
+// in three passes (2^8 cells per axis, or one bit less: a block of 256 is many cells even in
+// a ring), then all 30 or 31 in four.  545,000 points of two sets 3,731 and 3,699 us; two rings of
+// 262,144, whose cells hold two points, 23.2 ms both
+inline int key_bits(int64_t n, bool two_sets) { return n <= 1048576 ? 24 : two_sets ? 31 : 30; }
 
 // sequential sub-allocation of a workspace, 256-byte aligned
 struct Carve {

@@ -52,7 +52,7 @@ __device__ __forceinline__ float plain_limit(float lim) { return lim >= 0.0f ? l
 // and near-test rows, and targets: points, or panels' centroids with their limit
 template <int RULE>
 __global__ __launch_bounds__(256) void k_pf_rows(PanFarArgs a, const int* sperm, float4* sp, float4* sa, float4* tq,
-                                                 FFBounds sb, FFBounds tb, int* nn) {
+                                                 FFBounds sb, FFBounds tb, int* nn, int* tinv) {
   constexpr int N = RULE == PANFAR_POINTS7 ? 7 : 1;
   const int tid = threadIdx.x;
   if ((int)blockIdx.x >= a.f.ntiles) {
@@ -68,6 +68,7 @@ __global__ __launch_bounds__(256) void k_pf_rows(PanFarArgs a, const int* sperm,
         p = make_float4(a.p.tx[j], a.p.ty[j], a.p.tz[j], 0.0f);
       }
       tq[i] = p;
+      if (tinv) tinv[j] = (int)i;
     }
     ff_group_bounds<1>(i < a.f.nt, &p, nullptr, tb, b);
     if (tid == 0) nn[b] = 0;
@@ -217,10 +218,10 @@ __device__ __forceinline__ void pf_item(const PanFarArgs& a, int64_t b, int item
   }
   // particles -> panels: the pairs were summed with the roles reversed
   const double sg = RULE == PANFAR_PARTICLES ? -1.0 : 1.0;
-  double* slot = a.f.part + (int64_t)item * NOUT * FF_TB + tid;
+  double r[NOUT];
 #pragma unroll
   for (int d = 0; d < 3; ++d)
-    slot[d * FF_TB] = sg * (PREC == PREC_COMP ? (double)hi[d] + (double)lo[d] : (double)acc[d]);
+    r[d] = sg * (PREC == PREC_COMP ? (double)hi[d] + (double)lo[d] : (double)acc[d]);
   if (GRAD) {
     float g[9];
     if (PREC != PREC_COMP) {
@@ -232,8 +233,9 @@ __device__ __forceinline__ void pf_item(const PanFarArgs& a, int64_t b, int item
       }
     }
 #pragma unroll
-    for (int k = 0; k < 9; ++k) slot[(3 + k) * FF_TB] = PREC == PREC_COMP ? gd[k] : (double)g[k];
+    for (int k = 0; k < 9; ++k) r[3 + k] = PREC == PREC_COMP ? gd[k] : (double)g[k];
   }
+  ff_sum_store<NOUT>(a.f.part + (int64_t)item * NOUT * FF_TB, FF_TB, tid, a.f.rows, r);
   if (has_near && active) a.list[atomicAdd(a.count, 1u)] = (unsigned)item * FF_TB + tid;
 }
 
@@ -338,7 +340,8 @@ __global__ __launch_bounds__(BLOCK) void k_pf_walk(PanFarArgs a) {
       }
     }
     while (stack.n > 0) split();
-    double* slot = a.f.part + (int64_t)n.item * NOUT * FF_TB + n.tid;
+    double* slot = a.f.part + (int64_t)n.item * NOUT * FF_TB + (a.f.rows ? n.tid * NOUT : n.tid);
+    const int step = a.f.rows ? 1 : FF_TB;
     double u[3], g[9];
 #pragma unroll
     for (int d = 0; d < 3; ++d) u[d] = wave_sum((PART ? -1.0 : 1.0) * (double)acc[d]);
@@ -350,10 +353,10 @@ __global__ __launch_bounds__(BLOCK) void k_pf_walk(PanFarArgs a) {
     }
     if (lane != 0) continue;
 #pragma unroll
-    for (int d = 0; d < 3; ++d) slot[d * FF_TB] += u[d];
+    for (int d = 0; d < 3; ++d) slot[d * step] += u[d];
     if (GRAD) {
 #pragma unroll
-      for (int k = 0; k < 9; ++k) slot[(3 + k) * FF_TB] += g[k];
+      for (int k = 0; k < 9; ++k) slot[(3 + k) * step] += g[k];
     }
   }
 }
@@ -411,7 +414,8 @@ __global__ __launch_bounds__(BLOCK) void k_pf_near7(PanFarArgs a) {
       }
     }
     while (wave_any(head < tail)) drain();
-    double* slot = a.f.part + (int64_t)n.item * NOUT * FF_TB + n.tid;
+    double* slot = a.f.part + (int64_t)n.item * NOUT * FF_TB + (a.f.rows ? n.tid * NOUT : n.tid);
+    const int step = a.f.rows ? 1 : FF_TB;
 #pragma unroll
     for (int d = 0; d < 3; ++d) u[d] = quarter_sum(u[d]);
     if (GRAD) {
@@ -420,17 +424,17 @@ __global__ __launch_bounds__(BLOCK) void k_pf_near7(PanFarArgs a) {
     }
     if (ql != 0 || !has) continue;
 #pragma unroll
-    for (int d = 0; d < 3; ++d) slot[d * FF_TB] += u[d];
+    for (int d = 0; d < 3; ++d) slot[d * step] += u[d];
     if (GRAD) {
 #pragma unroll
-      for (int k = 0; k < 9; ++k) slot[(3 + k) * FF_TB] += g[k];
+      for (int k = 0; k < 9; ++k) slot[(3 + k) * step] += g[k];
     }
   }
 }
 
 struct PanFarLayout {
   unsigned *k_in, *k_out, *mask, *ctr, *list, *count;
-  int *i_in, *i_out, *nn, *items, *ioff, *mfold, *iblk;
+  int *i_in, *i_out, *tinv, *nn, *items, *ioff, *mfold, *iblk;
   void* tmp;
   float *box, *tcs, *tam, *tsg, *bcs;
   float4 *sp, *sa, *tq, *tsph, *bsph, *rec, *cen;
@@ -458,6 +462,7 @@ PanFarLayout layout(char* base, int rule, int64_t units, int64_t nt, int nout) {
   L.k_out = cv.take<unsigned>(units + nt);
   L.i_in = cv.take<int>(units + nt);
   L.i_out = cv.take<int>(units + nt);
+  L.tinv = cv.take<int>(nt);
   L.tmp = cv.take<char>(radix_tmp_bytes(units + nt));
   L.sp = cv.take<float4>((size_t)ntiles * T);
   L.sa = cv.take<float4>((size_t)ntiles * T);
@@ -528,8 +533,10 @@ int run(const PanArgs* p, const PtPanArgs* t, void* ws, hipStream_t st) {
   const int rc = factored_order(sets, L.box, L.k_in, L.i_in, L.k_out, L.i_out, L.tmp, st, &perm);
   if (rc != O3D_OK) return rc;
   f.tperm = perm + units;
+  f.tinv = L.tinv;
+  f.rows = nt >= FF_ROWS_MIN;
   hipLaunchKernelGGL((k_pf_rows<RULE>), dim3((unsigned)(ntiles + nb)), dim3(256), 0, st, a, perm, L.sp, L.sa, L.tq,
-                     FFBounds{L.tsph, L.tcs, L.tam, L.tsg}, FFBounds{L.bsph, L.bcs, nullptr, nullptr}, L.nn);
+                     FFBounds{L.tsph, L.tcs, L.tam, L.tsg}, FFBounds{L.bsph, L.bcs, nullptr, nullptr}, L.nn, nt >= FF_ROWS_MIN ? L.tinv : nullptr);
   hipLaunchKernelGGL((k_ff_classify<CORE_SING>), dim3(grid_of(nb * mwords, 256)), dim3(256), 0, st, L.bsph, L.bcs, nb,
                      L.tsph, L.tcs, ntiles, mwords, L.mask, L.nn);
   hipLaunchKernelGGL(k_ff_plan, dim3(1), dim3(FF_PLAN_THREADS), 0, st, L.nn, nb, near_split(nb, ntiles), L.items, L.ioff,
@@ -554,7 +561,8 @@ int run(const PanArgs* p, const PtPanArgs* t, void* ws, hipStream_t st) {
   else
     hipLaunchKernelGGL((k_pf_walk<RULE, GRAD, PREC>), dim3(gwalk), dim3(BLOCK), node_lds(PART ? t->maxlev : p->maxlev), st, a);
   HIPCHK(hipGetLastError());
-  hipLaunchKernelGGL((k_ff_combine<CORE_SING, GRAD>), dim3((unsigned)nb), dim3(FF_TB), 0, st, f);
+  if (f.rows) hipLaunchKernelGGL((k_ff_combine<CORE_SING, GRAD, true>), dim3((unsigned)nb), dim3(FF_TB), 0, st, f);
+  else hipLaunchKernelGGL((k_ff_combine<CORE_SING, GRAD, false>), dim3((unsigned)nb), dim3(FF_TB), 0, st, f);
   HIPCHK(hipGetLastError());
   return O3D_OK;
 }
