@@ -27,11 +27,16 @@
 // what bounds this kernel (HBM writes) -- and lists the others.  A first pass of
 // the same kernel only counts them, to size the list.  (Running the recursed
 // pairs on a second stream beside the writes was measured slower: the write
-// kernel's workgroups hold the CUs.)  k_bm_near: one wave per
-// listed pair: 16 lanes take the level-1 decisions and leave the open pairs'
-// triangles in LDS, the children of the open level-1 pairs are spread over the
-// wave, each lane walks what lies below its own, and a fixed
+// kernel's workgroups hold the CUs.)  k_bm_near: one wave per four
+// listed pairs: 16 lanes take a pair's level-1 decisions and leave the open pairs'
+// triangles in LDS, then pair by pair the children of the open level-1 pairs are
+// spread over the wave, and a fixed
 // butterfly adds the lanes' G in FP64, so results do not depend on scheduling.
+// 5,120 panels on themselves, three unknowns: k_bm_far 521 -> 221 us (4.3 TB/s written) with
+// near pairs listed 64 at a time and chunks of 64 sources instead of 256, k_bm_near 1,056 ->
+// 800 with four pairs per wave at level 1 and the deepest leaves gathered (986 with four
+// leaves per lane throughout): 1.61 -> 1.01 ms.  What is left is the FP64 of the leaves of
+// touching panels.
 // Every tree decision below the root is the reference's float arithmetic too, so
 // the GPU subdivides exactly where the reference does; leaves below the last
 // decision level take FP64 centroids of the float sub-triangle nodes.
@@ -168,6 +173,21 @@ __global__ __launch_bounds__(BLOCK) void k_bm_far(BmFarArgs a) {
   const int64_t j0 = (int64_t)blockIdx.y * a.schunk;
   const int64_t j1 = j0 + a.schunk < a.ns ? j0 + a.schunk : a.ns;
   unsigned long long cnt = 0;
+  // the wave's near pairs wait in LDS for 64 to be there: one counter add, whose answer the
+  // wave waits for, per 64 of them (one per source with a near pair: 0.52 ms on 5,120 panels)
+  __shared__ uint2 pends[BLOCK / 64][128];
+  uint2* pend = pends[tid >> 6];
+  int npend = 0;
+  auto flush = [&]() {
+    unsigned long long base = 0;
+    if (lane == 0) base = atomicAdd(a.count, (unsigned long long)npend);
+    base = __shfl(base, 0, 64);
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    for (int k = lane; k < npend; k += 64)
+      if (base + k < a.cap) a.list[base + k] = pend[k];
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    npend = 0;
+  };
   for (int64_t jt = j0; jt < j1; jt += BM_TILE) {
     const int n = (int)(j1 - jt < BM_TILE ? j1 - jt : BM_TILE);
     __syncthreads();
@@ -197,13 +217,11 @@ __global__ __launch_bounds__(BLOCK) void k_bm_far(BmFarArgs a) {
       }
       const unsigned long long m = __builtin_amdgcn_ballot_w64(nearp);
       if (m) {
-        const int first = __builtin_ctzll(m);
-        unsigned long long base = 0;
-        if (lane == first) base = atomicAdd(a.count, (unsigned long long)__builtin_popcountll(m));
-        base = __shfl(base, first, 64);
-        const unsigned long long slot = base + __builtin_amdgcn_mbcnt_hi((unsigned)(m >> 32),
-                                                                      __builtin_amdgcn_mbcnt_lo((unsigned)m, 0u));
-        if (nearp && slot < a.cap) a.list[slot] = make_uint2((unsigned)i, (unsigned)j);
+        if (nearp) pend[npend + __builtin_amdgcn_mbcnt_hi((unsigned)(m >> 32),
+                                                          __builtin_amdgcn_mbcnt_lo((unsigned)m, 0u))] =
+            make_uint2((unsigned)i, (unsigned)j);
+        npend += __builtin_popcountll(m);
+        if (npend >= 64) flush();
       }
       if (!vec && (!valid || nearp)) continue;
       // this pair's coefficients [unknown k][component m]
@@ -281,6 +299,7 @@ __global__ __launch_bounds__(BLOCK) void k_bm_far(BmFarArgs a) {
       }
     }
   }
+  if (MODE == BM_WRITE && npend > 0) flush();
   if (MODE == BM_COUNT) {
 #pragma unroll
     for (int o = 32; o >= 1; o >>= 1) cnt += __shfl_xor(cnt, o, 64);
@@ -414,31 +433,69 @@ __device__ __forceinline__ void bm_corners(const float4* r, float* v) {
   v[0] = a.x; v[1] = a.y; v[2] = a.z; v[3] = a.w; v[4] = b.x; v[5] = b.y; v[6] = b.z; v[7] = b.w; v[8] = c.x;
 }
 
-// One wave per listed pair.  Level 1: lane c < 16 decides child pair c (source
-// child c/4, target child c%4) and evaluates it if separated.  Level 2: the 16
-// children of each open level-1 pair are spread over the wave (item k: the
+// leaves of source child p with the 4 target children of node pair (sv, tv), as bm_leaves16
+__device__ __forceinline__ void bm_leaves4(const float* sv, const float* tv, int p, double w, double* G) {
+  double ct[4][3];
+  {
+    float tn[18];
+    bm_nodes(tv, tn);
+    bm_child_centroids(tn, ct);
+  }
+  float sc[9];
+  bm_child(sv, p, sc);
+  double cs[3];
+#pragma unroll
+  for (int d = 0; d < 3; ++d) cs[d] = ((double)sc[d] + (double)sc[3 + d] + (double)sc[6 + d]) * (1.0 / 3.0);
+#pragma unroll
+  for (int q = 0; q < 4; ++q) {
+    const double ex = ct[q][0] - cs[0], ey = ct[q][1] - cs[1], ez = ct[q][2] - cs[2];
+    const float rr = frsq((float)(ex * ex + ey * ey + ez * ez));
+    const double k = w * (double)(rr * rr * rr);
+    G[0] += k * ex; G[1] += k * ey; G[2] += k * ez;
+  }
+}
+
+// Four listed pairs per wave.  Level 1: the 16 lanes of a quarter decide its pair's 16
+// child pairs (source child c/4, target child c%4) and evaluate the separated ones, which
+// is all of most pairs.  Level 2, pair by pair, by the whole wave: the 16
+// children of each open level-1 pair are spread over it (item k: the
 // (k/16)-th open pair, child k%16); a separated one is a leaf, an open one below
-// maxlev is walked by its lane (level 3 all leaves when maxlev is 3).  The
+// maxlev is walked by its lane; with maxlev 3 the open ones are gathered first and their
+// leaves spread over the wave.  The
 // level-1 triangles of the open pairs pass through LDS.  The tree
 // decisions are the reference's float arithmetic; leaves below a decision level
 // take FP64 centroids of the float nodes.
 constexpr int BM_L1 = 20;   // floats per level-1 pair in LDS (18 used; rows 16-byte aligned)
 
+// level-1 triangles of row k in LDS, and of their children c2 = 4 s + t the triangles
+__device__ __forceinline__ void bm_level2(const float* l1, int k, int c2, float* s2v, float* t2v) {
+  const float4* row = (const float4*)(l1 + k * BM_L1);
+  const float4 r0 = row[0], r1 = row[1], r2 = row[2], r3 = row[3], r4 = row[4];
+  const float s1v[9] = {r0.x, r0.y, r0.z, r0.w, r1.x, r1.y, r1.z, r1.w, r2.x};
+  const float t1v[9] = {r2.y, r2.z, r2.w, r3.x, r3.y, r3.z, r3.w, r4.x, r4.y};
+  bm_child(s1v, c2 >> 2, s2v);
+  bm_child(t1v, c2 & 3, t2v);
+}
+
 template <int MAXLEV>
 __global__ __launch_bounds__(BLOCK) void k_bm_near(BmNearArgs a) {
-  // each wave's 16 level-1 triangle pairs, shared with its items through LDS; a
-  // wave reads only its own rows, and LDS operations of one wave complete in order
+  // each wave's 16 level-1 triangle pairs, shared with its items through LDS, and the open
+  // level-2 pairs; a wave touches only its own, and LDS operations of one wave complete in order
   __shared__ float4 l1s[(BLOCK / 64) * 16 * BM_L1 / 4];
-  const int lane = threadIdx.x & 63;
+  __shared__ unsigned char open2s[BLOCK / 64][256];
+  const int lane = threadIdx.x & 63, ql = lane & 15;
   float* l1 = (float*)l1s + (threadIdx.x >> 6) * 16 * BM_L1;
+  unsigned char* open2 = open2s[threadIdx.x >> 6];
   const int64_t wave = ((int64_t)blockIdx.x * BLOCK + threadIdx.x) >> 6;
   const int64_t nwaves = ((int64_t)gridDim.x * BLOCK) >> 6;
   const int64_t listed = (int64_t)(*a.count < a.cap ? *a.count : a.cap);
   const int nunk = a.nunk;
   constexpr int maxlev = MAXLEV;
   const int64_t R = (int64_t)nunk * a.nt;
-  for (int64_t e = wave; e < listed; e += nwaves) {
-    const uint2 p = a.list[e];
+  for (int64_t e = wave; 4 * e < listed; e += nwaves) {
+    const int64_t li = 4 * e + (lane >> 4);
+    const bool has = li < listed;
+    const uint2 p = a.list[has ? li : 4 * e];
     const int64_t i = p.x, j = p.y;
     const float4* sr = a.srec + j * BM_F4;
     const float4* tr = a.trec + i * BM_F4;
@@ -451,85 +508,109 @@ __global__ __launch_bounds__(BLOCK) void k_bm_near(BmNearArgs a) {
 #pragma clang fp contract(off)
       t4 = (sr[0].w + tr[0].w) * 4.0f;
     }
-    const float t41 = 0.5f * t4, t42 = 0.25f * t4, t43 = 0.125f * t4;
-    double G[3] = {0.0, 0.0, 0.0};
+    double G[3] = {0.0, 0.0, 0.0};   // of this lane's pair
     if constexpr (maxlev == 1) {
-      if (lane == 0) bm_leaves16(s0, t0, 0.0625, G);
+      if (ql == 0) bm_leaves16(s0, t0, 0.0625, G);
+#pragma unroll
+      for (int d = 0; d < 3; ++d) G[d] = quarter_sum(G[d]);
     } else {
-      // level 1 on lanes 0..15; the open pairs' triangles go to LDS for the items
+      // the open pairs' triangles go to LDS for the items
       bool open1 = false;
       float sv1[9], tv1[9];
-      if (lane < 16) {
-        bm_child(s0, lane >> 2, sv1);
-        bm_child(t0, lane & 3, tv1);
+      bm_child(s0, ql >> 2, sv1);
+      bm_child(t0, ql & 3, tv1);
+      {
         float ex, ey, ez, d2;
-        if (bm_sep(sv1, tv1, t41, ex, ey, ez, d2)) bm_leaf_d(ex, ey, ez, d2, 0.0625, G);
-        else open1 = true;
+        if (bm_sep(sv1, tv1, 0.5f * t4, ex, ey, ez, d2)) bm_leaf_d(ex, ey, ez, d2, 0.0625, G);
+        else open1 = has;
       }
+#pragma unroll
+      for (int d = 0; d < 3; ++d) G[d] = quarter_sum(G[d]);
       const unsigned long long m1 = __builtin_amdgcn_ballot_w64(open1);
-      if (open1) {
-        // the open pairs' rows in lane order, so that item k reads row k / 16
-        const unsigned rank = __builtin_amdgcn_mbcnt_hi((unsigned)(m1 >> 32),
-                                                        __builtin_amdgcn_mbcnt_lo((unsigned)m1, 0u));
-        float4* row = (float4*)(l1 + rank * BM_L1);
-        row[0] = make_float4(sv1[0], sv1[1], sv1[2], sv1[3]);
-        row[1] = make_float4(sv1[4], sv1[5], sv1[6], sv1[7]);
-        row[2] = make_float4(sv1[8], tv1[0], tv1[1], tv1[2]);
-        row[3] = make_float4(tv1[3], tv1[4], tv1[5], tv1[6]);
-        row[4] = make_float4(tv1[7], tv1[8], 0.f, 0.f);
-      }
-      __builtin_amdgcn_wave_barrier();
-      const int items = 16 * __builtin_popcountll(m1);
-      for (int k = lane; k < items; k += 64) {
-        const int c2 = k & 15;
-        float s1v[9], t1v[9];
-        {
-          const float4* row = (const float4*)(l1 + (k >> 4) * BM_L1);
-          const float4 r0 = row[0], r1 = row[1], r2 = row[2], r3 = row[3], r4 = row[4];
-          s1v[0] = r0.x; s1v[1] = r0.y; s1v[2] = r0.z; s1v[3] = r0.w;
-          s1v[4] = r1.x; s1v[5] = r1.y; s1v[6] = r1.z; s1v[7] = r1.w; s1v[8] = r2.x;
-          t1v[0] = r2.y; t1v[1] = r2.z; t1v[2] = r2.w; t1v[3] = r3.x; t1v[4] = r3.y;
-          t1v[5] = r3.z; t1v[6] = r3.w; t1v[7] = r4.x; t1v[8] = r4.y;
+      for (int q = 0; q < 4; ++q) {
+        const unsigned mq = (unsigned)(m1 >> (16 * q)) & 0xffffu;
+        if (mq == 0u) continue;
+        const float tq = __shfl(t4, 16 * q, 64);
+        const float t42 = 0.25f * tq, t43 = 0.125f * tq;
+        double D[3] = {0.0, 0.0, 0.0};
+        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+        if (open1 && lane >> 4 == q) {
+          // the open pairs' rows in lane order, so that item k reads row k / 16
+          float4* row = (float4*)(l1 + __builtin_popcount(mq & ((1u << ql) - 1u)) * BM_L1);
+          row[0] = make_float4(sv1[0], sv1[1], sv1[2], sv1[3]);
+          row[1] = make_float4(sv1[4], sv1[5], sv1[6], sv1[7]);
+          row[2] = make_float4(sv1[8], tv1[0], tv1[1], tv1[2]);
+          row[3] = make_float4(tv1[3], tv1[4], tv1[5], tv1[6]);
+          row[4] = make_float4(tv1[7], tv1[8], 0.f, 0.f);
         }
-        float s2v[9], t2v[9];
-        bm_child(s1v, c2 >> 2, s2v);
-        bm_child(t1v, c2 & 3, t2v);
-        float ex, ey, ez, d2;
-        if constexpr (maxlev == 2) {
-          float sx, sy, sz, tx, ty, tz;
-          bm_centroid(s2v, sx, sy, sz);
-          bm_centroid(t2v, tx, ty, tz);
-          d2 = dist2(tx, ty, tz, sx, sy, sz, ex, ey, ez);
-          bm_leaf_d(ex, ey, ez, d2, 0.00390625, G);
-          continue;
-        }
-        if (bm_sep(s2v, t2v, t42, ex, ey, ez, d2)) {
-          bm_leaf_d(ex, ey, ez, d2, 0.00390625, G);
-          continue;
+        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+        const int items = 16 * __builtin_popcount(mq);
+        int n2 = 0;   // open level-2 pairs gathered
+        for (int k0 = 0; k0 < items; k0 += 64) {
+          const int k = k0 + lane;
+          bool deeper = false;
+          if (k < items) {
+            float s2v[9], t2v[9];
+            bm_level2(l1, k >> 4, k & 15, s2v, t2v);
+            float ex, ey, ez, d2;
+            if constexpr (maxlev == 2) {
+              float sx, sy, sz, tx, ty, tz;
+              bm_centroid(s2v, sx, sy, sz);
+              bm_centroid(t2v, tx, ty, tz);
+              d2 = dist2(tx, ty, tz, sx, sy, sz, ex, ey, ez);
+              bm_leaf_d(ex, ey, ez, d2, 0.00390625, D);
+            } else if (bm_sep(s2v, t2v, t42, ex, ey, ez, d2)) {
+              bm_leaf_d(ex, ey, ez, d2, 0.00390625, D);
+            } else if constexpr (maxlev == 3) {
+              deeper = true;
+            } else {
+              for (int c3 = 0; c3 < 16; ++c3) {
+                float s3v[9], t3v[9];
+                bm_child(s2v, c3 >> 2, s3v);
+                bm_child(t2v, c3 & 3, t3v);
+                if (bm_sep(s3v, t3v, t43, ex, ey, ez, d2)) bm_leaf_d(ex, ey, ez, d2, 0.000244140625, D);
+                else bm_leaves16(s3v, t3v, 0.0000152587890625, D);
+              }
+            }
+          }
+          if constexpr (maxlev == 3) {
+            const unsigned long long m = __builtin_amdgcn_ballot_w64(deeper);
+            if (deeper)
+              open2[n2 + __builtin_amdgcn_mbcnt_hi((unsigned)(m >> 32), __builtin_amdgcn_mbcnt_lo((unsigned)m, 0u))] =
+                  (unsigned char)k;
+            n2 += __builtin_popcountll(m);
+          }
         }
         if constexpr (maxlev == 3) {
-          bm_leaves16(s2v, t2v, 0.000244140625, G);
-          continue;
-        } else {
-        for (int c3 = 0; c3 < 16; ++c3) {
-          float s3v[9], t3v[9];
-          bm_child(s2v, c3 >> 2, s3v);
-          bm_child(t2v, c3 & 3, t3v);
-          if (bm_sep(s3v, t3v, t43, ex, ey, ez, d2)) bm_leaf_d(ex, ey, ez, d2, 0.000244140625, G);
-          else bm_leaves16(s3v, t3v, 0.0000152587890625, G);
+          __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+          // 64 open pairs at a time with all 16 leaves each (a lane's set-up costs as much as six
+          // of them), the last 40 or fewer with four per lane
+          int k0 = 0;
+          for (; n2 - k0 > 40; k0 += 64) {
+            if (k0 + lane < n2) {
+              const int id = open2[k0 + lane];
+              float s2v[9], t2v[9];
+              bm_level2(l1, id >> 4, id & 15, s2v, t2v);
+              bm_leaves16(s2v, t2v, 0.000244140625, D);
+            }
+          }
+          for (int k = 4 * k0 + lane; k < 4 * n2; k += 64) {
+            const int id = open2[k >> 2];
+            float s2v[9], t2v[9];
+            bm_level2(l1, id >> 4, id & 15, s2v, t2v);
+            bm_leaves4(s2v, t2v, k & 3, 0.000244140625, D);
+          }
         }
+#pragma unroll
+        for (int d = 0; d < 3; ++d) {
+          const double all = wave_sum(D[d]);
+          if (lane >> 4 == q) G[d] += all;
         }
       }
     }
-    __builtin_amdgcn_wave_barrier();
-#pragma unroll
-    for (int d = 0; d < 3; ++d) {
-#pragma unroll
-      for (int o = 32; o >= 1; o >>= 1) G[d] += __shfl_xor(G[d], o, 64);
-    }
-    // lane k*nunk + m writes coefficient (unknown k, component m)
-    if (lane < nunk * nunk) {
-      const int k = lane / nunk, m = lane % nunk;
+    // lane k*nunk + m of a quarter writes coefficient (unknown k, component m) of its pair
+    if (has && ql < nunk * nunk) {
+      const int k = ql / nunk, m = ql % nunk;
       const float4 s1 = sr[1], s2 = sr[2];
       const float4 t1 = tr[1], t2 = tr[2], t3 = tr[3];
       const double w = (double)sa * (1.0 / (4.0 * M_PI));
@@ -629,15 +710,17 @@ int bem_matrix_dev(const o3d_panels* src, const o3d_panels* targ, int32_t nunk, 
   fa.nunk = nunk; fa.same = same ? 1 : 0; fa.maxlev = maxlev;
   fa.coeffs = coeffs; fa.count = cnt;
   fa.vec4 = ((uintptr_t)coeffs % 16 == 0) && ((int64_t)nunk * nt) % 4 == 0;
-  // about 8 workgroups per CU: target blocks x source chunks of whole LDS tiles
+  // about 8 workgroups per CU: target blocks x source chunks of at least 32 (whole LDS tiles
+  // of 256, as before, made 400 workgroups of 5,120 panels on themselves)
   const int64_t nbx = (nt + BLOCK - 1) / BLOCK;
-  const int64_t ntiles = (ns + BM_TILE - 1) / BM_TILE;
   int64_t ny = (8LL * num_cus() + nbx - 1) / nbx;
-  if (ny > ntiles) ny = ntiles;
-  if (ny > 65535) ny = 65535;
-  if (ny < 1) ny = 1;
-  fa.schunk = ((ntiles + ny - 1) / ny) * BM_TILE;
+  fa.schunk = (((ns + ny - 1) / ny + 31) / 32) * 32;
+  if (fa.schunk > BM_TILE) fa.schunk = ((fa.schunk + BM_TILE - 1) / BM_TILE) * BM_TILE;
   ny = (ns + fa.schunk - 1) / fa.schunk;
+  if (ny > 65535) {
+    fa.schunk = (((ns + 65534) / 65535 + BM_TILE - 1) / BM_TILE) * BM_TILE;
+    ny = (ns + fa.schunk - 1) / fa.schunk;
+  }
   const dim3 grid((unsigned)nbx, (unsigned)ny);
   hipLaunchKernelGGL(k_bm_far<BM_COUNT>, grid, dim3(BLOCK), 0, st, fa);
   HIPCHK(hipGetLastError());
@@ -657,8 +740,8 @@ int bem_matrix_dev(const o3d_panels* src, const o3d_panels* targ, int32_t nunk, 
   if (prof) HIPCHK(hipEventRecord(ev[2], st));
   if (nnear > 0 && maxlev > 0) {
     BmNearArgs na{srec, trec, list, cnt, nnear, nt, nunk, maxlev, coeffs};
-    const int64_t waves_per_block = BLOCK / 64;
-    int64_t nb = ((int64_t)nnear + waves_per_block - 1) / waves_per_block;
+    const int64_t pairs_per_block = 4 * (BLOCK / 64);
+    int64_t nb = ((int64_t)nnear + pairs_per_block - 1) / pairs_per_block;
     const int64_t maxb = 64LL * num_cus();
     if (nb > maxb) nb = maxb;
     if (maxlev == 1) hipLaunchKernelGGL(k_bm_near<1>, dim3((unsigned)nb), dim3(BLOCK), 0, st, na);

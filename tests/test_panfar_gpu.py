@@ -280,3 +280,16 @@ def test_auto_line(mods, core, grads, ns, nt):
     a = influence.p2p(core, p.pos[:, :m], p.str[:, :m], p.rad[:m], t[0], t[1], grads, "comp")
     b = influence.p2p(core, p.pos[:, :m], p.str[:, :m], p.rad[:m], t[0], t[1], grads, "comp", method="direct")
     assert np.array_equal(a[0], b[0]) and (not grads or np.array_equal(a[1], b[1]))
+
+
+@pytest.mark.parametrize("n,maxlev,nunk", [(1, 3, 3), (33, 3, 2), (65, 3, 3), (257, 3, 3), (120, 1, 3), (120, 2, 2), (70, 4, 3)])
+def test_bem_matrix_ragged(mods, n, maxlev, nunk):
+    """the influence matrix of a patch of n coarse panels, most pairs near: list remainders,
+    quarters without a pair, gathered leaves full and partial.  Against the oracle's FP64 leaves
+    on the same trees: leaf kernels in float (1e-7 each) and one rounding, 1e-6"""
+    torch, _lib, influence = mods
+    pan = scenes.icosphere_panels(levels=2)
+    S = oracle.surface(np.ascontiguousarray(pan.nodes, np.float32), np.asarray(pan.idx, np.uint32).reshape(-1, 3)[:n])
+    a = influence.bem_matrix(S[:3], None, nunk, maxlev)
+    b = oracle.bem_matrix("wl", S, S, nunk, True, maxlev, mode="f64t")
+    assert np.abs(a - b).max() <= 1e-6 * np.abs(b).max()
