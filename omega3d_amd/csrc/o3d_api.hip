@@ -143,13 +143,14 @@ hipError_t dispatch_p2p_split(int core, const P2PArgs& a, bool thick, bool grad,
 }
 
 // Source split of a call whose targets make fewer workgroups than the GPU holds at
-// once: slices of whole tiles, enough of them for about SPLIT_WGS_PER_CU
-// workgroups per compute unit, and a partial buffer of at most SPLIT_MAX_BYTES.
+// once: slices of whole tiles (of the smallest calls shorter), enough of them for about
+// SPLIT_WGS_PER_CU workgroups per compute unit, and a partial buffer of at most SPLIT_MAX_BYTES.
 // cap > 0 (a caller's fixed scratch of cap bytes): fewer slices when the partials
 // of the wanted slice count do not fit.  Returns the slice count (1: no split) and
 // the slice length.
 constexpr int SPLIT_WGS_PER_CU = 16;
 constexpr size_t SPLIT_MAX_BYTES = (size_t)256 << 20;
+constexpr int64_t SPLIT_SHORT = 32;
 int split_plan(int64_t nt, int64_t ns, int tile, bool grad, int prec, int64_t* slen, size_t* bytes, size_t cap) {
   const int64_t nb = (nt + BLOCK - 1) / BLOCK;
   const int64_t want = (int64_t)SPLIT_WGS_PER_CU * num_cus();
@@ -163,9 +164,22 @@ int split_plan(int64_t nt, int64_t ns, int tile, bool grad, int prec, int64_t* s
     const int64_t fit = (int64_t)(cap / ((size_t)nt * cols));
     if (nsl > fit) nsl = fit;
   }
-  if (nsl < 2) return 1;
+  if (nsl < 2 && ns <= 32) return 1;
+  nsl = std::max<int64_t>(nsl, 1);
   const int64_t tiles_per = (ntiles + nsl - 1) / nsl;
   *slen = tiles_per * tile;
+  // So few targets and sources that whole tiles leave the GPU mostly idle (less than two
+  // workgroups per CU): a wave's time is then its slice's sources one after another, so up to
+  // SPLIT_SHORT slices of 32 sources or more, as far as two workgroups per CU.  On themselves,
+  // compensated, with gradient, us before and with 16, 32 and 64 slices: RM 256 28.6 and 13.4
+  // (8 slices), 1,024 30.0 and 17.4, 17.6, 17.5, 2,048 30.5 and 22.6, 21.3, 26.7, 4,096 35.9 and
+  // 36.0, 34.5, 41.3; EXP 1,024 60.5 and 30.8, 25.1, 24.9, 4,096 66.3 and 64.8, 52.1, 49.9.
+  // 16,384 targets of 1,024 sources, 64 blocks: 34.6 and 36.3, 41.8, 41.1
+  if (nb * nsl < 2 * (int64_t)num_cus()) {
+    const int64_t most = std::min<int64_t>(SPLIT_SHORT, 2 * (int64_t)num_cus() / nb);
+    const int64_t len = (((ns + most - 1) / most + 31) / 32) * 32;
+    if (len < *slen && (cap == 0 || (size_t)((ns + len - 1) / len) * (size_t)nt * cols <= cap)) *slen = len;
+  }
   nsl = (ns + *slen - 1) / *slen;
   *bytes = (size_t)nsl * (size_t)nt * cols;
   if (nsl < 2 || *bytes > (cap > 0 ? cap : SPLIT_MAX_BYTES)) return 1;

@@ -293,3 +293,17 @@ def test_bem_matrix_ragged(mods, n, maxlev, nunk):
     a = influence.bem_matrix(S[:3], None, nunk, maxlev)
     b = oracle.bem_matrix("wl", S, S, nunk, True, maxlev, mode="f64t")
     assert np.abs(a - b).max() <= 1e-6 * np.abs(b).max()
+
+
+@pytest.mark.parametrize("core", ["rm", "exp"])
+@pytest.mark.parametrize("ns,nt", [(1, 1), (32, 5), (33, 300), (65, 257), (1025, 1), (1000, 16129), (4095, 255)])
+def test_short_slices(mods, core, ns, nt):
+    """the smallest calls, whose sources are cut below a tile: one source over a slice, the
+    last slice short, one target; within the compensated bar of the oracle"""
+    torch, _lib, influence = mods
+    p = scenes.ring(ns, seed=41)
+    t = (2.4 * np.random.default_rng(6).random((3, nt)) - 1.2).astype(np.float32)
+    v, g = influence.p2p(core, p.pos, p.str, p.rad, t, None, True, "comp")
+    k = np.arange(0, nt, max(1, nt // 400))
+    ov, og = oracle.p2p(core, p.pos, p.str, p.rad, t[:, k], None, True, "f64")
+    assert rel_errors(v[:, k], ov)[0] <= 2e-6 and rel_errors(g[:, k], og)[0] <= 2e-6
