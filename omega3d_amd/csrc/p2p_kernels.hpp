@@ -663,16 +663,135 @@ __global__ __launch_bounds__(BLOCK) void k_p2p_split(P2PArgs a, void* part, int6
 // pairs, the gradient's sums in FP64 (its cross-slice reduction) -- takes out the
 // self pair as p2p_span does, forms the gradient and adds into the outputs; with
 // a.tperm the slices are in that order and the outputs go to the original index.
-// A block takes COMBINE_TG targets, one per lane of each wave: wave w sums columns
-// w, w + COMBINE_NW, ..., each over every slice in order (so a column's sum is the
-// same chain of operations whatever wave runs it), loading COMBINE_CH slices of its
-// columns before adding them; the first wave finishes the targets from the column
-// sums in LDS.
-constexpr int COMBINE_TG = 64, COMBINE_NW = BLOCK / COMBINE_TG, COMBINE_CH = 8;
+// A block takes COMBINE_TG targets, one per lane of each wave, and has a wave per
+// column, which sums it over every slice in order, CH slices loaded before they
+// are added.  What bounds it is latency: the slices come from other XCDs' caches, a few
+// hundred KB in all.  So a column is a wave of its own (three or four per wave took a round of
+// loads per 8 slices), and the outputs and the self pair's inputs are asked for before the
+// sums.  In compensated mode a wave finishes its column's output itself; plain FP32 forms the
+// gradient from several columns, which pass through LDS.
+// Whole calls before and after, compensated with gradient: RM 1,024 particles 17.5 -> 13.9 us,
+// 4,096 34.8 -> 30.1, EXP 1,024 25.0 -> 21.4; plain FP32 RM 1,024 14.9 -> 11.6, 8,192 63.5 -> 59.6.
+// (A wave per output that reads the one or two columns of its entry again, without LDS and
+// barrier: FP32 1,024 15.1.)
+constexpr int COMBINE_TG = 64;
+// slices [y0, y0 + ny) of one column (vel: of the velocity) of one target, loaded and then
+// added in order
+template <int PREC, int CH, bool FULL, typename Elem>
+__device__ __forceinline__ void combine_chunk(const Elem* pe, int64_t step, int ny, bool vel, float& h, float& l,
+                                              double& sm) {
+  Elem v[CH];
+#pragma unroll
+  for (int k = 0; k < CH; ++k)
+    if (FULL || k < ny) v[k] = pe[k * step];
+  if (vel) {
+#pragma unroll
+    for (int k = 0; k < CH; ++k) {
+      if (!FULL && k >= ny) continue;
+      if (PREC == PREC_FP32) {
+        two_sum(h, l, (float)v[k]);
+      } else {
+        const float2 hl = __builtin_bit_cast(float2, (double)v[k]);
+        two_sum(h, l, hl.x);
+        l += hl.y;
+      }
+    }
+  } else {
+#pragma unroll
+    for (int k = 0; k < CH; ++k) {
+      if (FULL || k < ny) sm += (double)v[k];
+    }
+  }
+}
+template <int CORE, bool THICK, bool GRAD, int PREC, int CH>
+__global__ __launch_bounds__((COMBINE_TG * PartCols<GRAD, PREC>::n)) void k_p2p_combine(P2PArgs a, const void* part,
+                                                                                     int nslice) {
+  constexpr int NC = PartCols<GRAD, PREC>::n;
+  constexpr int NOUT = GRAD ? 12 : 3;
+  constexpr bool LDS = GRAD && PREC == PREC_FP32;
+  using Elem = typename std::conditional<PREC == PREC_FP32, float, double>::type;
+  __shared__ double cs[LDS ? NC : 1][COMBINE_TG];
+  const int64_t nt = a.nt;
+  const int lane = threadIdx.x % COMBINE_TG;
+  const int w = __builtin_amdgcn_readfirstlane((int)(threadIdx.x / COMBINE_TG));   // its column
+  const int64_t i = (int64_t)blockIdx.x * COMBINE_TG + lane;
+  const bool live = i < nt;
+  const bool vel = w < 3;
+  const int64_t io = live && a.tperm ? (int64_t)a.tperm[i] : i;
+  float* const out = w == 0 ? a.t.u : w == 1 ? a.t.v : w == 2 ? a.t.w : w < NOUT ? a.t.g[w - 3] : nullptr;
+  float old = 0.0f, sr = 0.0f, tr = 0.0f, ax = 0.0f, ay = 0.0f, az = 0.0f;
+  if (live && w < NOUT) old = out[io];
+  const bool self = GRAD && live && !vel && w < NOUT && a.self_excl;
+  if (self) {
+    sr = a.s.r[io];
+    if (THICK) tr = a.t.r[io];
+    ax = a.s.ax[io]; ay = a.s.ay[io]; az = a.s.az[io];
+  }
+  float h = 0.0f, l = 0.0f;
+  double sm = 0.0;
+  if (live) {
+    const Elem* pe = (const Elem*)part + (int64_t)w * nt + i;
+    const int64_t step = (int64_t)NC * nt;
+    int y0 = 0;
+    for (; y0 + CH <= nslice; y0 += CH)
+      combine_chunk<PREC, CH, true>(pe + y0 * step, step, CH, vel, h, l, sm);
+    if (y0 < nslice) combine_chunk<PREC, CH, false>(pe + y0 * step, step, nslice - y0, vel, h, l, sm);
+  }
+  if constexpr (LDS) {
+    if (!vel) cs[w][lane] = sm;
+    __syncthreads();
+  }
+  if (!live || w >= NOUT) return;
+  if (vel) {
+    out[io] = add_comp(old, h, l);
+    return;
+  }
+  if constexpr (GRAD) {
+    double kx = 0.0, ky = 0.0, kz = 0.0;
+    if (self) {
+      float ks, Bp;
+      kb<CORE>(0.0f, core_term<CORE>(sr) + (THICK ? core_term<CORE>(tr) : 0.0f), 0.0f, ks, Bp);
+      kx = (double)ks * ax; ky = (double)ks * ay; kz = (double)ks * az;
+    }
+    double r = sm;
+    if constexpr (PREC == PREC_FP32) {
+      // within the branch, so that a wave reads and forms what its own entry needs
+#pragma unroll
+      for (int c = 0; c < 9; ++c)
+        if (w == c + 3) {
+          double sum[NC], g[9];
+#pragma unroll
+          for (int k = 3; k < NC; ++k) sum[k] = cs[k][lane];
+          sum[11] -= kx; sum[12] -= ky; sum[13] -= kz;
+          grad_from<double>(sum, g);
+          r = g[c];
+        }
+    } else {
+      if (w == 4) r = sm - kz;
+      else if (w == 5) r = sm + ky;
+      else if (w == 6) r = sm + kz;
+      else if (w == 8) r = sm - kx;
+      else if (w == 9) r = sm - ky;
+      else if (w == 10) r = sm + kx;
+    }
+    out[io] = (float)((double)old + r);
+  }
+}
+
+// The same for fewer than combine_few slices (many targets, which fill the chip): four waves
+// to a block, wave w sums columns w, w + COMBINE_NW, ..., so that a wave has more than two or
+// three loads to itself; the first wave finishes the targets from the column sums in LDS.
+// Whole calls with this and with a wave per column, RM with gradient, plain FP32: 260 sources on
+// 500,000 targets (2 slices) 119.8 and 135.8 us, 3,000 on 262,144 (4 or more) 521.2 and 521.9;
+// compensated 126.2 and 127.5, 536.0 and 532.5
+// Plain FP32 with gradient, where a wave per column also waits at a barrier, from 8 slices: 800
+// on 300,000 (4 slices) 188.3 and 191.4, 1,024 on 16,384 (8) 26.7 and 23.3
+constexpr int combine_few(bool grad, int prec) { return grad && prec == PREC_FP32 ? 8 : 4; }
+constexpr int COMBINE_NW = BLOCK / COMBINE_TG, COMBINE_CH = 8;
 // the columns W, W + COMBINE_NW, ... below NC of one target: slices [y0, y0 + ny)
 // loaded, then added in order
 template <int NC, int PREC, int W, int CPT, bool FULL, typename Elem>
-__device__ __forceinline__ void combine_chunk(const Elem* pe, int64_t nt, int y0, int ny, float* h, float* l,
+__device__ __forceinline__ void combine_few_chunk(const Elem* pe, int64_t nt, int y0, int ny, float* h, float* l,
                                               double* sm) {
   Elem v[CPT][COMBINE_CH];
 #pragma unroll
@@ -701,9 +820,9 @@ __device__ __forceinline__ void combine_chunk(const Elem* pe, int64_t nt, int y0
     }
   }
 }
-// one wave's share of k_p2p_combine: the sums of its columns into LDS
+// one wave's share of k_p2p_combine_few: the sums of its columns into LDS
 template <int NC, int PREC, int W>
-__device__ __forceinline__ void combine_wave(const void* part, int64_t nt, int64_t i, int nslice, int lane,
+__device__ __forceinline__ void combine_few_wave(const void* part, int64_t nt, int64_t i, int nslice, int lane,
                                              double (*cs)[COMBINE_TG], float2 (*vs)[COMBINE_TG]) {
   constexpr int CPT = W < NC ? (NC - W + COMBINE_NW - 1) / COMBINE_NW : 0;
   if constexpr (CPT > 0) {
@@ -715,8 +834,8 @@ __device__ __forceinline__ void combine_wave(const void* part, int64_t nt, int64
     for (int m = 0; m < CPT; ++m) { h[m] = 0.f; l[m] = 0.f; sm[m] = 0.0; }
     int y0 = 0;
     for (; y0 + COMBINE_CH <= nslice; y0 += COMBINE_CH)
-      combine_chunk<NC, PREC, W, CPT, true>(pe, nt, y0, COMBINE_CH, h, l, sm);
-    if (y0 < nslice) combine_chunk<NC, PREC, W, CPT, false>(pe, nt, y0, nslice - y0, h, l, sm);
+      combine_few_chunk<NC, PREC, W, CPT, true>(pe, nt, y0, COMBINE_CH, h, l, sm);
+    if (y0 < nslice) combine_few_chunk<NC, PREC, W, CPT, false>(pe, nt, y0, nslice - y0, h, l, sm);
 #pragma unroll
     for (int m = 0; m < CPT; ++m) {
       const int c = W + m * COMBINE_NW;
@@ -726,7 +845,7 @@ __device__ __forceinline__ void combine_wave(const void* part, int64_t nt, int64
   }
 }
 template <int CORE, bool THICK, bool GRAD, int PREC>
-__global__ __launch_bounds__(BLOCK) void k_p2p_combine(P2PArgs a, const void* part, int nslice) {
+__global__ __launch_bounds__(BLOCK) void k_p2p_combine_few(P2PArgs a, const void* part, int nslice) {
   constexpr int NC = PartCols<GRAD, PREC>::n;
   static_assert(COMBINE_NW == 4, "one column group per wave of the block");
   __shared__ double cs[NC][COMBINE_TG];
@@ -736,10 +855,10 @@ __global__ __launch_bounds__(BLOCK) void k_p2p_combine(P2PArgs a, const void* pa
   const int w = __builtin_amdgcn_readfirstlane((int)(threadIdx.x / COMBINE_TG));
   const int64_t i = (int64_t)blockIdx.x * COMBINE_TG + lane;
   if (i < nt) {
-    if (w == 0) combine_wave<NC, PREC, 0>(part, nt, i, nslice, lane, cs, vs);
-    else if (w == 1) combine_wave<NC, PREC, 1>(part, nt, i, nslice, lane, cs, vs);
-    else if (w == 2) combine_wave<NC, PREC, 2>(part, nt, i, nslice, lane, cs, vs);
-    else combine_wave<NC, PREC, 3>(part, nt, i, nslice, lane, cs, vs);
+    if (w == 0) combine_few_wave<NC, PREC, 0>(part, nt, i, nslice, lane, cs, vs);
+    else if (w == 1) combine_few_wave<NC, PREC, 1>(part, nt, i, nslice, lane, cs, vs);
+    else if (w == 2) combine_few_wave<NC, PREC, 2>(part, nt, i, nslice, lane, cs, vs);
+    else combine_few_wave<NC, PREC, 3>(part, nt, i, nslice, lane, cs, vs);
   }
   __syncthreads();
   if (w != 0 || i >= nt) return;
@@ -923,7 +1042,15 @@ hipError_t launch_p2p_split_prec(const P2PArgs& a, int nslice, int64_t slen, voi
   hipError_t e = hipGetLastError();
   if (e != hipSuccess) return e;
   const unsigned nbc = (unsigned)((a.nt + COMBINE_TG - 1) / COMBINE_TG);
-  hipLaunchKernelGGL((k_p2p_combine<CORE, THICK, GRAD, PREC>), dim3(nbc), dim3(BLOCK), 0, st, a, (const void*)part,
+  if (nslice < combine_few(GRAD, PREC)) {
+    hipLaunchKernelGGL((k_p2p_combine_few<CORE, THICK, GRAD, PREC>), dim3(nbc), dim3(BLOCK), 0, st, a,
+                       (const void*)part, nslice);
+    return hipGetLastError();
+  }
+  // up to 8 slices a chunk of 8, whose fewer registers (42 against 86) let two blocks share a
+  // CU: 500 sources on 300,000 targets 133.5 us compensated, 146.5 with 32
+  const auto combine = nslice <= 8 ? k_p2p_combine<CORE, THICK, GRAD, PREC, 8> : k_p2p_combine<CORE, THICK, GRAD, PREC, 32>;
+  hipLaunchKernelGGL(combine, dim3(nbc), dim3(COMBINE_TG * PartCols<GRAD, PREC>::n), 0, st, a, (const void*)part,
                      nslice);
   return hipGetLastError();
 }

@@ -307,3 +307,27 @@ def test_short_slices(mods, core, ns, nt):
     k = np.arange(0, nt, max(1, nt // 400))
     ov, og = oracle.p2p(core, p.pos, p.str, p.rad, t[:, k], None, True, "f64")
     assert rel_errors(v[:, k], ov)[0] <= 2e-6 and rel_errors(g[:, k], og)[0] <= 2e-6
+
+
+@pytest.mark.parametrize("prec", ["comp", "fp32"])
+@pytest.mark.parametrize("core,ns,nt", [("rm", 257, 64), ("rm", 1024, 65), ("wl", 8192, 63), ("v2", 8449, 1),
+                                        ("exp", 16641, 129), ("rm", 20000, 1000)])
+def test_slices_added_by_column(mods, core, ns, nt, prec):
+    """slice counts at and about whole rounds of loads, last blocks of few targets, sums added
+    into values that are there, the self pair taken out.  Compensated: the oracle's bar.  Plain
+    FP32 adds up to 512 terms of a slice one after another, 512 roundings of 2^-24 of sums that
+    pass the result by less than a factor of three: 1e-4"""
+    torch, _lib, influence = mods
+    bar = 2e-6 if prec == "comp" else 1e-4
+    p = scenes.ring(ns, seed=43)
+    t = (2.4 * np.random.default_rng(8).random((3, nt)) - 1.2).astype(np.float32)
+    v0, g0 = np.full((3, nt), 0.25, np.float32), np.full((9, nt), -0.5, np.float32)
+    v, g = influence.p2p(core, p.pos, p.str, p.rad, t, None, True, prec, vel=v0.copy(), grad=g0.copy())
+    u, _ = influence.p2p(core, p.pos, p.str, p.rad, t, None, False, prec)
+    ov, og = oracle.p2p(core, p.pos, p.str, p.rad, t, None, True, "f64")
+    assert rel_errors(v, ov + v0)[0] <= bar and rel_errors(g, og + g0)[0] <= bar
+    assert rel_errors(u, ov)[0] <= bar
+    if ns <= 1024:
+        v, g = influence.p2p(core, p.pos, p.str, p.rad, p.pos, p.rad, True, prec, self_term=1)
+        w, h = influence.p2p(core, p.pos, p.str, p.rad, p.pos, p.rad, True, prec, self_term=1, tile=256, tpt=1)
+        assert rel_errors(v, w)[0] <= bar and rel_errors(g, h)[0] <= bar
