@@ -160,6 +160,9 @@ int run(const o3d_points* src, o3d_points* targ, bool self_excl, int T, hipStrea
   a.ns = ns; a.nt = nt;
   a.tile = T; a.mwords = mwords; a.ntiles = ntiles;
   a.self_excl = self_excl ? 1 : 0;
+  const bool fine = PREC == PREC_COMP && (a.ns < FF_FINE_BELOW || a.nt < FF_FINE_BELOW);
+  a.merge = fine ? FF_FINE_MERGE : ff_merge<CORE, GRAD>();
+  a.fold = fine ? FF_FINE_FOLD : ff_fold<CORE, GRAD>();
   const int nslice = far_slices(nb, ntiles, GRAD ? 2 : 3, num_cus());
   a.tslice = (ntiles + nslice - 1) / nslice;
   a.nslice = (ntiles + a.tslice - 1) / a.tslice;

@@ -94,6 +94,17 @@ constexpr int FF_SL = 40;           // far field: LDS row of a source's BF16 r2 
 // Cores that the direct kernel sums otherwise (4.6e-8): 2
 template <int CORE, bool GRAD>
 constexpr int ff_merge() { return GRAD && (CORE == CORE_RM || CORE == CORE_EXP || CORE == CORE_SING) ? 4 : 2; }
+// RM and EXP with gradient, compensated, of fewer points: both are finer, so that such a call
+// is no further from FP64 than the direct sum, which serves it below AUTO's line.  Normwise
+// errors of velocity and gradient, two rings of RM: 30,100 particles direct 3.6e-8 3.9e-8, as
+// above 4.1e-8 5.0e-8, with 2 tiles and 8 sources 3.5e-8 3.3e-8; 60,000 3.5e-8 3.5e-8, 3.8e-8
+// 4.2e-8, 3.4e-8 3.1e-8; EXP 24,600 4.2e-8 1.1e-7, 4.3e-8 1.1e-7, 3.9e-8 0.9e-7.  It costs 3.5%
+// (65,536 RM 1.64 and 1.70 ms), and at 1,048,576 EXP 2.6%; from FF_FINE_BELOW targets and
+// sources, where single calls have always come here, the coarser ones stay.
+constexpr int64_t FF_FINE_BELOW = 65536;
+constexpr int FF_FINE_MERGE = 2, FF_FINE_FOLD = 8;
+template <int CORE, bool GRAD>
+constexpr bool ff_sized() { return GRAD && (CORE == CORE_RM || CORE == CORE_EXP); }
 
 struct FFArgs {
   const float4* sp;    // sorted sources {x, y, z, core_term}, up to a whole tile: the last one again
@@ -125,6 +136,7 @@ struct FFArgs {
   int32_t mwords;
   int32_t ntiles;
   int32_t self_excl;
+  int32_t merge, fold;   // ff_sized: far tiles per fold, near sources per partial
 };
 
 // NOUT sums of one target: in a row, or each a whole array of n targets apart.  k_ff_combine
@@ -1181,7 +1193,7 @@ __global__ __launch_bounds__(FF_FAR_THREADS, 2) void k_ff_far(FFArgs a) {
     }
     // the run's scales fit a further tile when no factor passes 2^16 and none loses more
     // than 4 of its leading bits
-    more = ti >= 0 && !own && !wown && ++run < ff_merge<CORE, GRAD>() && (unsigned)(jw - wj + 1) <= 2u;
+    more = ti >= 0 && !own && !wown && ++run < (ff_sized<CORE, GRAD>() ? a.merge : ff_merge<CORE, GRAD>()) && (unsigned)(jw - wj + 1) <= 2u;
 #pragma unroll
     for (int g = 0; g < NG; ++g) more = more && (unsigned)(eg[g] - wg[g] + 4) <= 6u;
     } while (more);
@@ -1293,9 +1305,9 @@ __device__ __forceinline__ void near_item(const FFArgs& a, int64_t b, int r0, in
         // gradient's into FP64 and the velocity's into its TwoSum pair (the velocity
         // once per tile: error against FP64 on 65,536-131,072 particles in two rings
         // 9.1e-8 to 1.2e-7 instead of 4.8e-8 to 6.0e-8, near field 0-1% faster).
-        constexpr int FOLD = ff_fold<CORE, GRAD>();
-        for (int j0 = 0; j0 < cnt; j0 += FOLD) {
-          const int j1 = j0 + FOLD < cnt ? j0 + FOLD : cnt;
+        const int every = ff_sized<CORE, GRAD>() ? a.fold : ff_fold<CORE, GRAD>();
+        for (int j0 = 0; j0 < cnt; j0 += every) {
+          const int j1 = j0 + every < cnt ? j0 + every : cnt;
           for (int j = j0; j < j1; ++j)
             source_acc<CORE, GRAD, 1>(tx, ty, tz, tt, thr, sh[2 * j], sh[2 * j + 1], acc);
           if (GRAD) fold_grad_raw(acc[0], gr);
