@@ -360,13 +360,18 @@ bool ff_supported(int core, bool grad, int prec) {
 // and 830-884, WL 49,152 1,105 and 1,063-1,125, 65,536 faster.  100,000 particles on 16,384
 // field points and 8,192 on 262,144 fall on the same lines (less the preparation's recent
 // 0.07 ms: RM 1,134 and 1,064, 1,416 and 1,235; WL 1,235 and 1,402, 1,561 and 1,667), 2,048
-// on 262,144 not (EXP 631 and 645), nor do fewer targets.
+// on 262,144 not (EXP 631 and 645), nor do fewer targets.  Below FF_FEW_TARGETS the far kernel's
+// blocks are few, and a single ring crosses at 1.5 to 1.75 times the pairs: EXP 80,000 on 8,500
+// 583 and 596, 150,000 1,028 and 956; WL 240,000 1,571 and 1,670; velocity alone: RM 260,000 927
+// and 951, 400,000 1,386 and 1,391, EXP 120,000 520 and 581, 240,000 1,038 and 998.  RM with
+// gradient keeps its line there: 110,000 on 9,000 720 and 774 from one ring, 722 and 685 from two
+constexpr int64_t FF_FEW_TARGETS = 16384;
 bool ff_auto_pays(int core, bool grad, int prec, int64_t ns, int64_t nt) {
   if (!(prec == PREC_COMP || ff_supported(core, grad, prec))) return false;
   if (ns < 8192 || nt < 8192 || ns > INT_MAX || nt > INT_MAX) return false;
   const double least = core == CORE_EXP ? (grad ? 6.0e8 : 1.0e9) : core == CORE_RM ? (grad ? 9.0e8 : 2.2e9)
                                                                                  : (grad ? 2.0e9 : 3.0e9);
-  return (double)ns * (double)nt >= least && ns + nt <= INT_MAX;
+  return (double)ns * (double)nt >= (nt < FF_FEW_TARGETS && !(core == CORE_RM && grad) ? 1.75 * least : least) && ns + nt <= INT_MAX;
 }
 
 namespace {
