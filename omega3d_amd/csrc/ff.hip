@@ -57,7 +57,7 @@ struct Layout {
   int *i_in, *i_out, *tinv, *nn, *items, *ioff, *mfold;
   void* tmp;
   float4 *sp, *sa, *tq, *tsph, *bsph;
-  float *box, *tcs, *tam, *tsg, *bcs;
+  float *box, *tcs, *tcm, *tam, *tsg, *bcs, *bcm;
   double *farv, *part;
   unsigned long long* npair;
   size_t bytes;
@@ -82,10 +82,12 @@ Layout layout(char* base, int64_t ns, int64_t nt, bool same, int T, size_t tmp_b
   L.tq = cv.take<float4>(nt);
   L.tsph = cv.take<float4>(ntiles);
   L.tcs = cv.take<float>(ntiles);
+  L.tcm = cv.take<float>(ntiles);
   L.tam = cv.take<float>(ntiles);
   L.tsg = cv.take<float>(ntiles);
   L.bsph = cv.take<float4>(nb);
   L.bcs = cv.take<float>(nb);
+  L.bcm = cv.take<float>(nb);
   L.mask = cv.take<unsigned>((size_t)(nb * mwords));
   L.farv = cv.take<double>((size_t)nout * far_slices(nb, ntiles, nout == 3 ? 3 : 2, num_cus()) * nt);
   L.npair = cv.take<unsigned long long>(1);
@@ -142,18 +144,18 @@ int run(const o3d_points* src, o3d_points* targ, bool self_excl, int T, hipStrea
   int rc = factored_order(sets, L.box, L.k_in, L.i_in, L.k_out, L.i_out, L.tmp, st, &perm);
   if (rc != O3D_OK) return rc;
   const int *sperm = perm, *tperm = same ? perm : perm + ns;
+  const FFBounds tb{L.tsph, L.tcs, L.tcm, L.tam, L.tsg}, bb{L.bsph, L.bcs, L.bcm, nullptr, nullptr};
   hipLaunchKernelGGL((k_ff_rows<CORE, THICK>), dim3((unsigned)(ntiles + nb)), dim3(256), 0, st, sv, tv, sperm, tperm, ns,
-                     nt, T, ntiles, L.sp, L.sa, L.tq, FFBounds{L.tsph, L.tcs, L.tam, L.tsg},
-                     FFBounds{L.bsph, L.bcs, nullptr, nullptr}, L.nn, nt >= FF_ROWS_MIN ? L.tinv : nullptr);
-  hipLaunchKernelGGL((k_ff_classify<CORE>), dim3(grid_of(nb * mwords, 256)), dim3(256), 0, st, L.bsph, L.bcs, nb, L.tsph,
-                     L.tcs, ntiles, mwords, L.mask, L.nn);
+                     nt, T, ntiles, L.sp, L.sa, L.tq, tb, bb, L.nn, nt >= FF_ROWS_MIN ? L.tinv : nullptr);
+  hipLaunchKernelGGL((k_ff_classify<CORE>), dim3(grid_of(nb * mwords, 256)), dim3(256), 0, st, bb, nb, tb, ntiles, mwords,
+                     L.mask, L.nn);
   hipLaunchKernelGGL(k_ff_plan, dim3(1), dim3(FF_PLAN_THREADS), 0, st, L.nn, nb, near_split(nb, ntiles), L.items, L.ioff,
                      L.mfold, L.ctr, (unsigned*)nullptr);
   HIPCHK(hipGetLastError());
 
   FFArgs a{};
   a.sp = L.sp; a.sa = L.sa; a.tq = L.tq; a.tperm = tperm; a.tinv = L.tinv; a.rows = nt >= FF_ROWS_MIN;
-  a.tsph = L.tsph; a.tcs = L.tcs; a.tam = L.tam; a.bsph = L.bsph; a.bcs = L.bcs;
+  a.tsph = L.tsph; a.tcs = L.tcs; a.tcm = L.tcm; a.tam = L.tam; a.bsph = L.bsph; a.bcm = L.bcm;
   a.mask = L.mask; a.farv = L.farv; a.tsg = L.tsg;
   a.nn = L.nn; a.items = L.items; a.ioff = L.ioff; a.mfold = L.mfold; a.ctr = L.ctr; a.part = L.part;
   a.s = sv; a.t = tv;

@@ -45,6 +45,12 @@
 // pairs left near 21 -> 11% for 524,288 particles on 20,480 panels, 15 -> 8% for 65,537
 // points in a box around two rings of 100,002 (whole calls 5.13 -> 4.58 and 2.16 -> 2.00 ms).
 //
+// Nor may a block be so much smaller than the tile, or the core terms (RM and WL: part of
+// r2, V2: beside its square) so unlike each other, that one scale leaves a weight too few
+// bits: the largest r2 that a pair of the tile and the block can have is at most FF_RANGE
+// times the least, from which the scale is taken, cores included (a gap alone, beside cores
+// ten times as wide, left weights of 1e-5 times the scale, and fewer bits with each).
+//
 // Particles are sorted along a Hilbert curve first (keys on a 10-bit grid per axis) so
 // that blocks and tiles are compact; the decision per (block, tile) is computed
 // once into a bit mask read by both kernels.  The curve has no jumps: in Morton order a
@@ -79,6 +85,7 @@ constexpr int CORE_SING = 0;
 constexpr int FF_TB = 256;          // targets per workgroup: 4 waves x 64
 constexpr float FF_KAPPA = 1.0f;    // minimum gap, in radii of the block or the tile, whichever is smaller
 constexpr float FF_SPREAD = 1.0f / 3.0f;   // and in block radii, so that one scale serves the block's weights
+constexpr float FF_RANGE = 81.0f;   // largest to least r2: 9 to the fifth is 2^16, of a weight's 2^13 and 24 bits below
 // near field, compensated: sources per FP32 partial.  Gradient error against FP64 on two
 // rings: EXP, 1,048,576 particles, 5.9e-8 at 32 and 5.0e-8 at 16 (near field 30.3 and
 // 31.5 ms); RM, 262,144, 4.5e-8 and 4.3e-8, with the near field 6% slower at 16; WL,
@@ -113,9 +120,10 @@ struct FFArgs {
   const int* tperm;    // sorted target -> original target index
   const float4* tsph;  // per source tile: bounding sphere {cx, cy, cz, r}
   const float* tcs;    // per source tile: largest core term
+  const float* tcm;    // and the least
   const float* tam;    // per source tile: largest |alpha| and |q|
   const float4* bsph;  // per target block: bounding sphere
-  const float* bcs;    // per target block: largest core term
+  const float* bcm;    // per target block: least core term
   const unsigned* mask;  // far bit per (block, tile), mwords words per block
   double* farv;        // per slice and target, sorted: far-field velocity and gradient, 12 (3) (FFSum)
   const int* tinv;     // original target -> sorted target
@@ -419,12 +427,12 @@ static __global__ __launch_bounds__(256) void k_ff_bounds(const float4* p, int64
   }
 }
 
-// where a group's bounds go: sphere (bbox centre, largest distance), largest core term,
-// and of sources (am) a bound of |alpha| and |q| and the sign of the first nonzero strength
+// where a group's bounds go: sphere (bbox centre, largest distance), largest and least
+// (cmin, if given) core term, and of sources (am) a bound of |alpha| and |q| and the sign of the first nonzero strength
 // (0: none), by its first nonzero component
 struct FFBounds {
   float4* sph;
-  float *cs, *am, *sign;
+  float *cs, *cmin, *am, *sign;
 };
 // the bounds of the workgroup's points, N per thread (valid: this thread has some) with
 // core terms p.w; strengths a, of sources
@@ -432,7 +440,7 @@ template <int N>
 __device__ __forceinline__ void ff_group_bounds(bool valid, const float4* p, const float4* a, const FFBounds& out,
                                                 int64_t g) {
   const float inf = __builtin_huge_valf();
-  float v[7] = {-inf, -inf, -inf, -inf, -inf, -inf, 0.0f};
+  float v[8] = {-inf, -inf, -inf, -inf, -inf, -inf, 0.0f, -inf};
   if (valid)
 #pragma unroll
     for (int k = 0; k < N; ++k) {
@@ -440,8 +448,9 @@ __device__ __forceinline__ void ff_group_bounds(bool valid, const float4* p, con
 #pragma unroll
       for (int d = 0; d < 3; ++d) { v[d] = fmaxf(v[d], -q[d]); v[3 + d] = fmaxf(v[3 + d], q[d]); }
       v[6] = fmaxf(v[6], p[k].w);
+      v[7] = fmaxf(v[7], -p[k].w);
     }
-  wg_max_n<7>(v);
+  wg_max_n<8>(v);
   const float c[3] = {0.5f * v[3] - 0.5f * v[0], 0.5f * v[4] - 0.5f * v[1], 0.5f * v[5] - 0.5f * v[2]};
   float w[3] = {0.0f, 0.0f, -inf};   // squared radius, largest component, -(2 i + negative) of the first strength
   if (valid)
@@ -460,6 +469,7 @@ __device__ __forceinline__ void ff_group_bounds(bool valid, const float4* p, con
   // margin for the rounding of the distances above
   out.sph[g] = make_float4(c[0], c[1], c[2], __fsqrt_rn(w[0]) * 1.00001f + 1e-30f);
   out.cs[g] = v[6];
+  if (out.cmin) out.cmin[g] = -v[7];
   if (a) {
     out.am[g] = w[1] * 1.7321f;   // sqrt 3, rounded up
     out.sign[g] = w[2] == -inf ? 0.0f : ((int)-w[2] & 1) ? -1.0f : 1.0f;
@@ -499,28 +509,40 @@ __global__ __launch_bounds__(256) void k_ff_rows(SrcView s, TgtView t, const int
   }
 }
 
+// r2 at a distance of d with core terms c, as the far field's weights take it
+template <int CORE>
+__device__ __forceinline__ float ff_r2_with(float d, float c) {
+  const float d2 = d * d;
+  if (CORE == CORE_RM || CORE == CORE_WL) return d2 + c;
+  if (CORE == CORE_V2) return fmaxf(d2, __fsqrt_rn(fmaf(d2, d2, c)));
+  return d2;
+}
+
 // far bit of every (target block, source tile), and the near tiles counted into nn (cleared
 // before): one thread per 32 tiles of a block
 template <int CORE>
-__global__ __launch_bounds__(256) void k_ff_classify(const float4* bsph, const float* bcs, int64_t nb,
-                                                     const float4* tsph, const float* tcs, int ntiles, int mwords,
+__global__ __launch_bounds__(256) void k_ff_classify(FFBounds bb, int64_t nb, FFBounds tb, int ntiles, int mwords,
                                                      unsigned* mask, int* nn) {
+  constexpr bool CORES = CORE == CORE_RM || CORE == CORE_WL || CORE == CORE_V2;   // part of the weights
   const int64_t g = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
   if (g >= nb * mwords) return;
   const int64_t b = g / mwords;
   const int w = (int)(g - b * mwords);
-  const float4 cb = bsph[b];
-  const float csb = bcs[b];
+  const float4 cb = bb.sph[b];
+  const float csb = bb.cs[b], cmb = CORES ? bb.cmin[b] : 0.0f;
   unsigned bits = 0u;
   const int left = ntiles - 32 * w < 32 ? ntiles - 32 * w : 32;
   for (int k = 0; k < left; ++k) {
     const int ti = w * 32 + k;
-    const float4 ct = tsph[ti];
+    const float4 ct = tb.sph[ti];
+    const float cst = tb.cs[ti];
     const float dx = cb.x - ct.x, dy = cb.y - ct.y, dz = cb.z - ct.z;
     const float gap = __fsqrt_rn(fmaf(dz, dz, fmaf(dy, dy, dx * dx))) - cb.w - ct.w;
     bool far = gap > 0.0f && gap > FF_KAPPA * fmaxf(fminf(cb.w, ct.w), FF_SPREAD * cb.w);
-    if (CORE == CORE_EXP) far = far && gap * gap > exp_threshold(csb + tcs[ti]);
-    if (CORE == CORE_SING) far = far && gap > fmaxf(csb, tcs[ti]);
+    far = far && ff_r2_with<CORE>(gap + 2.0f * (cb.w + ct.w), csb + cst) <=
+                     FF_RANGE * ff_r2_with<CORE>(gap, CORES ? cmb + tb.cmin[ti] : 0.0f);
+    if (CORE == CORE_EXP) far = far && gap * gap > exp_threshold(csb + cst);
+    if (CORE == CORE_SING) far = far && gap > fmaxf(csb, cst);
     if (far) bits |= 1u << k;
   }
   mask[g] = bits;
@@ -770,7 +792,8 @@ __device__ __forceinline__ void ff_load_lds16(const float4* src, float4* dst) {
 // The moment products keep about 22 significant bits per product (hi hi + lo hi +
 // hi lo), the accuracy of the FP32 products they replace.  Weights are scaled by
 // powers of 2^(1/2): r2 -> r2 2^-jw through the staged source terms and the targets'
-// a, so Bp takes 2^(5 jw / 2) and K 2^(3 jw / 2) (from Bp <= 3.5 gap^-5), and each moment
+// a, so Bp takes 2^(5 jw / 2) and K 2^(3 jw / 2) (from Bp <= 3.5 r^-5 at the least r of the
+// gap and the cores), and each moment
 // group by 2^eg (from the tile's largest |alpha| and source distance), so that every
 // FP16 factor stays below 2^16.  Consecutive tiles keep the scales of the first as
 // long as they fit (ff_merge tiles at most) and share one fold into FP64, where the
@@ -984,7 +1007,8 @@ __global__ __launch_bounds__(FF_FAR_THREADS, 2) void k_ff_far(FFArgs a) {
       const float ddx = cb.x - ct.x, ddy = cb.y - ct.y, ddz = cb.z - ct.z;
       const float dc = __fsqrt_rn(fmaf(ddz, ddz, fmaf(ddy, ddy, ddx * ddx)));
       const float gap = dc - cb.w - ct.w;   // > 0 for a far tile
-      const float lgap = __builtin_amdgcn_logf(fmaxf(gap, 1e-37f));
+      float lr = __builtin_amdgcn_logf(fmaxf(gap, 1e-37f));   // of the least distance that the weights see
+      if (COREA || TAU) lr = fmaxf(lr, 0.5f * __builtin_amdgcn_logf(ff_r2_with<CORE>(gap, a.bcm[blk] + a.tcm[t])));
       const bool own = !(gap > FF_KAPPA * cb.w);   // a tile nearer than the block is wide: its own centre
       const float rs = own ? fmaxf(ct.w, gap * 0x1p-12f) : dc + ct.w;   // |s'| bound
       const float lrs = __builtin_amdgcn_logf(rs);
@@ -998,7 +1022,7 @@ __global__ __launch_bounds__(FF_FAR_THREADS, 2) void k_ff_far(FFArgs a) {
       int wg[5];
 #pragma unroll
       for (int g = 0; g < 5; ++g) wg[g] = (int)fminf(fmaxf(floorf(13.0f - lg[g]) - (float)ea, -126.0f), 126.0f) & 255;
-      pk0 = ((int)floorf(2.0f * (lgap + top)) << 16) | (wg[1] << 8) | wg[0];
+      pk0 = ((int)floorf(2.0f * (lr + top)) << 16) | (wg[1] << 8) | wg[0];
       pk1 = (own ? 1 << 24 : 0) | (wg[4] << 16) | (wg[3] << 8) | wg[2];
     }
     const int t = __builtin_ctz(bits);

@@ -512,7 +512,7 @@ int run(const PanArgs* p, const PtPanArgs* t, void* ws, hipStream_t st) {
   const PanFarLayout L = layout(static_cast<char*>(ws), RULE, units, nt, GRAD ? 12 : 3);
   FFArgs& f = a.f;
   f.sp = L.sp; f.sa = L.sa; f.tq = L.tq;
-  f.tsph = L.tsph; f.tcs = L.tcs; f.tam = L.tam; f.tsg = L.tsg; f.bsph = L.bsph; f.bcs = L.bcs;
+  f.tsph = L.tsph; f.tcs = L.tcs; f.tam = L.tam; f.tsg = L.tsg; f.bsph = L.bsph;
   f.mask = L.mask; f.farv = L.farv;
   f.nn = L.nn; f.items = L.items; f.ioff = L.ioff; f.mfold = L.mfold; f.ctr = L.ctr; f.part = L.part;
   f.nt = nt; f.ns = (int64_t)ntiles * T;
@@ -535,10 +535,11 @@ int run(const PanArgs* p, const PtPanArgs* t, void* ws, hipStream_t st) {
   f.tperm = perm + units;
   f.tinv = L.tinv;
   f.rows = nt >= FF_ROWS_MIN;
-  hipLaunchKernelGGL((k_pf_rows<RULE>), dim3((unsigned)(ntiles + nb)), dim3(256), 0, st, a, perm, L.sp, L.sa, L.tq,
-                     FFBounds{L.tsph, L.tcs, L.tam, L.tsg}, FFBounds{L.bsph, L.bcs, nullptr, nullptr}, L.nn, nt >= FF_ROWS_MIN ? L.tinv : nullptr);
-  hipLaunchKernelGGL((k_ff_classify<CORE_SING>), dim3(grid_of(nb * mwords, 256)), dim3(256), 0, st, L.bsph, L.bcs, nb,
-                     L.tsph, L.tcs, ntiles, mwords, L.mask, L.nn);
+  const FFBounds tb{L.tsph, L.tcs, nullptr, L.tam, L.tsg}, bb{L.bsph, L.bcs, nullptr, nullptr, nullptr};
+  hipLaunchKernelGGL((k_pf_rows<RULE>), dim3((unsigned)(ntiles + nb)), dim3(256), 0, st, a, perm, L.sp, L.sa, L.tq, tb, bb,
+                     L.nn, nt >= FF_ROWS_MIN ? L.tinv : nullptr);
+  hipLaunchKernelGGL((k_ff_classify<CORE_SING>), dim3(grid_of(nb * mwords, 256)), dim3(256), 0, st, bb, nb, tb, ntiles,
+                     mwords, L.mask, L.nn);
   hipLaunchKernelGGL(k_ff_plan, dim3(1), dim3(FF_PLAN_THREADS), 0, st, L.nn, nb, near_split(nb, ntiles), L.items, L.ioff,
                      L.mfold, L.ctr, L.count);
   HIPCHK(hipGetLastError());

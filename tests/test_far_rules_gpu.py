@@ -1,0 +1,81 @@
+"""What the factored far field may take: pairs whose weights keep their bits, whatever the
+core radii, the shape of a block or the values of its strengths, and calls that it is
+chosen for."""
+import ctypes as C
+
+import numpy as np
+import pytest
+
+from omega3d_amd import scenes
+from omega3d_amd.metrics import rel_errors
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.fixture(scope="module")
+def infl():
+    pytest.importorskip("torch")   # before the library, as the other modules have it
+    from omega3d_amd import _lib, influence
+    assert _lib.lib.o3d_init(-1) == 0, _lib.last_error()
+    return influence
+
+
+@pytest.mark.parametrize("over", [1.0, 0.3, 0.1, 0.03])
+@pytest.mark.parametrize("core,grads,n", [("rm", True, 30001), ("wl", True, 44801), ("v2", True, 44801),
+                                          ("rm", False, 47001), ("wl", False, 54901), ("v2", False, 54901)])
+def test_cores_wider_than_the_gap(infl, core, grads, n, over):
+    """a cube `over` core radii wide, which AUTO sends to the far field: the gaps between
+    tiles are small beside the cores.  Within the compensated bar of the FP64 sums"""
+    rng = np.random.default_rng(n)
+    pos = rng.random((3, n)).astype(np.float32)
+    st = (rng.normal(size=(3, n)) / n).astype(np.float32)
+    rad = (rng.uniform(0.8, 1.25, n) / over).astype(np.float32)
+    k = np.arange(0, n, n // 500)
+    v, g = infl.p2p(core, pos, st, rad, pos, rad, grads, "comp")
+    d, dg = infl.p2p(core, pos, st, rad, pos[:, k], rad[k], grads, "fp64")
+    e = [rel_errors(v[:, k], d), rel_errors(g[:, k], dg) if grads else None]
+    print(core, grads, over, e)
+    assert e[0][0] <= 2e-6 and (not grads or e[1][0] <= 2e-6)
+
+
+def _pair_sums(core, sp, ss, sr, t, grads):
+    """sums of |K alpha x d| (and of |Bp d (alpha x d)| + |K alpha|) of one target in FP64"""
+    d = t[:, None].astype(np.float64) - sp
+    q = (d * d).sum(0)
+    s2 = sr.astype(np.float64) ** 2
+    if core == "rm":
+        K, B = (q + s2) ** -1.5, 3 * (q + s2) ** -2.5
+    elif core == "wl":
+        K = (q + 2.5 * s2) * (q + s2) ** -2.5
+        B = 3 * (q + 3.5 * s2) * (q + s2) ** -3.5
+    elif core == "v2":
+        K, B = (q * q + s2 * s2) ** -0.75, 3 * q * (q * q + s2 * s2) ** -1.75
+    else:
+        K, B = q ** -1.5, 3 * q ** -2.5   # beyond the core; within it less
+    a, c = np.linalg.norm(ss, axis=0), np.linalg.norm(np.cross(ss, d, axis=0), axis=0)
+    return (K * c).sum(), (B * np.sqrt(q) * c + K * a).sum() if grads else 0.0
+
+
+@pytest.mark.parametrize("sigma", [0.05, 0.003])
+@pytest.mark.parametrize("core,grads", [("rm", True), ("wl", True), ("v2", True), ("exp", True), ("rm", False),
+                                        ("wl", False), ("v2", False), ("exp", False)])
+def test_blocks_without_extent(infl, core, grads, sigma):
+    """65 blocks of 256 coincident points and a block of one, inside a dense ring: a tile may
+    lie as near to such a block as its own sphere ends.  Each point for itself against FP64:
+    a pair keeps 22 bits of its weight and moments, at most four times its own size, 1e-6 of
+    the sum of its pairs' sizes in all"""
+    rng = np.random.default_rng(5)
+    ns, nb = 200000, 65
+    ph, th, r = 6.2831853 * rng.random(ns), 6.2831853 * rng.random(ns), 0.1 * np.sqrt(rng.random(ns))
+    sp = np.stack([(1 + r * np.cos(ph)) * np.cos(th), (1 + r * np.cos(ph)) * np.sin(th), r * np.sin(ph)]).astype(np.float32)
+    ss = (rng.normal(size=(3, ns)) / ns).astype(np.float32)
+    sr = np.full(ns, sigma, np.float32)
+    at = sp[:, rng.choice(ns, nb, replace=False)] + np.float32(1e-4)
+    tp = np.concatenate([np.repeat(at, 256, 1), at[:, -1:]], 1)
+    v, g = infl.p2p(core, sp, ss, sr, tp, None, grads, "comp")
+    d, dg = infl.p2p(core, sp, ss, sr, at, None, grads, "fp64")
+    for b in range(nb):
+        size = _pair_sums(core, sp, ss, sr, at[:, b], grads)
+        for t in (256 * b, 256 * b + 255) + ((256 * nb,) if b == nb - 1 else ()):
+            e = [np.linalg.norm(v[:, t] - d[:, b]) / size[0], np.linalg.norm(g[:, t] - dg[:, b]) / size[1] if grads else 0.0]
+            assert max(e) <= 1e-6, (core, grads, sigma, b, t, e)
