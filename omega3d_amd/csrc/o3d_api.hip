@@ -700,7 +700,9 @@ int o3d_factored_profile_dev(const o3d_points* src, o3d_points* targ, const o3d_
   if ((rc = check_self(src, targ, o)) != O3D_OK) return rc;
   if ((rc = ensure_init()) != O3D_OK) return rc;
   if (src->n == 0 || targ->n == 0) return O3D_OK;
-  return p2p_factored(src, targ, o, (hipStream_t)o->stream, out);
+  o3d_opts of = *o;   // whatever the field says: what FACTORED does not serve is refused
+  of.method = O3D_METHOD_FACTORED;
+  return p2p_factored(src, targ, &of, (hipStream_t)o->stream, out);
 }
 
 int o3d_points_affect_points64(const o3d_points64* src, o3d_points64* targ, const o3d_opts* o, o3d_stats* stats) {

@@ -79,3 +79,24 @@ def test_blocks_without_extent(infl, core, grads, sigma):
         for t in (256 * b, 256 * b + 255) + ((256 * nb,) if b == nb - 1 else ()):
             e = [np.linalg.norm(v[:, t] - d[:, b]) / size[0], np.linalg.norm(g[:, t] - dg[:, b]) / size[1] if grads else 0.0]
             assert max(e) <= 1e-6, (core, grads, sigma, b, t, e)
+
+
+@pytest.mark.parametrize("core,grads,prec", [("wl", True, "comp"), ("v2", True, "fp32"), ("rm", False, "comp"),
+                                             ("exp", False, "fp32"), ("rm", True, "fp64"), ("exp", True, "fp64")])
+def test_profile_refuses_what_factored_refuses(infl, core, grads, prec):
+    """the profile is of method FACTORED whatever the method field says: calls that it does not
+    serve are refused, and the outputs stay as they were"""
+    from omega3d_amd import _lib
+    p, D = scenes.ring(2048), _lib.DeviceArray.from_host
+    x, s, r = D(p.pos), D(p.str), D(p.rad)
+    out = D(np.full((12, p.n), 0.5, np.float32))
+    q = _lib.Points()
+    q.n, q.r = p.n, r.ptr
+    for d in range(3):
+        q.x[d], q.s[d], q.u[d] = x.row(d), s.row(d), out.row(d)
+    for k in range(9):
+        q.ug[k] = out.row(3 + k)
+    for method in ("auto", "direct"):
+        o = _lib.make_opts(core, grads, prec, method=method)
+        assert _lib.lib.o3d_factored_profile_dev(C.byref(q), C.byref(q), C.byref(o), C.byref(_lib.FactoredProfile())) == 1
+    assert (out.to_host() == 0.5).all()
