@@ -459,7 +459,12 @@ __device__ __forceinline__ void ff_group_bounds(bool valid, const float4* p, con
       const float dx = p[k].x - c[0], dy = p[k].y - c[1], dz = p[k].z - c[2];
       w[0] = fmaxf(w[0], fmaf(dz, dz, fmaf(dy, dy, dx * dx)));
       if (a) {   // no square that could leave the range
-        w[1] = fmaxf(fmaxf(fmaxf(w[1], fabsf(a[k].x)), fmaxf(fabsf(a[k].y), fabsf(a[k].z))), fabsf(a[k].w));
+        // one that is no number counts as infinite
+#pragma unroll
+        for (int c = 0; c < 4; ++c) {
+          const float m = fabsf(c == 0 ? a[k].x : c == 1 ? a[k].y : c == 2 ? a[k].z : a[k].w);
+          w[1] = m <= w[1] ? w[1] : m < inf ? m : inf;
+        }
         const float f = a[k].x != 0.0f ? a[k].x : a[k].y != 0.0f ? a[k].y : a[k].z != 0.0f ? a[k].z : a[k].w;
         if (f != 0.0f) w[2] = fmaxf(w[2], -(float)(2 * (N * (int)threadIdx.x + k) + (f < 0.0f ? 1 : 0)));
       }
@@ -519,7 +524,9 @@ __device__ __forceinline__ float ff_r2_with(float d, float c) {
 }
 
 // far bit of every (target block, source tile), and the near tiles counted into nn (cleared
-// before): one thread per 32 tiles of a block
+// before): one thread per 32 tiles of a block.  A tile with a strength that is infinite or no
+// number is near, as its products would leave nothing of the finite components, and so is one
+// whose r2 can leave the range
 template <int CORE>
 __global__ __launch_bounds__(256) void k_ff_classify(FFBounds bb, int64_t nb, FFBounds tb, int ntiles, int mwords,
                                                      unsigned* mask, int* nn) {
@@ -539,8 +546,9 @@ __global__ __launch_bounds__(256) void k_ff_classify(FFBounds bb, int64_t nb, FF
     const float dx = cb.x - ct.x, dy = cb.y - ct.y, dz = cb.z - ct.z;
     const float gap = __fsqrt_rn(fmaf(dz, dz, fmaf(dy, dy, dx * dx))) - cb.w - ct.w;
     bool far = gap > 0.0f && gap > FF_KAPPA * fmaxf(fminf(cb.w, ct.w), FF_SPREAD * cb.w);
-    far = far && ff_r2_with<CORE>(gap + 2.0f * (cb.w + ct.w), csb + cst) <=
-                     FF_RANGE * ff_r2_with<CORE>(gap, CORES ? cmb + tb.cmin[ti] : 0.0f);
+    const float most = ff_r2_with<CORE>(gap + 2.0f * (cb.w + ct.w), csb + cst);
+    far = far && most <= FF_RANGE * ff_r2_with<CORE>(gap, CORES ? cmb + tb.cmin[ti] : 0.0f);
+    far = far && most < __builtin_huge_valf() && tb.am[ti] < __builtin_huge_valf();
     if (CORE == CORE_EXP) far = far && gap * gap > exp_threshold(csb + cst);
     if (CORE == CORE_SING) far = far && gap > fmaxf(csb, cst);
     if (far) bits |= 1u << k;

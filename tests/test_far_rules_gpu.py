@@ -100,3 +100,79 @@ def test_profile_refuses_what_factored_refuses(infl, core, grads, prec):
         o = _lib.make_opts(core, grads, prec, method=method)
         assert _lib.lib.o3d_factored_profile_dev(C.byref(q), C.byref(q), C.byref(o), C.byref(_lib.FactoredProfile())) == 1
     assert (out.to_host() == 0.5).all()
+
+
+@pytest.mark.parametrize("what", ["strength inf", "strength nan", "radius inf", "place 3e19"])
+@pytest.mark.parametrize("core,grads", [("rm", True), ("wl", True), ("v2", True), ("exp", True), ("rm", False), ("wl", False)])
+def test_values_that_are_no_numbers(infl, core, grads, what):
+    """a strength component that is infinite or no number, an infinite core or a distance whose
+    square overflows touches the components that it touches in the direct sums, no others"""
+    n = 56001
+    p = scenes.colliding_rings((n + 1) // 2, sigma=0.03)
+    pos, st, rad = p.pos[:, :n].copy(), p.str[:, :n].copy(), p.rad[:n].copy()
+    tp = pos[:, ::3].copy()
+    if what.startswith("strength"):
+        st[0, 5] = float(what.split()[1])
+    elif what == "radius inf":
+        rad[5] = np.inf
+    else:
+        pos[0, 5] = 3e19
+    for t, tr in ((pos, rad), (tp, None)):
+        ns = n if tr is not None else 6 * n
+        s = (pos, st, rad) if tr is not None else tuple(np.concatenate([a] * 6, -1) for a in (pos, st / 6, rad))
+        v, g = infl.p2p(core, *s, t, tr, grads, "comp")
+        w, h = infl.p2p(core, *s, t, tr, grads, "comp", method="direct", tile=256, tpt=1)
+        for a, b in [(v, w)] + ([(g, h)] if grads else []):
+            fa, fb = np.isfinite(a), np.isfinite(b)
+            assert np.array_equal(fa, fb), (what, ns, fa.mean(1), fb.mean(1))
+            rows = fb.all(1)
+            if rows.any():
+                assert rel_errors(a[rows], b[rows])[0] <= 4e-6
+
+
+@pytest.mark.parametrize("bad", [np.inf, np.nan])
+def test_panel_strengths_that_are_no_numbers(infl, bad):
+    """the same of a panel's strength by both rules and of a particle's on panels"""
+    from omega3d_amd import _lib
+    pan, D = scenes.icosphere_panels(levels=3), _lib.DeviceArray.from_host
+    ts = pan.ts.astype(np.float32).copy()
+    ts[1, 7] = bad
+    tp = scenes.shell_points(3000, 1.02, 3.0, seed=4).astype(np.float32)
+    nodes, idx, ar = D(pan.nodes.astype(np.float32)), D(pan.idx.astype(np.uint32)), D(pan.area.astype(np.float32))
+    dts, dtp = D(ts), D(tp)
+    p, q = _lib.Panels(), _lib.Points()
+    p.np, p.nn, p.idx, p.area, q.n = pan.np, pan.nodes.shape[1], idx.ptr, ar.ptr, tp.shape[1]
+    out = _lib.DeviceArray((12, q.n))
+    for d in range(3):
+        p.x[d], p.ts[d], q.x[d], q.u[d] = nodes.row(d), dts.row(d), dtp.row(d), out.row(d)
+    for k in range(9):
+        q.ug[k] = out.row(3 + k)
+    for method in ("auto", "gauss7"):
+        res = []
+        for tile in (0, 128):
+            out.zero()
+            o = _lib.make_opts("rm", True, "comp", method=method, tile=tile)
+            _lib.check(_lib.lib.o3d_panels_affect_points_dev(C.byref(p), C.byref(q), C.byref(o), None))
+            res.append(np.isfinite(out.to_host()))
+        assert np.array_equal(*res), (method, [r.mean(1) for r in res])
+    st = np.full((3, 40000), 1e-5, np.float32)
+    st[1, 7] = bad
+    sp = D(scenes.shell_points(40000, 1.05, 3.0, seed=5).astype(np.float32))
+    dst = D(st)
+    q.n = 40000
+    for d in range(3):
+        q.x[d], q.s[d] = sp.row(d), dst.row(d)
+    few = scenes.icosphere_panels(levels=2)
+    nodes, idx, ar = D(few.nodes.astype(np.float32)), D(few.idx.astype(np.uint32)), D(few.area.astype(np.float32))
+    p.np, p.nn, p.idx, p.area = few.np, few.nodes.shape[1], idx.ptr, ar.ptr
+    for d in range(3):
+        p.x[d] = nodes.row(d)
+    vel = _lib.DeviceArray((3, few.np))
+    pv = (C.c_void_p * 3)(*[vel.row(d) for d in range(3)])
+    res = []
+    for tile in (0, 256):
+        vel.zero()
+        o = _lib.make_opts("rm", False, "comp", tile=tile)
+        _lib.check(_lib.lib.o3d_points_affect_panels_dev(C.byref(q), C.byref(p), pv, C.byref(o), None))
+        res.append(np.isfinite(vel.to_host()))
+    assert np.array_equal(*res), [r.mean(1) for r in res]
