@@ -176,3 +176,32 @@ def test_panel_strengths_that_are_no_numbers(infl, bad):
         _lib.check(_lib.lib.o3d_points_affect_panels_dev(C.byref(q), C.byref(p), pv, C.byref(o), None))
         res.append(np.isfinite(vel.to_host()))
     assert np.array_equal(*res), [r.mean(1) for r in res]
+
+
+def _far_fraction(pos):
+    """share of the pairs that one factored RM evaluation of particles on themselves takes far"""
+    from omega3d_amd import _lib
+    n, D = pos.shape[1], _lib.DeviceArray.from_host
+    x, s, r, out = D(pos.astype(np.float32)), D(np.full((3, n), 1e-3, np.float32)), D(np.full(n, 0.02, np.float32)), _lib.DeviceArray((12, n))
+    q = _lib.Points()
+    q.n, q.r = n, r.ptr
+    for d in range(3):
+        q.x[d], q.s[d], q.u[d] = x.row(d), s.row(d), out.row(d)
+    for k in range(9):
+        q.ug[k] = out.row(3 + k)
+    prof, o = _lib.FactoredProfile(), _lib.make_opts("rm", True, "comp", method="factored")
+    _lib.check(_lib.lib.o3d_factored_profile_dev(C.byref(q), C.byref(q), C.byref(o), C.byref(prof)))
+    return prof.far_tile_fraction
+
+
+@pytest.mark.parametrize("share,far", [(1e-4, 100), (1e-3, 1000), (0.05, 300)])
+def test_few_particles_far_away_leave_the_order(infl, share, far):
+    """a few particles many radii away widen the box, not the blocks of the rest: at most 5% of
+    the pairs less are far, beside those of blocks that a stray particle is in"""
+    p = scenes.colliding_rings(30000)
+    pos, rng = p.pos.copy(), np.random.default_rng(3)
+    base, m = _far_fraction(pos), int(share * p.n)
+    pos[:, rng.choice(p.n, m, replace=False)] = far * rng.normal(size=(3, m))
+    got = _far_fraction(pos)
+    print(share, far, base, got)
+    assert got >= base - 0.05 - 2 * share
