@@ -1510,11 +1510,13 @@ static __global__ void k_ff_zero_u64(unsigned long long* p) {
 
 // ---- host side shared by the factored calls ----------------------------------------
 
-// Key bits, the set's bit included, of n points in all: up to 1,048,576 points 24, which sort
+// Key bits, the set's bit included, of n points in all: up to 131,072 points 24, which sort
 // in three passes (2^8 cells per axis, or one bit less: a block of 256 is many cells even in
-// a ring), then all 30 or 31 in four.  545,000 points of two sets 3,731 and 3,699 us; two rings of
-// 262,144, whose cells hold two points, 23.2 ms both
-inline int key_bits(int64_t n, bool two_sets) { return n <= 1048576 ? 24 : two_sets ? 31 : 30; }
+// a ring), then all 30 or 31 in four, which collections of parts far apart need.  With 24 and
+// 30 bits: two RM rings of 150,000 each 300 radii apart 49.0 and 30.2 ms, of 50,000 5.5 and
+// 3.7; near each other 28.4 and 28.5, 3.74 and 3.77; 165,540 points of two sets 1,766 and
+// 1,781 us, 544,768 4.51 and 4.54 ms; 30,000 EXP particles 693 and 712 us
+inline int key_bits(int64_t n, bool two_sets) { return n <= 131072 ? 24 : two_sets ? 31 : 30; }
 
 // sequential sub-allocation of a workspace, 256-byte aligned
 struct Carve {

@@ -205,3 +205,23 @@ def test_few_particles_far_away_leave_the_order(infl, share, far):
     got = _far_fraction(pos)
     print(share, far, base, got)
     assert got >= base - 0.05 - 2 * share
+
+
+def test_rings_far_apart_keep_their_order(infl):
+    """two rings 300 radii apart, a few cells of the grid across each: the pairs that the
+    far field takes are at least those of blocks cut from a Hilbert order of 2^10 cells per axis"""
+    from test_panfar_gpu import _hilbert_order
+    p, q = scenes.ring(100000), scenes.ring(100000, seed=3)
+    pos = np.concatenate([p.pos, q.pos + np.float32(300) * np.array([[1], [0.3], [0.1]], np.float32)], 1).astype(np.float32)
+    n, s = pos.shape[1], pos[:, _hilbert_order(pos)].astype(float)
+    c, r = [], []
+    for i in range(0, n, 256):
+        b = s[:, i:i + 256]
+        c.append(0.5 * (b.min(1) + b.max(1)))
+        r.append(np.linalg.norm(b - c[-1][:, None], axis=0).max())
+    c, r, m = np.array(c), np.array(r), np.minimum(256, n - 256 * np.arange(len(r)))
+    gap = np.linalg.norm(c[:, None] - c[None], axis=2) - r[:, None] - r[None]
+    want = (m[:, None] * m[None] * (gap > np.maximum(r[:, None], r[None]))).sum() / float(n) ** 2
+    got = _far_fraction(pos)
+    print(got, want)
+    assert got >= want - 0.002
