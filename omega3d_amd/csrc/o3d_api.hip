@@ -278,14 +278,20 @@ int p2p_dev(const o3d_points* src, o3d_points* targ, const o3d_opts* o, hipStrea
   if (o->method == O3D_METHOD_FACTORED) return p2p_factored(src, targ, o, st);
   if (o->method == O3D_METHOD_AUTO && !tun && o->tile == 0 && o->tpt == 0 && 
       ff_auto_pays(o->core, grad, o->precision, src->n, targ->n)) {
-    // under graph capture the stream's workspace cannot grow: when it is too small
-    // for the factored method, the direct kernel (which needs none) takes the call
+    // under graph capture the stream's workspace cannot grow, and memory can be short: when
+    // the factored method's scratch cannot be had, the direct kernel (which needs little or
+    // none) takes the call
     bool ff = true;
     if (stream_capturing(st)) {
       std::lock_guard<std::mutex> lk(stream_ws_mutex());
       ff = stream_workspace_fits(st, ff_workspace_bytes(src->n, targ->n, ff_same_points(src, targ), 0, grad));
     }
-    if (ff) return p2p_factored(src, targ, o, st);
+    if (ff) {
+      const int rc = p2p_factored(src, targ, o, st);   // asks for its scratch before anything else
+      if (rc != O3D_ENOMEM) return rc;
+      clear_error();
+      (void)hipGetLastError();
+    }
   }
   return p2p_direct(src, targ, o, st, tun, nullptr, 0);
 }

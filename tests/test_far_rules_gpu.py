@@ -225,3 +225,43 @@ def test_rings_far_apart_keep_their_order(infl):
     got = _far_fraction(pos)
     print(got, want)
     assert got >= want - 0.002
+
+
+def test_auto_without_room_for_the_far_field(infl):
+    """a call whose far field would need more memory than the GPU has is the direct kernel's
+    (7e8 targets in one place: outputs of 34 GB, 290 GB of scratch), bit for bit;
+    the method asked for by name has no other way and says so"""
+    from omega3d_amd import _lib
+    n, p, D = 700_000_000, scenes.ring(8192, sigma=0.05), _lib.DeviceArray.from_host
+    x, s, r = D(p.pos), D(p.str), D(p.rad)
+    zero, out = C.c_void_p(), C.c_void_p()
+    for a, rows in ((zero, 1), (out, 12)):
+        if _lib.lib.o3d_dev_malloc(C.byref(a), 4 * n * rows):
+            pytest.skip("no room for the outputs")
+        _lib.check(_lib.lib.o3d_memset_dev(a, 0, 4 * n * rows))
+    src, t = _lib.Points(), _lib.Points()
+    src.n, src.r, t.n = p.n, r.ptr, n
+    for d in range(3):
+        src.x[d], src.s[d], t.x[d], t.u[d] = x.row(d), s.row(d), zero.value, out.value + 4 * n * d
+    for k in range(9):
+        t.ug[k] = out.value + 4 * n * (3 + k)
+    _lib.synchronize()   # the stream below does not wait for the fills
+    stream = C.c_void_p()
+    _lib.check(_lib.lib.o3d_stream_create(C.byref(stream)))
+    try:
+        o = _lib.make_opts("rm", True, "fp32", method="factored", stream=stream)
+        assert _lib.lib.o3d_points_affect_points_dev(C.byref(src), C.byref(t), C.byref(o), None) == 2
+        o = _lib.make_opts("wl", True, "comp", stream=stream)
+        _lib.check(_lib.lib.o3d_points_affect_points_dev(C.byref(src), C.byref(t), C.byref(o), None))
+        _lib.check(_lib.lib.o3d_stream_synchronize(stream))
+        got = np.empty((12, 2), np.float32)
+        for k in range(12):
+            for e, i in enumerate((0, n - 1)):
+                _lib.check(_lib.lib.o3d_memcpy_dtoh(got[k, e:].ctypes.data, out.value + 4 * (n * k + i), 4))
+    finally:
+        _lib.lib.o3d_stream_destroy(stream)
+        for a in (zero, out):
+            _lib.lib.o3d_dev_free(a)
+    v, g = infl.p2p("wl", p.pos, p.str, p.rad, np.zeros((3, 1)), None, True, "comp", method="direct", tile=256, tpt=1)
+    for e in (0, 1):
+        assert np.array_equal(got[:3, e:e + 1], v) and np.array_equal(got[3:, e:e + 1], g)
