@@ -373,7 +373,7 @@ bool ff_auto_pays(int core, bool grad, int prec, int64_t ns, int64_t nt) {
   if (ns < 8192 || nt < 8192 || ns > INT_MAX || nt > INT_MAX) return false;
   const double least = core == CORE_EXP ? (grad ? 6.0e8 : 1.0e9) : core == CORE_RM ? (grad ? 9.0e8 : 2.2e9)
                                                                                  : (grad ? 2.0e9 : 3.0e9);
-  return (double)ns * (double)nt >= (nt < FF_FEW_TARGETS && !(core == CORE_RM && grad) ? 1.75 * least : least) && ns + nt <= INT_MAX;
+  return (double)ns * (double)nt >= (nt < FF_FEW_TARGETS && !(core == CORE_RM && grad) ? 1.75 * least : least);
 }
 
 namespace {

@@ -185,7 +185,9 @@ size_t radix_tmp_bytes(int64_t n) {
 
 int radix_sort_pairs(unsigned* ka, int* va, unsigned* kb, int* vb, int64_t n, int bits, void* tmp, hipStream_t st,
                      unsigned** keys, int** vals) {
-  if (n < 0 || n > INT32_MAX || bits < 1 || bits > 32 || !tmp)
+  // places are 32 bits; the values are the caller's (two sets sorted together keep their own
+  // indices, each below INT32_MAX)
+  if (n < 0 || n > UINT32_MAX || bits < 1 || bits > 32 || !tmp)
     return fail(O3D_EINVAL, "radix sort: n %lld, bits %d", (long long)n, bits);
   unsigned* kin = ka;
   int* vin = va;

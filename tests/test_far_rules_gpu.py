@@ -265,3 +265,47 @@ def test_auto_without_room_for_the_far_field(infl):
     v, g = infl.p2p("wl", p.pos, p.str, p.rad, np.zeros((3, 1)), None, True, "comp", method="direct", tile=256, tpt=1)
     for e in (0, 1):
         assert np.array_equal(got[:3, e:e + 1], v) and np.array_equal(got[3:, e:e + 1], g)
+
+
+def test_factored_counts_whose_sum_passes_the_int_range(infl):
+    """FACTORED takes up to INT_MAX sources and targets each, also where both together are more
+    (one sort orders both): sources and targets in one place, whose gradient is that of the
+    summed strengths, N K(0) alpha with RM's K(0) = 1 / sigma^3, within the compensated bar"""
+    from omega3d_amd import _lib
+    ns, nt = 2**31 - 601, 1000
+    bufs, fill = [], (0, 0x3d, 0x2e)   # places 0, radii 0.0462, strengths 4e-11
+    out, D = _lib.DeviceArray.from_host(np.zeros((12, nt), np.float32)), None
+    sigma, alpha = (float(np.frombuffer(bytes([b] * 4), np.float32)[0]) for b in fill[1:])
+    try:
+        for b in fill:
+            p = C.c_void_p()
+            if _lib.lib.o3d_dev_malloc(C.byref(p), 4 * ns):
+                pytest.skip("no room for the sources")
+            bufs.append(p)
+            _lib.check(_lib.lib.o3d_memset_dev(p, b, 4 * ns))
+        _lib.synchronize()
+        s, t = _lib.Points(), _lib.Points()
+        s.n, s.r, t.n = ns, bufs[1].value, nt
+        for d in range(3):
+            s.x[d], s.s[d], t.x[d], t.u[d] = bufs[0].value, bufs[2].value, bufs[0].value, out.row(d)
+        for k in range(9):
+            t.ug[k] = out.row(3 + k)
+        stream = C.c_void_p()
+        _lib.check(_lib.lib.o3d_stream_create(C.byref(stream)))
+        try:
+            o = _lib.make_opts("rm", True, "comp", method="factored", stream=stream)
+            rc = _lib.lib.o3d_points_affect_points_dev(C.byref(s), C.byref(t), C.byref(o), None)
+            if rc == 2:
+                pytest.skip("no room for the scratch")
+            _lib.check(rc)
+            _lib.check(_lib.lib.o3d_stream_synchronize(stream))
+        finally:
+            _lib.lib.o3d_stream_destroy(stream)
+        got = out.to_host().astype(np.float64)
+    finally:
+        for p in bufs:
+            _lib.lib.o3d_dev_free(p)
+    W = ns * alpha / sigma ** 3
+    want = np.array([0, W, -W, -W, 0, W, W, -W, 0])[:, None]   # skew of (W, W, W)
+    assert not got[:3].any()
+    assert np.abs(got[3:] - want).max() <= 2e-6 * W
