@@ -586,16 +586,30 @@ int run_points(const PanArgs& p, int prec, void* ws, hipStream_t st) {
 // and 0.89 ms; 3,600 on 262,144 1.30 and 1.11, 5,120 1.89 and 1.33.  7-point rule: 960
 // panels on 1,024 points 511 and 212 us, 1,280 on 131,072 1.45 and 1.03 ms (velocity alone
 // 0.87 and 0.77); 640 panels on 65,536 520 and 498 us (311 and 429), 320 on 524,288 points
-// 4.86 and 2.57 ms.  Particles on panels: 20 panels and 8,192 particles 751 and 309 us, 320
-// and 16,384 257 and 292, 320 and 32,768 447 and 351, 20,480 and 180,000 1.85 and 1.63 ms,
-// 5,120 and 262,144 0.85 and 1.14, 524,288 2.43 and 1.89; 1,280 and 400,000 2.42 and 1.37,
-// 2,560 and 400,000 0.76 and 1.05.  A call that names its method or a tile is the direct
-// kernels'.
+// 4.86 and 2.57 ms.  Both rules gain alike in plain FP32
+// (5,120 panels on 100,000 points 848 and 506 us, 7-point rule 3,426 and 2,077), with errors
+// against FP64 that are no larger (7.1e-7 and 3.6e-7).
+//
+// Particles on panels: the direct kernel keeps eight near particles per panel and slice and
+// scans a slice with more again, so the particles per panel decide for few panels, and the
+// pairs for many; how near the particles lie decides as much and is not known here.  us direct
+// and here of whole spheres, particles in the shells 1.01-2.5, 1.005-1.1, 1.02-1.5 and 1.5-4:
+//   320 panels,  32,768 particles    192  214     686   359     457   254      80  184
+//   320         100,000              488  359   2,002   652   1,300   464     185  238
+//   1,280       180,000              409  463   1,781 1,058     617   626     407  350
+//   1,280       262,144              425  585   2,765 1,372   1,604   821     398  409
+//   1,280       400,000              626  729   4,280 1,992   2,438 1,112     583  508
+//   5,120       262,144              760  759   3,822 1,435     847   954     769  620
+//   5,120       400,000                         6,489 1,944   1,470 1,297   1,096  820
+//   20,480       65,536              715  680     783   842     731   751     695  551
+//   20,480      131,072            1,327  999   1,660 1,307   1,371 1,182   1,318  888
+// With 8,192 particles 20 panels take 183 and 160, 80 panels 189 and 171; from 512 panels on
+// the launches are worth 200 particles per panel instead of 100 (640 and 131,072 270 354,
+// 1,239 625, 410 456, 275 278).  A call that names its method or a tile is the direct kernels'.
 bool panfar_pays(int rule, int64_t units, int64_t nt, int method, int tile, int prec) {
   if (method != O3D_METHOD_AUTO || tile > 0 || prec == PREC_FP64 || units > (1 << 26) || nt > (1 << 26)) return false;
   if (rule == PANFAR_PARTICLES) {
-    if (nt < 512) return units >= 8192 && units >= 100 * nt;
-    return units * nt >= 2500000000LL || (units >= 400000 && nt <= 2048);
+    return units >= 8192 && (units >= (nt < 512 ? 100 : 200) * nt || units * nt >= 1800000000LL);
   }
   if (nt < 32) return false;
   if (rule == PANFAR_POINTS7) return units >= 1024 || units * nt >= 160000000LL;

@@ -309,3 +309,26 @@ def test_factored_counts_whose_sum_passes_the_int_range(infl):
     want = np.array([0, W, -W, -W, 0, W, W, -W, 0])[:, None]   # skew of (W, W, W)
     assert not got[:3].any()
     assert np.abs(got[3:] - want).max() <= 2e-6 * W
+
+
+@pytest.mark.parametrize("levels,np_,below,beyond", [(3, 1280, 255999, 256001), (3, 640, 127999, 128001), (4, 5120, 351562, 351563)])
+def test_line_of_particles_on_panels(infl, levels, np_, below, beyond):
+    """200 particles per panel or 1.8e9 pairs: the direct kernel's bits below, others beyond"""
+    from omega3d_amd import _lib
+    pan, D = scenes.icosphere_panels(levels=levels), _lib.DeviceArray.from_host
+    sp, st = D(scenes.shell_points(beyond, 1.02, 1.5, seed=4).astype(np.float32)), D(np.full((3, beyond), 1e-5, np.float32))
+    nodes, idx, ar = D(pan.nodes.astype(np.float32)), D(pan.idx.astype(np.uint32)), D(pan.area.astype(np.float32))
+    q, p, vel = _lib.Points(), _lib.Panels(), _lib.DeviceArray((3, np_))
+    p.np, p.nn, p.idx, p.area = np_, pan.nodes.shape[1], idx.ptr, ar.ptr
+    for d in range(3):
+        p.x[d], q.x[d], q.s[d] = nodes.row(d), sp.row(d), st.row(d)
+    pv = (C.c_void_p * 3)(*[vel.row(d) for d in range(3)])
+    for n in (below, beyond):
+        q.n, res = n, []
+        for tile in (0, 256):
+            vel.zero()
+            o = _lib.make_opts("rm", False, "comp", tile=tile)
+            _lib.check(_lib.lib.o3d_points_affect_panels_dev(C.byref(q), C.byref(p), pv, C.byref(o), None))
+            res.append(vel.to_host())
+        assert np.array_equal(*res) == (n == below)
+        assert rel_errors(*res)[0] <= 4e-6
