@@ -65,10 +65,10 @@ enum o3d_self { O3D_SELF_INCLUDE = 0, O3D_SELF_EXCLUDE = 1 };
  *             cores; other pairs as in DIRECT.  RM and EXP cores, velocity and
  *             gradient, FP32 or compensated precision; tile 64, 128 or 256.
  *   AUTO:     FACTORED where it applies with tile and tpt left at 0 and enough pairs
- *             (both counts >= 8192 and, with gradient, about 24,500 particles on
- *             themselves for EXP and 30,000 for RM; 1.75 times the pairs for fewer than
- *             16,384 targets but RM's), DIRECT otherwise.  In compensated
- *             precision AUTO takes the far tiles of the other cores (WL, V2: about
+ *             (compensated: both counts >= 8192 and, with gradient, about 24,500
+ *             particles on themselves for EXP and 30,000 for RM; 1.75 times the pairs for
+ *             fewer than 16,384 targets but RM's.  FP32: both counts >= 65,536) and memory
+ *             for its scratch, DIRECT otherwise.  In compensated precision AUTO takes the far tiles of the other cores (WL, V2: about
  *             45,000) and of velocities alone (EXP 32,000, RM 47,000, WL and V2 55,000)
  *             to the matrix cores as well.
  * For panel sources (o3d_panels_affect_points[_dev]) the field selects the rule:

@@ -368,9 +368,16 @@ bool ff_supported(int core, bool grad, int prec) {
 // and 951, 400,000 1,386 and 1,391, EXP 120,000 520 and 581, 240,000 1,038 and 998.  RM with
 // gradient keeps its line there: 110,000 on 9,000 720 and 774 from one ring, 722 and 685 from two
 constexpr int64_t FF_FEW_TARGETS = 16384;
+// Plain FP32 sums from here on only: below, the far field is faster (RM 40,000 particles 1,162
+// and 796 us, EXP 28,672 1,227 and 584), but its near tiles are one FP32 sum where the direct
+// kernel adds slices: rms error of the velocity on one ring RM 30,100 0.99e-7 and 1.7e-7, 49,152
+// 1.6e-7 and 2.1e-7, 65,000 2.2e-7 and 2.3e-7; EXP 28,672 1.0e-7 and 2.0e-7; 40,000 EXP
+// particles on as many points in a box five times as wide 1.8e-7 and 3.0e-7
+constexpr int64_t FF_FP32_MIN = 65536;
 bool ff_auto_pays(int core, bool grad, int prec, int64_t ns, int64_t nt) {
   if (!(prec == PREC_COMP || ff_supported(core, grad, prec))) return false;
   if (ns < 8192 || nt < 8192 || ns > INT_MAX || nt > INT_MAX) return false;
+  if (prec == PREC_FP32) return ns >= FF_FP32_MIN && nt >= FF_FP32_MIN;
   const double least = core == CORE_EXP ? (grad ? 6.0e8 : 1.0e9) : core == CORE_RM ? (grad ? 9.0e8 : 2.2e9)
                                                                                  : (grad ? 2.0e9 : 3.0e9);
   return (double)ns * (double)nt >= (nt < FF_FEW_TARGETS && !(core == CORE_RM && grad) ? 1.75 * least : least);

@@ -332,3 +332,15 @@ def test_line_of_particles_on_panels(infl, levels, np_, below, beyond):
             res.append(vel.to_host())
         assert np.array_equal(*res) == (n == below)
         assert rel_errors(*res)[0] <= 4e-6
+
+
+@pytest.mark.parametrize("core,ns,nt,far", [("rm", 65535, 65535, False), ("exp", 65535, 65535, False), ("exp", 32768, 32768, False),
+                                            ("rm", 110000, 65535, False), ("exp", 65535, 70000, False),
+                                            ("rm", 65536, 65536, True), ("exp", 65536, 66000, True)])
+def test_line_of_plain_sums(infl, core, ns, nt, far):
+    """plain FP32 takes the far field from 65,536 sources and targets on: the direct bits below"""
+    p = scenes.ring(ns, seed=5)
+    t = (p.pos, p.rad) if ns == nt else (scenes.ring(nt, a=0.2, seed=6).pos, None)
+    args = (core, p.pos, p.str, p.rad, *t, True, "fp32")
+    (v, g), (w, h) = infl.p2p(*args), infl.p2p(*args, method="direct")
+    assert (np.array_equal(v, w) and np.array_equal(g, h)) != far
