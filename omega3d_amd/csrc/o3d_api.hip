@@ -147,11 +147,19 @@ hipError_t dispatch_p2p_split(int core, const P2PArgs& a, bool thick, bool grad,
 // SPLIT_WGS_PER_CU workgroups per compute unit, and a partial buffer of at most SPLIT_MAX_BYTES.
 // cap > 0 (a caller's fixed scratch of cap bytes): fewer slices when the partials
 // of the wanted slice count do not fit.  Returns the slice count (1: no split) and
-// the slice length.
+// the slice length.  Fewer than `least` sources of one tile are not worth the second launch.
 constexpr int SPLIT_WGS_PER_CU = 16;
 constexpr size_t SPLIT_MAX_BYTES = (size_t)256 << 20;
 constexpr int64_t SPLIT_SHORT = 32;
-int split_plan(int64_t nt, int64_t ns, int tile, bool grad, int prec, int64_t* slen, size_t* bytes, size_t cap) {
+// us in one pass and in slices, on themselves and on 1,000 points: RM compensated with gradient
+// 64 sources 9.0 9.1, 10.6 11.4, 96 11.8 9.7, 13.4 11.5; plain FP32 96 11.3 10.4, 12.9 12.5, 97
+// (one slice more) 11.5 13.0, 13.0 13.2, 112 12.8 12.8, 14.4 13.3; velocities 96 7.2 7.9, 8.0
+// 8.8, 112 7.9 7.6, 8.6 8.0; WL alike.  EXP, whose sources take twice as long: with gradient
+// 40 16.3 16.8, 15.7 17.1, 48 18.4 16.8, 16.7 16.9, 56 20.5 16.7, 17.6 16.4; velocities 48
+// 14.8 13.2, 12.1 13.5, 56 16.4 13.3, 13.1 13.3
+int64_t split_least(int core) { return core == CORE_EXP ? 49 : 112; }
+int split_plan(int64_t nt, int64_t ns, int tile, bool grad, int prec, int64_t least, int64_t* slen, size_t* bytes,
+               size_t cap) {
   const int64_t nb = (nt + BLOCK - 1) / BLOCK;
   const int64_t want = (int64_t)SPLIT_WGS_PER_CU * num_cus();
   if (nb >= want) return 1;
@@ -164,7 +172,7 @@ int split_plan(int64_t nt, int64_t ns, int tile, bool grad, int prec, int64_t* s
     const int64_t fit = (int64_t)(cap / ((size_t)nt * cols));
     if (nsl > fit) nsl = fit;
   }
-  if (nsl < 2 && ns <= 32) return 1;
+  if (nsl < 2 && ns < least) return 1;
   nsl = std::max<int64_t>(nsl, 1);
   const int64_t tiles_per = (ntiles + nsl - 1) / nsl;
   *slen = tiles_per * tile;
@@ -324,8 +332,8 @@ int p2p_direct(const o3d_points* src, o3d_points* targ, const o3d_opts* o, hipSt
   // batched and served kernels share)
   int64_t slen = 0;
   size_t pbytes = 0;
-  const int nsl = auto_cfg && tpt == 1 ? split_plan(a.nt, a.ns, tile, grad, o->precision, &slen, &pbytes,
-                                                    ws ? ws_bytes : 0)
+  const int nsl = auto_cfg && tpt == 1 ? split_plan(a.nt, a.ns, tile, grad, o->precision, split_least(o->core), &slen,
+                                                    &pbytes, ws ? ws_bytes : 0)
                                        : 1;
   if (nsl > 1) {
     void* part = ws;

@@ -344,3 +344,14 @@ def test_line_of_plain_sums(infl, core, ns, nt, far):
     args = (core, p.pos, p.str, p.rad, *t, True, "fp32")
     (v, g), (w, h) = infl.p2p(*args), infl.p2p(*args, method="direct")
     assert (np.array_equal(v, w) and np.array_equal(g, h)) != far
+
+
+@pytest.mark.parametrize("core,ns", [("rm", 33), ("rm", 64), ("rm", 111), ("wl", 97), ("v2", 80), ("exp", 33), ("exp", 48)])
+def test_fewest_sources_take_one_pass(infl, core, ns):
+    """so few sources are not cut: the bits of the one-pass kernel"""
+    p = scenes.ring(ns, seed=7)
+    t = (2.4 * np.random.default_rng(9).random((3, 1000)) - 1.2).astype(np.float32)
+    for grads, prec in ((True, "comp"), (False, "comp"), (True, "fp32")):
+        a = infl.p2p(core, p.pos, p.str, p.rad, t, None, grads, prec)
+        b = infl.p2p(core, p.pos, p.str, p.rad, t, None, grads, prec, tile=256, tpt=1)
+        assert np.array_equal(a[0], b[0]) and (not grads or np.array_equal(a[1], b[1]))
