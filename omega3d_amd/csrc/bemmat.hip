@@ -477,7 +477,10 @@ __device__ __forceinline__ void bm_level2(const float* l1, int k, int c2, float*
   bm_child(t1v, c2 & 3, t2v);
 }
 
-template <int MAXLEV>
+// PAIRS 1: a pair per wave, in its first 16 lanes at level 1, where a wave's pairs one after
+// another are what the call waits for: few pairs (20 panels, maxlev 3, 400 pairs: 94 us with
+// four and 74 with one), and maxlev 4, whose walks differ most (1,280 panels 2.33 and 1.58 ms)
+template <int MAXLEV, int PAIRS>
 __global__ __launch_bounds__(BLOCK) void k_bm_near(BmNearArgs a) {
   // each wave's 16 level-1 triangle pairs, shared with its items through LDS, and the open
   // level-2 pairs; a wave touches only its own, and LDS operations of one wave complete in order
@@ -492,10 +495,10 @@ __global__ __launch_bounds__(BLOCK) void k_bm_near(BmNearArgs a) {
   const int nunk = a.nunk;
   constexpr int maxlev = MAXLEV;
   const int64_t R = (int64_t)nunk * a.nt;
-  for (int64_t e = wave; 4 * e < listed; e += nwaves) {
-    const int64_t li = 4 * e + (lane >> 4);
-    const bool has = li < listed;
-    const uint2 p = a.list[has ? li : 4 * e];
+  for (int64_t e = wave; PAIRS * e < listed; e += nwaves) {
+    const int64_t li = PAIRS * e + (lane >> 4);
+    const bool has = (lane >> 4) < PAIRS && li < listed;
+    const uint2 p = a.list[has ? li : PAIRS * e];
     const int64_t i = p.x, j = p.y;
     const float4* sr = a.srec + j * BM_F4;
     const float4* tr = a.trec + i * BM_F4;
@@ -527,7 +530,7 @@ __global__ __launch_bounds__(BLOCK) void k_bm_near(BmNearArgs a) {
 #pragma unroll
       for (int d = 0; d < 3; ++d) G[d] = quarter_sum(G[d]);
       const unsigned long long m1 = __builtin_amdgcn_ballot_w64(open1);
-      for (int q = 0; q < 4; ++q) {
+      for (int q = 0; q < PAIRS; ++q) {
         const unsigned mq = (unsigned)(m1 >> (16 * q)) & 0xffffu;
         if (mq == 0u) continue;
         const float tq = __shfl(t4, 16 * q, 64);
@@ -740,14 +743,16 @@ int bem_matrix_dev(const o3d_panels* src, const o3d_panels* targ, int32_t nunk, 
   if (prof) HIPCHK(hipEventRecord(ev[2], st));
   if (nnear > 0 && maxlev > 0) {
     BmNearArgs na{srec, trec, list, cnt, nnear, nt, nunk, maxlev, coeffs};
-    const int64_t pairs_per_block = 4 * (BLOCK / 64);
+    const bool one = maxlev == 4 || (int64_t)nnear <= 16LL * num_cus();   // up to four waves per SIMD
+    const int64_t pairs_per_block = (one ? 1 : 4) * (BLOCK / 64);
     int64_t nb = ((int64_t)nnear + pairs_per_block - 1) / pairs_per_block;
     const int64_t maxb = 64LL * num_cus();
     if (nb > maxb) nb = maxb;
-    if (maxlev == 1) hipLaunchKernelGGL(k_bm_near<1>, dim3((unsigned)nb), dim3(BLOCK), 0, st, na);
-    else if (maxlev == 2) hipLaunchKernelGGL(k_bm_near<2>, dim3((unsigned)nb), dim3(BLOCK), 0, st, na);
-    else if (maxlev == 3) hipLaunchKernelGGL(k_bm_near<3>, dim3((unsigned)nb), dim3(BLOCK), 0, st, na);
-    else hipLaunchKernelGGL(k_bm_near<4>, dim3((unsigned)nb), dim3(BLOCK), 0, st, na);
+    const auto near = maxlev == 1   ? (one ? k_bm_near<1, 1> : k_bm_near<1, 4>)
+                      : maxlev == 2 ? (one ? k_bm_near<2, 1> : k_bm_near<2, 4>)
+                      : maxlev == 3 ? (one ? k_bm_near<3, 1> : k_bm_near<3, 4>)
+                                    : k_bm_near<4, 1>;
+    hipLaunchKernelGGL(near, dim3((unsigned)nb), dim3(BLOCK), 0, st, na);
     HIPCHK(hipGetLastError());
   }
   if (prof) {
