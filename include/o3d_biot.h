@@ -68,9 +68,9 @@ enum o3d_self { O3D_SELF_INCLUDE = 0, O3D_SELF_EXCLUDE = 1 };
  *             (compensated: both counts >= 8192 and, with gradient, about 24,500
  *             particles on themselves for EXP and 30,000 for RM; 1.75 times the pairs for
  *             fewer than 16,384 targets but RM's.  FP32: both counts >= 65,536) and memory
- *             for its scratch, DIRECT otherwise.  In compensated precision AUTO takes the far tiles of the other cores (WL, V2: about
- *             45,000) and of velocities alone (EXP 32,000, RM 47,000, WL and V2 55,000)
- *             to the matrix cores as well.
+ *             for its scratch, DIRECT otherwise.  In compensated precision AUTO takes the
+ *             far tiles of the other cores (WL, V2: about 45,000) and of velocities alone
+ *             (EXP 32,000, RM 47,000, WL and V2 55,000) to the matrix cores as well.
  * For panel sources (o3d_panels_affect_points[_dev]) the field selects the rule:
  *   AUTO / DIRECT:      the reference's recursive centroid rule (Kernels.h:1028-1211);
  *             AUTO takes the separated pairs of large calls with tile 0, of both rules

@@ -355,3 +355,20 @@ def test_fewest_sources_take_one_pass(infl, core, ns):
         a = infl.p2p(core, p.pos, p.str, p.rad, t, None, grads, prec)
         b = infl.p2p(core, p.pos, p.str, p.rad, t, None, grads, prec, tile=256, tpt=1)
         assert np.array_equal(a[0], b[0]) and (not grads or np.array_equal(a[1], b[1]))
+
+
+@pytest.mark.parametrize("core,grads,below,nt", [("exp", True, 24494, 0), ("rm", True, 29999, 0), ("wl", True, 44721, 0),
+                                                 ("v2", True, 44721, 0), ("exp", False, 31622, 0), ("rm", False, 46904, 0),
+                                                 ("wl", False, 54772, 0), ("v2", False, 54772, 0), ("exp", True, 104999, 10000),
+                                                 ("wl", True, 213636, 16383), ("rm", False, 320833, 12000),
+                                                 ("rm", True, 109863, 8192), ("exp", True, 73242, 8191)])
+def test_both_sides_of_autos_lines(infl, core, grads, below, nt):
+    """compensated calls a particle below AUTO's line have the direct kernel's bits, a particle
+    beyond it others (nt 0: on themselves; fewer than 8,192 targets are direct at any count)"""
+    for ns in (below, below + 1):
+        p = scenes.ring(ns, seed=12)
+        t = (p.pos, p.rad) if nt == 0 else (scenes.ring(nt, a=0.3, seed=13).pos, None)
+        args = (core, p.pos, p.str, p.rad, *t, grads, "comp")
+        (v, g), (w, h) = infl.p2p(*args), infl.p2p(*args, method="direct")
+        same = np.array_equal(v, w) and (not grads or np.array_equal(g, h))
+        assert same == (ns == below or nt == 8191)
