@@ -56,8 +56,8 @@ struct Layout {
   unsigned *k_in, *k_out, *mask, *ctr;
   int *i_in, *i_out, *tinv, *nn, *items, *ioff, *mfold;
   void* tmp;
-  float4 *sp, *sa, *tq, *tsph, *bsph;
-  float *box, *tcs, *tcm, *tam, *tsg, *bcs, *bcm;
+  float4 *sp, *sa, *tq, *tsph, *tlim, *bsph, *blim;
+  float* box;
   double *farv, *part;
   unsigned long long* npair;
   size_t bytes;
@@ -70,7 +70,7 @@ Layout layout(char* base, int64_t ns, int64_t nt, bool same, int T, size_t tmp_b
   Carve cv{base};
   Layout L{};
   const int64_t n = same ? ns : ns + nt;
-  L.box = cv.take<float>(6 * FF_BOX_GRID);
+  L.box = cv.take<float>(FF_BOX_FLOATS);
   L.k_in = cv.take<unsigned>(n);
   L.k_out = cv.take<unsigned>(n);
   L.i_in = cv.take<int>(n);
@@ -81,13 +81,9 @@ Layout layout(char* base, int64_t ns, int64_t nt, bool same, int T, size_t tmp_b
   L.sa = cv.take<float4>((size_t)ntiles * T);
   L.tq = cv.take<float4>(nt);
   L.tsph = cv.take<float4>(ntiles);
-  L.tcs = cv.take<float>(ntiles);
-  L.tcm = cv.take<float>(ntiles);
-  L.tam = cv.take<float>(ntiles);
-  L.tsg = cv.take<float>(ntiles);
+  L.tlim = cv.take<float4>(ntiles);
   L.bsph = cv.take<float4>(nb);
-  L.bcs = cv.take<float>(nb);
-  L.bcm = cv.take<float>(nb);
+  L.blim = cv.take<float4>(nb);
   L.mask = cv.take<unsigned>((size_t)(nb * mwords));
   L.farv = cv.take<double>((size_t)nout * far_slices(nb, ntiles, nout == 3 ? 3 : 2, num_cus()) * nt);
   L.npair = cv.take<unsigned long long>(1);
@@ -144,7 +140,7 @@ int run(const o3d_points* src, o3d_points* targ, bool self_excl, int T, hipStrea
   int rc = factored_order(sets, L.box, L.k_in, L.i_in, L.k_out, L.i_out, L.tmp, st, &perm);
   if (rc != O3D_OK) return rc;
   const int *sperm = perm, *tperm = same ? perm : perm + ns;
-  const FFBounds tb{L.tsph, L.tcs, L.tcm, L.tam, L.tsg}, bb{L.bsph, L.bcs, L.bcm, nullptr, nullptr};
+  const FFBounds tb{L.tsph, L.tlim}, bb{L.bsph, L.blim};
   hipLaunchKernelGGL((k_ff_rows<CORE, THICK>), dim3((unsigned)(ntiles + nb)), dim3(256), 0, st, sv, tv, sperm, tperm, ns,
                      nt, T, ntiles, L.sp, L.sa, L.tq, tb, bb, L.nn, nt >= FF_ROWS_MIN ? L.tinv : nullptr);
   hipLaunchKernelGGL((k_ff_classify<CORE>), dim3(grid_of(nb * mwords, 256)), dim3(256), 0, st, bb, nb, tb, ntiles, mwords,
@@ -155,8 +151,8 @@ int run(const o3d_points* src, o3d_points* targ, bool self_excl, int T, hipStrea
 
   FFArgs a{};
   a.sp = L.sp; a.sa = L.sa; a.tq = L.tq; a.tperm = tperm; a.tinv = L.tinv; a.rows = nt >= FF_ROWS_MIN;
-  a.tsph = L.tsph; a.tcs = L.tcs; a.tcm = L.tcm; a.tam = L.tam; a.bsph = L.bsph; a.bcm = L.bcm;
-  a.mask = L.mask; a.farv = L.farv; a.tsg = L.tsg;
+  a.tsph = L.tsph; a.tlim = L.tlim; a.bsph = L.bsph; a.blim = L.blim;
+  a.mask = L.mask; a.farv = L.farv;
   a.nn = L.nn; a.items = L.items; a.ioff = L.ioff; a.mfold = L.mfold; a.ctr = L.ctr; a.part = L.part;
   a.s = sv; a.t = tv;
   a.ns = ns; a.nt = nt;
@@ -226,8 +222,9 @@ int factored_order(const FFSets& s, float* box, unsigned* ka, int* va, unsigned*
   const int64_t n = s.n[0] + s.n[1];
   const int bits = key_bits(n, s.n[1] > 0);
   const unsigned g = std::min<unsigned>(FF_BOX_GRID, grid_of(n, 1024));
-  hipLaunchKernelGGL(k_ff_box, dim3(g), dim3(256), 0, st, s, box);
-  hipLaunchKernelGGL(k_ff_hkeys, dim3(std::min(1024u, grid_of(n, 256))), dim3(256), 0, st, s, box, (int)g,
+  float* where = box + 12 * FF_BOX_GRID;
+  hipLaunchKernelGGL(k_ff_box, dim3(g + 2), dim3(256), 0, st, s, box, (int)g, where);
+  hipLaunchKernelGGL(k_ff_hkeys, dim3(std::min(1024u, grid_of(n, 256))), dim3(256), 0, st, s, box, (int)g, where,
                      s.n[1] > 0 ? bits - 1 : bits, ka, va);
   HIPCHK(hipGetLastError());
   unsigned* keys = nullptr;

@@ -119,15 +119,12 @@ struct FFArgs {
   const float4* tq;    // sorted targets {x, y, z, core_term or 0 for point targets}
   const int* tperm;    // sorted target -> original target index
   const float4* tsph;  // per source tile: bounding sphere {cx, cy, cz, r}
-  const float* tcs;    // per source tile: largest core term
-  const float* tcm;    // and the least
-  const float* tam;    // per source tile: largest |alpha| and |q|
+  const float4* tlim;  // per source tile and target block: FFBounds::lim
   const float4* bsph;  // per target block: bounding sphere
-  const float* bcm;    // per target block: least core term
+  const float4* blim;
   const unsigned* mask;  // far bit per (block, tile), mwords words per block
   double* farv;        // per slice and target, sorted: far-field velocity and gradient, 12 (3) (FFSum)
   const int* tinv;     // original target -> sorted target
-  const float* tsg;    // per source tile: sign of its first nonzero strength, 0: none
   int32_t nslice;      // slices of the far field: slice y takes tiles [y * tslice, (y + 1) * tslice)
   int32_t tslice;
   const int* nn;       // near tiles per block
@@ -140,7 +137,7 @@ struct FFArgs {
   SrcView s;           // original sources (self-pair exclusion)
   TgtView t;           // original targets (outputs, accumulated)
   int64_t ns, nt;
-  int32_t tile;        // sources per tile (multiple of 32, <= 512)
+  int32_t tile;        // sources per tile: 64, 128 or 256
   int32_t mwords;
   int32_t ntiles;
   int32_t self_excl;
@@ -322,102 +319,121 @@ __device__ __forceinline__ void wg_max_n(float* v) {
   for (int k = 0; k < N; ++k) v[k] = fmaxf(fmaxf(red[0][k], red[1][k]), fmaxf(red[2][k], red[3][k]));
 }
 
-// each workgroup's box {-lo, hi} over its strided share of both sets
-constexpr int FF_BOX_GRID = 256;
-static __global__ __launch_bounds__(256) void k_ff_box(FFSets s, float* part) {
-  float v[6];
+// middle one of a wave's values (no NaN), in every lane: the largest that at most half
+// are below
+__device__ __forceinline__ float wave_median(float x) {
+  int below = 0;
 #pragma unroll
-  for (int d = 0; d < 6; ++d) v[d] = -__builtin_huge_valf();
+  for (int j = 0; j < 64; ++j) below += __uint_as_float(__builtin_amdgcn_readlane(__float_as_uint(x), j)) < x;
+  float m = below <= 32 ? x : -__builtin_huge_valf();
+#pragma unroll
+  for (int off = 32; off > 0; off >>= 1) m = fmaxf(m, __shfl_xor(m, off));
+  return m;
+}
+
+// Each workgroup's boxes {-lo, hi} of both sets over its strided share of them; and, one
+// workgroup per set beside these, where its points are: of 64 of them, per axis, the median
+// and the median distance from it, {median 3, distance 3} in `where`
+constexpr int FF_BOX_GRID = 256;
+constexpr int FF_BOX_FLOATS = 12 * FF_BOX_GRID + 12;   // boxes, then where
+static __global__ __launch_bounds__(256) void k_ff_box(FFSets s, float* part, int nparts, float* where) {
+  const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
+  if ((int)blockIdx.x >= nparts) {
+    const int set = (int)blockIdx.x - nparts;
+    if (w > 2) return;
+    float p[3] = {0.0f, 0.0f, 0.0f};
+    if (s.n[set] > 0) ff_position(s, set, s.n[set] * lane / 64, p);
+    const float x = w == 0 ? p[0] : w == 1 ? p[1] : p[2];
+    const float m = wave_median(x == x ? x : 0.0f);
+    const float r = wave_median(x == x ? fabsf(x - m) : 0.0f);
+    if (lane == 0) { where[6 * set + w] = m; where[6 * set + 3 + w] = r; }
+    return;
+  }
+  float v[12];
+#pragma unroll
+  for (int d = 0; d < 12; ++d) v[d] = -__builtin_huge_valf();
+#pragma unroll
   for (int set = 0; set < 2; ++set)
-    for (int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x; i < s.n[set]; i += (int64_t)gridDim.x * 256) {
+    for (int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x; i < s.n[set]; i += (int64_t)nparts * 256) {
       float p[3];
       ff_position(s, set, i, p);
 #pragma unroll
-      for (int d = 0; d < 3; ++d) { v[d] = fmaxf(v[d], -p[d]); v[3 + d] = fmaxf(v[3 + d], p[d]); }
+      for (int d = 0; d < 3; ++d) {
+        v[6 * set + d] = fmaxf(v[6 * set + d], -p[d]);
+        v[6 * set + 3 + d] = fmaxf(v[6 * set + 3 + d], p[d]);
+      }
     }
-  wg_max_n<6>(v);
+  wg_max_n<12>(v);
   if (threadIdx.x == 0)
 #pragma unroll
-    for (int d = 0; d < 6; ++d) part[6 * blockIdx.x + d] = v[d];
+    for (int d = 0; d < 12; ++d) part[12 * blockIdx.x + d] = v[d];
 }
 
-// middle one of a wave's values (no NaN), in every lane
-__device__ __forceinline__ float wave_median(float x) {
-  int rank = 0;
-#pragma unroll
-  for (int j = 0; j < 64; ++j) {
-    const float y = __uint_as_float(__builtin_amdgcn_readlane(__float_as_uint(x), j));
-    rank += y < x || (y == x && j < (int)(threadIdx.x & 63));
-  }
-  const uint64_t m = __builtin_amdgcn_ballot_w64(rank == 32);
-  return __shfl(x, m ? __builtin_ctzll(m) : 0);
-}
-
-// Where the box says little about where the points are (a few particles that have left, a
-// dense collection in a wide field), a grid of 2^8 or 2^10 cells per axis has the collection
-// in a few cells and its blocks in no order.  So each axis is laid out about the median of 64
-// points, linear up to twice their spread (the median distance from it, of the widest axis)
+// Where a set's box says little about where its points are (a few particles that have left,
+// a dense collection in a wide field), a grid of 2^8 or 2^10 cells per axis has the collection
+// in a few cells and its blocks in no order.  So each axis is laid out about the median,
+// linear up to twice the points' spread (the median distance from it, of the widest axis)
 // and logarithmic beyond; a box within FF_WIDE spreads, as of any collection that fills its
 // box somehow, stays linear.  Ring pairs, RM with gradient, one particle in 10,000 100 radii
 // away: of 100,000 7.2 ms without and 3.7 with (3.7 without such particles), of 300,000 63
 // and 29.6 (28.5); a tenth of 100,000 WL particles 300 radii away 9.9 and 6.2
 constexpr float FF_WIDE = 8.0f;
 struct FFAxes {
-  float mid[3], core;   // core: half the width of the linear part, 0: linear throughout
+  float mid[3], lo[3], sc;
+  float core;   // half the width of the linear part, 0: linear throughout
   __device__ __forceinline__ float at(int d, float x) const {
     if (core == 0.0f) return x;
     const float u = x - mid[d], a = fabsf(u);
     return copysignf(a <= core ? a : core * (1.0f + 0.69314718f * __builtin_amdgcn_logf(a / core)), u);
   }
+  // v: the set's box {-lo, hi}
+  __device__ __forceinline__ FFAxes(const float* v, const float* where) {
+    float far = 0.0f, ext = 0.0f;
+    core = 0.0f;
+#pragma unroll
+    for (int d = 0; d < 3; ++d) {
+      mid[d] = where[d];
+      core = fmaxf(core, 2.0f * where[3 + d]);
+      far = fmaxf(far, fmaxf(v[3 + d] - mid[d], v[d] + mid[d]));
+    }
+    if (!(far > 0.5f * FF_WIDE * core && far < __builtin_huge_valf())) core = 0.0f;
+#pragma unroll
+    for (int d = 0; d < 3; ++d) {
+      lo[d] = -at(d, -v[d]);
+      ext = fmaxf(ext, at(d, v[3 + d]) + lo[d]);
+    }
+    sc = ext > 0.0f ? 1023.0f / ext : 0.0f;
+  }
 };
 
-// the top `bits` bits of the 30-bit Hilbert keys on the common box, below the set's bit,
-// and each set's identity permutation
-static __global__ __launch_bounds__(256) void k_ff_hkeys(FFSets s, const float* part, int nparts, int bits,
-                                                  unsigned* keys, int* idx) {
-  const int64_t n = s.n[0] + s.n[1];
-  const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
-  float v[6];
+// the top `bits` bits of the 30-bit Hilbert keys, each set's on a grid of its own (they are
+// sorted apart, so nothing has to match), below the set's bit, and each set's identity
+// permutation
+static __global__ __launch_bounds__(256) void k_ff_hkeys(FFSets s, const float* part, int nparts, const float* where,
+                                                  int bits, unsigned* keys, int* idx) {
+  float v[12];
 #pragma unroll
-  for (int d = 0; d < 6; ++d) v[d] = -__builtin_huge_valf();
+  for (int d = 0; d < 12; ++d) v[d] = -__builtin_huge_valf();
   for (int k = threadIdx.x; k < nparts; k += 256)
 #pragma unroll
-    for (int d = 0; d < 6; ++d) v[d] = fmaxf(v[d], part[6 * k + d]);
-  __shared__ float spread[3][2];
-  if (w < 3) {   // axis w of the 64 points
-    const int64_t i = n * lane / 64;
-    float p[3];
-    ff_position(s, i >= s.n[0], i >= s.n[0] ? i - s.n[0] : i, p);
-    const float x = w == 0 ? p[0] : w == 1 ? p[1] : p[2];
-    const float m = wave_median(x == x ? x : 0.0f);
-    const float r = wave_median(x == x ? fabsf(x - m) : 0.0f);
-    if (lane == 0) { spread[w][0] = m; spread[w][1] = r; }
-  }
-  wg_max_n<6>(v);   // (a barrier before and after)
-  FFAxes ax;
-  float far = 0.0f;
-  ax.core = 0.0f;
+    for (int d = 0; d < 12; ++d) v[d] = fmaxf(v[d], part[12 * k + d]);
+  if (s.n[1] > 0) wg_max_n<12>(v);
+  else wg_max_n<6>(v);
 #pragma unroll
-  for (int d = 0; d < 3; ++d) {
-    ax.mid[d] = spread[d][0];
-    ax.core = fmaxf(ax.core, 2.0f * spread[d][1]);
-    far = fmaxf(far, fmaxf(v[3 + d] - ax.mid[d], v[d] + ax.mid[d]));
-  }
-  if (!(far > 0.5f * FF_WIDE * ax.core && far < __builtin_huge_valf())) ax.core = 0.0f;
+  for (int set = 0; set < 2; ++set) {
+    if (s.n[set] == 0) continue;
+    const FFAxes ax(v + 6 * set, where + 6 * set);
+    for (int64_t j = (int64_t)blockIdx.x * 256 + threadIdx.x; j < s.n[set]; j += (int64_t)gridDim.x * 256) {
+      float p[3];
+      ff_position(s, set, j, p);
+      unsigned c[3];
 #pragma unroll
-  for (int d = 0; d < 3; ++d) { v[d] = -ax.at(d, -v[d]); v[3 + d] = ax.at(d, v[3 + d]); }
-  const float ext = fmaxf(fmaxf(v[3] + v[0], v[4] + v[1]), v[5] + v[2]);
-  const float sc = ext > 0.0f ? 1023.0f / ext : 0.0f;
-  for (int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x; i < n; i += (int64_t)gridDim.x * 256) {
-    const int set = i >= s.n[0];
-    const int64_t j = set ? i - s.n[0] : i;
-    float p[3];
-    ff_position(s, set, j, p);
-    unsigned c[3];
-#pragma unroll
-    for (int d = 0; d < 3; ++d) c[d] = (unsigned)fminf(fmaxf((ax.at(d, p[d]) + v[d]) * sc, 0.0f), 1023.0f);   // NaN -> 0
-    keys[i] = ((unsigned)set << bits) | (hilbert30(c[0], c[1], c[2]) >> (30 - bits));
-    idx[i] = (int)j;
+      for (int d = 0; d < 3; ++d)
+        c[d] = (unsigned)fminf(fmaxf((ax.at(d, p[d]) + ax.lo[d]) * ax.sc, 0.0f), 1023.0f);   // NaN -> 0
+      const int64_t i = set ? s.n[0] + j : j;
+      keys[i] = ((unsigned)set << bits) | (hilbert30(c[0], c[1], c[2]) >> (30 - bits));
+      idx[i] = (int)j;
+    }
   }
 }
 
@@ -480,12 +496,11 @@ static __global__ __launch_bounds__(256) void k_ff_bounds(const float4* p, int64
   }
 }
 
-// where a group's bounds go: sphere (bbox centre, largest distance), largest and least
-// (cmin, if given) core term, and of sources (am) a bound of |alpha| and |q| and the sign of the first nonzero strength
-// (0: none), by its first nonzero component
+// where a group's bounds go: sphere (bbox centre, largest distance), and {largest and least
+// core term, of sources a bound of |alpha| and |q|, and the sign of the first nonzero strength
+// (0: none), by its first nonzero component}
 struct FFBounds {
-  float4* sph;
-  float *cs, *cmin, *am, *sign;
+  float4 *sph, *lim;
 };
 // the bounds of the workgroup's points, N per thread (valid: this thread has some) with
 // core terms p.w; strengths a, of sources
@@ -526,12 +541,8 @@ __device__ __forceinline__ void ff_group_bounds(bool valid, const float4* p, con
   if (threadIdx.x != 0) return;
   // margin for the rounding of the distances above
   out.sph[g] = make_float4(c[0], c[1], c[2], __fsqrt_rn(w[0]) * 1.00001f + 1e-30f);
-  out.cs[g] = v[6];
-  if (out.cmin) out.cmin[g] = -v[7];
-  if (a) {
-    out.am[g] = w[1] * 1.7321f;   // sqrt 3, rounded up
-    out.sign[g] = w[2] == -inf ? 0.0f : ((int)-w[2] & 1) ? -1.0f : 1.0f;
-  }
+  // w[1] times sqrt 3, rounded up
+  out.lim[g] = make_float4(v[6], -v[7], w[1] * 1.7321f, w[2] == -inf ? 0.0f : ((int)-w[2] & 1) ? -1.0f : 1.0f);
 }
 
 // rows and bounds, one workgroup per source tile and then one per target block: sources up
@@ -588,22 +599,23 @@ __global__ __launch_bounds__(256) void k_ff_classify(FFBounds bb, int64_t nb, FF
   if (g >= nb * mwords) return;
   const int64_t b = g / mwords;
   const int w = (int)(g - b * mwords);
-  const float4 cb = bb.sph[b];
-  const float csb = bb.cs[b], cmb = CORES ? bb.cmin[b] : 0.0f;
+  const float4 cb = bb.sph[b], lb = bb.lim[b];
   unsigned bits = 0u;
   const int left = ntiles - 32 * w < 32 ? ntiles - 32 * w : 32;
+#pragma unroll 8
   for (int k = 0; k < left; ++k) {
-    const int ti = w * 32 + k;
-    const float4 ct = tb.sph[ti];
-    const float cst = tb.cs[ti];
+    const float4 ct = tb.sph[32 * w + k], lt = tb.lim[32 * w + k];
     const float dx = cb.x - ct.x, dy = cb.y - ct.y, dz = cb.z - ct.z;
     const float gap = __fsqrt_rn(fmaf(dz, dz, fmaf(dy, dy, dx * dx))) - cb.w - ct.w;
-    bool far = gap > 0.0f && gap > FF_KAPPA * fmaxf(fminf(cb.w, ct.w), FF_SPREAD * cb.w);
-    const float most = ff_r2_with<CORE>(gap + 2.0f * (cb.w + ct.w), csb + cst);
-    far = far && most <= FF_RANGE * ff_r2_with<CORE>(gap, CORES ? cmb + tb.cmin[ti] : 0.0f);
-    far = far && most < __builtin_huge_valf() && tb.am[ti] < __builtin_huge_valf();
-    if (CORE == CORE_EXP) far = far && gap * gap > exp_threshold(csb + cst);
-    if (CORE == CORE_SING) far = far && gap > fmaxf(csb, cst);
+    const float most = ff_r2_with<CORE>(gap + 2.0f * (cb.w + ct.w), lb.x + lt.x);
+    const float least = ff_r2_with<CORE>(gap, CORES ? lb.y + lt.y : 0.0f);
+    // no branches: the loads of the next tiles go ahead
+    bool far = gap > 0.0f;
+    far &= gap > FF_KAPPA * fmaxf(fminf(cb.w, ct.w), FF_SPREAD * cb.w);
+    far &= most <= FF_RANGE * least;
+    far &= fmaxf(most, lt.z) < __builtin_huge_valf();
+    if (CORE == CORE_EXP) far &= gap * gap > exp_threshold(lb.x + lt.x);
+    if (CORE == CORE_SING) far &= gap > fmaxf(lb.x, lt.x);
     if (far) bits |= 1u << k;
   }
   mask[g] = bits;
@@ -906,8 +918,8 @@ __global__ __launch_bounds__(FF_FAR_THREADS, 2) void k_ff_far(FFArgs a) {
   const int64_t blk = blockIdx.x;
   const int64_t base = blk * FF_TB + w * 64;
   const float4 cb = a.bsph[blk];
-  float sgn = a.tsg[0];   // of the first nonzero strength of all
-  for (int t = 1; sgn == 0.0f && t < a.ntiles; ++t) sgn = a.tsg[t];
+  float sgn = a.tlim[0].w;   // of the first nonzero strength of all
+  for (int t = 1; sgn == 0.0f && t < a.ntiles; ++t) sgn = a.tlim[t].w;
   sgn = sgn < 0.0f ? -1.0f : 1.0f;
 
   // targets; and the current run's centre, the block's or its one tile's
@@ -1064,20 +1076,20 @@ __global__ __launch_bounds__(FF_FAR_THREADS, 2) void k_ff_far(FFArgs a) {
       if (32 * word + 32 > end_tile) bits &= (1u << (end_tile & 31)) - 1u;
       if (bits == 0u) continue;
       const int t = word * 32 + col < a.ntiles ? word * 32 + col : a.ntiles - 1;
-      const float4 ct = a.tsph[t];
+      const float4 ct = a.tsph[t], lt = a.tlim[t];
       const float ddx = cb.x - ct.x, ddy = cb.y - ct.y, ddz = cb.z - ct.z;
       const float dc = __fsqrt_rn(fmaf(ddz, ddz, fmaf(ddy, ddy, ddx * ddx)));
       const float gap = dc - cb.w - ct.w;   // > 0 for a far tile
       float lr = __builtin_amdgcn_logf(fmaxf(gap, 1e-37f));   // of the least distance that the weights see
-      if (COREA || TAU) lr = fmaxf(lr, 0.5f * __builtin_amdgcn_logf(ff_r2_with<CORE>(gap, a.bcm[blk] + a.tcm[t])));
+      if (COREA || TAU) lr = fmaxf(lr, 0.5f * __builtin_amdgcn_logf(ff_r2_with<CORE>(gap, a.blim[blk].y + lt.y)));
       const bool own = !(gap > FF_KAPPA * cb.w);   // a tile nearer than the block is wide: its own centre
       const float rs = own ? fmaxf(ct.w, gap * 0x1p-12f) : dc + ct.w;   // |s'| bound
       const float lrs = __builtin_amdgcn_logf(rs);
       // strengths by exponent and mantissa, so that scaling all by a power of two moves the
       // scales by just that and the results with them, exactly
       int ea;
-      const float lam = __builtin_amdgcn_logf(fmaxf(frexpf(a.tam[t], &ea), 0.5f));
-      const float lbm = __builtin_amdgcn_logf(fmaf(rs, rs, COREA ? a.tcs[t] : 0.0f));
+      const float lam = __builtin_amdgcn_logf(fmaxf(frexpf(lt.z, &ea), 0.5f));
+      const float lbm = __builtin_amdgcn_logf(fmaf(rs, rs, COREA ? lt.x : 0.0f));
       const float top = (TAU ? 11.0f : 13.0f) * (HASB ? 1.0f / 5.0f : 1.0f / 3.0f);
       const float lg[5] = {lam, lam + lrs, lam + 2.0f * lrs, lam + lbm, lam + lbm + lrs};
       int wg[5];
@@ -1383,7 +1395,7 @@ __device__ __forceinline__ void near_item(const FFArgs& a, int64_t b, int r0, in
         sh[2 * j + 1] = a.sa[s0 + j];
       }
       __syncthreads();
-      float thr[1] = {CORE == CORE_EXP ? exp_threshold(a.tcs[ti] + tt[0]) : 0.0f};
+      float thr[1] = {CORE == CORE_EXP ? exp_threshold(a.tlim[ti].x + tt[0]) : 0.0f};
       if (PREC == PREC_COMP) {
         // In this order a near tile holds the target's closest sources, whose large
         // terms cancel; the FP32 partials are therefore folded every ff_fold sources, the

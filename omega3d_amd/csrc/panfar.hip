@@ -436,8 +436,8 @@ struct PanFarLayout {
   unsigned *k_in, *k_out, *mask, *ctr, *list, *count;
   int *i_in, *i_out, *tinv, *nn, *items, *ioff, *mfold, *iblk;
   void* tmp;
-  float *box, *tcs, *tam, *tsg, *bcs;
-  float4 *sp, *sa, *tq, *tsph, *bsph, *rec, *cen;
+  float* box;
+  float4 *sp, *sa, *tq, *tsph, *tlim, *bsph, *blim, *rec, *cen;
   double *farv, *part;
   size_t bytes;
 };
@@ -457,7 +457,7 @@ PanFarLayout layout(char* base, int rule, int64_t units, int64_t nt, int nout) {
   const int f4 = rule == PANFAR_POINTS ? PAN_F4 : rule == PANFAR_POINTS7 ? G7_F4 : 0;
   Carve cv{base};
   PanFarLayout L{};
-  L.box = cv.take<float>(6 * FF_BOX_GRID);
+  L.box = cv.take<float>(FF_BOX_FLOATS);
   L.k_in = cv.take<unsigned>(units + nt);
   L.k_out = cv.take<unsigned>(units + nt);
   L.i_in = cv.take<int>(units + nt);
@@ -470,11 +470,9 @@ PanFarLayout layout(char* base, int rule, int64_t units, int64_t nt, int nout) {
   L.cen = cv.take<float4>(f4 ? units : 0);
   L.tq = cv.take<float4>(nt);
   L.tsph = cv.take<float4>(ntiles);
-  L.tcs = cv.take<float>(ntiles);
-  L.tam = cv.take<float>(ntiles);
-  L.tsg = cv.take<float>(ntiles);
+  L.tlim = cv.take<float4>(ntiles);
   L.bsph = cv.take<float4>(nb);
-  L.bcs = cv.take<float>(nb);
+  L.blim = cv.take<float4>(nb);
   L.mask = cv.take<unsigned>((size_t)(nb * mwords));
   L.farv = cv.take<double>((size_t)nout * far_slices(nb, ntiles, nout == 3 ? 3 : 2, num_cus()) * nt);
   L.nn = cv.take<int>(nb);
@@ -512,7 +510,7 @@ int run(const PanArgs* p, const PtPanArgs* t, void* ws, hipStream_t st) {
   const PanFarLayout L = layout(static_cast<char*>(ws), RULE, units, nt, GRAD ? 12 : 3);
   FFArgs& f = a.f;
   f.sp = L.sp; f.sa = L.sa; f.tq = L.tq;
-  f.tsph = L.tsph; f.tcs = L.tcs; f.tam = L.tam; f.tsg = L.tsg; f.bsph = L.bsph;
+  f.tsph = L.tsph; f.tlim = L.tlim; f.bsph = L.bsph; f.blim = L.blim;
   f.mask = L.mask; f.farv = L.farv;
   f.nn = L.nn; f.items = L.items; f.ioff = L.ioff; f.mfold = L.mfold; f.ctr = L.ctr; f.part = L.part;
   f.nt = nt; f.ns = (int64_t)ntiles * T;
@@ -535,7 +533,7 @@ int run(const PanArgs* p, const PtPanArgs* t, void* ws, hipStream_t st) {
   f.tperm = perm + units;
   f.tinv = L.tinv;
   f.rows = nt >= FF_ROWS_MIN;
-  const FFBounds tb{L.tsph, L.tcs, nullptr, L.tam, L.tsg}, bb{L.bsph, L.bcs, nullptr, nullptr, nullptr};
+  const FFBounds tb{L.tsph, L.tlim}, bb{L.bsph, L.blim};
   hipLaunchKernelGGL((k_pf_rows<RULE>), dim3((unsigned)(ntiles + nb)), dim3(256), 0, st, a, perm, L.sp, L.sa, L.tq, tb, bb,
                      L.nn, nt >= FF_ROWS_MIN ? L.tinv : nullptr);
   hipLaunchKernelGGL((k_ff_classify<CORE_SING>), dim3(grid_of(nb * mwords, 256)), dim3(256), 0, st, bb, nb, tb, ntiles,

@@ -372,3 +372,25 @@ def test_both_sides_of_autos_lines(infl, core, grads, below, nt):
         (v, g), (w, h) = infl.p2p(*args), infl.p2p(*args, method="direct")
         same = np.array_equal(v, w) and (not grads or np.array_equal(g, h))
         assert same == (ns == below or nt == 8191)
+
+
+def test_field_points_do_not_widen_the_sources_grid(infl):
+    """rings among field points of a box 30 times as wide: each set is ordered on a grid of its
+    own, so as many pairs are far as with the points in a box that just holds the rings"""
+    from omega3d_amd import _lib
+    p, D = scenes.colliding_rings(30000), _lib.DeviceArray.from_host
+    box, f = 4.0 * np.random.default_rng(6).random((3, 20000)) - 2.0, []
+    x, s, r, out = D(p.pos.astype(np.float32)), D(p.str.astype(np.float32)), D(p.rad.astype(np.float32)), _lib.DeviceArray((12, 20000))
+    for wide in (1, 30):
+        tp = D((wide * box).astype(np.float32))
+        q, t = _lib.Points(), _lib.Points()
+        q.n, q.r, t.n = p.n, r.ptr, 20000
+        for d in range(3):
+            q.x[d], q.s[d], t.x[d], t.u[d] = x.row(d), s.row(d), tp.row(d), out.row(d)
+        for k in range(9):
+            t.ug[k] = out.row(3 + k)
+        prof, o = _lib.FactoredProfile(), _lib.make_opts("rm", True, "comp", method="factored")
+        _lib.check(_lib.lib.o3d_factored_profile_dev(C.byref(q), C.byref(t), C.byref(o), C.byref(prof)))
+        f.append(prof.far_tile_fraction)
+    print(f)
+    assert f[1] >= f[0]
