@@ -1,11 +1,11 @@
 // ff.hip -- host side of the factored far-field evaluation (method "factored").
 //
 // One call enqueues, on the caller's stream and without synchronising:
-//   bounding box -> Hilbert keys -> radix sort (sort.hip) of sources (and of targets
-//   when they are a different collection) -> gather into sorted float4 rows ->
-//   bounding spheres of source tiles and target blocks -> far/near bit per
-//   (block, tile) -> near-field plan -> far-field kernel (matrix cores) -> near-field kernel, which
-//   also adds the far part and accumulates into the caller's arrays.
+//   bounding boxes and medians -> Hilbert keys -> radix sort (sort.hip) of sources (and of
+//   targets when they are a different collection) -> sorted float4 rows, bounding spheres
+//   and limits of source tiles and target blocks -> far/near bit per (block, tile) ->
+//   near-field plan -> far-field kernel (matrix cores) -> near-field kernel -> combine, which
+//   adds the parts and accumulates into the caller's arrays.
 // Scratch lives in one device workspace per stream (calls on one stream are
 // ordered, so they can share it); it grows when a larger call comes, after the
 // stream has drained.  A caller that owns its scratch (a batch) passes it in
@@ -353,8 +353,9 @@ bool ff_supported(int core, bool grad, int prec) {
 
 // AUTO also sends compensated sums of the other cores and of velocities alone.  The line is
 // drawn in pairs, where both methods' times cross, us direct and factored on one or two
-// rings: EXP 24,576 particles 600-630 and 505; RM 24,576 452 and 468, 32,768 750 and 570-645;
-// WL (V2 alike) 32,768 829 and 798-869, 49,152 1,833 and 1,573-1,641; velocity alone: EXP
+// rings (particles that fill a cube cross later, having more near tiles: RM 30,100 720-770 and
+// 841, 40,000 1,161 and 1,116; EXP velocity alone and WL about 5% at their lines): EXP 24,576
+// particles 600-630 and 505; RM 24,576 452 and 468, 32,768 750 and 570-645; WL (V2 alike) 32,768 829 and 798-869, 49,152 1,833 and 1,573-1,641; velocity alone: EXP
 // 24,576 376-396 and 410-420, 32,768 675 and 493-562, RM 32,768 441 and 456-504, 49,152 980
 // and 830-884, WL 49,152 1,105 and 1,063-1,125, 65,536 faster.  100,000 particles on 16,384
 // field points and 8,192 on 262,144 fall on the same lines (less the preparation's recent

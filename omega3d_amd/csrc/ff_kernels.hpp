@@ -24,8 +24,9 @@
 // the weight into two FP16 values per pair on the vector ALUs.  Two rings, compensated,
 // far field of one call, before and after the pipelined form of k_ff_far, its slices and
 // its cheaper staging: 65,536 particles 1.67 -> 1.32 ms, 131,072 5.7 -> 4.9, 262,144
-// 21.6 -> 19.8, 1,048,576 323 -> 311 (3.4e12 pairs/s).  At the last size the clock is what
-// the power allows: 12% fewer cycles ran at 2.11 GHz instead of 2.26.
+// 21.6 -> 19.8, 1,048,576 323 -> 311.  By counter the last takes 303 ms now (3.55e12 pairs/s
+// at 2.14 GHz): 7.2 vector instructions per pair, the vector units active 89% of the time
+// and the matrix cores 41%.
 //
 // Separation: a tile is "far" for a block when the gap between their bounding
 // spheres is at least one block radius (then every term above is at most

@@ -1,10 +1,9 @@
 // sort.hip -- stable LSD radix sort of (key, index) pairs for gfx950.
 //
-// Used for the Morton order of particles (the factored method's sources and
-// targets, the direct EXP kernel's target order) and for the factored method's
-// work plan.  Everything here is plain kernel launches on the caller's stream:
-// no memory fills, no allocation, no host synchronisation, so a call can be
-// recorded into a HIP graph.
+// Used for the Hilbert order of the factored method's sources and targets (panels too),
+// and for the Morton order of the direct EXP kernel's targets and of o3d_morton_order_dev.
+// Everything here is plain kernel launches on the caller's stream: no memory fills, no
+// allocation, no host synchronisation, so a call can be recorded into a HIP graph.
 //
 // One pass per RS_BITS-bit digit, three kernels per pass:
 //   k_rs_hist     per workgroup tile of RS_TILE keys: digit histogram ->
